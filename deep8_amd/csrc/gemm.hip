@@ -698,7 +698,7 @@ bool gemm_tiled_run_pair(int dtype, GemmArgs &gx, GemmArgs &gy, void *workspace,
     const bool off = getenv("D8_CONV_GRADS_APART") != nullptr;  // tuning and test aid (read at every call)
     if (off || dtype == D8_FLOAT64) return false;
     if (gx.virt != VIRT_A_ROWS || gy.virt != VIRT_B_KROWS || gx.batch != 1 || gy.batch != 1) return false;
-    if (!gemm_tiled_eligible(dtype, gx, 0, 0) || !gemm_tiled_eligible(dtype, gy, 1, 0)) return false;
+    if (!gemm_tiled_eligible(dtype, gx, 0, 0, true) || !gemm_tiled_eligible(dtype, gy, 1, 0, true)) return false;
     // More workgroups than the chip holds at once (two per compute unit): in half the shared launch still gains
     // (3x3 Conv2d, B32: 56x56x64 49.9 -> 47.0 us, 14x14x256 46.0 -> 34.9, 56x56x64->128 74.2 -> 65.0; DeConv2d 4x4 s2
     // B64 14x14x256 60.7 -> 47.9), gx's remainder band riding along as it does alone.  In fp32, bound by the matrix

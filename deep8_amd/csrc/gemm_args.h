@@ -100,8 +100,9 @@ int launch_bias_relu(int dtype, void *z, const void *bias, long rows, int cols, 
 
 // Tiled kernels (fp16 and fp32) for shapes whose operands can be moved in 16-byte pieces.
 int gemm_tiled_k_step(int dtype);  // K elements per step: 64 (fp16) or 32 (fp32)
-// Whether the shape qualifies (g.splits / g.tiles_per_split need not be set yet).
-bool gemm_tiled_eligible(int dtype, const GemmArgs &g, int transA, int transB);
+// Whether the shape qualifies (g.splits / g.tiles_per_split need not be set yet).  whole_steps: among products with a
+// patch-matrix operand only those whose K steps are all whole and whose output is no smaller than a tile.
+bool gemm_tiled_eligible(int dtype, const GemmArgs &g, int transA, int transB, bool whole_steps = false);
 // Launch; with g.splits > 1 the fp32 partial sums go to g.ws for the caller to reduce.
 int gemm_tiled_launch(int dtype, const GemmArgs &g, int transA, int transB, hipStream_t stream);
 // Two patch-matrix products as ONE launch: gx with patch rows as A (NN: a convolution's gradient of its input), gy with

@@ -34,7 +34,7 @@
 // pixels per grid layer (OutClass) -- DeConv2d forward and Conv2d's gradient of x for strides
 // above 1, whose rows of C are then pixels of the output image rather than consecutive rows.
 //
-// The same device covers ragged reductions and skinny matrices of real operands: in a last K step that is
+// The same device covers ragged reductions and skinny matrices: in a last K step that is
 // partly past K the pieces beyond K are fetched at an offset outside the buffer (zeros), and a matrix with
 // fewer rows or columns than the tile is covered by a tile that starts at 0 and reaches past it -- what
 // its loads bring in from there only enters results that are not stored.
@@ -458,23 +458,41 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
             va_base[p] = (((img * pg.H + va_iy[p]) * pg.W + va_ix[p]) * pg.C + a_c * EPV) * ES;
         }
     }
-    // patch k-rows as B: this thread's tap and channel never change; a step selects the rows
-    // (with column passes, Tile::B_COLS: this thread's k-row within the step never changes; piece p has its own tap and channel)
-    int vb_dy = 0, vb_dx = 0, vb_c = 0;
-    int vb_ty[B_IT], vb_tx[B_IT], vb_off[B_IT];
-    if constexpr (T::B_COLS) {
+    // patch k-rows as B: this thread's taps and channels never change; a step selects the rows.  A row is one output
+    // pixel, and each of the rows a thread fetches moves on by BK pixels per step: its source coordinates and byte
+    // offset are kept and advanced by uniform amounts with a carry per axis, so a step costs a dozen additions and
+    // selects per row instead of two divisions by multiplication and four further multiplications (a quarter of
+    // the vector rate each).  A row past the last is in an image past the last, i.e. outside the buffer: zeros.
+    // (with column passes, Tile::B_COLS: one row per thread and step, and piece p has its own tap and channel)
+    constexpr int VB_N = VIRT == VIRT_B_KROWS ? (T::B_COLS ? 1 : B_IT) : 1;
+    int vb_y[VB_N], vb_x[VB_N], vb_off[VB_N];  // source row, column and byte offset of this thread's rows
+    int vb_ty[B_IT], vb_tx[B_IT], vb_toff[B_IT];  // column passes: tap displacement and byte offset of each piece
+    int vb_y_end = 0, vb_x_end = 0;
+    if constexpr (VIRT == VIRT_B_KROWS) {
+        int cy = -pg.pt, cx = -pg.pl, cc = 0;  // what the tap and channel add to an output pixel's source coordinates
+        if constexpr (T::B_COLS) {
 #pragma unroll
-        for (int p = 0; p < B_IT; ++p) {
-            const int n = n0 + p * T::B_PASS + b_c * EPV, t = n / pg.C, fy = t / pg.FW, fx = t - fy * pg.FW;
-            vb_ty[p] = fy * pg.dy;
-            vb_tx[p] = fx * pg.dx;
-            vb_off[p] = ((vb_ty[p] * pg.W + vb_tx[p]) * pg.C + (n - t * pg.C)) * ES;
+            for (int p = 0; p < B_IT; ++p) {
+                const int n = n0 + p * T::B_PASS + b_c * EPV, t = n / pg.C, fy = t / pg.FW, fx = t - fy * pg.FW;
+                vb_ty[p] = fy * pg.dy;
+                vb_tx[p] = fx * pg.dx;
+                vb_toff[p] = ((vb_ty[p] * pg.W + vb_tx[p]) * pg.C + (n - t * pg.C)) * ES;
+            }
+        } else {
+            const int n = n0 + b_c * EPV, t = n / pg.C, fy = t / pg.FW, fx = t - fy * pg.FW;
+            cc = n - t * pg.C;
+            cy += fy * pg.dy;
+            cx += fx * pg.dx;
         }
-    } else if constexpr (VIRT == VIRT_B_KROWS) {
-        const int n = n0 + b_c * EPV, t = n / pg.C, fy = t / pg.FW, fx = t - fy * pg.FW;
-        vb_c = n - t * pg.C;
-        vb_dy = fy * pg.dy - pg.pt;
-        vb_dx = fx * pg.dx - pg.pl;
+        vb_y_end = pg.OH * pg.sy + cy, vb_x_end = pg.OW * pg.sx + cx;
+        const int plane = pg.OH * pg.OW;
+#pragma unroll
+        for (int p = 0; p < VB_N; ++p) {
+            const int m = split * tps * BK + b_r + p * T::B_ROWS, img = m / plane, rem = m - img * plane, oy = rem / pg.OW;
+            vb_y[p] = oy * pg.sy + cy;
+            vb_x[p] = (rem - oy * pg.OW) * pg.sx + cx;
+            vb_off[p] = (((img * pg.H + vb_y[p]) * pg.W + vb_x[p]) * pg.C + cc) * ES;
+        }
     }
 
     // ---- per-lane LDS offsets of its MFMA operands
@@ -492,93 +510,105 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
     // ---- this workgroup's steps x0 .. x0 + nsteps - 1 of the extended reduction; step x reads
-    // product x / ktiles at K offset (x % ktiles) * BK (all uniform: scalar arithmetic)
-    // K need not be a multiple of the K step for real matrices: the last step of a product is then partly past
-    // K, and the pieces that lie past it are fetched at an offset beyond the buffer, i.e. as zeros.
-    const int ktiles = (g.K + BK - 1) / BK, tail_len = g.K % BK;
+    // product x / ktiles at K offset (x % ktiles) * BK (all uniform: scalar arithmetic, counted on from step to step)
+    // K need not be a multiple of the K step: the last step of a product (of a filter tap, where K is its channels) is then
+    // partly past K, and the pieces that lie past it are fetched at an offset beyond the buffer, i.e. as zeros.  Where the
+    // reduction runs over patch rows or over the rows of a real matrix, rows past the last lie outside the buffer anyway.
+    const int ktiles = (g.K + BK - 1) / BK, last_len = g.K - (ktiles - 1) * BK;
     const unsigned av_plain = (unsigned)ES * ((unsigned)a_r * (unsigned)g.lda + a_c * EPV);
     const unsigned bv_plain = (unsigned)ES * ((unsigned)b_r * (unsigned)g.ldb + b_c * EPV);
     const int x0 = split * tps, nsteps = min(red * ktiles, x0 + tps) - x0;
     const unsigned a_prod = (unsigned)ES * (unsigned)g.sA, b_prod = (unsigned)ES * (unsigned)g.sB;
     const unsigned b_prod_row = (unsigned)ES * (unsigned)g.sB_row, b_first = (unsigned)ES * b_cls;
-    auto step_a = [&](int i) -> unsigned {
-        const int x = x0 + min(i, nsteps - 1), r = x / ktiles;  // past the end: refetch the last step, never used
+    // The step that is fetched next: its product, K step and filter tap are counted on from step to step (every step is
+    // fetched once, in order), because four divisions by runtime numbers at the head of each step -- some 35 dependent
+    // scalar instructions that no matrix instruction covers -- were a fifth of a short half step's time.
+    int ld_i = 0, ld_r = x0 / ktiles, ld_kx = x0 - ld_r * ktiles;
+    int ld_fy = VA ? ld_r / pg.FW : 0, ld_fx = VA ? ld_r - ld_fy * pg.FW : 0;
+    // patch k-rows: what BK more pixels add, and the corrections when a row or an image is complete
+    int vb_dy = 0, vb_dx = 0, vb_d = 0, vb_d_row = 0, vb_d_img = 0;
+    if constexpr (VIRT == VIRT_B_KROWS) {
+        const int plane = pg.OH * pg.OW, img = BK / plane, rem = BK - img * plane, oy = rem / pg.OW;
+        vb_dy = oy * pg.sy, vb_dx = (rem - oy * pg.OW) * pg.sx;
+        vb_d = ((img * pg.H + vb_dy) * pg.W + vb_dx) * pg.C * ES;
+        vb_d_row = (pg.sy * pg.W - pg.OW * pg.sx) * pg.C * ES;
+        vb_d_img = (pg.H - pg.OH * pg.sy) * pg.W * pg.C * ES;
+    }
+    // How much of the step that is fetched lies within K: all of it, or what is left of K in a product's last step.  (Where
+    // K is a multiple of the K step -- an instantiation without TAIL -- nothing asks: on patch rows in fp32 the
+    // comparisons alone cost 2 % of a launch.)
+    constexpr bool PARTIAL = TAIL && VIRT != VIRT_B_KROWS;
+    auto k_left = [&]() -> int { return ld_kx == ktiles - 1 ? last_len : BK; };
+    auto step_a = [&]() -> unsigned {
         if constexpr (VA) {
-            const int fy = r / pg.FW, fx = r - fy * pg.FW, tdy = fy * pg.dy, tdx = fx * pg.dx;
-            const int toff = ((tdy * pg.W + tdx) * pg.C + (x - r * ktiles) * BK) * ES;
+            const int tdy = ld_fy * pg.dy, tdx = ld_fx * pg.dx;
+            const int toff = ((tdy * pg.W + tdx) * pg.C + ld_kx * BK) * ES;
+            const bool live = !PARTIAL || a_c * EPV < k_left();
 #pragma unroll
             for (int p = 0; p < A_IT; ++p) {
                 const bool inside = (unsigned)(va_iy[p] + tdy) < (unsigned)pg.H && (unsigned)(va_ix[p] + tdx) < (unsigned)pg.W;
-                av[p] = inside ? (unsigned)(va_base[p] + toff) : OUTSIDE;
+                av[p] = inside && live ? (unsigned)(va_base[p] + toff) : OUTSIDE;
             }
             return 0u;
         } else {
-            const int kx = x - r * ktiles;
-            if constexpr (VIRT == VIRT_NONE) {
-                if constexpr (TAIL) {
-                    const bool tail = kx == ktiles - 1;
+            if constexpr (PARTIAL) {
+                const int left = k_left();
 #pragma unroll
-                    for (int p = 0; p < A_IT; ++p) {
-                        const bool past = A_KC ? a_c * EPV >= tail_len : a_r + p * T::A_ROWS >= tail_len;
-                        av[p] = tail && past ? OUTSIDE : av_plain;
-                    }
-                }
+                for (int p = 0; p < A_IT; ++p) av[p] = (A_KC ? a_c * EPV : a_r + p * T::A_ROWS) < left ? av_plain : OUTSIDE;
             }
-            return Au + (g.red > 1 ? r * a_prod : 0u) + kx * a_step;
+            return Au + ld_r * a_prod + ld_kx * a_step;
         }
     };
-    auto step_b = [&](int i) -> unsigned {
-        const int x = x0 + min(i, nsteps - 1), r = x / ktiles;
-        if constexpr (T::B_COLS) {
-            const unsigned plane = pg.OH * pg.OW, m = (unsigned)x * BK + b_r;
-            unsigned img = __umulhi(m, pg.mg_plane), rem = m - img * plane;
-            if (rem >= plane) ++img, rem -= plane;
-            unsigned oy = __umulhi(rem, pg.mg_ow), ox = rem - oy * pg.OW;
-            if (ox >= (unsigned)pg.OW) ++oy, ox -= pg.OW;
-            const int iy0 = (int)oy * pg.sy - pg.pt, ix0 = (int)ox * pg.sx - pg.pl;
-            const int base = (((int)img * pg.H + iy0) * pg.W + ix0) * pg.C * ES;
+    auto step_b = [&]() -> unsigned {
+        if constexpr (VIRT == VIRT_B_KROWS) {
 #pragma unroll
             for (int p = 0; p < B_IT; ++p) {
-                const bool inside = (unsigned)(iy0 + vb_ty[p]) < (unsigned)pg.H && (unsigned)(ix0 + vb_tx[p]) < (unsigned)pg.W;
-                bv[p] = inside ? (unsigned)(base + vb_off[p]) : OUTSIDE;
-            }
-            return 0u;
-        } else if constexpr (VIRT == VIRT_B_KROWS) {
-            const unsigned plane = pg.OH * pg.OW;
-#pragma unroll
-            for (int p = 0; p < B_IT; ++p) {
-                const unsigned m = (unsigned)x * BK + b_r + p * T::B_ROWS;
-                unsigned img = __umulhi(m, pg.mg_plane), rem = m - img * plane;
-                if (rem >= plane) ++img, rem -= plane;
-                unsigned oy = __umulhi(rem, pg.mg_ow), ox = rem - oy * pg.OW;
-                if (ox >= (unsigned)pg.OW) ++oy, ox -= pg.OW;
-                const int iy = (int)oy * pg.sy + vb_dy, ix = (int)ox * pg.sx + vb_dx;
+                const int q = T::B_COLS ? 0 : p;
+                const int iy = vb_y[q] + (T::B_COLS ? vb_ty[p] : 0), ix = vb_x[q] + (T::B_COLS ? vb_tx[p] : 0);
                 const bool inside = (unsigned)iy < (unsigned)pg.H && (unsigned)ix < (unsigned)pg.W;
-                bv[p] = inside ? (unsigned)(((((int)img * pg.H + iy) * pg.W + ix) * pg.C + vb_c) * ES) : OUTSIDE;
+                bv[p] = inside ? (unsigned)(vb_off[q] + (T::B_COLS ? vb_toff[p] : 0)) : OUTSIDE;
             }
             return 0u;
-        } else if constexpr (VIRT == VIRT_A_CLASSES) {
-            const int fy = r / pg.FW, fx = r - fy * pg.FW;
-            return Bu + b_first + fy * b_prod_row + fx * b_prod + (x - r * ktiles) * b_step;
-        } else {
-            const int kx = x - r * ktiles;
-            if constexpr (VIRT == VIRT_NONE) {
-                if constexpr (TAIL) {
-                    const bool tail = kx == ktiles - 1;
+        }
+        if constexpr (PARTIAL) {
+            const int left = k_left();
 #pragma unroll
-                    for (int p = 0; p < B_IT; ++p) {
-                        const bool past = B_KC ? b_c * EPV >= tail_len : b_r + p * T::B_ROWS >= tail_len;
-                        bv[p] = tail && past ? OUTSIDE : bv_plain;
-                    }
-                }
+            for (int p = 0; p < B_IT; ++p) bv[p] = (B_KC ? b_c * EPV : b_r + p * T::B_ROWS) < left ? bv_plain : OUTSIDE;
+        }
+        if constexpr (VIRT == VIRT_A_CLASSES) return Bu + b_first + ld_fy * b_prod_row + ld_fx * b_prod + ld_kx * b_step;
+        return Bu + ld_r * b_prod + ld_kx * b_step;
+    };
+    // (selects, no branches: around a branch the compiler moves all accumulators out of the AGPRs and back.  Past the end
+    // the last step is fetched again, or zeros where patch k-rows move on past it; never used)
+    auto step_on = [&]() {
+        ld_kx += ++ld_i < nsteps ? 1 : 0;
+        const int done = ld_kx == ktiles ? 1 : 0;
+        ld_kx = done ? 0 : ld_kx;
+        ld_r += done;
+        if constexpr (VA) {
+            ld_fx += done;
+            const int row = ld_fx == pg.FW ? 1 : 0;
+            ld_fx = row ? 0 : ld_fx;
+            ld_fy += row;
+        }
+        if constexpr (VIRT == VIRT_B_KROWS) {
+#pragma unroll
+            for (int q = 0; q < VB_N; ++q) {
+                vb_x[q] += vb_dx;
+                const bool row = vb_x[q] >= vb_x_end;
+                vb_x[q] -= row ? pg.OW * pg.sx : 0;
+                vb_y[q] += vb_dy + (row ? pg.sy : 0);
+                const bool img = vb_y[q] >= vb_y_end;
+                vb_y[q] -= img ? pg.OH * pg.sy : 0;
+                vb_off[q] += vb_d + (row ? vb_d_row : 0) + (img ? vb_d_img : 0);
             }
-            return Bu + (g.red > 1 ? r * b_prod : 0u) + kx * b_step;
         }
     };
 
     // ---- prologue: step 0 into LDS half 0, step 1 into registers, first operands of step 0
     {
-        const unsigned pa = step_a(0), pb = step_b(0);
+        const unsigned pa = step_a(), pb = step_b();
+        step_on();
 #pragma unroll
         for (int p = 0; p < NP; ++p)
             R[p] = p < A_IT ? __builtin_amdgcn_raw_buffer_load_b128(ra, av[p < A_IT ? p : 0], pa + p * a_pass, 0)
@@ -588,7 +618,8 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     for (int p = 0; p < NP; ++p)
         *(u32x4 *)(p < A_IT ? As0 + a_dst + p * T::A_PASS : Bs0 + b_dst + (p - A_IT) * T::B_PASS) = R[p];
     {
-        const unsigned pa = step_a(1), pb = step_b(1);
+        const unsigned pa = step_a(), pb = step_b();
+        step_on();
 #pragma unroll
         for (int p = 0; p < NP; ++p)
             R[p] = p < A_IT ? __builtin_amdgcn_raw_buffer_load_b128(ra, av[p < A_IT ? p : 0], pa + p * a_pass, 0)
@@ -606,12 +637,14 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     // ---- main loop, two steps per trip so that the LDS half of every access is known statically;
     for (int i = 0; i < nsteps; i += 2) {
         {
-            const unsigned pa = step_a(i + 2), pb = step_b(i + 2);
+            const unsigned pa = step_a(), pb = step_b();
+            step_on();
             k_step<T>(As0 + a_frag, Bs0 + b_frag, As1 + a_frag, Bs1 + b_frag, As1 + a_dst, Bs1 + b_dst, ra, rb, pa, pb,
                       a_pass, b_pass, av, bv, R, fa, fb, acc);
         }
         if (i + 1 < nsteps) {
-            const unsigned pa = step_a(i + 3), pb = step_b(i + 3);
+            const unsigned pa = step_a(), pb = step_b();
+            step_on();
             k_step<T>(As1 + a_frag, Bs1 + b_frag, As0 + a_frag, Bs0 + b_frag, As0 + a_dst, Bs0 + b_dst, ra, rb, pa, pb,
                       a_pass, b_pass, av, bv, R, fa, fb, acc);
         }
@@ -645,7 +678,7 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
 }
 
 // TAIL: K is not a multiple of the K step (an instantiation of its own, so that the per-piece offsets of the
-// ordinary case stay constants)
+// ordinary case stay constants; patch k-rows as B need none)
 template <typename T, bool TAIL = false>
 __global__ __launch_bounds__(T::NT) void gemm_tiled_kernel(GemmArgs g, int tilesM, int tilesN) {
     typedef typename T::E E;
@@ -686,6 +719,12 @@ __global__ __launch_bounds__(T0::NT) void gemm_tiled_pair_kernel(GemmArgs g0, Ge
 extern unsigned long long *phase_rec_buf;
 extern size_t phase_rec_bytes;
 
+// Launches of one product, one translation unit each (gemm_tiled_launch.h)
+int gemm_tiled_plain_f16(const GemmArgs &g, int transA, int transB, hipStream_t stream);
+int gemm_tiled_plain_f32(const GemmArgs &g, int transA, int transB, hipStream_t stream);
+int gemm_tiled_patch_f16(const GemmArgs &g, int transB, hipStream_t stream);
+int gemm_tiled_patch_f32(const GemmArgs &g, int transB, hipStream_t stream);
+
 // Which tile a product runs on.
 enum TileId { TILE_WIDE, TILE_256, TILE_128x64, TILE_64x64, TILE_64x128, TILE_128x128 };
 
@@ -702,6 +741,8 @@ static TileId choose_tile(const GemmArgs &g) {
         if (big && VIRT == VIRT_NONE && !(wide && atoi(wide) == 0) && gemm_wide_eligible(g, !A_KC, B_KC)) return TILE_WIDE;
         if (big) return TILE_256;
     }
+    // a filter gradient smaller than a tile both ways (few channels, few taps)
+    if (VIRT == VIRT_B_KROWS && g.M < 128 && g.N < 128) return TILE_64x64;
     // a 64-wide side gets a tile of that width (im2col products with 64 output channels)
     if (g.N < 128) return TILE_128x64;
     // a patch-matrix product whose last 128-column tile would be at most half full: 64 x 64 tiles, no padding

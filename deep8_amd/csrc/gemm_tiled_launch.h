@@ -1,0 +1,75 @@
+// The launch of one product on the tile its shape asks for.  Included by the translation units that instantiate the tiled
+// kernels: one per element type and kind of operands, so that they compile side by side.
+#ifndef DEEP8_AMD_GEMM_TILED_LAUNCH_H
+#define DEEP8_AMD_GEMM_TILED_LAUNCH_H
+
+#include "gemm_tiled_kernel.h"
+
+namespace d8 {
+
+template <typename E, int BM, int BN, int WGM, int WGN, bool A_KC, bool B_KC, int VIRT>
+static int launch_tiled(const GemmArgs &g0, hipStream_t stream) {
+    GemmArgs g = g0;
+    typedef Tile<E, BM, BN, WGM, WGN, A_KC, B_KC, VIRT> T;
+    const bool tail = g.tail_splits > 0;  // (gemm_tiled_run sets it only for 128-row tiles and a tail_m0 that is a multiple of them)
+    const int tilesM = ceil_div(tail ? g.tail_m0 : g.M, BM), tilesN = ceil_div(g.N, BN);
+    const int extra = tail ? ceil_div(g.M - g.tail_m0, BM) * tilesN * g.tail_splits : 0;
+    // A launch of at most two workgroups per CU is spread evenly only if a CU cannot take a third:
+    // where the tile's own LDS would let three in, unused dynamic LDS is requested on top.
+    constexpr long lds = 2L * (T::A_SZ + T::B_SZ) * T::ES, third = 160 * 1024 / 3;
+    const int layers = VIRT == VIRT_A_CLASSES ? g.ncls : g.batch * g.splits;  // for classes g.M is the largest one's
+    const long wgs = (long)tilesM * tilesN * layers, cus = cu_count();
+    const unsigned pad = (lds <= third && wgs > cus && wgs <= 2 * cus) ? (unsigned)(third + 512 - lds) : 0u;
+    // a launch whose records would not fit the caller's buffer writes none
+    g.phase_rec = (size_t)(tilesM * tilesN + extra) * layers * 64 <= phase_rec_bytes ? phase_rec_buf : nullptr;
+    if (VIRT != VIRT_B_KROWS && g.K % T::BK)
+        hipLaunchKernelGGL((gemm_tiled_kernel<T, VIRT != VIRT_B_KROWS>), dim3(tilesM * tilesN + extra, 1, layers), dim3(T::NT), pad, stream, g, tilesM, tilesN);
+    else
+        hipLaunchKernelGGL((gemm_tiled_kernel<T, false>), dim3(tilesM * tilesN + extra, 1, layers), dim3(T::NT), pad, stream, g, tilesM, tilesN);
+    D8_LAUNCH_CHECK();
+    return 0;
+}
+
+template <typename E, bool A_KC, bool B_KC, int VIRT = VIRT_NONE>
+static int pick_tile(const GemmArgs &g, hipStream_t stream) {
+    switch (choose_tile<E, A_KC, B_KC, VIRT>(g)) {
+        case TILE_WIDE: return gemm_wide_launch(g, !A_KC, B_KC, stream);
+        case TILE_256:
+            if constexpr (sizeof(E) == 2) return launch_tiled<E, 256, 256, 4, 2, A_KC, B_KC, VIRT>(g, stream);
+            break;
+        case TILE_128x64: return launch_tiled<E, 128, 64, 2, 2, A_KC, B_KC, VIRT>(g, stream);
+        case TILE_64x64:
+            if constexpr (VIRT == VIRT_B_KROWS) return launch_tiled<E, 64, 64, 2, 2, A_KC, B_KC, VIRT>(g, stream);
+            break;
+        case TILE_64x128: return launch_tiled<E, 64, 128, 2, 2, A_KC, B_KC, VIRT>(g, stream);
+        default: break;
+    }
+    return launch_tiled<E, 128, 128, 2, 2, A_KC, B_KC, VIRT>(g, stream);
+}
+
+// Real matrices as both operands.
+template <typename E>
+static int launch_plain(const GemmArgs &g, int transA, int transB, hipStream_t stream) {
+    if (!transA && !transB) return pick_tile<E, true, false>(g, stream);
+    if (!transA && transB) return pick_tile<E, true, true>(g, stream);
+    return pick_tile<E, false, false>(g, stream);
+}
+
+// A patch matrix as one of them.
+template <typename E>
+static int launch_patch(const GemmArgs &g, int transB, hipStream_t stream) {
+    if (g.virt == VIRT_A_CLASSES) {  // every class has at least 128 rows (checked by eligible)
+        if (transB) {
+            if (g.N < 128) return launch_tiled<E, 128, 64, 2, 2, true, true, VIRT_A_CLASSES>(g, stream);
+            return launch_tiled<E, 128, 128, 2, 2, true, true, VIRT_A_CLASSES>(g, stream);
+        }
+        if (g.N < 128) return launch_tiled<E, 128, 64, 2, 2, true, false, VIRT_A_CLASSES>(g, stream);
+        return launch_tiled<E, 128, 128, 2, 2, true, false, VIRT_A_CLASSES>(g, stream);
+    }
+    if (g.virt == VIRT_A_ROWS) return transB ? pick_tile<E, true, true, VIRT_A_ROWS>(g, stream) : pick_tile<E, true, false, VIRT_A_ROWS>(g, stream);
+    return pick_tile<E, false, false, VIRT_B_KROWS>(g, stream);
+}
+
+}  // namespace d8
+
+#endif

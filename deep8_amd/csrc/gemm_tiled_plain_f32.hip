@@ -1,0 +1,8 @@
+// Tiled GEMM, fp32: products of real matrices (gemm_tiled_launch.h).
+#include "gemm_tiled_launch.h"
+
+namespace d8 {
+
+int gemm_tiled_plain_f32(const GemmArgs &g, int transA, int transB, hipStream_t stream) { return launch_plain<float>(g, transA, transB, stream); }
+
+}  // namespace d8

@@ -134,9 +134,11 @@ struct ConvShape {
 static unsigned magic_of(unsigned d) { return d <= 1 ? 0xFFFFFFFFu : (unsigned)((1ull << 32) / d); }
 
 // Whether a product with a patch-matrix operand can run: the tiled kernels have their alignment and size rules,
-// the fp64 kernel moves single elements and takes any shape.
+// the fp64 kernel moves single elements and takes any shape.  A scratch query (no tensors) counts on it only for products of
+// whole K steps and whole tiles: where a channel count leaves a partial step in every filter tap, or an output is smaller
+// than a tile, the query keeps asking for the interim matrix, and the call uses what it needs of that for its split.
 static bool implicit_eligible(int dtype, const GemmArgs &g, int ta, int tb) {
-    return dtype == D8_FLOAT64 ? true : gemm_tiled_eligible(dtype, g, ta, tb);
+    return dtype == D8_FLOAT64 ? true : gemm_tiled_eligible(dtype, g, ta, tb, g.A == nullptr);
 }
 // Workspace such a product may use (the split of its reduction).
 static size_t implicit_workspace(int dtype, const GemmArgs &g) {

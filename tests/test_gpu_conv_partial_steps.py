@@ -1,0 +1,65 @@
+"""Convolutions whose channel counts leave a partial K step in every filter tap, whose pixel count is no multiple of the K
+step, or whose output is smaller than a tile: all of them read their patch matrix in the GEMM's loader.  Called without
+scratch (the staged route would refuse) and with it (the reduction may then be split); integers bit for bit against the
+oracle."""
+import numpy as np
+import pytest
+
+from util import f, h, ints, rng
+
+pytestmark = pytest.mark.gpu
+
+# B, IH, IW, IC, OC, FH, FW, covered, sy, sx, dy, dx
+CONV = [
+    (2, 9, 7, 8, 8, 3, 3, True, 1, 1, 1, 1),       # a lone partial step per tap, fewer rows and columns than any tile
+    (1, 12, 11, 72, 40, 3, 3, True, 1, 1, 1, 1),   # a whole step and a piece of one
+    (3, 15, 15, 96, 136, 3, 3, True, 2, 2, 1, 1),  # strided: the gradient of x by classes
+    (2, 14, 13, 56, 64, 1, 1, True, 1, 1, 1, 1),   # one tap
+    (2, 13, 17, 24, 160, 5, 5, False, 1, 1, 1, 1),
+    (4, 21, 10, 40, 16, 3, 3, True, 1, 1, 2, 2),
+]
+# B, IH, IW, IC, OC, FH, FW, covered, sy, sx
+DECONV = [
+    (2, 7, 7, 96, 40, 4, 4, False, 2, 2),
+    (1, 5, 6, 8, 8, 3, 3, False, 2, 2),            # classes of a few pixels
+    (3, 6, 9, 40, 72, 2, 2, False, 2, 2),
+    (2, 10, 10, 24, 136, 3, 3, True, 1, 1),
+]
+
+
+def _call(lib, name, dt, bufs, shape, filt, geo, out, scratch_bytes):
+    from deep8_amd.capi import DeviceArray, check
+    a, b, c = bufs
+    ws = DeviceArray((max(scratch_bytes, 16),), np.uint8)
+    check(getattr(lib, name)(dt, a.ptr, *shape, b.ptr, *filt, c.ptr, *geo, ws.ptr if scratch_bytes else None, scratch_bytes, None))
+    return f(out.numpy())
+
+
+@pytest.mark.parametrize("op,cfg", [("conv2d", c) for c in CONV] + [("deconv2d", c) for c in DECONV])
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+def test_partial_steps_without_interim_matrix(oracle_port, op, cfg, dtype):
+    from deep8_amd import capi, ops
+    from deep8_amd.capi import DeviceArray
+    lib = capi.init()
+    B, IH, IW, IC, OC, FH, FW = cfg[:7]
+    geo = cfg[7:]
+    OH, OW, _, _ = getattr(ops, op + "_geometry")(IH, IW, FH, FW, *geo)
+    r = rng(sum(cfg[:7]))
+    hi = 3 if dtype == np.float16 else 10
+    c = (lambda v: h(v)) if dtype == np.float16 else (lambda v: v)
+    x, w, gz = ints(r, (B, IH, IW, IC), hi), ints(r, (OC, FH, FW, IC), hi), ints(r, (B, OH, OW, OC), hi)
+    if dtype == np.float16:  # thinned, so that every sum stays a whole number that half can hold
+        x, w, gz = x * (r.random(x.shape) < 0.3), w * (r.random(w.shape) < 0.3), gz * (r.random(gz.shape) < 0.3)
+    port = oracle_port
+    want = [getattr(port, op)(x, w, *geo), getattr(port, op + "_grad_x")(x, w, gz, *geo), getattr(port, op + "_grad_y")(x, w, gz, *geo)]
+    assert dtype == np.float32 or max(np.abs(t).max() for t in want) < 2048
+    dt = capi.dtype_id(np.dtype(dtype))
+    shape, filt, g = (B, IH, IW, IC), (OC, FH, FW), (int(geo[0]),) + tuple(geo[1:])
+    for which, name in enumerate(("d8_" + op, "d8_%s_grad_x_overwrite" % op, "d8_%s_grad_y_overwrite" % op)):
+        nan = DeviceArray.from_numpy(np.full(want[which].shape, np.nan, dtype))
+        bufs = [DeviceArray.from_numpy(c(x)), DeviceArray.from_numpy(c(w)), DeviceArray.from_numpy(c(gz))]
+        bufs[(2, 0, 1)[which]] = nan
+        asked = getattr(lib, "d8_%s_scratch_bytes" % op)(dt, which, *shape, *filt, *g)
+        for scratch in (0, asked):
+            got = _call(lib, name, dt, bufs, shape, filt, g, nan, scratch)
+            assert np.array_equal(got, want[which]), (which, scratch)
