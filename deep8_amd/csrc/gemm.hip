@@ -77,7 +77,8 @@ __device__ inline void wave_mma(const float *As, const float *Bs, int arow, int 
 }
 
 // ------------------------------------------------------------------------------------------
-// General kernel: any M, N, K, leading dimension and alignment.  128 x 128 tile, 4 waves in a
+// General kernel: what the tiled kernels refuse -- operands of 2 GiB and more, sums over half matrices that lie an odd
+// number of elements apart.  128 x 128 tile, 4 waves in a
 // 2 x 2 arrangement, 64 x 64 per wave; element-wise, bounds-checked tile loads.
 // ------------------------------------------------------------------------------------------
 template <typename T, bool TA, bool TB>
@@ -324,87 +325,78 @@ static bool gemm_is_small(int M, int N, int K, int batch, int red) {
 
 // C[b][m][n] = beta * C + sum_s ws[b][s][m][n].  A workgroup covers 32 groups of 4 consecutive
 // outputs; its 8 thread rows each add every 8th partial (16-byte loads), and the 8 sums meet in
-// LDS in a fixed order, so the result does not depend on scheduling.
-template <typename T>
+// LDS in a fixed order, so the result does not depend on scheduling.  The groups count through an output's elements
+// whatever the length of its rows: with rows of an odd length a group starts at any 4-byte aligned address (which is what
+// a 16-byte load needs) and may go on in the next row.  An output a thread, as rows of an odd length had it first, took
+// 17.3 us for four partial sums of 1024 x 1001, this takes 8.0 us.
+typedef f32x4 f32x4_any __attribute__((aligned(4)));
+
+// (ROWS: the rows are multiples of 4, so a group lies in one row and may be stored at once)
+template <typename T, bool ROWS>
 __device__ __forceinline__ void gemm_split_reduce_body(const GemmArgs &g, const long block, f32x4 (*part)[32]) {
-    const long mn = (long)g.M * g.N;
+    typedef T T4 __attribute__((ext_vector_type(4)));
+    const long mn = (long)g.M * g.N, groups = ROWS ? mn / 4 : (mn + 3) / 4;
     const int lane = threadIdx.x & 31, row = threadIdx.x >> 5;
-    const long e = (block * 32 + lane) * 4;  // first of this thread's 4 outputs (N % 4 == 0)
-    const bool live = e < mn * g.batch;
-    const int b = live ? (int)(e / mn) : 0;
-    const long r = e - (long)b * mn;
+    const long id = block * 32 + lane;  // this thread's group of 4 outputs
+    const bool live = id < groups * g.batch;
+    const int b = live && g.batch > 1 ? (int)(id / groups) : 0;
+    const long r = (id - (long)b * groups) * 4;
+    const int n_out = ROWS || mn - r >= 4 ? 4 : (int)(mn - r);
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
     if (live) {
         const float *p = g.ws + (long)b * g.splits * mn + r;
-        for (int s = row; s < g.splits; s += 8) v += *(const f32x4 *)(p + (long)s * mn);
+        if (n_out == 4) {
+            for (int s = row; s < g.splits; s += 8) v += *(const f32x4_any *)(p + (long)s * mn);
+        } else {
+            for (int s = row; s < g.splits; s += 8)
+                for (int k = 0; k < n_out; ++k) v[k] += p[(long)s * mn + k];
+        }
     }
     part[row][lane] = v;
     __syncthreads();
     if (row == 0 && live) {
 #pragma unroll
         for (int k = 1; k < 8; ++k) v += part[k][lane];
-        const int m = (int)(r / g.N), n = (int)(r - (long)m * g.N);
+        int m = (int)(r / g.N), n = (int)(r - (long)m * g.N);
         T *c0 = (T *)g.C + (long)b * g.sC;
+        auto finish = [&](float o, float old, float bias) {
+            if (g.beta != 0.f) o += old;
+            if (g.bias) o = (g.round_first ? to_f32((T)o) : o) + bias;
+            return (T)(g.relu && !(o > 0.f) ? 0.f : o);
+        };
+        if (ROWS && !g.perm_OC && g.ldc % 4 == 0 && (((size_t)c0 | (size_t)g.bias) & (4 * sizeof(T) - 1)) == 0) {
+            T4 *c = (T4 *)(c0 + (long)m * g.ldc + n);
+            T4 old = {}, bias = {}, out;
+            if (g.beta != 0.f) old = *c;
+            if (g.bias) bias = *(const T4 *)((const T *)g.bias + n);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) out[k] = finish(v[k], to_f32(old[k]), to_f32(bias[k]));
+            *c = out;
+            return;
+        }
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            T *c = c0 + c_index(g, m, n + k);
-            float o = v[k];
-            if (g.beta != 0.f) o += to_f32(*c);
-            if (g.bias) o += to_f32(((const T *)g.bias)[n + k]);
-            *c = (T)(g.relu && !(o > 0.f) ? 0.f : o);
+            if (ROWS || k < n_out) {
+                T *c = c0 + c_index(g, m, n);
+                *c = finish(v[k], g.beta != 0.f ? to_f32(*c) : 0.f, g.bias ? to_f32(((const T *)g.bias)[n]) : 0.f);
+            }
+            if (++n == g.N && !ROWS) n = 0, ++m;
         }
     }
 }
 
-template <typename T>
+template <typename T, bool ROWS>
 __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(GemmArgs g) {
     __shared__ f32x4 part[8][32];
-    gemm_split_reduce_body<T>(g, (long)blockIdx.x, part);
+    gemm_split_reduce_body<T, ROWS>(g, (long)blockIdx.x, part);
 }
 
 // The reductions of two products in one launch: the first blocks0 workgroups are g0's, the rest g1's.
 template <typename T>
 __global__ __launch_bounds__(256) void gemm_split_reduce_pair_kernel(GemmArgs g0, GemmArgs g1, unsigned blocks0) {
     __shared__ f32x4 part[8][32];
-    if (blockIdx.x < blocks0) gemm_split_reduce_body<T>(g0, (long)blockIdx.x, part);
-    else gemm_split_reduce_body<T>(g1, (long)(blockIdx.x - blocks0), part);
-}
-
-// The same for N not a multiple of 4: a workgroup covers 32 outputs; its 8 thread rows each add every 8th
-// partial (four loads in flight) and the 8 sums meet in LDS in a fixed order.
-template <typename T>
-__global__ __launch_bounds__(256) void gemm_split_reduce_scalar_kernel(GemmArgs g) {
-    __shared__ float part[8][32];
-    const long mn = (long)g.M * g.N;
-    const int lane = threadIdx.x & 31, row = threadIdx.x >> 5;
-    const long i = (long)blockIdx.x * 32 + lane;
-    const bool live = i < mn * g.batch;
-    const int b = live ? (int)(i / mn) : 0;
-    const long e = i - (long)b * mn;
-    float v = 0.f;
-    if (live) {
-        const float *p = g.ws + (long)b * g.splits * mn + e;
-        int s = row;
-        for (; s + 24 < g.splits; s += 32) {
-            float t[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) t[u] = p[(long)(s + 8 * u) * mn];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) v += t[u];
-        }
-        for (; s < g.splits; s += 8) v += p[(long)s * mn];
-    }
-    part[row][lane] = v;
-    __syncthreads();
-    if (row == 0 && live) {
-#pragma unroll
-        for (int k = 1; k < 8; ++k) v += part[k][lane];
-        const int m = (int)(e / g.N), n = (int)(e - (long)m * g.N);
-        T *c = (T *)g.C + (long)b * g.sC + c_index(g, m, n);
-        if (g.beta != 0.f) v += to_f32(*c);
-        if (g.bias) v += to_f32(((const T *)g.bias)[n]);
-        *c = (T)(g.relu && !(v > 0.f) ? 0.f : v);
-    }
+    if (blockIdx.x < blocks0) gemm_split_reduce_body<T, true>(g0, (long)blockIdx.x, part);
+    else gemm_split_reduce_body<T, true>(g1, (long)(blockIdx.x - blocks0), part);
 }
 
 // ---- planning a product whose 128 x 128 tiles are fewer than the CUs -----------------------------------------
@@ -516,33 +508,29 @@ static int plan_splits(int BK, int M, int N, int K, int batch, int red, size_t w
 }
 
 // C = beta * C + the g.splits partial sums in g.ws (+ bias, ReLu)
+static long reduce_blocks(const GemmArgs &g) { return (((long)g.M * g.N + 3) / 4 * g.batch + 31) / 32; }
+
 template <typename T>
 static int launch_reduce(const GemmArgs &g, hipStream_t stream) {
-    const long total = (long)g.M * g.N * g.batch;
-    if (g.N % 4 == 0 && ((size_t)g.ws & 15) == 0) {
-        hipLaunchKernelGGL((gemm_split_reduce_kernel<T>), dim3((unsigned)((total / 4 + 31) / 32)), dim3(256), 0, stream, g);
-    } else {
-        hipLaunchKernelGGL((gemm_split_reduce_scalar_kernel<T>), dim3((unsigned)((total + 31) / 32)), dim3(256), 0, stream, g);
-    }
+    const dim3 grid((unsigned)reduce_blocks(g));
+    if (g.N % 4 == 0) hipLaunchKernelGGL((gemm_split_reduce_kernel<T, true>), grid, dim3(256), 0, stream, g);
+    else hipLaunchKernelGGL((gemm_split_reduce_kernel<T, false>), grid, dim3(256), 0, stream, g);
     D8_LAUNCH_CHECK();
     return 0;
 }
 
-// The reductions that follow a launch of two products (either may be unsplit): one launch for both where both take
-// the 16-byte form.
+// The reductions that follow a launch of two products (either may be unsplit): one launch for both (whose rows are
+// multiples of 4, or they would not have shared the first).
 static int launch_reduce_pair(int dtype, const GemmArgs &g0, const GemmArgs &g1, hipStream_t stream) {
     const bool r0 = g0.splits > 1, r1 = g1.splits > 1;
-    auto vec = [](const GemmArgs &g) { return g.N % 4 == 0 && ((size_t)g.ws & 15) == 0; };
-    if (r0 && r1 && vec(g0) && vec(g1)) {
-        const long b0 = ((long)g0.M * g0.N * g0.batch / 4 + 31) / 32, b1 = ((long)g1.M * g1.N * g1.batch / 4 + 31) / 32;
-        if (b0 + b1 < 0x7fffffffL) {
-            if (dtype == D8_FLOAT16)
-                hipLaunchKernelGGL((gemm_split_reduce_pair_kernel<f16>), dim3((unsigned)(b0 + b1)), dim3(256), 0, stream, g0, g1, (unsigned)b0);
-            else
-                hipLaunchKernelGGL((gemm_split_reduce_pair_kernel<float>), dim3((unsigned)(b0 + b1)), dim3(256), 0, stream, g0, g1, (unsigned)b0);
-            D8_LAUNCH_CHECK();
-            return 0;
-        }
+    const long b0 = reduce_blocks(g0), b1 = reduce_blocks(g1);
+    if (r0 && r1 && g0.N % 4 == 0 && g1.N % 4 == 0 && b0 + b1 < 0x7fffffffL) {
+        if (dtype == D8_FLOAT16)
+            hipLaunchKernelGGL((gemm_split_reduce_pair_kernel<f16>), dim3((unsigned)(b0 + b1)), dim3(256), 0, stream, g0, g1, (unsigned)b0);
+        else
+            hipLaunchKernelGGL((gemm_split_reduce_pair_kernel<float>), dim3((unsigned)(b0 + b1)), dim3(256), 0, stream, g0, g1, (unsigned)b0);
+        D8_LAUNCH_CHECK();
+        return 0;
     }
     if (r0)
         if (int rc = dtype == D8_FLOAT16 ? launch_reduce<f16>(g0, stream) : launch_reduce<float>(g0, stream)) return rc;
@@ -698,7 +686,7 @@ bool gemm_tiled_run_pair(int dtype, GemmArgs &gx, GemmArgs &gy, void *workspace,
     const bool off = getenv("D8_CONV_GRADS_APART") != nullptr;  // tuning and test aid (read at every call)
     if (off || dtype == D8_FLOAT64) return false;
     if (gx.virt != VIRT_A_ROWS || gy.virt != VIRT_B_KROWS || gx.batch != 1 || gy.batch != 1) return false;
-    if (!gemm_tiled_eligible(dtype, gx, 0, 0, true) || !gemm_tiled_eligible(dtype, gy, 1, 0, true)) return false;
+    if (!gemm_tiled_eligible(dtype, gx, 0, 0, TILED_WHOLE) || !gemm_tiled_eligible(dtype, gy, 1, 0, TILED_WHOLE)) return false;
     // More workgroups than the chip holds at once (two per compute unit): in half the shared launch still gains
     // (3x3 Conv2d, B32: 56x56x64 49.9 -> 47.0 us, 14x14x256 46.0 -> 34.9, 56x56x64->128 74.2 -> 65.0; DeConv2d 4x4 s2
     // B64 14x14x256 60.7 -> 47.9), gx's remainder band riding along as it does alone.  In fp32, bound by the matrix
@@ -748,7 +736,7 @@ bool gemm_tiled_run_plain_pair(int dtype, GemmArgs &g0, int ta0, int tb0, GemmAr
     const bool off = getenv("D8_MATMUL_GRADS_APART") != nullptr;  // tuning and test aid (read at every call)
     if (off || dtype == D8_FLOAT64 || ta0 || !tb0 || !ta1 || tb1) return false;
     if (g0.virt != VIRT_NONE || g1.virt != VIRT_NONE || g0.K < 1 || g1.K < 1) return false;
-    if (!gemm_tiled_eligible(dtype, g0, ta0, tb0) || !gemm_tiled_eligible(dtype, g1, ta1, tb1)) return false;
+    if (!gemm_tiled_eligible(dtype, g0, ta0, tb0, TILED_PIECES) || !gemm_tiled_eligible(dtype, g1, ta1, tb1, TILED_PIECES)) return false;
     if (gemm_is_small(g0.M, g0.N, g0.K, g0.batch, g0.red) || gemm_is_small(g1.M, g1.N, g1.K, g1.batch, g1.red)) return false;
     if (balanced_rows(g0) || balanced_rows(g1)) return false;
     const size_t usable = (workspace && ((size_t)workspace & 15) == 0) ? workspace_bytes : 0;
@@ -768,12 +756,12 @@ bool gemm_tiled_run_plain_pair(int dtype, GemmArgs &g0, int ta0, int tb0, GemmAr
     return true;
 }
 
-bool gemm_fuses_store(int dtype, const GemmArgs &g, int transA, int transB) {
+bool gemm_fuses_store(int dtype, const GemmArgs &g, int transA, int transB, TiledRule rule) {
     // (a product beyond one launch's limits -- more than 448 outputs, more than 65535 * 128 rows -- is cut into several
     // by d8_gemm; the fused store stays out of that: the caller runs the product and one pass over its result)
     if (dtype == D8_FLOAT64 || g.K < 1 || g.beta != 0.f || g.red != 1 || g.batch > 448 || g.M > 65535 * 128) return false;
     if (g.virt == VIRT_NONE && gemm_is_small(g.M, g.N, g.K, g.batch, g.red)) return false;  // gemm_small_kernel has no fused store
-    return gemm_tiled_eligible(dtype, g, transA, transB);
+    return gemm_tiled_eligible(dtype, g, transA, transB, rule);
 }
 
 int gemm_run_fused(int dtype, GemmArgs &g, int transA, int transB, void *workspace, size_t workspace_bytes, hipStream_t stream) {

@@ -77,6 +77,10 @@ struct GemmArgs {
     // ReLu do as separate passes over C in the reference (deep8/src/math/Add.cu:21-52, ReLu.cu:20-59).
     const void *bias;
     int relu;
+    // Half: the product is rounded to half before the bias is added, as a separate pass over it would find it.  Set where
+    // product and bias + ReLu used to be two passes: a gate decided by the sum that is rounded once opens for other
+    // elements (about one in five thousand), and a layer keeps the gates it had.
+    int round_first;
     // Remainder band in the same launch (tail_splits > 0; unsplit, unbatched products only): rows tail_m0 .. M - 1
     // are not tiled by the launch's first tiles(tail_m0) x tiles(N) workgroups but by further ones, tail_splits per
     // tile, each walking tail_tps K steps and writing fp32 partial sums to ws[piece][row - tail_m0][n].  They start
@@ -90,9 +94,11 @@ struct GemmArgs {
     unsigned long long *phase_rec;
 };
 
+enum TiledRule { TILED_ANY, TILED_PIECES, TILED_WHOLE };  // see gemm_tiled_eligible
+
 // Whether a product with these arguments would run on a kernel that applies GemmArgs::bias / relu in its store
 // (else the caller runs the plain product and launch_bias_relu).
-bool gemm_fuses_store(int dtype, const GemmArgs &g, int transA, int transB);
+bool gemm_fuses_store(int dtype, const GemmArgs &g, int transA, int transB, TiledRule rule = TILED_ANY);
 // The product of d8_gemm (beta = 0, no summed batch) with the fused store; the shape must pass gemm_fuses_store.
 int gemm_run_fused(int dtype, GemmArgs &g, int transA, int transB, void *workspace, size_t workspace_bytes, hipStream_t stream);
 // z[r][c] = relu?(z[r][c] + bias[c]) in place, one pass (bias may be null): the fallback for shapes the fused store does not take.
@@ -100,9 +106,15 @@ int launch_bias_relu(int dtype, void *z, const void *bias, long rows, int cols, 
 
 // Tiled kernels (fp16 and fp32) for shapes whose operands can be moved in 16-byte pieces.
 int gemm_tiled_k_step(int dtype);  // K elements per step: 64 (fp16) or 32 (fp32)
-// Whether the shape qualifies (g.splits / g.tiles_per_split need not be set yet).  whole_steps: among products with a
-// patch-matrix operand only those whose K steps are all whole and whose output is no smaller than a tile.
-bool gemm_tiled_eligible(int dtype, const GemmArgs &g, int transA, int transB, bool whole_steps = false);
+// Whether the shape qualifies (g.splits / g.tiles_per_split need not be set yet).
+//   TILED_ANY     whatever a single launch takes: real matrices of any shape and alignment, patch matrices whose channels
+//                 can be moved in 16-byte pieces
+//   TILED_PIECES  ... real matrices too only in 16-byte pieces, and at least one side of the output as long as a tile (what
+//                 a launch of two products takes)
+//   TILED_WHOLE   ... and patch matrices only where all K steps are whole and the output is no smaller than a tile (what
+//                 a launch of a convolution's two gradients takes, and what the scratch queries plan without an interim
+//                 matrix)
+bool gemm_tiled_eligible(int dtype, const GemmArgs &g, int transA, int transB, TiledRule rule = TILED_ANY);
 // Launch; with g.splits > 1 the fp32 partial sums go to g.ws for the caller to reduce.
 int gemm_tiled_launch(int dtype, const GemmArgs &g, int transA, int transB, hipStream_t stream);
 // Two patch-matrix products as ONE launch: gx with patch rows as A (NN: a convolution's gradient of its input), gy with

@@ -12,10 +12,8 @@ void gemm_tiled_phase_record(void *records, size_t bytes) {
     phase_rec_bytes = records ? bytes : 0;
 }
 
-// whole_steps: only products whose K steps are whole inside every filter tap / over the patch rows, and whose outputs fill
-// a tile -- the shapes that the scratch queries plan without an interim matrix and that a launch of two products takes.
 template <typename E>
-static bool eligible(const GemmArgs &g, int transA, int transB, bool whole_steps) {
+static bool eligible(const GemmArgs &g, int transA, int transB, TiledRule rule) {
     constexpr long ES = sizeof(E), EPV = 16 / ES, BK = 128 / ES;
     const bool va = g.virt == VIRT_A_ROWS || g.virt == VIRT_A_CLASSES, vb = g.virt == VIRT_B_KROWS;
     if (g.virt == VIRT_A_CLASSES && (g.splits > 1 || g.ncls < 1 || g.ncls > MAX_CLASSES)) return false;
@@ -26,10 +24,14 @@ static bool eligible(const GemmArgs &g, int transA, int transB, bool whole_steps
     if (!va && ((g.red - 1) * g.sA + (long)(transA ? g.K : g.M) * g.lda) * ES >= (1L << 31)) return false;
     if (!vb && ((g.red - 1) * g.sB + (long)(transB ? g.N : g.K) * g.ldb) * ES >= (1L << 31)) return false;
     if (g.K < 1) return false;  // (a K below one K step is a lone partial step)
+    if ((long)ceil_div(g.M, 128) * ceil_div(g.N, 128) > 0x7fffffffL || (long)g.batch * 128 > 65535) return false;
+    if (g.virt == VIRT_NONE && rule == TILED_ANY)
+        // rows may start at any element (EDGE_ANY); a thread's shift must hold for all products of a sum
+        return in_pieces<E>(g, !transA, transB) || g.red == 1 || ((g.sA | g.sB) * ES) % 4 == 0;
     // one side may be shorter than any tile (a few rows against a wide matrix: the 64 x 128 / 128 x 64 tile
     // then reaches past it) when the other side fills a tile; a patch-matrix product may have both short
-    if (g.M < 128 && g.N < 128 && (g.virt == VIRT_NONE || whole_steps)) return false;
-    if (whole_steps && g.virt != VIRT_NONE && (g.K % BK || g.M < (g.virt == VIRT_A_CLASSES ? 128 : 64) || (vb && g.N < 64))) return false;
+    if (g.M < 128 && g.N < 128 && (g.virt == VIRT_NONE || rule == TILED_WHOLE)) return false;
+    if (rule == TILED_WHOLE && g.virt != VIRT_NONE && (g.K % BK || g.M < (g.virt == VIRT_A_CLASSES ? 128 : 64) || (vb && g.N < 64))) return false;
     // a 16-byte piece of an operand stored along K must lie wholly on one side of K
     if (g.K % BK && (!transA || transB) && g.K % EPV) return false;
     if (!va && (g.lda % EPV || g.sA % EPV)) return false;
@@ -37,15 +39,14 @@ static bool eligible(const GemmArgs &g, int transA, int transB, bool whole_steps
     if (((size_t)g.A | (size_t)g.B) & 15) return false;
     if (transA && g.M % EPV) return false;
     if (!transB && g.N % EPV) return false;
-    if ((long)ceil_div(g.M, 128) * ceil_div(g.N, 128) > 0x7fffffffL || (long)g.batch * 128 > 65535) return false;
     return true;
 }
 
 int gemm_tiled_k_step(int dtype) { return dtype == D8_FLOAT16 ? 64 : 32; }
 
-bool gemm_tiled_eligible(int dtype, const GemmArgs &g, int transA, int transB, bool whole_steps) {
+bool gemm_tiled_eligible(int dtype, const GemmArgs &g, int transA, int transB, TiledRule rule) {
     if (dtype == D8_FLOAT64) return false;
-    return dtype == D8_FLOAT16 ? eligible<f16>(g, transA, transB, whole_steps) : eligible<float>(g, transA, transB, whole_steps);
+    return dtype == D8_FLOAT16 ? eligible<f16>(g, transA, transB, rule) : eligible<float>(g, transA, transB, rule);
 }
 
 int gemm_tiled_launch(int dtype, const GemmArgs &g, int transA, int transB, hipStream_t stream) {

@@ -56,6 +56,19 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 #define SG_DS_READ 0x100
 #define SG_DS_WRITE 0x200
 
+// What a product's operands look like at their edges (a template argument of the kernels):
+//   EDGE_NONE    K is a multiple of the K step
+//   EDGE_PIECES  a last, partial K step; a 16-byte piece of an operand lies on one side of K
+//   EDGE_ANY     rows that start anywhere: any leading dimension, any K, any element-aligned pointer.  A piece is fetched
+//                from a 4-byte aligned address (which is all a buffer load needs), for half from the one at or before it,
+//                with one more dword where the row starts in the middle of a dword, and shifted into place on its way to
+//                LDS; what a piece of a row stored along K brings in from past K is cut off there as well.  Rows
+//                keep their parity from step to step (K steps and passes are even numbers of rows), so shift and extra
+//                dword are constants of a thread.  Half 4096 x 1024 by 1024 x 1001, which a kernel that moved single elements
+//                served before: product with bias and ReLu 68 -> 29 us, its gradients 50 and 68 -> 21 and 22 us.  Bound by
+//                the K loop's latency as the other variants, plus 60 vector instructions a step.
+enum { EDGE_NONE = 0, EDGE_PIECES = 1, EDGE_ANY = 2 };
+
 // ---- per element type: operand fragments and how to multiply one k group --------------------
 template <typename E>
 struct Elem;
@@ -131,7 +144,8 @@ struct Tile {
     __device__ __host__ static constexpr int kc_row(int r) { return r * BK + (r >> 1) * EPV; }
     static constexpr int KC_BLK = kc_row(32);  // elements between rows 32 apart (from an even row)
     static constexpr int A_LD = BM + EL::TR_PAD / ES, B_LD = BN + EL::TR_PAD / ES;
-    static constexpr int A_SZ = A_KC ? kc_row(BM) : BK * A_LD;
+    static constexpr int A_TILE = A_KC ? kc_row(BM) : BK * A_LD, PATCHES = NT / 128 * 32 * 36 * 4 / ES;  // (patches: the epilogue's, see below)
+    static constexpr int A_SZ = A_TILE > PATCHES ? A_TILE : PATCHES;
     static constexpr int B_SZ = B_KC ? kc_row(BN) : BK * B_LD;
     // 16-byte pieces each thread moves per K step, and the rows one pass of all threads covers
     static constexpr int A_IT = BM * 8 / NT, B_IT = BN * 8 / NT, NP = A_IT + B_IT;
@@ -159,16 +173,51 @@ __device__ __host__ constexpr int piece_lo(int q) { return q * NP / 3; }
 // The t-th of n events of a quarter goes right after MFMA number (t * MQ) / n.
 __device__ __host__ constexpr int slot_of(int t, int n, int MQ) { return t * MQ / n; }
 
+// EDGE_ANY: what a thread needs to put its pieces into place
+template <typename T, int EDGE>
+struct Loose {
+    static constexpr bool ANY = EDGE == EDGE_ANY, ODD = ANY && T::ES == 2;
+    unsigned X[ODD ? T::NP : 1];  // the dword after each piece
+    unsigned shift[2], next[2];   // per operand: bits to shift by, byte offset of that dword (outside the buffer where it is not needed)
+    u32x4 keep[2];                // ... and which bits of a piece are within K (operands stored along K)
+    __device__ __forceinline__ u32x4 place(int p, u32x4 v) const {
+        if constexpr (ANY) {
+            const int o = p < T::A_IT ? 0 : 1;
+            if constexpr (ODD) {
+                u32x4 w;
+#pragma unroll
+                for (int d = 0; d < 4; ++d) w[d] = __builtin_amdgcn_alignbit(d < 3 ? v[d < 3 ? d + 1 : 3] : X[p], v[d], shift[o]);
+                v = w;
+            }
+            if (o == 0 ? T::A_KC : T::B_KC) v &= keep[o];
+        }
+        return v;
+    }
+    __device__ __forceinline__ void fetch(int p, __amdgpu_buffer_rsrc_t r, unsigned v, unsigned s) {
+        if constexpr (ODD) X[p] = __builtin_amdgcn_raw_buffer_load_b32(r, v + next[p < T::A_IT ? 0 : 1], s, 0);
+    }
+    // the pieces of operand o written next have `left` elements of K from this thread's first on
+    __device__ __forceinline__ void keep_first(int o, int left) {
+        if constexpr (ANY) {
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+                if constexpr (T::ES == 2) keep[o][d] = left > 2 * d + 1 ? 0xffffffffu : left > 2 * d ? 0xffffu : 0u;
+                else keep[o][d] = left > d ? 0xffffffffu : 0u;
+            }
+        }
+    }
+};
+
 // One K step.  Ar/Br: this lane's operand addresses in the LDS half being multiplied; An/Bn: the
 // same in the other half (next step); Aw/Bw: where this thread's pieces of the next step go;
 // ra/rb: buffer descriptors of the A and B matrices; ga/gb: wave-uniform byte offset (tile origin +
 // K step) of the pieces of the step after that, av/bv: this thread's byte offset for each piece.
-template <typename T>
+template <typename T, int EDGE>
 __device__ __forceinline__ void k_step(const typename T::E *Ar, const typename T::E *Br, const typename T::E *An,
                                        const typename T::E *Bn, typename T::E *Aw, typename T::E *Bw,
                                        __amdgpu_buffer_rsrc_t ra, __amdgpu_buffer_rsrc_t rb, unsigned ga, unsigned gb,
                                        unsigned a_pass, unsigned b_pass, const unsigned (&av)[T::A_IT],
-                                       const unsigned (&bv)[T::B_IT], u32x4 (&R)[T::NP], typename T::EL::Frag (&fa)[2][T::TM],
+                                       const unsigned (&bv)[T::B_IT], u32x4 (&R)[T::NP], Loose<T, EDGE> &L, typename T::EL::Frag (&fa)[2][T::TM],
                                        typename T::EL::Frag (&fb)[2][T::TN], f32x16 (&acc)[T::TM][T::TN]) {
     typedef typename T::E E;
     typedef typename T::EL EL;
@@ -189,7 +238,7 @@ __device__ __forceinline__ void k_step(const typename T::E *Ar, const typename T
                 if (slot_of(t, w_n, MQ) == m) {
                     const int p = w_lo + t;
                     E *dst = p < A_IT ? Aw + p * T::A_PASS : Bw + (p - A_IT) * T::B_PASS;
-                    *(u32x4 *)dst = R[p];
+                    *(u32x4 *)dst = L.place(p, R[p]);
                 }
 #pragma unroll
             for (int t = 0; t < g_n; ++t)
@@ -197,6 +246,7 @@ __device__ __forceinline__ void k_step(const typename T::E *Ar, const typename T
                     const int p = g_lo + t;
                     R[p] = p < A_IT ? __builtin_amdgcn_raw_buffer_load_b128(ra, av[p < A_IT ? p : 0], ga + p * a_pass, 0)
                                     : __builtin_amdgcn_raw_buffer_load_b128(rb, bv[p < A_IT ? 0 : p - A_IT], gb + (p - A_IT) * b_pass, 0);
+                    L.fetch(p, p < A_IT ? ra : rb, p < A_IT ? av[p < A_IT ? p : 0] : bv[p < A_IT ? 0 : p - A_IT], p < A_IT ? ga + p * a_pass : gb + (p - A_IT) * b_pass);
                 }
             // operands of the next quarter (of the next step's first quarter when q == 3)
 #pragma unroll
@@ -221,7 +271,7 @@ __device__ __forceinline__ void k_step(const typename T::E *Ar, const typename T
                 if (slot_of(t, w_n, MQ) == m) __builtin_amdgcn_sched_group_barrier(SG_DS_WRITE, 1, 0);
 #pragma unroll
             for (int t = 0; t < g_n; ++t)
-                if (slot_of(t, g_n, MQ) == m) __builtin_amdgcn_sched_group_barrier(SG_VMEM_READ, 1, 0);
+                if (slot_of(t, g_n, MQ) == m) __builtin_amdgcn_sched_group_barrier(SG_VMEM_READ, Loose<T, EDGE>::ODD ? 2 : 1, 0);
 #pragma unroll
             for (int f = 0; f < NF; ++f)
                 if (slot_of(f, NF, MQ) == m) {
@@ -268,7 +318,7 @@ struct RowMap {
 template <typename T, typename O>
 __device__ __forceinline__ void store_tile(f32x16 (&acc)[T::TM][T::TN], float *lds0, float *lds1, O *C, int ldc, float beta,
                                            bool aligned, int N, const Origin &o, const RowMap &crow,
-                                           const O *bias = nullptr, bool relu = false) {
+                                           const O *bias = nullptr, bool relu = false, bool round_first = false) {
     constexpr int TM = T::TM, TN = T::TN, OPV = 16 / sizeof(O);
     typedef O OV __attribute__((ext_vector_type(OPV)));
     constexpr int HALF_WAVES = T::NT / 128;
@@ -302,7 +352,7 @@ __device__ __forceinline__ void store_tile(f32x16 (&acc)[T::TM][T::TN], float *l
                             if (bias) {
                                 const OV bv = *(const OV *)(bias + n + h * OPV);
 #pragma unroll
-                                for (int e = 0; e < OPV; ++e) v[h * OPV + e] += as_f32(bv[e]);
+                                for (int e = 0; e < OPV; ++e) v[h * OPV + e] = (round_first ? as_f32((O)v[h * OPV + e]) : v[h * OPV + e]) + as_f32(bv[e]);
                             }
 #pragma unroll
                             for (int e = 0; e < OPV; ++e) out[e] = (O)(relu && !(v[h * OPV + e] > 0.f) ? 0.f : v[h * OPV + e]);
@@ -313,28 +363,33 @@ __device__ __forceinline__ void store_tile(f32x16 (&acc)[T::TM][T::TN], float *l
             }
         return;
     }
+    // element by element: 32 lanes store 32 consecutive columns of a row.  (A row's address is formed once per row, the
+    // bias read once per column.)
+    const bool plain_rows = !crow.plane && !crow.perm_OC;
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int j = 0; j < TN; ++j) {
+        const int n = o.n0 + o.wn0 + j * 32 + l32;
+        const bool in_n = n >= o.n_own && n < o.n_end;
+        const float bias_n = bias && in_n ? as_f32(bias[n]) : 0.f;
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const int n = o.n0 + o.wn0 + j * 32 + l32;
+        for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int m = o.m0 + o.wm0 + i * 32 + (r >> 2) * 8 + lhi * 4 + (r & 3);
-                if (m >= o.m_own && n >= o.n_own && m < o.m_end && n < o.n_end) {
-                    O *c = C + crow.at(m, n, ldc);
+                if (in_n && m >= o.m_own && m < o.m_end) {
+                    O *c = C + (plain_rows ? (long)m * ldc + n : crow.at(m, n, ldc));
                     float v = acc[i][j][r];
                     if (beta != 0.f) v += as_f32(*c);
-                    if (bias) v += as_f32(bias[n]);
+                    if (bias) v = (round_first ? as_f32((O)v) : v) + bias_n;
                     *c = (O)(relu && !(v > 0.f) ? 0.f : v);
                 }
             }
-        }
+    }
 }
 
 // The work of one workgroup: workgroup (bx, bz) of a grid of nbx x layers (the launch's own blockIdx / gridDim, or what a
 // launch of two products makes of them).  As0 .. Bs1: the two halves of both operand areas in LDS.
-template <typename T, bool TAIL>
+template <typename T, int EDGE>
 __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, const int tilesN, const int bx, const int bz, const int nbx,
                                                 typename T::E *As0, typename T::E *As1, typename T::E *Bs0, typename T::E *Bs1) {
     typedef typename T::E E;
@@ -419,17 +474,22 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     // number of rows below piece 0, in global memory and in LDS alike.  Global memory is read
     // through buffer descriptors: byte offset = uniform part (tile origin, K step, piece; scalar
     // registers) + per-thread part (one VGPR per operand).
+    // EDGE_ANY: the buffers start at the dword that holds the operand's first element and end with the one that holds its
+    // last (a dword at a multiple of 4 never reaches into another page); at the elements before and after sit no results.
+    constexpr bool ANY = EDGE == EDGE_ANY, ODD = Loose<T, EDGE>::ODD;
     const long a_rows = A_KC ? g.M : g.K, b_rows = B_KC ? g.N : g.K;
+    const E *Ab = (const E *)g.A + (long)b * g.sA, *Bb = (const E *)g.B + (long)b * g.sB;
+    const unsigned a_odd = ODD ? (unsigned)((size_t)Ab & 2) >> 1 : 0u, b_odd = ODD ? (unsigned)((size_t)Bb & 2) >> 1 : 0u;
+    const long a_len = ANY ? (g.red - 1) * g.sA + (a_rows - 1) * g.lda + (A_KC ? g.K : g.M) + a_odd : (g.red - 1) * g.sA + a_rows * g.lda;
+    // (the taps of a filter interleave inside its rows: the filter ends with its last row)
+    const long b_len = ANY ? (g.red - 1) * g.sB + (b_rows - 1) * g.ldb + (B_KC ? g.K : g.N) + b_odd : (VA ? 0 : (g.red - 1) * g.sB) + b_rows * g.ldb;
     const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)((const E *)g.A + (long)b * g.sA), 0,
-        VA ? (int)pg.bytes : (int)(ES * ((g.red - 1) * g.sA + a_rows * g.lda)), 0x00020000);
+        (void *)(Ab - a_odd), 0, VA ? (int)pg.bytes : (int)((ES * a_len + 3) & ~3L), 0x00020000);
     const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)((const E *)g.B + (long)b * g.sB), 0,
-        VIRT == VIRT_B_KROWS ? (int)pg.bytes
-                             // (the taps of a filter interleave inside its rows: the filter ends with its last row)
-                             : (int)(ES * ((VA ? 0 : (g.red - 1) * g.sB) + b_rows * g.ldb)), 0x00020000);
-    const unsigned Au = (unsigned)ES * (A_KC ? (unsigned)m0 * g.lda : (unsigned)m0);
-    const unsigned Bu = (unsigned)ES * (B_KC ? (unsigned)n0 * g.ldb : (unsigned)n0);
+        (void *)(Bb - b_odd), 0, VIRT == VIRT_B_KROWS ? (int)pg.bytes : (int)((ES * b_len + 3) & ~3L), 0x00020000);
+    // where the tile starts, in elements: uniform, but for half rows at any element only the dword part of it is
+    const unsigned a_tile = (A_KC ? (unsigned)m0 * g.lda : (unsigned)m0) + a_odd, b_tile = (B_KC ? (unsigned)n0 * g.ldb : (unsigned)n0) + b_odd;
+    const unsigned Au = (unsigned)ES * (ODD ? a_tile & ~1u : a_tile), Bu = (unsigned)ES * (ODD ? b_tile & ~1u : b_tile);
     const int a_r = A_KC ? tid >> 3 : tid / (BM / EPV), a_c = A_KC ? tid & 7 : tid % (BM / EPV);
     const int b_r = (B_KC || T::B_COLS) ? tid >> 3 : tid / (BN / EPV), b_c = (B_KC || T::B_COLS) ? tid & 7 : tid % (BN / EPV);
     const int a_dst = (A_KC ? T::kc_row(a_r) : a_r * A_LD) + a_c * EPV, b_dst = (B_KC ? T::kc_row(b_r) : b_r * B_LD) + b_c * EPV;
@@ -440,11 +500,19 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     // per-thread byte offset of each piece: one value for a real matrix, recomputed every step
     // for a patch matrix (an offset beyond the image makes the buffer load return zeros)
     constexpr unsigned OUTSIDE = 0x80000000u;
+    const unsigned a_first = (unsigned)a_r * (unsigned)g.lda + a_c * EPV + (ODD ? a_tile & 1u : 0u);
+    const unsigned b_first_el = (unsigned)b_r * (unsigned)g.ldb + b_c * EPV + (ODD ? b_tile & 1u : 0u);
+    const unsigned av_plain = (unsigned)ES * (ODD ? a_first & ~1u : a_first), bv_plain = (unsigned)ES * (ODD ? b_first_el & ~1u : b_first_el);
     unsigned av[A_IT], bv[B_IT];
 #pragma unroll
-    for (int p = 0; p < A_IT; ++p) av[p] = (unsigned)ES * ((unsigned)a_r * (unsigned)g.lda + a_c * EPV);
+    for (int p = 0; p < A_IT; ++p) av[p] = av_plain;
 #pragma unroll
-    for (int p = 0; p < B_IT; ++p) bv[p] = (unsigned)ES * ((unsigned)b_r * (unsigned)g.ldb + b_c * EPV);
+    for (int p = 0; p < B_IT; ++p) bv[p] = bv_plain;
+    Loose<T, EDGE> L;
+    if constexpr (ODD) {
+        L.shift[0] = (a_first & 1u) * 16, L.shift[1] = (b_first_el & 1u) * 16;
+        L.next[0] = a_first & 1u ? 16u : OUTSIDE, L.next[1] = b_first_el & 1u ? 16u : OUTSIDE;
+    }
     // patch rows as A: this thread's rows never change; a step selects the tap
     int va_base[A_IT], va_iy[A_IT], va_ix[A_IT];
     if constexpr (VA) {
@@ -515,8 +583,6 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     // partly past K, and the pieces that lie past it are fetched at an offset beyond the buffer, i.e. as zeros.  Where the
     // reduction runs over patch rows or over the rows of a real matrix, rows past the last lie outside the buffer anyway.
     const int ktiles = (g.K + BK - 1) / BK, last_len = g.K - (ktiles - 1) * BK;
-    const unsigned av_plain = (unsigned)ES * ((unsigned)a_r * (unsigned)g.lda + a_c * EPV);
-    const unsigned bv_plain = (unsigned)ES * ((unsigned)b_r * (unsigned)g.ldb + b_c * EPV);
     const int x0 = split * tps, nsteps = min(red * ktiles, x0 + tps) - x0;
     const unsigned a_prod = (unsigned)ES * (unsigned)g.sA, b_prod = (unsigned)ES * (unsigned)g.sB;
     const unsigned b_prod_row = (unsigned)ES * (unsigned)g.sB_row, b_first = (unsigned)ES * b_cls;
@@ -535,9 +601,9 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
         vb_d_img = (pg.H - pg.OH * pg.sy) * pg.W * pg.C * ES;
     }
     // How much of the step that is fetched lies within K: all of it, or what is left of K in a product's last step.  (Where
-    // K is a multiple of the K step -- an instantiation without TAIL -- nothing asks: on patch rows in fp32 the
+    // K is a multiple of the K step -- EDGE_NONE -- nothing asks: on patch rows in fp32 the
     // comparisons alone cost 2 % of a launch.)
-    constexpr bool PARTIAL = TAIL && VIRT != VIRT_B_KROWS;
+    constexpr bool PARTIAL = EDGE != EDGE_NONE && VIRT != VIRT_B_KROWS;
     auto k_left = [&]() -> int { return ld_kx == ktiles - 1 ? last_len : BK; };
     auto step_a = [&]() -> unsigned {
         if constexpr (VA) {
@@ -605,26 +671,35 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
         }
     };
 
-    // ---- prologue: step 0 into LDS half 0, step 1 into registers, first operands of step 0
-    {
-        const unsigned pa = step_a(), pb = step_b();
+    // EDGE_ANY: the pieces that are written next are those of the step before the one fetched next
+    int written_left = BK;
+    auto next_step = [&](unsigned &pa, unsigned &pb) {
+        if constexpr (ANY) {
+            L.keep_first(0, written_left - a_c * EPV);
+            L.keep_first(1, written_left - b_c * EPV);
+            written_left = k_left();
+        }
+        pa = step_a(), pb = step_b();
         step_on();
+    };
+    auto fetch_all = [&](unsigned pa, unsigned pb) {
 #pragma unroll
-        for (int p = 0; p < NP; ++p)
+        for (int p = 0; p < NP; ++p) {
             R[p] = p < A_IT ? __builtin_amdgcn_raw_buffer_load_b128(ra, av[p < A_IT ? p : 0], pa + p * a_pass, 0)
                             : __builtin_amdgcn_raw_buffer_load_b128(rb, bv[p < A_IT ? 0 : p - A_IT], pb + (p - A_IT) * b_pass, 0);
-    }
+            L.fetch(p, p < A_IT ? ra : rb, p < A_IT ? av[p < A_IT ? p : 0] : bv[p < A_IT ? 0 : p - A_IT], p < A_IT ? pa + p * a_pass : pb + (p - A_IT) * b_pass);
+        }
+    };
+
+    // ---- prologue: step 0 into LDS half 0, step 1 into registers, first operands of step 0
+    unsigned pa, pb;
+    next_step(pa, pb);
+    fetch_all(pa, pb);
+    next_step(pa, pb);
 #pragma unroll
     for (int p = 0; p < NP; ++p)
-        *(u32x4 *)(p < A_IT ? As0 + a_dst + p * T::A_PASS : Bs0 + b_dst + (p - A_IT) * T::B_PASS) = R[p];
-    {
-        const unsigned pa = step_a(), pb = step_b();
-        step_on();
-#pragma unroll
-        for (int p = 0; p < NP; ++p)
-            R[p] = p < A_IT ? __builtin_amdgcn_raw_buffer_load_b128(ra, av[p < A_IT ? p : 0], pa + p * a_pass, 0)
-                            : __builtin_amdgcn_raw_buffer_load_b128(rb, bv[p < A_IT ? 0 : p - A_IT], pb + (p - A_IT) * b_pass, 0);
-    }
+        *(u32x4 *)(p < A_IT ? As0 + a_dst + p * T::A_PASS : Bs0 + b_dst + (p - A_IT) * T::B_PASS) = L.place(p, R[p]);
+    fetch_all(pa, pb);
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -636,17 +711,13 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     if (g.phase_rec) st_w[1] = wall_clock64(), st_c[0] = __builtin_readcyclecounter();
     // ---- main loop, two steps per trip so that the LDS half of every access is known statically;
     for (int i = 0; i < nsteps; i += 2) {
-        {
-            const unsigned pa = step_a(), pb = step_b();
-            step_on();
-            k_step<T>(As0 + a_frag, Bs0 + b_frag, As1 + a_frag, Bs1 + b_frag, As1 + a_dst, Bs1 + b_dst, ra, rb, pa, pb,
-                      a_pass, b_pass, av, bv, R, fa, fb, acc);
-        }
+        next_step(pa, pb);
+        k_step<T, EDGE>(As0 + a_frag, Bs0 + b_frag, As1 + a_frag, Bs1 + b_frag, As1 + a_dst, Bs1 + b_dst, ra, rb, pa, pb,
+                        a_pass, b_pass, av, bv, R, L, fa, fb, acc);
         if (i + 1 < nsteps) {
-            const unsigned pa = step_a(), pb = step_b();
-            step_on();
-            k_step<T>(As1 + a_frag, Bs1 + b_frag, As0 + a_frag, Bs0 + b_frag, As0 + a_dst, Bs0 + b_dst, ra, rb, pa, pb,
-                      a_pass, b_pass, av, bv, R, fa, fb, acc);
+            next_step(pa, pb);
+            k_step<T, EDGE>(As1 + a_frag, Bs1 + b_frag, As0 + a_frag, Bs0 + b_frag, As0 + a_dst, Bs0 + b_dst, ra, rb, pa, pb,
+                            a_pass, b_pass, av, bv, R, L, fa, fb, acc);
         }
     }
 
@@ -663,7 +734,8 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
         store_tile<T, float>(acc, patches, patches1, g.ws + ((long)(b * g.splits + split) * g.M) * g.N, g.N, 0.f, true, g.N, o, plain);
     else
         store_tile<T, E>(acc, patches, patches1, (E *)g.C + (long)b * g.sC, g.ldc, g.beta,
-                         g.ldc % EPV == 0 && g.sC % EPV == 0 && ((size_t)g.C & 15) == 0, g.N, o, crow, (const E *)g.bias, g.relu != 0);
+                         g.ldc % EPV == 0 && g.sC % EPV == 0 && ((size_t)g.C & 15) == 0, g.N, o, crow, (const E *)g.bias, g.relu != 0,
+                         ES == 2 && g.round_first != 0);
     if (g.phase_rec) {
         __builtin_amdgcn_s_waitcnt(0x0f70);  // this wave's stores have been acknowledged
         st_w[3] = wall_clock64();
@@ -677,9 +749,9 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     }
 }
 
-// TAIL: K is not a multiple of the K step (an instantiation of its own, so that the per-piece offsets of the
-// ordinary case stay constants; patch k-rows as B need none)
-template <typename T, bool TAIL = false>
+// (EDGE: instantiations of their own, so that the per-piece offsets of the ordinary case stay constants; patch k-rows as B
+// need none)
+template <typename T, int EDGE = EDGE_NONE>
 __global__ __launch_bounds__(T::NT) void gemm_tiled_kernel(GemmArgs g, int tilesM, int tilesN) {
     typedef typename T::E E;
     // four separate arrays, so that reads of one half are known not to touch the other
@@ -687,7 +759,7 @@ __global__ __launch_bounds__(T::NT) void gemm_tiled_kernel(GemmArgs g, int tiles
     __shared__ __attribute__((aligned(16))) E As1[T::A_SZ];
     __shared__ __attribute__((aligned(16))) E Bs0[T::B_SZ];
     __shared__ __attribute__((aligned(16))) E Bs1[T::B_SZ];
-    gemm_tiled_body<T, TAIL>(g, tilesM, tilesN, (int)blockIdx.x, (int)blockIdx.z, (int)gridDim.x, As0, As1, Bs0, Bs1);
+    gemm_tiled_body<T, EDGE>(g, tilesM, tilesN, (int)blockIdx.x, (int)blockIdx.z, (int)gridDim.x, As0, As1, Bs0, Bs1);
 }
 
 // Two products in one launch: the first nx0 * nz0 workgroups are the first product's grid (x fastest), the rest the
@@ -707,10 +779,10 @@ __global__ __launch_bounds__(T0::NT) void gemm_tiled_pair_kernel(GemmArgs g0, Ge
     __shared__ __attribute__((aligned(16))) E Bs1[B_SZ];
     const int id = (int)blockIdx.x, first = nx0 * nz0;
     if (id < first) {
-        gemm_tiled_body<T0, false>(g0, tilesM0, tilesN0, id % nx0, id / nx0, nx0, As0, As1, Bs0, Bs1);
+        gemm_tiled_body<T0, EDGE_NONE>(g0, tilesM0, tilesN0, id % nx0, id / nx0, nx0, As0, As1, Bs0, Bs1);
     } else {
         const int j = id - first;
-        gemm_tiled_body<T1, false>(g1, tilesM1, tilesN1, j % nx1, j / nx1, nx1, As0, As1, Bs0, Bs1);
+        gemm_tiled_body<T1, EDGE_NONE>(g1, tilesM1, tilesN1, j % nx1, j / nx1, nx1, As0, As1, Bs0, Bs1);
     }
 }
 
@@ -728,21 +800,31 @@ int gemm_tiled_patch_f32(const GemmArgs &g, int transB, hipStream_t stream);
 // Which tile a product runs on.
 enum TileId { TILE_WIDE, TILE_256, TILE_128x64, TILE_64x64, TILE_64x128, TILE_128x128 };
 
+// Whether both operands of a product of real matrices can be moved in 16-byte pieces that K does not cut (else EDGE_ANY).
+template <typename E>
+static bool in_pieces(const GemmArgs &g, bool a_kc, bool b_kc) {
+    constexpr int EPV = 16 / (int)sizeof(E), BK = 128 / (int)sizeof(E);
+    if ((g.lda | g.ldb) % EPV || (g.sA | g.sB) % EPV || (((size_t)g.A | (size_t)g.B) & 15)) return false;
+    if ((a_kc || b_kc) && g.K % BK && g.K % EPV) return false;
+    return (a_kc || g.M % EPV == 0) && (b_kc || g.N % EPV == 0);
+}
+
 template <typename E, bool A_KC, bool B_KC, int VIRT = VIRT_NONE>
-static TileId choose_tile(const GemmArgs &g) {
+static TileId choose_tile(const GemmArgs &g, bool any = false) {
     static const char *force = getenv("D8_GEMM_TILE");  // tuning aid
     const long big_tiles = (long)ceil_div(g.M, 256) * ceil_div(g.N, 256) * g.batch * g.splits;
     bool big = g.M >= 256 && g.N >= 256 && big_tiles >= (long)cu_count() * 3 / 4;
     if (force && g.M >= 256 && g.N >= 256) big = atoi(force) != 128;
     // fp32 runs 64-cycle MFMAs on a quarter of the bytes per flop: the 128 x 128 tile already
     // keeps the matrix pipe fed, and the compiler cannot hold the 256 x 256 variant in registers
+    if (any) big = false;  // (and rows that start anywhere have no kernel of 256 x 256 tiles)
     if constexpr (sizeof(E) == 2) {
         static const char *wide = getenv("D8_GEMM_WIDE");  // tuning aid: 0 keeps the 32x32x16 kernel
         if (big && VIRT == VIRT_NONE && !(wide && atoi(wide) == 0) && gemm_wide_eligible(g, !A_KC, B_KC)) return TILE_WIDE;
         if (big) return TILE_256;
     }
-    // a filter gradient smaller than a tile both ways (few channels, few taps)
-    if (VIRT == VIRT_B_KROWS && g.M < 128 && g.N < 128) return TILE_64x64;
+    // an output smaller than a tile both ways (a filter gradient of few channels and taps)
+    if ((VIRT == VIRT_B_KROWS || any) && g.M < 128 && g.N < 128) return TILE_64x64;
     // a 64-wide side gets a tile of that width (im2col products with 64 output channels)
     if (g.N < 128) return TILE_128x64;
     // a patch-matrix product whose last 128-column tile would be at most half full: 64 x 64 tiles, no padding

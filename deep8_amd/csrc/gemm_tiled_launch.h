@@ -8,7 +8,7 @@
 namespace d8 {
 
 template <typename E, int BM, int BN, int WGM, int WGN, bool A_KC, bool B_KC, int VIRT>
-static int launch_tiled(const GemmArgs &g0, hipStream_t stream) {
+static int launch_tiled(const GemmArgs &g0, hipStream_t stream, bool any = false) {
     GemmArgs g = g0;
     typedef Tile<E, BM, BN, WGM, WGN, A_KC, B_KC, VIRT> T;
     const bool tail = g.tail_splits > 0;  // (gemm_tiled_run sets it only for 128-row tiles and a tail_m0 that is a multiple of them)
@@ -22,29 +22,34 @@ static int launch_tiled(const GemmArgs &g0, hipStream_t stream) {
     const unsigned pad = (lds <= third && wgs > cus && wgs <= 2 * cus) ? (unsigned)(third + 512 - lds) : 0u;
     // a launch whose records would not fit the caller's buffer writes none
     g.phase_rec = (size_t)(tilesM * tilesN + extra) * layers * 64 <= phase_rec_bytes ? phase_rec_buf : nullptr;
-    if (VIRT != VIRT_B_KROWS && g.K % T::BK)
-        hipLaunchKernelGGL((gemm_tiled_kernel<T, VIRT != VIRT_B_KROWS>), dim3(tilesM * tilesN + extra, 1, layers), dim3(T::NT), pad, stream, g, tilesM, tilesN);
+    const dim3 grid(tilesM * tilesN + extra, 1, layers);
+    constexpr int ANY = VIRT == VIRT_NONE && BM <= 128 ? EDGE_ANY : EDGE_NONE, PIECES = VIRT != VIRT_B_KROWS ? EDGE_PIECES : EDGE_NONE;
+    if (ANY == EDGE_ANY && any)
+        hipLaunchKernelGGL((gemm_tiled_kernel<T, ANY>), grid, dim3(T::NT), pad, stream, g, tilesM, tilesN);
+    else if (VIRT != VIRT_B_KROWS && g.K % T::BK)
+        hipLaunchKernelGGL((gemm_tiled_kernel<T, PIECES>), grid, dim3(T::NT), pad, stream, g, tilesM, tilesN);
     else
-        hipLaunchKernelGGL((gemm_tiled_kernel<T, false>), dim3(tilesM * tilesN + extra, 1, layers), dim3(T::NT), pad, stream, g, tilesM, tilesN);
+        hipLaunchKernelGGL((gemm_tiled_kernel<T, EDGE_NONE>), grid, dim3(T::NT), pad, stream, g, tilesM, tilesN);
     D8_LAUNCH_CHECK();
     return 0;
 }
 
 template <typename E, bool A_KC, bool B_KC, int VIRT = VIRT_NONE>
 static int pick_tile(const GemmArgs &g, hipStream_t stream) {
-    switch (choose_tile<E, A_KC, B_KC, VIRT>(g)) {
+    const bool any = VIRT == VIRT_NONE && !in_pieces<E>(g, A_KC, B_KC);
+    switch (choose_tile<E, A_KC, B_KC, VIRT>(g, any)) {
         case TILE_WIDE: return gemm_wide_launch(g, !A_KC, B_KC, stream);
         case TILE_256:
             if constexpr (sizeof(E) == 2) return launch_tiled<E, 256, 256, 4, 2, A_KC, B_KC, VIRT>(g, stream);
             break;
-        case TILE_128x64: return launch_tiled<E, 128, 64, 2, 2, A_KC, B_KC, VIRT>(g, stream);
+        case TILE_128x64: return launch_tiled<E, 128, 64, 2, 2, A_KC, B_KC, VIRT>(g, stream, any);
         case TILE_64x64:
-            if constexpr (VIRT == VIRT_B_KROWS) return launch_tiled<E, 64, 64, 2, 2, A_KC, B_KC, VIRT>(g, stream);
+            if constexpr (VIRT == VIRT_B_KROWS || VIRT == VIRT_NONE) return launch_tiled<E, 64, 64, 2, 2, A_KC, B_KC, VIRT>(g, stream, any);
             break;
-        case TILE_64x128: return launch_tiled<E, 64, 128, 2, 2, A_KC, B_KC, VIRT>(g, stream);
+        case TILE_64x128: return launch_tiled<E, 64, 128, 2, 2, A_KC, B_KC, VIRT>(g, stream, any);
         default: break;
     }
-    return launch_tiled<E, 128, 128, 2, 2, A_KC, B_KC, VIRT>(g, stream);
+    return launch_tiled<E, 128, 128, 2, 2, A_KC, B_KC, VIRT>(g, stream, any);
 }
 
 // Real matrices as both operands.

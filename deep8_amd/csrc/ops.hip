@@ -60,6 +60,7 @@ static int run_bias_relu(int dtype, const Gemm &p, const void *bias, int relu, v
     if (bias || relu) {
         GemmArgs g = to_args(p);
         g.bias = bias, g.relu = relu;
+        g.round_first = !gemm_fuses_store(dtype, g, p.ta, p.tb, TILED_PIECES);
         if (gemm_fuses_store(dtype, g, p.ta, p.tb)) return gemm_run_fused(dtype, g, p.ta, p.tb, ws, ws_bytes, as_stream(stream));
     }
     if (int rc = run(dtype, p, ws, ws_bytes, stream)) return rc;
@@ -138,7 +139,7 @@ static unsigned magic_of(unsigned d) { return d <= 1 ? 0xFFFFFFFFu : (unsigned)(
 // whole K steps and whole tiles: where a channel count leaves a partial step in every filter tap, or an output is smaller
 // than a tile, the query keeps asking for the interim matrix, and the call uses what it needs of that for its split.
 static bool implicit_eligible(int dtype, const GemmArgs &g, int ta, int tb) {
-    return dtype == D8_FLOAT64 ? true : gemm_tiled_eligible(dtype, g, ta, tb, g.A == nullptr);
+    return dtype == D8_FLOAT64 ? true : gemm_tiled_eligible(dtype, g, ta, tb, g.A ? TILED_ANY : TILED_WHOLE);
 }
 // Workspace such a product may use (the split of its reduction).
 static size_t implicit_workspace(int dtype, const GemmArgs &g) {
@@ -494,6 +495,8 @@ static int conv2d_impl(int dtype, const void *x, int B, int IH, int IW, int IC,
         int ta, tb;
         if (conv_implicit_plan(dtype, 0, cs, x, w, z, ga, ta, tb)) {
             ga.bias = bias, ga.relu = relu;  // applied in the tile store (and in the remainder band's reduction)
+            ga.round_first = !gemm_tiled_eligible(dtype, ga, ta, tb, TILED_WHOLE) &&
+                             !gemm_fuses_store(dtype, to_args(conv_plan(0, M, K, OC, nullptr, w, z)), 0, 1, TILED_PIECES);
             return implicit_run(dtype, ga, ta, tb, scratch, scratch_bytes, as_stream(stream));
         }
     }
