@@ -1,0 +1,580 @@
+// Conv2d on an image of few channels (a network's first layer: 1 or 3 channels), forward and filter gradient.
+//
+// The patch rows of such an image (25, 27, 75, 147 elements) cannot be cut into 16-byte pieces of one tap's channels, which is
+// what the tiled GEMM's patch loader fetches, and writing the patch matrix out moves the image FH * FW / stride^2 times.
+// What a filter row covers is contiguous, though: FW * C elements of one image row.  A workgroup therefore keeps the image
+// rows under a TR x TC block of output pixels in LDS, with zeros where they leave the image, and the matrix instructions'
+// operands are read straight from there:
+//   forward   D[oc][pixel] = w[oc][k] . patch[k][pixel]: k runs over FH runs of FW * C elements, each filled up to P pieces of
+//             16 bytes.  The filter stays in registers (one fragment per pair of pieces), a patch fragment is 16 bytes at
+//             pixel + run + piece, and what a run's last piece brings in from behind the run is cut off (not merely met by a
+//             zero weight: it may be an infinity).  Channels are D's rows, so a lane holds four consecutive channels of a
+//             pixel; in half two lanes exchange halves and store 16 bytes each.
+//   gradient  D[oc][n] = dz^T[oc][pixel] . patch[pixel][n], n = (fy, fx, c) unpadded: a wave owns 32 n, a lane one n and 8 (4
+//             in fp32) consecutive pixels of a row, i.e. strided single elements; dz is staged beside the image and read
+//             transposed.  Waves beyond the n blocks take every other group of pixels and meet in LDS, workgroups leave
+//             partial sums that conv_direct_reduce_kernel adds in a fixed order.
+#include "conv_direct.h"
+#include "gemm_tiled_kernel.h"
+
+namespace d8 {
+
+namespace {
+
+struct DirectArgs {
+    DirectShape s;
+    const void *x, *w, *bias;
+    void *z;
+    float *ws;
+    int relu, round_first;
+    int K, run, P;              // FH * FW * C; FW * C; 16-byte pieces of a run
+    int TR, TC, TCp;            // tile of output pixels; TC rounded up to what a lane's fragment covers
+    int tiles_y, tiles_x, ntiles;
+    int rows, pitch;            // image rows of a tile, and elements an image row takes in LDS
+    int vec_x, vec_z;           // elements a staging access of the image / of z moves
+    unsigned mg_chunks, mg_tc;  // ceil(2^32 / (pitch / vec_x)), ceil(2^32 / TC or TCp)
+    int kb, pixels_p;           // gradient: blocks of 32 n; pixels of a tile with its rows filled up, a multiple of a k group
+};
+
+// quotient by multiplication: exact for n, d < 2^16
+__device__ __forceinline__ int quotient(int n, unsigned magic, int d) { return d == 1 ? n : (int)__umulhi((unsigned)n, magic); }
+
+struct TileAt {
+    int b, oy0, ox0, first, skip;  // first: image column (in elements) LDS column 0 holds; skip: LDS column of the tile's first patch
+};
+
+__device__ __forceinline__ TileAt tile_at(const DirectArgs &a, int t) {
+    TileAt r;
+    const int plane = a.tiles_y * a.tiles_x;
+    r.b = t / plane;
+    t -= r.b * plane;
+    r.oy0 = t / a.tiles_x;
+    r.ox0 = (t - r.oy0 * a.tiles_x) * a.TC;
+    r.oy0 *= a.TR;
+    const int lead = (r.ox0 * a.s.sx - a.s.pl) * a.s.C;
+    r.skip = lead & (a.vec_x - 1);  // (vec_x is a power of two)
+    r.first = lead - r.skip;
+    return r;
+}
+
+// Piece `idx` of the tile's image rows: where it lies in LDS, and its elements (zeros outside the image: a piece lies
+// inside or outside as a whole, because a row's length and `first` are multiples of it)
+template <typename E, typename V>
+__device__ __forceinline__ V image_piece(const DirectArgs &a, const TileAt &t, int idx, int total, int &dst) {
+    constexpr int N = sizeof(V) / sizeof(E);
+    const int per_row = a.pitch / N, r = quotient(idx, a.mg_chunks, per_row), col = (idx - r * per_row) * N;
+    dst = r * a.pitch + col;
+    const int iy = t.oy0 * a.s.sy - a.s.pt + r, el = t.first + col, row = a.s.IW * a.s.C;
+    V v = {};
+    if (idx < total && (unsigned)iy < (unsigned)a.s.IH && el >= 0 && el < row)
+        v = *(const V *)((const E *)a.x + ((long)t.b * a.s.IH + iy) * row + el);
+    return v;
+}
+
+template <typename E, typename V>
+__device__ __forceinline__ void stage_image_as(const DirectArgs &a, const TileAt &t, E *img) {
+    constexpr int N = sizeof(V) / sizeof(E), AHEAD = 4;
+    const int total = a.rows * (a.pitch / N);
+    for (int i = threadIdx.x; i < total; i += AHEAD * blockDim.x) {
+        V v[AHEAD];
+        int dst[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) v[u] = image_piece<E, V>(a, t, i + u * blockDim.x, total, dst[u]);
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u)
+            if (i + u * (int)blockDim.x < total) *(V *)(img + dst[u]) = v[u];
+    }
+}
+
+template <typename E>
+__device__ __forceinline__ void stage_image(const DirectArgs &a, const TileAt &t, E *img) {
+    if (a.vec_x * sizeof(E) == 16) stage_image_as<E, u32x4>(a, t, img);
+    else if (sizeof(E) == 4 || a.vec_x == 2) stage_image_as<E, unsigned>(a, t, img);
+    else stage_image_as<E, E>(a, t, img);
+}
+
+// 16 bytes from any element of LDS
+template <typename E, bool ODD>
+__device__ __forceinline__ u32x4 piece_at(const E *lds, int el) {
+    u32x4 v;
+    if constexpr (sizeof(E) == 4) {
+        const unsigned *p = (const unsigned *)lds + el;
+        v[0] = p[0], v[1] = p[1], v[2] = p[2], v[3] = p[3];
+    } else {
+        const unsigned *p = (const unsigned *)lds + (el >> 1);
+        v[0] = p[0], v[1] = p[1], v[2] = p[2], v[3] = p[3];
+        if constexpr (ODD) {
+            const unsigned x = p[4], shift = (el & 1) * 16;
+            v[0] = __builtin_amdgcn_alignbit(v[1], v[0], shift), v[1] = __builtin_amdgcn_alignbit(v[2], v[1], shift);
+            v[2] = __builtin_amdgcn_alignbit(v[3], v[2], shift), v[3] = __builtin_amdgcn_alignbit(x, v[3], shift);
+        }
+    }
+    return v;
+}
+
+// the bits of dword d of a piece whose first n elements count
+template <typename E>
+__device__ __forceinline__ unsigned first_mask(int n, int d) {
+    if constexpr (sizeof(E) == 4) return n > d ? 0xffffffffu : 0u;
+    else return n > 2 * d + 1 ? 0xffffffffu : n > 2 * d ? 0xffffu : 0u;
+}
+
+}  // namespace
+
+// G: k groups (pairs of pieces) a wave keeps of the filter; NB: blocks of 32 channels per workgroup; ODD: half patches may
+// start in the middle of a dword.  A workgroup walks every gridDim.x-th tile, its four waves every fourth block of 32 pixels.
+// Bound by the store of z and the latency of a tile's image rows, which two workgroups per compute unit hide from each
+// other; figures at conv_direct_forward.
+template <typename E, int G, int NB, bool ODD>
+__global__ __launch_bounds__(256) void conv_direct_forward_kernel(DirectArgs a) {
+    typedef Elem<E> EL;
+    typedef typename EL::Frag Frag;
+    constexpr int EPV = 16 / sizeof(E);
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds_bytes[];
+    __shared__ float bias_s[NB * 32];
+    E *lds = (E *)lds_bytes;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, half = lane >> 5;
+    const int oc0 = blockIdx.y * (NB * 32), ocs = min(NB * 32, a.s.OC - oc0);
+
+    // ---- the filter: through LDS (rows of K elements, as they lie in memory) into fragments; rows past OC and pieces past
+    // the last run are zeros
+    {
+        const E *w = (const E *)a.w + (long)oc0 * a.K;
+        const int n = ocs * a.K;
+        if (((size_t)w & 15) == 0) {
+            for (int i = threadIdx.x * EPV; i + EPV <= n; i += 256 * EPV) *(u32x4 *)(lds + i) = *(const u32x4 *)(w + i);
+            for (int i = n / EPV * EPV + threadIdx.x; i < n; i += 256) lds[i] = w[i];
+        } else {
+            for (int i = threadIdx.x; i < n; i += 256) lds[i] = w[i];
+        }
+        if (threadIdx.x < NB * 32) bias_s[threadIdx.x] = a.bias && (int)threadIdx.x < ocs ? (float)((const E *)a.bias)[oc0 + threadIdx.x] : 0.f;
+    }
+    __syncthreads();
+    Frag wf[NB][G];
+    int koff[G];              // element offset of this lane's piece of each group from its pixel's first element
+    unsigned some[G], all[G];  // all ones: the piece has elements of the patch (may be a run's last one) / only such
+    const int tail = a.run - (a.P - 1) * EPV;  // elements of a run's last piece
+    unsigned tail_mask[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) tail_mask[d] = first_mask<E>(tail, d);
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        const int p = 2 * g + half, fy = p / a.P, j = p - fy * a.P;
+        const bool in = fy < a.s.FH, last = j == a.P - 1;
+        koff[g] = in ? fy * a.s.dy * a.pitch + j * EPV : 0;
+        some[g] = in ? 0xffffffffu : 0u;
+        all[g] = in && !last ? 0xffffffffu : 0u;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            const int oc = nb * 32 + l32;
+            u32x4 v = piece_at<E, true>(lds, in && oc < ocs ? oc * a.K + fy * a.run + j * EPV : 0);
+#pragma unroll
+            for (int d = 0; d < 4; ++d) v[d] &= oc < ocs ? (tail_mask[d] & some[g]) | all[g] : 0u;
+            wf[nb][g] = __builtin_bit_cast(Frag, v);
+        }
+    }
+
+    const int blocks = (a.TR * a.TC + 31) / 32;
+    const bool vec = a.s.OC % EPV == 0 && ((size_t)a.z & 15) == 0;
+    for (int t = blockIdx.x; t < a.ntiles; t += gridDim.x) {
+        const TileAt at = tile_at(a, t);
+        __syncthreads();  // the filter's fragments have been read; every wave is done with the tile before
+        stage_image<E>(a, at, lds);
+        __syncthreads();
+        for (int blk = wave; blk < blocks; blk += 4) {
+            const int q = blk * 32 + l32, qc = min(q, a.TR * a.TC - 1), r = quotient(qc, a.mg_tc, a.TC), c = qc - r * a.TC;
+            const int base = r * a.s.sy * a.pitch + c * a.s.sx * a.s.C + at.skip;
+            f32x16 acc[NB];
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[nb][i] = 0.f;
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                u32x4 v = piece_at<E, ODD>(lds, base + koff[g]);
+#pragma unroll
+                for (int d = 0; d < 4; ++d) v[d] &= (tail_mask[d] & some[g]) | all[g];
+                const Frag f = __builtin_bit_cast(Frag, v);
+#pragma unroll
+                for (int e = 0; e < EL::MFMA_PER_FRAG; ++e)
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb) acc[nb] = EL::mfma(wf[nb][g], f, acc[nb], e);
+            }
+            const int oy = at.oy0 + r, ox = at.ox0 + c;
+            const bool mine = q < a.TR * a.TC && oy < a.s.OH && ox < a.s.OW;
+            E *z = (E *)a.z + (((long)at.b * a.s.OH + oy) * a.s.OW + ox) * a.s.OC + oc0;
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                // register i of the block is channel 8 * (i / 4) + 4 * half + i % 4 of this lane's pixel
+                E o[16];
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    float v = acc[nb][i];
+                    if (a.bias) v = (sizeof(E) == 2 && a.round_first ? (float)(E)v : v) + bias_s[nb * 32 + 8 * (i >> 2) + 4 * half + (i & 3)];
+                    o[i] = (E)(a.relu && !(v > 0.f) ? 0.f : v);
+                }
+                if (vec) {
+                    if constexpr (sizeof(E) == 4) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const int n = nb * 32 + 8 * i + 4 * half;
+                            if (mine && n < ocs) *(f32x4 *)(z + n) = (f32x4){(float)o[4 * i], (float)o[4 * i + 1], (float)o[4 * i + 2], (float)o[4 * i + 3]};
+                        }
+                    } else {
+                        // the lower half of the wave takes channels 16 i .. + 7 of its pixel, the upper 16 i + 8 .. + 15
+#pragma unroll
+                        for (int i = 0; i < 2; ++i) {
+                            u32x4 out;
+#pragma unroll
+                            for (int d = 0; d < 2; ++d) {
+                                const f16x2 lo = {(f16)o[8 * i + 2 * d], (f16)o[8 * i + 2 * d + 1]}, hi = {(f16)o[8 * i + 4 + 2 * d], (f16)o[8 * i + 5 + 2 * d]};
+                                const auto s = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, lo), __builtin_bit_cast(unsigned, hi), false, false);
+                                out[d] = s[0], out[d + 2] = s[1];
+                            }
+                            const int n = nb * 32 + 16 * i + 8 * half;
+                            if (mine && n < ocs) *(u32x4 *)(z + n) = out;
+                        }
+                    }
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        const int n = nb * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
+                        if (mine && n < ocs) z[n] = o[i];
+                    }
+                }
+            }
+        }
+    }
+}
+
+// Filter gradient.  blockDim = 64 * kb * (a power of two of waves that share the pixels of a tile).  The next tile's image
+// rows and dz are fetched into registers while the present one is multiplied (where both move in 16-byte pieces and fit).
+// Bound by the LDS reads of single patch elements (8 per 32 x 32 x 16 block in half) and the first tile's way from memory.
+template <typename E, int NB>
+__global__ __launch_bounds__(768) void conv_direct_grad_kernel(DirectArgs a) {
+    typedef Elem<E> EL;
+    typedef typename EL::Frag Frag;
+    constexpr int EPV = 16 / sizeof(E);
+    constexpr int LD = NB * 32 + (sizeof(E) == 4 ? 8 : NB == 2 ? 32 : 16);  // elements a pixel's channels take in LDS
+    constexpr int PARTS = NB * 32 / EPV, IMG_AHEAD = 3, DZ_AHEAD = 4;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds_bytes[];
+    E *dzs = (E *)lds_bytes, *img = dzs + a.pixels_p * LD;
+    const int nt = blockDim.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, half = lane >> 5;
+    const int sharers = (nt >> 6) / a.kb, kb = wave % a.kb, ps = wave / a.kb;
+    const int oc0 = blockIdx.y * (NB * 32), ocs = min(NB * 32, a.s.OC - oc0);
+    const int n = kb * 32 + l32, fy = n / a.run;
+    const int noff = n < a.K ? fy * a.s.dy * a.pitch + (n - fy * a.run) : 0;
+    const int step = a.s.sx * a.s.C;
+    const E *gz = (const E *)a.w;
+    const int img_total = a.rows * (a.pitch / EPV), dz_total = a.pixels_p * PARTS;
+    const bool ahead = a.vec_x == EPV && a.vec_z == EPV && img_total <= IMG_AHEAD * nt && dz_total <= DZ_AHEAD * nt;
+
+    // piece idx of dz: PARTS pieces per pixel, zeros for the pixels that fill a row up or lie outside z
+    auto dz_at = [&](const TileAt &t, int px, int ch, const E *&src) -> bool {
+        const int r = quotient(px, a.mg_tc, a.TCp), c = px - r * a.TCp, oy = t.oy0 + r, ox = t.ox0 + c;
+        src = gz + (((long)t.b * a.s.OH + oy) * a.s.OW + ox) * a.s.OC + oc0 + ch;
+        return r < a.TR && c < a.TC && oy < a.s.OH && ox < a.s.OW && ch < ocs;
+    };
+    u32x4 ri[IMG_AHEAD], rd[DZ_AHEAD];
+    auto fetch = [&](const TileAt &t) {
+#pragma unroll
+        for (int u = 0; u < IMG_AHEAD; ++u) {
+            int dst;
+            ri[u] = image_piece<E, u32x4>(a, t, tid + u * nt, img_total, dst);
+        }
+#pragma unroll
+        for (int u = 0; u < DZ_AHEAD; ++u) {
+            const int i = tid + u * nt;
+            const E *src;
+            rd[u] = (u32x4){0, 0, 0, 0};
+            if (i < dz_total && dz_at(t, i / PARTS, i % PARTS * EPV, src)) rd[u] = *(const u32x4 *)src;
+        }
+    };
+    auto put = [&](const TileAt &t) {
+#pragma unroll
+        for (int u = 0; u < IMG_AHEAD; ++u) {
+            const int i = tid + u * nt, per_row = a.pitch / EPV, r = quotient(i, a.mg_chunks, per_row);
+            if (i < img_total) *(u32x4 *)(img + r * a.pitch + (i - r * per_row) * EPV) = ri[u];
+        }
+#pragma unroll
+        for (int u = 0; u < DZ_AHEAD; ++u) {
+            const int i = tid + u * nt;
+            if (i < dz_total) *(u32x4 *)(dzs + i / PARTS * LD + i % PARTS * EPV) = rd[u];
+        }
+    };
+
+    f32x16 acc[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[nb][i] = 0.f;
+
+    TileAt at = tile_at(a, blockIdx.x);  // (the grid has no more workgroups than there are tiles)
+    if (ahead) fetch(at);
+    for (int t = blockIdx.x; t < a.ntiles; t += gridDim.x) {
+        __syncthreads();
+        if (ahead) {
+            put(at);
+        } else {
+            stage_image<E>(a, at, img);
+            if (a.vec_z == EPV) {
+                for (int i = tid; i < dz_total; i += nt) {
+                    const E *src;
+                    u32x4 v = {0, 0, 0, 0};
+                    if (dz_at(at, i / PARTS, i % PARTS * EPV, src)) v = *(const u32x4 *)src;
+                    *(u32x4 *)(dzs + i / PARTS * LD + i % PARTS * EPV) = v;
+                }
+            } else {
+                for (int i = tid; i < a.pixels_p * (NB * 32); i += nt) {
+                    const E *src;
+                    const int px = i / (NB * 32), ch = i % (NB * 32);
+                    dzs[px * LD + ch] = dz_at(at, px, ch, src) ? *src : (E)0.f;
+                }
+            }
+        }
+        __syncthreads();
+        const int skip = at.skip, rows_here = min(a.TR, a.s.OH - at.oy0), cols_here = min(a.TC, a.s.OW - at.ox0);
+        if (t + (int)gridDim.x < a.ntiles) {
+            at = tile_at(a, t + gridDim.x);
+            if (ahead) fetch(at);
+        }
+        for (int g = ps; g < a.pixels_p / (2 * EPV); g += sharers) {
+            // this lane's EPV pixels: consecutive ones of a tile row (rows are filled up to a multiple of EPV)
+            const int q = (2 * g + half) * EPV, r = quotient(q, a.mg_tc, a.TCp), c = q - r * a.TCp;
+            const int valid = r < rows_here ? cols_here - c : 0;
+            const E *p = img + (r < a.TR ? r * a.s.sy * a.pitch + c * step + skip : 0) + noff;
+            Frag b;
+            if constexpr (sizeof(E) == 4) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) b[e] = p[r < a.TR ? e * step : 0];
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) b[e] = p[r < a.TR ? e * step : 0];
+            }
+            u32x4 v = __builtin_bit_cast(u32x4, b);
+#pragma unroll
+            for (int d = 0; d < 4; ++d) v[d] &= first_mask<E>(valid, d);
+            b = __builtin_bit_cast(Frag, v);
+            Frag fa[NB];
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) fa[nb] = EL::read_tr(dzs + 2 * g * EPV * LD + EL::tr_offset(lane, LD, nb * 32), LD);
+#pragma unroll
+            for (int e = 0; e < EL::MFMA_PER_FRAG; ++e)
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) acc[nb] = EL::mfma(fa[nb], b, acc[nb], e);
+        }
+    }
+
+    // ---- the waves that shared the pixels of an n block meet: the upper half hands its sums to the lower until one is left
+    float *meet = (float *)lds_bytes;
+    for (int s = sharers >> 1; s >= 1; s >>= 1) {
+        __syncthreads();
+        if (ps >= s && ps < 2 * s) {
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) meet[(((ps - s) * a.kb + kb) * (NB * 16) + nb * 16 + i) * 64 + lane] = acc[nb][i];
+        }
+        __syncthreads();
+        if (ps < s) {
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[nb][i] += meet[((ps * a.kb + kb) * (NB * 16) + nb * 16 + i) * 64 + lane];
+        }
+    }
+    if (ps == 0 && n < a.K) {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int oc = nb * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
+                if (oc < ocs) a.ws[((long)blockIdx.x * a.s.OC + oc0 + oc) * a.K + n] = acc[nb][i];
+            }
+    }
+}
+
+// gw[i] = beta * gw[i] + the sum of `parts` partial sums ws[.][i]: 64 outputs per workgroup, 16 waves that take every
+// sixteenth part each (four loads in flight) and meet in LDS in wave order.
+template <typename E>
+__global__ __launch_bounds__(1024) void conv_direct_reduce_kernel(const float *ws, E *gw, int n, int parts, float beta) {
+    __shared__ float met[16][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = blockIdx.x * 64 + lane;
+    float sum[4] = {0.f, 0.f, 0.f, 0.f};
+    if (i < n) {
+        int p = wave;
+        for (; p + 48 < parts; p += 64)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) sum[u] += ws[(long)(p + 16 * u) * n + i];
+        for (; p < parts; p += 16) sum[0] += ws[(long)p * n + i];
+    }
+    met[wave][lane] = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+    __syncthreads();
+    if (wave == 0 && i < n) {
+        float v = 0.f;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) v += met[w][lane];
+        if (beta != 0.f) v += (float)gw[i];
+        gw[i] = (E)v;
+    }
+}
+
+// ---- host ------------------------------------------------------------------------------------------------------------
+namespace {
+
+constexpr int LDS_LIMIT = 64 * 1024;
+
+unsigned magic_up(int d) { return d == 1 ? 0u : (unsigned)(((1UL << 32) + d - 1) / d); }
+
+int pieces_of(int dtype, const DirectShape &s) {
+    const int epv = 16 / (int)dtype_bytes(dtype);
+    return s.FH * ceil_div((long)s.FW * s.C, epv);
+}
+int most_groups(int dtype) { return dtype == D8_FLOAT16 ? 11 : 21; }
+
+// Everything of a launch but the pointers.  `grain`: pixels a tile row is filled up to (1 forward, a fragment's for the
+// gradient); `pixels`: how many a tile may have; `px_bytes`: LDS of a pixel besides the image.  False where no tile fits.
+bool plan_tiles(int dtype, const DirectShape &s, const void *x, int grain, int pixels, int px_bytes, int min_bytes, DirectArgs &a, size_t &lds) {
+    const int es = (int)dtype_bytes(dtype), epv = 16 / es;
+    memset(&a, 0, sizeof(a));
+    a.s = s, a.x = x;
+    a.run = s.FW * s.C, a.K = s.FH * a.run, a.P = ceil_div(a.run, epv);
+    const long row = (long)s.IW * s.C;
+    a.vec_x = row % epv == 0 && ((size_t)x & 15) == 0 ? epv : es == 2 && row % 2 == 0 && ((size_t)x & 3) == 0 ? 2 : 1;
+    a.TC = ceil_div(s.OW, ceil_div(s.OW, pixels));
+    a.TR = 1;
+    auto fits = [&](int TR, int TC) {
+        const int TCp = ceil_div(TC, grain) * grain, k_group = grain > 1 ? 2 * grain : 1;
+        const long px = (long)ceil_div((long)TR * TCp, k_group) * k_group;
+        const long rows = (long)(TR - 1) * s.sy + (long)(s.FH - 1) * s.dy + 1;
+        // the last pixel's pieces, the part of a staging access before the first, and a dword for the odd start
+        long pitch = (long)(TCp - 1) * s.sx * s.C + (long)a.P * epv + (a.vec_x - 1) + 2;
+        const int unit = a.vec_x > 2 / es ? a.vec_x : 2;
+        pitch = (pitch + unit - 1) / unit * unit;
+        const long bytes = ((rows * pitch * es + 15) & ~15L) + 16 + px * px_bytes;
+        if (px > pixels + k_group || rows * pitch >= (1 << 15) || bytes > LDS_LIMIT) return false;
+        a.TR = TR, a.TC = TC, a.TCp = TCp, a.pixels_p = (int)px, a.rows = (int)rows, a.pitch = (int)pitch, lds = (size_t)bytes;
+        return true;
+    };
+    int TC = a.TC;
+    while (!fits(1, TC)) {
+        if (TC == 1) return false;
+        TC = (TC + 1) / 2;
+    }
+    TC = ceil_div(s.OW, ceil_div(s.OW, TC));
+    int TR = pixels / a.TCp;
+    TR = TR < 1 ? 1 : TR > s.OH ? s.OH : TR;
+    while (TR > 1 && !fits(TR, TC)) --TR;
+    if (!fits(ceil_div(s.OH, ceil_div(s.OH, TR)), TC)) return false;
+    a.tiles_y = ceil_div(s.OH, a.TR), a.tiles_x = ceil_div(s.OW, a.TC);
+    const long tiles = (long)s.B * a.tiles_y * a.tiles_x;
+    if (tiles >= (1L << 30)) return false;
+    a.ntiles = (int)tiles;
+    a.mg_chunks = magic_up(a.pitch / a.vec_x);
+    a.mg_tc = magic_up(grain > 1 ? a.TCp : a.TC);
+    if (lds < (size_t)min_bytes) lds = min_bytes;
+    return lds <= (size_t)LDS_LIMIT;
+}
+
+template <typename E, int G, int NB>
+int launch_forward(const DirectArgs &a, size_t lds, bool odd, hipStream_t stream) {
+    const dim3 grid((unsigned)(a.ntiles < 2 * cu_count() ? a.ntiles : 2 * cu_count()), (unsigned)ceil_div(a.s.OC, NB * 32));
+    if (sizeof(E) == 2 && odd) hipLaunchKernelGGL((conv_direct_forward_kernel<E, G, NB, sizeof(E) == 2>), grid, dim3(256), lds, stream, a);
+    else hipLaunchKernelGGL((conv_direct_forward_kernel<E, G, NB, false>), grid, dim3(256), lds, stream, a);
+    D8_LAUNCH_CHECK();
+    return 0;
+}
+
+// channels per workgroup: the filter's fragments are what fills the registers (8 dwords a group for 64 channels)
+int forward_channels(int dtype, const DirectShape &s) { return dtype == D8_FLOAT16 && s.OC > 32 ? 64 : 32; }
+
+bool plan_forward(int dtype, const DirectShape &s, const void *x, DirectArgs &a, size_t &lds) {
+    const int es = (int)dtype_bytes(dtype), filter = (forward_channels(dtype, s) * s.FH * s.FW * s.C + 8) * es + 16;
+    return plan_tiles(dtype, s, x, 1, 256, 0, filter, a, lds);
+}
+
+int grad_waves(int kb) { return kb == 1 ? 8 : kb == 2 ? 8 : kb == 3 ? 6 : 2 * kb; }
+
+bool plan_grad(int dtype, const DirectShape &s, const void *x, const void *gz, DirectArgs &a, size_t &lds) {
+    const int es = (int)dtype_bytes(dtype), epv = 16 / es, nb = s.OC > 32 ? 2 : 1, kb = ceil_div((long)s.FH * s.FW * s.C, 32);
+    if (kb > 6) return false;
+    const int ld = nb * 32 + (es == 4 ? 8 : nb == 2 ? 32 : 16), meet = grad_waves(kb) / 2 * nb * 16 * 64 * 4;
+    if (!plan_tiles(dtype, s, x, epv, es == 2 ? 224 : 128, ld * es, meet, a, lds)) return false;
+    a.kb = kb;
+    a.vec_z = s.OC % epv == 0 && ((size_t)gz & 15) == 0 ? epv : 1;
+    return true;
+}
+
+}  // namespace
+
+bool conv_direct_eligible(int dtype, const DirectShape &s) {
+    if (dtype != D8_FLOAT16 && dtype != D8_FLOAT32) return false;
+    if (s.dx != 1 || (long)s.FH * s.FW * s.C >= 4096 || pieces_of(dtype, s) > 2 * most_groups(dtype)) return false;
+    DirectArgs a;
+    size_t lds;
+    return plan_forward(dtype, s, nullptr, a, lds) && plan_grad(dtype, s, nullptr, nullptr, a, lds);
+}
+
+// Every layer of the shape qualifies: on these sizes the interim matrix lost everywhere it was measured.  Half 16 x
+// 224x224x3 -> 64, 7x7 stride 2 (K = 147): patch matrix + padded filter + product 81 -> 23 us (26 MB are stored: 5 us at a
+// copy's rate; what the rest goes on is the way of a tile's rows from memory to the first fragment); fp32 64 x 28x28x1 -> 32,
+// 5x5: patch matrix + product 18 -> 11 us.
+int conv_direct_forward(int dtype, const DirectShape &s, const void *x, const void *w, void *z, const void *bias, int relu,
+                        int round_first, hipStream_t stream) {
+    DirectArgs a;
+    size_t lds;
+    D8_REQUIRE(conv_direct_eligible(dtype, s) && plan_forward(dtype, s, x, a, lds), "conv_direct_forward: the layer does not fit");
+    a.w = w, a.z = z, a.bias = bias, a.relu = relu, a.round_first = round_first;
+    const int groups = ceil_div(pieces_of(dtype, s), 2);
+    if (dtype == D8_FLOAT32) {
+        if (groups <= 5) return launch_forward<float, 5, 1>(a, lds, false, stream);
+        if (groups <= 10) return launch_forward<float, 10, 1>(a, lds, false, stream);
+        return launch_forward<float, 21, 1>(a, lds, false, stream);
+    }
+    // every patch starts at an even element of an even pitch
+    const bool odd = (s.sx * s.C) % 2 != 0 || (s.pl * s.C) % 2 != 0;
+    if (s.OC > 32) {
+        if (groups <= 3) return launch_forward<f16, 3, 2>(a, lds, odd, stream);
+        if (groups <= 5) return launch_forward<f16, 5, 2>(a, lds, odd, stream);
+        return launch_forward<f16, 11, 2>(a, lds, odd, stream);
+    }
+    if (groups <= 3) return launch_forward<f16, 3, 1>(a, lds, odd, stream);
+    if (groups <= 5) return launch_forward<f16, 5, 1>(a, lds, odd, stream);
+    return launch_forward<f16, 11, 1>(a, lds, odd, stream);
+}
+
+// One workgroup per compute unit (10 waves for 147 columns): the partial sums are OC * K floats each, and a second workgroup
+// would double what is written and read again.  The layers above: 82 -> 28 us, 29 -> 13 us, both with the reduction.
+bool conv_direct_grad_y(int dtype, const DirectShape &s, const void *x, void *gw, const void *gz, float beta, void *ws,
+                        size_t ws_bytes, hipStream_t stream, int *rc) {
+    DirectArgs a;
+    size_t lds;
+    if (!plan_grad(dtype, s, x, gz, a, lds)) return false;
+    const int nb = s.OC > 32 ? 2 : 1, oc_tiles = ceil_div(s.OC, nb * 32);
+    const size_t one = (size_t)s.OC * a.K * sizeof(float);
+    long wgs = ceil_div(cu_count(), oc_tiles);
+    if (wgs > a.ntiles) wgs = a.ntiles;
+    if (wgs > (long)(ws_bytes / one)) wgs = (long)(ws_bytes / one);
+    if (wgs < 1 || ((size_t)ws & 3)) return false;
+    a.w = gz, a.ws = (float *)ws;
+    const dim3 grid((unsigned)wgs, (unsigned)oc_tiles), block(64 * grad_waves(a.kb));
+    if (dtype == D8_FLOAT32) {
+        if (nb == 2) hipLaunchKernelGGL((conv_direct_grad_kernel<float, 2>), grid, block, lds, stream, a);
+        else hipLaunchKernelGGL((conv_direct_grad_kernel<float, 1>), grid, block, lds, stream, a);
+    } else {
+        if (nb == 2) hipLaunchKernelGGL((conv_direct_grad_kernel<f16, 2>), grid, block, lds, stream, a);
+        else hipLaunchKernelGGL((conv_direct_grad_kernel<f16, 1>), grid, block, lds, stream, a);
+    }
+    auto launched = [&]() -> int {
+        D8_LAUNCH_CHECK();
+        return 0;
+    };
+    if ((*rc = launched())) return true;
+    const int n = s.OC * a.K;
+    if (dtype == D8_FLOAT32) hipLaunchKernelGGL((conv_direct_reduce_kernel<float>), dim3(ceil_div(n, 64)), dim3(1024), 0, stream, (const float *)ws, (float *)gw, n, (int)wgs, beta);
+    else hipLaunchKernelGGL((conv_direct_reduce_kernel<f16>), dim3(ceil_div(n, 64)), dim3(1024), 0, stream, (const float *)ws, (f16 *)gw, n, (int)wgs, beta);
+    *rc = launched();
+    return true;
+}
+
+}  // namespace d8

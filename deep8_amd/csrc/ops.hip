@@ -7,6 +7,7 @@
 //   DeConv2d         deep8/src/math/DeConv2d.cu:76-131, :371-429, :642-700, pads :99-100
 #include <atomic>
 
+#include "conv_direct.h"
 #include "conv_maps.h"
 #include "gemm_args.h"
 
@@ -454,6 +455,12 @@ static PaddedScratch conv_padded_scratch(int dtype, int which, int M, int OC, in
     return s;
 }
 
+// Layers that stage a patch matrix only because the tile loader cannot read their image (1 or 3 channels) run on the
+// kernels that read it from LDS.
+static bool conv_direct(int dtype, const DirectShape &s) {
+    return getenv("D8_CONV_EXPLICIT") == nullptr && conv_direct_eligible(dtype, s);
+}
+
 size_t d8_conv2d_scratch_bytes(int dtype, int which, int B, int IH, int IW, int IC,
                                int OC, int FH, int FW, int covered, int sy, int sx, int dy, int dx) {
     if (which == 3)  // for d8_conv2d_grad_xy: both gradients' scratch side by side (they may share a launch)
@@ -501,6 +508,15 @@ static int conv2d_impl(int dtype, const void *x, int B, int IH, int IW, int IC,
         }
     }
     if (int rc = need_scratch("d8_conv2d", scratch, scratch_bytes, (size_t)M * K * dtype_bytes(dtype), x, w, z)) return rc;
+    {
+        const DirectShape ds = {B, IH, IW, IC, OC, FH, FW, g[0], g[1], sy, sx, dy, dx, g[2], g[3]};
+        if (conv_direct(dtype, ds)) {
+            // (in half the layers whose bias used to be added by a pass of its own find the product rounded)
+            const int pitch = conv_padded_pitch(dtype, K, OC);
+            const int round_first = !gemm_fuses_store(dtype, to_args(conv_plan(0, M, pitch ? pitch : K, OC, nullptr, pitch ? nullptr : w, z)), 0, 1, TILED_PIECES);
+            return conv_direct_forward(dtype, ds, x, w, z, bias, relu, round_first, as_stream(stream));
+        }
+    }
     if (const int pitch = conv_padded_pitch(dtype, K, OC)) {
         const PaddedScratch ps = conv_padded_scratch(dtype, 0, M, OC, pitch);
         if (scratch_bytes >= ps.total && ((size_t)scratch & 15) == 0) {  // a smaller scratch still serves the plain route
@@ -603,6 +619,11 @@ static int d8_conv2d_grad_y_impl(int dtype, const void *x, int B, int IH, int IW
         }
     }
     if (int rc = need_scratch("d8_conv2d_grad_y", scratch, scratch_bytes, (size_t)M * K * dtype_bytes(dtype), x, gw, gz)) return rc;
+    {
+        const DirectShape ds = {B, IH, IW, IC, OC, FH, FW, g[0], g[1], sy, sx, dy, dx, g[2], g[3]};
+        int rc = 0;
+        if (conv_direct(dtype, ds) && conv_direct_grad_y(dtype, ds, x, gw, gz, beta, scratch, scratch_bytes, as_stream(stream), &rc)) return rc;
+    }
     if (const int pitch = conv_padded_pitch(dtype, K, OC)) {
         const PaddedScratch ps = conv_padded_scratch(dtype, 2, M, OC, pitch);
         if (scratch_bytes >= ps.total && ((size_t)scratch & 15) == 0) {
