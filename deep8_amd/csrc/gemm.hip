@@ -13,6 +13,7 @@
 // Both LDS tiles are kept K-contiguous ([row][k]), so one 16-byte LDS read feeds an MFMA
 // operand; the transposed-operand cases differ only in how the tile loader walks global memory.
 #include <atomic>
+#include <cmath>
 
 #include "gemm_args.h"
 
@@ -614,16 +615,60 @@ size_t gemm_tiled_workspace(int dtype, int M, int N, int K, int red, int virt) {
     return splits > 1 ? (size_t)splits * rows * N * sizeof(float) : 0;
 }
 
+// fp32, whose K step is bound by the matrix pipe: 64 x 64 tiles where the 128-wide ones leave compute units idle.  A step of
+// theirs is a quarter of the work and their ends are shorter, so the same pieces (or none) spread over four times as many
+// workgroups.  The estimate counts as plan_few_tiles does, in steps of a 128 x 128 tile (about 2 us of a CU), for the plan that
+// g holds (splits set) and for 64 x 64 tiles in 1 .. as many pieces as that plan; 7 % or more decide.
+// NN, us before and after (M x K x N): 512 x 512 x 512 16.4 -> 10.2, 784 x 1152 x 128 16.0 -> 10.3, 1024 x 1024 x 1024
+// 33.6 -> 23.5, 12544 x 800 x 64 24.0 -> 17.0, 3136 x 576 x 256 24.5 -> 12.7, 1536 x 1536 x 1536 76.8 -> 72.5 (NT and TN alike).  A narrow
+// output (128 x 32 tiles, below) counts its pieces the same way.
+static double tile_cost(int bm, int bn, const GemmArgs &g, long total, long s) {
+    const long cus = cu_count(), n = (ceil_div(g.M, bm) * (long)ceil_div(g.N, bn) * g.batch * s + cus - 1) / cus, len = (total + s - 1) / s;
+    const double step = bm * bn / 16384.0;
+    return n * len * step * (n == 1 ? 1.1 : 1.0) + 0.5 + 2.0 * sqrt(step) + 0.3 * (n - 1) + (s > 1 ? 2.0 + s * ((double)g.M * g.N * g.batch / 2e6) : 0.0);
+}
+
+static void few_tiles_small(GemmArgs &g, size_t usable) {
+    // (a filter gradient's pieces stay those of the launch it may share with the input's: one sum, one result)
+    if (g.virt == VIRT_A_CLASSES || g.virt == VIRT_B_KROWS || gemm_is_small(g.M, g.N, g.K, g.batch, g.red)) return;
+    if ((long)ceil_div(g.M, 128) * ceil_div(g.N, 128) * g.batch >= cu_count()) return;
+    const long total = (long)g.red * ceil_div(g.K, 32);
+    const bool half = g.splits == 1 && gemm_tiled_half_tiles(g.M, g.N, g.batch, total, 32);
+    const bool narrow = g.tile_hint == HINT_128x32;
+    const double now = narrow ? 1e30 : g.N < 128 ? tile_cost(128, 64, g, total, g.splits) : tile_cost(g.M < 128 || half ? 64 : 128, 128, g, total, g.splits);
+    long most = (long)(usable / ((size_t)g.batch * g.M * g.N * sizeof(float)));
+    int tps;  // (no more pieces than the 128-wide plan would have: what the scratch queries provide for, whatever is passed)
+    const long planned = plan_splits(32, g.M, g.N, g.K, g.batch, g.red, (size_t)-1, &tps, g.virt);
+    if (most > planned) most = planned;
+    if (most > total / 2) most = total / 2;
+    double best = 0.93 * now;
+    long pieces = 0;
+    for (long s = 1; s == 1 || s <= most; ++s)
+        if (const double c = narrow ? tile_cost(128, 32, g, total, s) : tile_cost(64, 64, g, total, s); c < best) best = c, pieces = s;
+    if (!pieces) return;
+    if (!narrow) g.tile_hint = HINT_64x64;
+    g.tiles_per_split = (int)((total + pieces - 1) / pieces);
+    g.splits = (int)((total + g.tiles_per_split - 1) / g.tiles_per_split);
+}
+
+// fp32 outputs of at most 32 columns (an input gradient of few channels): 128 x 32 tiles, because half of a 128 x 64 tile's
+// matrix instructions would multiply columns that are not there.  50000 x 288 x 32: 22.0 -> 14.3 us.
+static bool narrow_output(int dtype, const GemmArgs &g) {
+    return dtype == D8_FLOAT32 && g.N <= 32 && g.M >= 128 && (g.virt == VIRT_NONE || g.virt == VIRT_A_ROWS);
+}
+
 static int gemm_tiled_run_whole(int dtype, GemmArgs &g, int transA, int transB, void *workspace, size_t workspace_bytes,
                                 hipStream_t stream) {
     g.ws = (float *)workspace;
-    g.splits = plan_splits(gemm_tiled_k_step(dtype), g.M, g.N, g.K, g.batch, g.red, (workspace && ((size_t)workspace & 15) == 0) ? workspace_bytes : 0,
-                           &g.tiles_per_split, g.virt);
+    const size_t usable = (workspace && ((size_t)workspace & 15) == 0) ? workspace_bytes : 0;
+    g.splits = plan_splits(gemm_tiled_k_step(dtype), g.M, g.N, g.K, g.batch, g.red, usable, &g.tiles_per_split, g.virt);
+    if (dtype == D8_FLOAT32) few_tiles_small(g, usable);
     return dtype == D8_FLOAT16 ? launch<f16>(g, transA, transB, true, stream) : launch<float>(g, transA, transB, true, stream);
 }
 
 int gemm_tiled_run(int dtype, GemmArgs &g, int transA, int transB, void *workspace, size_t workspace_bytes,
                    hipStream_t stream) {
+    if (narrow_output(dtype, g)) g.tile_hint = HINT_128x32;
     static const bool no_cut = getenv("D8_GEMM_NO_ROW_CUT") != nullptr;  // tuning and test aid
     const int head = (no_cut || transA) ? 0 : balanced_rows(g);
     if (!head) return gemm_tiled_run_whole(dtype, g, transA, transB, workspace, workspace_bytes, stream);
@@ -744,6 +789,7 @@ bool gemm_tiled_run_plain_pair(int dtype, GemmArgs &g0, int ta0, int tb0, GemmAr
     // each split as it would be alone, the partial sums of the two side by side in the workspace
     g0.splits = plan_splits(BK, g0.M, g0.N, g0.K, g0.batch, g0.red, usable, &g0.tiles_per_split);
     g1.splits = plan_splits(BK, g1.M, g1.N, g1.K, g1.batch, g1.red, usable, &g1.tiles_per_split);
+    if (dtype == D8_FLOAT32) few_tiles_small(g0, usable), few_tiles_small(g1, usable);
     const size_t need0 = g0.splits > 1 ? ((size_t)g0.splits * g0.batch * g0.M * g0.N * sizeof(float) + 255) & ~(size_t)255 : 0;
     const size_t need1 = g1.splits > 1 ? (size_t)g1.splits * g1.batch * g1.M * g1.N * sizeof(float) : 0;
     if (need0 + need1 > usable) return false;

@@ -81,6 +81,8 @@ struct GemmArgs {
     // product and bias + ReLu used to be two passes: a gate decided by the sum that is rounded once opens for other
     // elements (about one in five thousand), and a layer keeps the gates it had.
     int round_first;
+    // fp32: a smaller tile than the shape's own, chosen by gemm_tiled_run (few_tiles_small, narrow_output)
+    int tile_hint;
     // Remainder band in the same launch (tail_splits > 0; unsplit, unbatched products only): rows tail_m0 .. M - 1
     // are not tiled by the launch's first tiles(tail_m0) x tiles(N) workgroups but by further ones, tail_splits per
     // tile, each walking tail_tps K steps and writing fp32 partial sums to ws[piece][row - tail_m0][n].  They start
@@ -93,6 +95,8 @@ struct GemmArgs {
     // product of a launch of two it belongs to (bit 1: gemm_tiled_pair_launch's gx)
     unsigned long long *phase_rec;
 };
+
+enum { HINT_NONE = 0, HINT_64x64 = 1, HINT_128x32 = 2 };  // GemmArgs::tile_hint
 
 enum TiledRule { TILED_ANY, TILED_PIECES, TILED_WHOLE };  // see gemm_tiled_eligible
 

@@ -798,7 +798,7 @@ int gemm_tiled_patch_f16(const GemmArgs &g, int transB, hipStream_t stream);
 int gemm_tiled_patch_f32(const GemmArgs &g, int transB, hipStream_t stream);
 
 // Which tile a product runs on.
-enum TileId { TILE_WIDE, TILE_256, TILE_128x64, TILE_64x64, TILE_64x128, TILE_128x128 };
+enum TileId { TILE_WIDE, TILE_256, TILE_128x64, TILE_64x64, TILE_64x128, TILE_128x128, TILE_128x32 };
 
 // Whether both operands of a product of real matrices can be moved in 16-byte pieces that K does not cut (else EDGE_ANY).
 template <typename E>
@@ -812,6 +812,7 @@ static bool in_pieces(const GemmArgs &g, bool a_kc, bool b_kc) {
 template <typename E, bool A_KC, bool B_KC, int VIRT = VIRT_NONE>
 static TileId choose_tile(const GemmArgs &g, bool any = false) {
     static const char *force = getenv("D8_GEMM_TILE");  // tuning aid
+    if (sizeof(E) == 4 && g.tile_hint) return g.tile_hint == HINT_128x32 ? TILE_128x32 : TILE_64x64;
     const long big_tiles = (long)ceil_div(g.M, 256) * ceil_div(g.N, 256) * g.batch * g.splits;
     bool big = g.M >= 256 && g.N >= 256 && big_tiles >= (long)cu_count() * 3 / 4;
     if (force && g.M >= 256 && g.N >= 256) big = atoi(force) != 128;

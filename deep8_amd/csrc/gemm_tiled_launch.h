@@ -44,7 +44,10 @@ static int pick_tile(const GemmArgs &g, hipStream_t stream) {
             break;
         case TILE_128x64: return launch_tiled<E, 128, 64, 2, 2, A_KC, B_KC, VIRT>(g, stream, any);
         case TILE_64x64:
-            if constexpr (VIRT == VIRT_B_KROWS || VIRT == VIRT_NONE) return launch_tiled<E, 64, 64, 2, 2, A_KC, B_KC, VIRT>(g, stream, any);
+            if constexpr (VIRT == VIRT_B_KROWS || VIRT == VIRT_NONE || sizeof(E) == 4) return launch_tiled<E, 64, 64, 2, 2, A_KC, B_KC, VIRT>(g, stream, any);
+            break;
+        case TILE_128x32:
+            if constexpr (VIRT != VIRT_B_KROWS && sizeof(E) == 4) return launch_tiled<E, 128, 32, 4, 1, A_KC, B_KC, VIRT>(g, stream, any);
             break;
         case TILE_64x128: return launch_tiled<E, 64, 128, 2, 2, A_KC, B_KC, VIRT>(g, stream, any);
         default: break;
@@ -64,6 +67,10 @@ static int launch_plain(const GemmArgs &g, int transA, int transB, hipStream_t s
 template <typename E>
 static int launch_patch(const GemmArgs &g, int transB, hipStream_t stream) {
     if (g.virt == VIRT_A_CLASSES) {  // every class has at least 128 rows (checked by eligible)
+        if constexpr (sizeof(E) == 4)
+            if (g.N <= 32)  // (see narrow_output in gemm.hip)
+                return transB ? launch_tiled<E, 128, 32, 4, 1, true, true, VIRT_A_CLASSES>(g, stream)
+                              : launch_tiled<E, 128, 32, 4, 1, true, false, VIRT_A_CLASSES>(g, stream);
         if (transB) {
             if (g.N < 128) return launch_tiled<E, 128, 64, 2, 2, true, true, VIRT_A_CLASSES>(g, stream);
             return launch_tiled<E, 128, 128, 2, 2, true, true, VIRT_A_CLASSES>(g, stream);
