@@ -201,18 +201,21 @@ __device__ inline long c_index(const GemmArgs &g, int m, int n) {
 // ------------------------------------------------------------------------------------------
 // Small products: a handful of 128 x 128 tiles would leave the chip to a few workgroups, each
 // walking its whole reduction at one MFMA per 64 (fp32) cycles behind one load latency per K step.
-// Here a workgroup owns a 32 x 32 tile of C and its four waves take every fourth chunk of the
+// Here a workgroup owns a 32 x 32 tile of C and its eight waves take every eighth chunk of the
 // reduction each (8 k values for fp32, 16 for fp16: one MFMA operand per lane).  A lane fetches
 // its operand values of ALL its chunks straight from global memory into registers before the
-// first MFMA, so the whole product costs one load latency; the four partial tiles meet in LDS in
-// wave order, so the result does not depend on scheduling.  Any M, N, K, leading dimension and
-// alignment; element-wise, bounds-checked loads.
+// first MFMA, so the whole product costs one load latency: no branch lies between the loads (an
+// index past the matrix is clamped and the value replaced by zero) and no division (unless products
+// are summed).  The eight partial tiles meet in LDS in wave order, every wave adding up and storing
+// an eighth, so the result does not depend on scheduling.  Any M, N, K, leading dimension and alignment.
+// fp32 64 x 128 x 256: forward 6.3 -> 3.8 us, both gradients 7.4 -> 5.4 us (four waves, each value behind a bounds check of its
+// own before); an empty kernel takes 1.3 us.
 // ------------------------------------------------------------------------------------------
 template <typename T>
 struct SmallOp;
 template <>
 struct SmallOp<float> {
-    static constexpr int PER = 4, KG = 8, MAXC = 16;  // values per lane and chunk, k per chunk, chunks per wave
+    static constexpr int PER = 4, KG = 8;  // values per lane and chunk, k per chunk
     typedef f32x4 Frag;
     __device__ static void mma(const Frag &a, const Frag &b, f32x16 &acc) {
 #pragma unroll
@@ -221,84 +224,104 @@ struct SmallOp<float> {
 };
 template <>
 struct SmallOp<f16> {
-    static constexpr int PER = 8, KG = 16, MAXC = 8;
+    static constexpr int PER = 8, KG = 16;
     typedef f16x8 Frag;
     __device__ static void mma(const Frag &a, const Frag &b, f32x16 &acc) {
         acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, acc, 0, 0, 0);
     }
 };
+enum { SMALL_WAVES = 8, SMALL_MAXC = 8 };  // chunks per wave: gemm_is_small admits 64 in all
+typedef float SmallParts[SMALL_WAVES][32 * 32];
 
-// (the work of workgroup (bx, by) of output b; part: 3 x 32 x 32 floats of LDS)
-template <typename T, bool TA, bool TB>
-__device__ __forceinline__ void gemm_small_body(const GemmArgs &g, const int bx, const int by, const int b, float (*part)[32 * 32]) {
-    typedef SmallOp<T> OP;
-    constexpr int BT = 32, PER = OP::PER, KG = OP::KG, MAXC = OP::MAXC;
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int l32 = lane & 31, lhi = lane >> 5;
-    const int gm = by * BT + l32, gn = bx * BT + l32;  // this lane's row of A and column of B
-    const int kchunks = (g.K + KG - 1) / KG, total = g.red * kchunks;   // total <= 4 * MAXC (gemm_is_small)
-
-    // a K-contiguous operand whose rows can be read 16 bytes at a time gives a lane its values in one load
-    const bool vec_a = !TA && g.lda % PER == 0 && g.sA % PER == 0 && g.K % PER == 0 && ((size_t)g.A & 15) == 0;
-    const bool vec_b = TB && g.ldb % PER == 0 && g.sB % PER == 0 && g.K % PER == 0 && ((size_t)g.B & 15) == 0;
-    typename OP::Frag fa[MAXC], fb[MAXC];
+// One operand's values of a chunk, PER consecutive k of row (column) `line`, as they lie in memory (VEC: in one load; K and
+// with it every piece are then multiples of PER) ...
+template <typename T, bool KC, bool VEC, typename Index>
+__device__ __forceinline__ void small_fetch(T (&v)[SmallOp<T>::PER], const T *p, int ld, int line, int k0, int K) {
+    constexpr int PER = SmallOp<T>::PER;
+    if constexpr (VEC) {
+        *(typename SmallOp<T>::Frag *)v = *(const typename SmallOp<T>::Frag *)(p + (Index)line * (Index)ld + (Index)min(k0, K - PER));
+    } else {
 #pragma unroll
-    for (int c = 0; c < MAXC; ++c) {
-        const int t = wave + 4 * c;
-#pragma unroll
-        for (int e = 0; e < PER; ++e) fa[c][e] = (T)0, fb[c][e] = (T)0;
-        if (t < total) {
-            const int r = t / kchunks, k0 = (t - r * kchunks) * KG + lhi * PER;
-            const T *Ap = (const T *)g.A + (long)(b + r) * g.sA;
-            const T *Bp = (const T *)g.B + (long)(b + r) * g.sB;
-            if (vec_a) {
-                if (gm < g.M && k0 < g.K) fa[c] = *(const typename OP::Frag *)(Ap + (long)gm * g.lda + k0);
-            } else {
-#pragma unroll
-                for (int e = 0; e < PER; ++e)
-                    if (gm < g.M && k0 + e < g.K) fa[c][e] = TA ? Ap[(long)(k0 + e) * g.lda + gm] : Ap[(long)gm * g.lda + k0 + e];
-            }
-            if (vec_b) {
-                if (gn < g.N && k0 < g.K) fb[c] = *(const typename OP::Frag *)(Bp + (long)gn * g.ldb + k0);
-            } else {
-#pragma unroll
-                for (int e = 0; e < PER; ++e)
-                    if (gn < g.N && k0 + e < g.K) fb[c][e] = TB ? Bp[(long)gn * g.ldb + k0 + e] : Bp[(long)(k0 + e) * g.ldb + gn];
-            }
+        for (int e = 0; e < PER; ++e) {
+            const int k = min(k0 + e, K - 1);
+            v[e] = p[KC ? (Index)line * (Index)ld + (Index)k : (Index)k * (Index)ld + (Index)line];
         }
     }
+}
+// ... and with zeros past K, once all loads are under way
+template <typename T>
+__device__ __forceinline__ typename SmallOp<T>::Frag small_cut(const T (&v)[SmallOp<T>::PER], int k0, int K) {
+    typename SmallOp<T>::Frag f;
+#pragma unroll
+    for (int e = 0; e < SmallOp<T>::PER; ++e) f[e] = k0 + e < K ? v[e] : (T)0;
+    return f;
+}
+
+template <typename T, bool TA, bool TB, bool VECA, bool VECB, typename Index>
+__device__ __forceinline__ void small_multiply(const GemmArgs &g, int gm, int gn, int b, int wave, int lhi, f32x16 &acc) {
+    typedef SmallOp<T> OP;
+    constexpr int PER = OP::PER, KG = OP::KG;
+    const int kchunks = (g.K + KG - 1) / KG, total = g.red * kchunks;
+    const int lm = min(gm, g.M - 1), ln = min(gn, g.N - 1);  // (rows and columns past the matrix: results that are not stored)
+    T va[SMALL_MAXC][PER], vb[SMALL_MAXC][PER];
+    int k0[SMALL_MAXC];
+#pragma unroll
+    for (int c = 0; c < SMALL_MAXC; ++c) {
+        const int t = wave + SMALL_WAVES * c;
+        k0[c] = 0;
+        if (t < total) {
+            const int r = g.red == 1 ? 0 : t / kchunks;
+            k0[c] = (t - r * kchunks) * KG + lhi * PER;
+            small_fetch<T, !TA, VECA, Index>(va[c], (const T *)g.A + (long)(b + r) * g.sA, g.lda, lm, k0[c], g.K);
+            small_fetch<T, TB, VECB, Index>(vb[c], (const T *)g.B + (long)(b + r) * g.sB, g.ldb, ln, k0[c], g.K);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < SMALL_MAXC; ++c)
+        if (wave + SMALL_WAVES * c < total) OP::mma(small_cut<T>(va[c], k0[c], g.K), small_cut<T>(vb[c], k0[c], g.K), acc);
+}
+
+// (the work of workgroup (bx, by) of output b)
+template <typename T, bool TA, bool TB>
+__device__ __forceinline__ void gemm_small_body(const GemmArgs &g, const int bx, const int by, const int b, SmallParts &part) {
+    constexpr int BT = 32;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, lhi = lane >> 5;
     f32x16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    const int gm = by * BT + l32, gn = bx * BT + l32;
+    constexpr int PER = SmallOp<T>::PER;
+    const bool vec_a = !TA && g.lda % PER == 0 && g.sA % PER == 0 && g.K % PER == 0 && ((size_t)g.A & 15) == 0;
+    const bool vec_b = TB && g.ldb % PER == 0 && g.sB % PER == 0 && g.K % PER == 0 && ((size_t)g.B & 15) == 0;
+    // (32-bit offsets where both operands allow them)
+    if ((long)(TA ? g.K : g.M) * g.lda * (long)sizeof(T) >= (1L << 31) || (long)(TB ? g.N : g.K) * g.ldb * (long)sizeof(T) >= (1L << 31))
+        small_multiply<T, TA, TB, false, false, long>(g, gm, gn, b, wave, lhi, acc);
+    else if ((TA || vec_a) && (!TB || vec_b))
+        small_multiply<T, TA, TB, !TA, TB, unsigned>(g, gm, gn, b, wave, lhi, acc);
+    else
+        small_multiply<T, TA, TB, false, false, unsigned>(g, gm, gn, b, wave, lhi, acc);
 #pragma unroll
-    for (int c = 0; c < MAXC; ++c)
-        if (wave + 4 * c < total) OP::mma(fa[c], fb[c], acc);
-
-    if (wave > 0) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) part[wave - 1][((r >> 2) * 8 + lhi * 4 + (r & 3)) * BT + l32] = acc[r];
-    }
+    for (int r = 0; r < 16; ++r) part[wave][((r >> 2) * 8 + lhi * 4 + (r & 3)) * BT + l32] = acc[r];
     __syncthreads();
-    if (wave == 0) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int row = (r >> 2) * 8 + lhi * 4 + (r & 3), m = by * BT + row;
-            float v = acc[r];
+    for (int i = 0; i < BT * BT / (SMALL_WAVES * 64); ++i) {
+        const int e = tid + i * (SMALL_WAVES * 64), m = by * BT + e / BT, gn = bx * BT + e % BT;
+        float v = part[0][e];
 #pragma unroll
-            for (int w = 0; w < 3; ++w) v += part[w][row * BT + l32];
-            if (m < g.M && gn < g.N) {
-                T *c = (T *)g.C + (long)b * g.sC + (long)m * g.ldc + gn;
-                if (g.beta != 0.f) v += to_f32(*c);
-                *c = (T)v;
-            }
+        for (int w = 1; w < SMALL_WAVES; ++w) v += part[w][e];
+        if (m < g.M && gn < g.N) {
+            T *c = (T *)g.C + (long)b * g.sC + (long)m * g.ldc + gn;
+            if (g.beta != 0.f) v += to_f32(*c);
+            if (g.bias) v = (g.round_first ? to_f32((T)v) : v) + to_f32(((const T *)g.bias)[gn]);
+            *c = (T)(g.relu && !(v > 0.f) ? 0.f : v);
         }
     }
 }
 
 template <typename T, bool TA, bool TB>
-__global__ __launch_bounds__(256) void gemm_small_kernel(GemmArgs g) {
-    __shared__ float part[3][32 * 32];
+__global__ __launch_bounds__(SMALL_WAVES * 64) void gemm_small_kernel(GemmArgs g) {
+    __shared__ SmallParts part;
     gemm_small_body<T, TA, TB>(g, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, part);
 }
 
@@ -306,8 +329,8 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(GemmArgs g) {
 // a MatrixMultiply's first input), the rest g1's (TN: the gradient of its second).  Each of them is one load
 // latency and a few matrix instructions long; what a launch of its own costs on top is most of its time.
 template <typename T>
-__global__ __launch_bounds__(256) void gemm_small_pair_kernel(GemmArgs g0, GemmArgs g1, int nx0, int ny0, int n0, int nx1, int ny1) {
-    __shared__ float part[3][32 * 32];
+__global__ __launch_bounds__(SMALL_WAVES * 64) void gemm_small_pair_kernel(GemmArgs g0, GemmArgs g1, int nx0, int ny0, int n0, int nx1, int ny1) {
+    __shared__ SmallParts part;
     int id = (int)blockIdx.x;
     if (id < n0) {
         gemm_small_body<T, false, true>(g0, id % nx0, (id / nx0) % ny0, id / (nx0 * ny0), part);
@@ -545,11 +568,11 @@ static int launch(GemmArgs &g, int transA, int transB, bool tiled, hipStream_t s
     if (g.virt == VIRT_NONE && g.splits == 1 && gemm_is_small(g.M, g.N, g.K, g.batch, g.red)) {
         dim3 grid(ceil_div(g.N, 32), ceil_div(g.M, 32), g.batch);
         if (!transA && !transB)
-            hipLaunchKernelGGL((gemm_small_kernel<T, false, false>), grid, dim3(256), 0, stream, g);
+            hipLaunchKernelGGL((gemm_small_kernel<T, false, false>), grid, dim3(SMALL_WAVES * 64), 0, stream, g);
         else if (!transA && transB)
-            hipLaunchKernelGGL((gemm_small_kernel<T, false, true>), grid, dim3(256), 0, stream, g);
+            hipLaunchKernelGGL((gemm_small_kernel<T, false, true>), grid, dim3(SMALL_WAVES * 64), 0, stream, g);
         else
-            hipLaunchKernelGGL((gemm_small_kernel<T, true, false>), grid, dim3(256), 0, stream, g);
+            hipLaunchKernelGGL((gemm_small_kernel<T, true, false>), grid, dim3(SMALL_WAVES * 64), 0, stream, g);
         D8_LAUNCH_CHECK();
         return 0;
     }
@@ -713,9 +736,9 @@ bool gemm_small_pair_run(int dtype, const GemmArgs &g0, int ta0, int tb0, const 
     GemmArgs a = g0, b = g1;
     a.splits = b.splits = 1;
     if (dtype == D8_FLOAT16)
-        hipLaunchKernelGGL((gemm_small_pair_kernel<f16>), dim3((unsigned)(n0 + n1)), dim3(256), 0, stream, a, b, nx0, ny0, (int)n0, nx1, ny1);
+        hipLaunchKernelGGL((gemm_small_pair_kernel<f16>), dim3((unsigned)(n0 + n1)), dim3(SMALL_WAVES * 64), 0, stream, a, b, nx0, ny0, (int)n0, nx1, ny1);
     else
-        hipLaunchKernelGGL((gemm_small_pair_kernel<float>), dim3((unsigned)(n0 + n1)), dim3(256), 0, stream, a, b, nx0, ny0, (int)n0, nx1, ny1);
+        hipLaunchKernelGGL((gemm_small_pair_kernel<float>), dim3((unsigned)(n0 + n1)), dim3(SMALL_WAVES * 64), 0, stream, a, b, nx0, ny0, (int)n0, nx1, ny1);
     const hipError_t e = hipGetLastError();
     *rc = e == hipSuccess ? 0 : fail((int)e, "kernel launch: %s", hipGetErrorString(e));
     return true;
@@ -806,7 +829,8 @@ bool gemm_fuses_store(int dtype, const GemmArgs &g, int transA, int transB, Tile
     // (a product beyond one launch's limits -- more than 448 outputs, more than 65535 * 128 rows -- is cut into several
     // by d8_gemm; the fused store stays out of that: the caller runs the product and one pass over its result)
     if (dtype == D8_FLOAT64 || g.K < 1 || g.beta != 0.f || g.red != 1 || g.batch > 448 || g.M > 65535 * 128) return false;
-    if (g.virt == VIRT_NONE && gemm_is_small(g.M, g.N, g.K, g.batch, g.red)) return false;  // gemm_small_kernel has no fused store
+    // (gemm_small_kernel had no fused store: asked by the other rules, which say where two passes used to round twice, it has none)
+    if (rule != TILED_ANY && g.virt == VIRT_NONE && gemm_is_small(g.M, g.N, g.K, g.batch, g.red)) return false;
     return gemm_tiled_eligible(dtype, g, transA, transB, rule);
 }
 
