@@ -347,21 +347,26 @@ static bool gemm_is_small(int M, int N, int K, int batch, int red) {
            batch * 1L < 65536;
 }
 
-// C[b][m][n] = beta * C + sum_s ws[b][s][m][n].  A workgroup covers 32 groups of 4 consecutive
-// outputs; its 8 thread rows each add every 8th partial (16-byte loads), and the 8 sums meet in
-// LDS in a fixed order, so the result does not depend on scheduling.  The groups count through an output's elements
+// C[b][m][n] = beta * C + sum_s ws[b][s][m][n].  A workgroup covers groups of 4 consecutive outputs.
+// Few pieces (LANES = 1): 256 groups, a thread adds all pieces of its group in order, four loads in
+// flight.  Many (LANES = 8): 32 groups, 8 thread rows each add every 8th piece, and the 8 sums meet in
+// LDS in a fixed order.  Either way the result does not depend on scheduling, and up to 8 pieces
+// it is the same.  Five pieces of 12544 x 32: 4.9 -> 4.0 us, four of 1024 x 1001 in half: 7.1 -> 5.4 us (3 us of which is
+// what any launch behind one that wrote a lot takes).  The groups count through an output's elements
 // whatever the length of its rows: with rows of an odd length a group starts at any 4-byte aligned address (which is what
 // a 16-byte load needs) and may go on in the next row.  An output a thread, as rows of an odd length had it first, took
 // 17.3 us for four partial sums of 1024 x 1001, this takes 8.0 us.
 typedef f32x4 f32x4_any __attribute__((aligned(4)));
+__host__ __device__ static inline int reduce_lanes(const GemmArgs &g) { return g.splits <= 8 ? 1 : 8; }
 
 // (ROWS: the rows are multiples of 4, so a group lies in one row and may be stored at once)
-template <typename T, bool ROWS>
+template <typename T, bool ROWS, int LANES>
 __device__ __forceinline__ void gemm_split_reduce_body(const GemmArgs &g, const long block, f32x4 (*part)[32]) {
     typedef T T4 __attribute__((ext_vector_type(4)));
     const long mn = (long)g.M * g.N, groups = ROWS ? mn / 4 : (mn + 3) / 4;
-    const int lane = threadIdx.x & 31, row = threadIdx.x >> 5;
-    const long id = block * 32 + lane;  // this thread's group of 4 outputs
+    constexpr int GROUPS = 256 / LANES;
+    const int lane = threadIdx.x % GROUPS, row = threadIdx.x / GROUPS;
+    const long id = block * GROUPS + lane;  // this thread's group of 4 outputs
     const bool live = id < groups * g.batch;
     const int b = live && g.batch > 1 ? (int)(id / groups) : 0;
     const long r = (id - (long)b * groups) * 4;
@@ -370,17 +375,28 @@ __device__ __forceinline__ void gemm_split_reduce_body(const GemmArgs &g, const 
     if (live) {
         const float *p = g.ws + (long)b * g.splits * mn + r;
         if (n_out == 4) {
-            for (int s = row; s < g.splits; s += 8) v += *(const f32x4_any *)(p + (long)s * mn);
+            int s = row;
+            for (; s + 3 * LANES < g.splits; s += 4 * LANES) {
+                f32x4 t[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) t[u] = *(const f32x4_any *)(p + (long)(s + u * LANES) * mn);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) v += t[u];
+            }
+            for (; s < g.splits; s += LANES) v += *(const f32x4_any *)(p + (long)s * mn);
         } else {
-            for (int s = row; s < g.splits; s += 8)
+            for (int s = row; s < g.splits; s += LANES)
                 for (int k = 0; k < n_out; ++k) v[k] += p[(long)s * mn + k];
         }
     }
-    part[row][lane] = v;
-    __syncthreads();
+    if constexpr (LANES > 1) {
+        part[row][lane] = v;
+        __syncthreads();
+    }
     if (row == 0 && live) {
+        if constexpr (LANES > 1)
 #pragma unroll
-        for (int k = 1; k < 8; ++k) v += part[k][lane];
+            for (int k = 1; k < LANES; ++k) v += part[k][lane];
         int m = (int)(r / g.N), n = (int)(r - (long)m * g.N);
         T *c0 = (T *)g.C + (long)b * g.sC;
         auto finish = [&](float o, float old, float bias) {
@@ -409,18 +425,20 @@ __device__ __forceinline__ void gemm_split_reduce_body(const GemmArgs &g, const 
     }
 }
 
-template <typename T, bool ROWS>
+template <typename T, bool ROWS, int LANES>
 __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(GemmArgs g) {
     __shared__ f32x4 part[8][32];
-    gemm_split_reduce_body<T, ROWS>(g, (long)blockIdx.x, part);
+    gemm_split_reduce_body<T, ROWS, LANES>(g, (long)blockIdx.x, part);
 }
 
 // The reductions of two products in one launch: the first blocks0 workgroups are g0's, the rest g1's.
 template <typename T>
 __global__ __launch_bounds__(256) void gemm_split_reduce_pair_kernel(GemmArgs g0, GemmArgs g1, unsigned blocks0) {
     __shared__ f32x4 part[8][32];
-    if (blockIdx.x < blocks0) gemm_split_reduce_body<T, true>(g0, (long)blockIdx.x, part);
-    else gemm_split_reduce_body<T, true>(g1, (long)(blockIdx.x - blocks0), part);
+    const GemmArgs &g = blockIdx.x < blocks0 ? g0 : g1;
+    const long block = blockIdx.x < blocks0 ? blockIdx.x : blockIdx.x - blocks0;
+    if (reduce_lanes(g) == 1) gemm_split_reduce_body<T, true, 1>(g, block, part);
+    else gemm_split_reduce_body<T, true, 8>(g, block, part);
 }
 
 // ---- planning a product whose 128 x 128 tiles are fewer than the CUs -----------------------------------------
@@ -532,13 +550,19 @@ static int plan_splits(int BK, int M, int N, int K, int batch, int red, size_t w
 }
 
 // C = beta * C + the g.splits partial sums in g.ws (+ bias, ReLu)
-static long reduce_blocks(const GemmArgs &g) { return (((long)g.M * g.N + 3) / 4 * g.batch + 31) / 32; }
+static long reduce_blocks(const GemmArgs &g, int lanes) {
+    const int groups = 256 / lanes;
+    return (((long)g.M * g.N + 3) / 4 * g.batch + groups - 1) / groups;
+}
 
 template <typename T>
 static int launch_reduce(const GemmArgs &g, hipStream_t stream) {
-    const dim3 grid((unsigned)reduce_blocks(g));
-    if (g.N % 4 == 0) hipLaunchKernelGGL((gemm_split_reduce_kernel<T, true>), grid, dim3(256), 0, stream, g);
-    else hipLaunchKernelGGL((gemm_split_reduce_kernel<T, false>), grid, dim3(256), 0, stream, g);
+    const int lanes = reduce_lanes(g);
+    const dim3 grid((unsigned)reduce_blocks(g, lanes));
+    if (g.N % 4 == 0 && lanes == 1) hipLaunchKernelGGL((gemm_split_reduce_kernel<T, true, 1>), grid, dim3(256), 0, stream, g);
+    else if (g.N % 4 == 0) hipLaunchKernelGGL((gemm_split_reduce_kernel<T, true, 8>), grid, dim3(256), 0, stream, g);
+    else if (lanes == 1) hipLaunchKernelGGL((gemm_split_reduce_kernel<T, false, 1>), grid, dim3(256), 0, stream, g);
+    else hipLaunchKernelGGL((gemm_split_reduce_kernel<T, false, 8>), grid, dim3(256), 0, stream, g);
     D8_LAUNCH_CHECK();
     return 0;
 }
@@ -547,12 +571,12 @@ static int launch_reduce(const GemmArgs &g, hipStream_t stream) {
 // multiples of 4, or they would not have shared the first).
 static int launch_reduce_pair(int dtype, const GemmArgs &g0, const GemmArgs &g1, hipStream_t stream) {
     const bool r0 = g0.splits > 1, r1 = g1.splits > 1;
-    const long b0 = reduce_blocks(g0), b1 = reduce_blocks(g1);
+    const long b0 = reduce_blocks(g0, reduce_lanes(g0)), b1 = reduce_blocks(g1, reduce_lanes(g1));
     if (r0 && r1 && g0.N % 4 == 0 && g1.N % 4 == 0 && b0 + b1 < 0x7fffffffL) {
         if (dtype == D8_FLOAT16)
-            hipLaunchKernelGGL((gemm_split_reduce_pair_kernel<f16>), dim3((unsigned)(b0 + b1)), dim3(256), 0, stream, g0, g1, (unsigned)b0);
+            hipLaunchKernelGGL(gemm_split_reduce_pair_kernel<f16>, dim3((unsigned)(b0 + b1)), dim3(256), 0, stream, g0, g1, (unsigned)b0);
         else
-            hipLaunchKernelGGL((gemm_split_reduce_pair_kernel<float>), dim3((unsigned)(b0 + b1)), dim3(256), 0, stream, g0, g1, (unsigned)b0);
+            hipLaunchKernelGGL(gemm_split_reduce_pair_kernel<float>, dim3((unsigned)(b0 + b1)), dim3(256), 0, stream, g0, g1, (unsigned)b0);
         D8_LAUNCH_CHECK();
         return 0;
     }
