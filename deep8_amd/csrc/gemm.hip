@@ -662,36 +662,43 @@ size_t gemm_tiled_workspace(int dtype, int M, int N, int K, int red, int virt) {
     return splits > 1 ? (size_t)splits * rows * N * sizeof(float) : 0;
 }
 
-// fp32, whose K step is bound by the matrix pipe: 64 x 64 tiles where the 128-wide ones leave compute units idle.  A step of
-// theirs is a quarter of the work and their ends are shorter, so the same pieces (or none) spread over four times as many
-// workgroups.  The estimate counts as plan_few_tiles does, in steps of a 128 x 128 tile (about 2 us of a CU), for the plan that
-// g holds (splits set) and for 64 x 64 tiles in 1 .. as many pieces as that plan; 7 % or more decide.
-// NN, us before and after (M x K x N): 512 x 512 x 512 16.4 -> 10.2, 784 x 1152 x 128 16.0 -> 10.3, 1024 x 1024 x 1024
-// 33.6 -> 23.5, 12544 x 800 x 64 24.0 -> 17.0, 3136 x 576 x 256 24.5 -> 12.7, 1536 x 1536 x 1536 76.8 -> 72.5 (NT and TN alike).  A narrow
-// output (128 x 32 tiles, below) counts its pieces the same way.
-static double tile_cost(int bm, int bn, const GemmArgs &g, long total, long s) {
+// 64 x 64 tiles where the 128-wide ones leave compute units idle.  In fp32, whose K step is bound by the matrix pipe, a step of
+// theirs is a quarter of the work; in half, whose step waits longer than it multiplies, half of it (0.25 us against 0.38 for a
+// 64 x 128 tile and 0.46 for 128 x 128).  The same pieces -- or none, and no second pass -- spread over four times as many
+// workgroups.  The estimate counts as plan_few_tiles does, in steps of a 128 x 128 tile (about 2 us of a CU in fp32, 0.5 us in
+// half), for the plan that g holds (splits set) and for 64 x 64 tiles in 1 .. as many pieces as that plan; 7 % or more decide.
+// A narrow output (128 x 32 tiles, below) counts its pieces the same way.
+// NN, us before and after (M x K x N; NT and TN alike): fp32 512 x 512 x 512 16.4 -> 10.2, 784 x 1152 x 128 16.0 -> 10.3,
+// 1024 x 1024 x 1024 33.6 -> 23.5, 12544 x 800 x 64 24.0 -> 17.0, 3136 x 576 x 256 24.5 -> 12.7, 1536 x 1536 x 1536
+// 76.8 -> 72.5; half 512 x 512 x 512 8.6 -> 5.5, 256 x 1024 x 1024 11.8 -> 7.5, 1024 x 1024 x 1024 9.6 -> 8.2,
+// 1600 x 2304 x 256 18.2 -> 12.6 (in pieces 18.7), 300 x 3136 x 256 10.6 -> 9.1 (whole 15.7); left alone, and slower if not:
+// 1536 x 1536 x 1536 16.5 (19.8), 1024 x 2048 x 2048 18.2 (19.3).
+static double tile_cost(bool half_elems, int bm, int bn, const GemmArgs &g, long total, long s) {
     const long cus = cu_count(), n = (ceil_div(g.M, bm) * (long)ceil_div(g.N, bn) * g.batch * s + cus - 1) / cus, len = (total + s - 1) / s;
-    const double step = bm * bn / 16384.0;
-    return n * len * step * (n == 1 ? 1.1 : 1.0) + 0.5 + 2.0 * sqrt(step) + 0.3 * (n - 1) + (s > 1 ? 2.0 + s * ((double)g.M * g.N * g.batch / 2e6) : 0.0);
+    const double area = bm * bn / 16384.0, mn = (double)g.M * g.N * g.batch;
+    if (half_elems) return n * len * (area < 0.3 ? 0.5 : area < 0.6 ? 0.76 : 1.0) + 7.0 + 0.5 * (n - 1) + (s > 1 ? 6.5 + s * (mn / 0.25e6) : 0.0);
+    return n * len * area * (n == 1 ? 1.1 : area < 0.3 ? 1.08 : 1.0) + 0.5 + 2.0 * sqrt(area) + 0.3 * (n - 1) + (s > 1 ? 2.0 + s * (mn / 2e6) : 0.0);
 }
 
-static void few_tiles_small(GemmArgs &g, size_t usable) {
+static void few_tiles_small(int dtype, GemmArgs &g, size_t usable) {
     // (a filter gradient's pieces stay those of the launch it may share with the input's: one sum, one result)
     if (g.virt == VIRT_A_CLASSES || g.virt == VIRT_B_KROWS || gemm_is_small(g.M, g.N, g.K, g.batch, g.red)) return;
     if ((long)ceil_div(g.M, 128) * ceil_div(g.N, 128) * g.batch >= cu_count()) return;
-    const long total = (long)g.red * ceil_div(g.K, 32);
-    const bool half = g.splits == 1 && gemm_tiled_half_tiles(g.M, g.N, g.batch, total, 32);
+    const bool half_elems = dtype == D8_FLOAT16;
+    const int BK = gemm_tiled_k_step(dtype);
+    const long total = (long)g.red * ceil_div(g.K, BK);
+    const bool half = g.splits == 1 && gemm_tiled_half_tiles(g.M, g.N, g.batch, total, BK);
     const bool narrow = g.tile_hint == HINT_128x32;
-    const double now = narrow ? 1e30 : g.N < 128 ? tile_cost(128, 64, g, total, g.splits) : tile_cost(g.M < 128 || half ? 64 : 128, 128, g, total, g.splits);
+    const double now = narrow ? 1e30 : g.N < 128 ? tile_cost(half_elems, 128, 64, g, total, g.splits) : tile_cost(half_elems, g.M < 128 || half ? 64 : 128, 128, g, total, g.splits);
     long most = (long)(usable / ((size_t)g.batch * g.M * g.N * sizeof(float)));
     int tps;  // (no more pieces than the 128-wide plan would have: what the scratch queries provide for, whatever is passed)
-    const long planned = plan_splits(32, g.M, g.N, g.K, g.batch, g.red, (size_t)-1, &tps, g.virt);
+    const long planned = plan_splits(BK, g.M, g.N, g.K, g.batch, g.red, (size_t)-1, &tps, g.virt);
     if (most > planned) most = planned;
     if (most > total / 2) most = total / 2;
     double best = 0.93 * now;
     long pieces = 0;
     for (long s = 1; s == 1 || s <= most; ++s)
-        if (const double c = narrow ? tile_cost(128, 32, g, total, s) : tile_cost(64, 64, g, total, s); c < best) best = c, pieces = s;
+        if (const double c = narrow ? tile_cost(half_elems, 128, 32, g, total, s) : tile_cost(half_elems, 64, 64, g, total, s); c < best) best = c, pieces = s;
     if (!pieces) return;
     if (!narrow) g.tile_hint = HINT_64x64;
     g.tiles_per_split = (int)((total + pieces - 1) / pieces);
@@ -709,7 +716,7 @@ static int gemm_tiled_run_whole(int dtype, GemmArgs &g, int transA, int transB, 
     g.ws = (float *)workspace;
     const size_t usable = (workspace && ((size_t)workspace & 15) == 0) ? workspace_bytes : 0;
     g.splits = plan_splits(gemm_tiled_k_step(dtype), g.M, g.N, g.K, g.batch, g.red, usable, &g.tiles_per_split, g.virt);
-    if (dtype == D8_FLOAT32) few_tiles_small(g, usable);
+    few_tiles_small(dtype, g, usable);
     return dtype == D8_FLOAT16 ? launch<f16>(g, transA, transB, true, stream) : launch<float>(g, transA, transB, true, stream);
 }
 
@@ -836,7 +843,12 @@ bool gemm_tiled_run_plain_pair(int dtype, GemmArgs &g0, int ta0, int tb0, GemmAr
     // each split as it would be alone, the partial sums of the two side by side in the workspace
     g0.splits = plan_splits(BK, g0.M, g0.N, g0.K, g0.batch, g0.red, usable, &g0.tiles_per_split);
     g1.splits = plan_splits(BK, g1.M, g1.N, g1.K, g1.batch, g1.red, usable, &g1.tiles_per_split);
-    if (dtype == D8_FLOAT32) few_tiles_small(g0, usable), few_tiles_small(g1, usable);
+    // (in half the two products fill the chip together on larger tiles, which sum an unsplit reduction in the same order)
+    for (GemmArgs *g : {&g0, &g1}) {
+        const int whole = g->splits == 1 && dtype == D8_FLOAT16;
+        few_tiles_small(dtype, *g, usable);
+        if (whole) g->tile_hint = HINT_NONE;
+    }
     const size_t need0 = g0.splits > 1 ? ((size_t)g0.splits * g0.batch * g0.M * g0.N * sizeof(float) + 255) & ~(size_t)255 : 0;
     const size_t need1 = g1.splits > 1 ? (size_t)g1.splits * g1.batch * g1.M * g1.N * sizeof(float) : 0;
     if (need0 + need1 > usable) return false;

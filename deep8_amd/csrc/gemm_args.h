@@ -81,7 +81,7 @@ struct GemmArgs {
     // product and bias + ReLu used to be two passes: a gate decided by the sum that is rounded once opens for other
     // elements (about one in five thousand), and a layer keeps the gates it had.
     int round_first;
-    // fp32: a smaller tile than the shape's own, chosen by gemm_tiled_run (few_tiles_small, narrow_output)
+    // a smaller tile than the shape's own (128 x 32: fp32 only), chosen by gemm_tiled_run (few_tiles_small, narrow_output)
     int tile_hint;
     // Remainder band in the same launch (tail_splits > 0; unsplit, unbatched products only): rows tail_m0 .. M - 1
     // are not tiled by the launch's first tiles(tail_m0) x tiles(N) workgroups but by further ones, tail_splits per

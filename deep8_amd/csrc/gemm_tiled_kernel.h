@@ -812,7 +812,7 @@ static bool in_pieces(const GemmArgs &g, bool a_kc, bool b_kc) {
 template <typename E, bool A_KC, bool B_KC, int VIRT = VIRT_NONE>
 static TileId choose_tile(const GemmArgs &g, bool any = false) {
     static const char *force = getenv("D8_GEMM_TILE");  // tuning aid
-    if (sizeof(E) == 4 && g.tile_hint) return g.tile_hint == HINT_128x32 ? TILE_128x32 : TILE_64x64;
+    if (g.tile_hint) return g.tile_hint == HINT_128x32 ? TILE_128x32 : TILE_64x64;
     const long big_tiles = (long)ceil_div(g.M, 256) * ceil_div(g.N, 256) * g.batch * g.splits;
     bool big = g.M >= 256 && g.N >= 256 && big_tiles >= (long)cu_count() * 3 / 4;
     if (force && g.M >= 256 && g.N >= 256) big = atoi(force) != 128;

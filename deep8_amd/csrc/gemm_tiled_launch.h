@@ -43,9 +43,7 @@ static int pick_tile(const GemmArgs &g, hipStream_t stream) {
             if constexpr (sizeof(E) == 2) return launch_tiled<E, 256, 256, 4, 2, A_KC, B_KC, VIRT>(g, stream);
             break;
         case TILE_128x64: return launch_tiled<E, 128, 64, 2, 2, A_KC, B_KC, VIRT>(g, stream, any);
-        case TILE_64x64:
-            if constexpr (VIRT == VIRT_B_KROWS || VIRT == VIRT_NONE || sizeof(E) == 4) return launch_tiled<E, 64, 64, 2, 2, A_KC, B_KC, VIRT>(g, stream, any);
-            break;
+        case TILE_64x64: return launch_tiled<E, 64, 64, 2, 2, A_KC, B_KC, VIRT>(g, stream, any);
         case TILE_128x32:
             if constexpr (VIRT != VIRT_B_KROWS && sizeof(E) == 4) return launch_tiled<E, 128, 32, 4, 1, A_KC, B_KC, VIRT>(g, stream, any);
             break;

@@ -9,7 +9,7 @@ namespace d8 {
 template <typename E>
 static bool plain_pair_tiles(const GemmArgs &g0, const GemmArgs &g1, TileId &t0, TileId &t1) {
     t0 = choose_tile<E, true, true>(g0), t1 = choose_tile<E, false, false>(g1);
-    auto ok = [](TileId t) { return t == TILE_64x128 || t == TILE_128x128 || t == TILE_128x64 || (sizeof(E) == 4 && t == TILE_64x64); };
+    auto ok = [](TileId t) { return t == TILE_64x128 || t == TILE_128x128 || t == TILE_128x64 || t == TILE_64x64; };
     constexpr int BK = 128 / (int)sizeof(E);
     return ok(t0) && ok(t1) && g0.K % BK == 0 && g1.K % BK == 0;
 }
@@ -22,17 +22,14 @@ static int launch_plain_pair(const GemmArgs &g0, const GemmArgs &g1, hipStream_t
     switch (t1) {                                                                                                   \
         case TILE_128x128: return launch_pair_tiles<T0T, Tile<E, 128, 128, 2, 2, false, false>>(g0, g1, stream);    \
         case TILE_64x128: return launch_pair_tiles<T0T, Tile<E, 64, 128, 2, 2, false, false>>(g0, g1, stream);      \
-        case TILE_64x64:                                                                                            \
-            if constexpr (sizeof(E) == 4) return launch_pair_tiles<T0T, Tile<E, 64, 64, 2, 2, false, false>>(g0, g1, stream); \
-            [[fallthrough]];                                                                                        \
+        case TILE_64x64: return launch_pair_tiles<T0T, Tile<E, 64, 64, 2, 2, false, false>>(g0, g1, stream);        \
         default: return launch_pair_tiles<T0T, Tile<E, 128, 64, 2, 2, false, false>>(g0, g1, stream);               \
     }
     typedef Tile<E, 64, 128, 2, 2, true, true> A0;
     typedef Tile<E, 128, 128, 2, 2, true, true> A1;
     typedef Tile<E, 128, 64, 2, 2, true, true> A2;
     typedef Tile<E, 64, 64, 2, 2, true, true> A3;
-    if constexpr (sizeof(E) == 4)
-        if (t0 == TILE_64x64) { D8_PAIR_1(A3) }
+    if (t0 == TILE_64x64) { D8_PAIR_1(A3) }
     if (t0 == TILE_64x128) { D8_PAIR_1(A0) }
     if (t0 == TILE_128x128) { D8_PAIR_1(A1) }
     D8_PAIR_1(A2)

@@ -1,9 +1,9 @@
-"""fp32 products on the smaller tiles: 64 x 64 where 128-wide tiles would leave compute units idle, 128 x 32 for outputs of at
-most 32 columns; with and without a split reduction, as matrices and as convolutions.  Integers, bit for bit."""
+"""Products on the smaller tiles: 64 x 64 where 128-wide tiles would leave compute units idle, 128 x 32 for outputs of at
+most 32 columns in fp32; with and without a split reduction, as matrices and as convolutions.  Integers, bit for bit."""
 import numpy as np
 import pytest
 
-from util import ints, rng
+from util import f, ints, rng
 
 pytestmark = pytest.mark.gpu
 
@@ -14,23 +14,26 @@ SHAPES = [(784, 128, 1152), (130, 191, 608), (65, 260, 999), (1000, 64, 32), (32
 
 @pytest.mark.parametrize("M,N,K", SHAPES)
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0)])
-def test_products(oracle_port, M, N, K, ta, tb):
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+def test_products(oracle_port, M, N, K, ta, tb, dtype):
     from deep8_amd import capi
     from deep8_amd.capi import DeviceArray, check
     lib = capi.init()
-    r = rng(M + 3 * N + 7 * K)
+    r, dt = rng(M + 3 * N + 7 * K), capi.dtype_id(np.dtype(dtype))
+    hi = 2 if dtype == np.float16 else 9
     for batch in (1,) if M > 1000 else (1, 3):
-        A = ints(r, (batch,) + ((K, M) if ta else (M, K)), 9)
-        B = ints(r, (batch,) + ((N, K) if tb else (K, N)), 9)
+        A = ints(r, (batch,) + ((K, M) if ta else (M, K)), hi)
+        B = ints(r, (batch,) + ((N, K) if tb else (K, N)), hi)
         C = ints(r, (batch, M, N), 5)
         want = np.stack([oracle_port.gemm(ta, tb, A[i], B[i]) for i in range(batch)])
-        dA, dB = DeviceArray.from_numpy(A), DeviceArray.from_numpy(B)
-        asked = lib.d8_gemm_workspace_bytes(capi.FLOAT32, ta, tb, M, N, K, batch, M * N)
+        assert dtype == np.float32 or want.max() < 2040
+        dA, dB = DeviceArray.from_numpy(A.astype(dtype)), DeviceArray.from_numpy(B.astype(dtype))
+        asked = lib.d8_gemm_workspace_bytes(dt, ta, tb, M, N, K, batch, M * N)
         for nb, beta in ((asked, 0.0), (asked, 1.0), (0, 0.0), (2 * batch * M * N * 4 + 64, 0.0)):
-            dC, ws = DeviceArray.from_numpy(C), DeviceArray((max(nb, 16),), np.uint8)
-            check(lib.d8_gemm(capi.FLOAT32, ta, tb, M, N, K, dA.ptr, A.shape[2], A[0].size, dB.ptr, B.shape[2], B[0].size, beta, dC.ptr, N,
+            dC, ws = DeviceArray.from_numpy(C.astype(dtype)), DeviceArray((max(nb, 16),), np.uint8)
+            check(lib.d8_gemm(dt, ta, tb, M, N, K, dA.ptr, A.shape[2], A[0].size, dB.ptr, B.shape[2], B[0].size, beta, dC.ptr, N,
                               M * N, batch, ws.ptr if nb else None, nb, None))
-            assert np.array_equal(dC.numpy(), want + beta * C), (batch, nb, beta)
+            assert np.array_equal(f(dC.numpy()), want + beta * C), (batch, nb, beta)
 
 
 # B, IH, IW, IC, OC, FH, FW, covered, sy, sx, dy, dx: few input channels (the gradient of x is narrow), few output channels
