@@ -196,49 +196,58 @@ __global__ __launch_bounds__(256) void column_sum_finish_kernel(const float *__r
 // column sums are taken on the way, with column_sum_kernel's chunks, row order and LDS meeting order, so the sums
 // are bit for bit those of d8_add_grad run on dpre afterwards.  z is the layer's output relu(pre): z > 0 exactly
 // where pre > 0 (deep8/src/math/ReLu.cu:61-116 gates on pre; Add.cu:64-133 sums).  dpre may be dz (in place).
-template <typename T, int VEC>
+//
+// ANY: rows that start at any element (an odd number of columns, an element-aligned tensor).  The same 16-byte accesses
+// at the alignment of an element, which the compiler is told; the last vector of a row is moved back to end with the row,
+// and of the columns that it then shares with its neighbour only the neighbour writes dpre and the sums.
+template <typename T, int VEC, bool ANY>
 __global__ __launch_bounds__(256) void relu_gate_column_sum_kernel(const T *__restrict__ z, const T *dz, T *dpre,
                                                                    T *__restrict__ g, float *__restrict__ partial, int R, int C,
                                                                    int TX, int rows_per_chunk, int chunks, float keep) {
     typedef T VT __attribute__((ext_vector_type(VEC)));
+    typedef VT MT __attribute__((aligned(ANY ? sizeof(T) : sizeof(VT))));  // a vector as it lies in memory
     __shared__ float part[256][VEC];
     const int tx = threadIdx.x % TX, ty = threadIdx.x / TX, lanes = 256 / TX;
     const int cv = blockIdx.x * TX + tx;
     const int chunk = blockIdx.y;
     const bool live = (long)cv * VEC < C;
+    const long col = ANY ? min((long)cv * VEC, (long)C - VEC) : (long)cv * VEC;
+    const int skip = ANY ? (int)((long)cv * VEC - col) : 0;  // leading elements that are the neighbour's
     float acc[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) acc[e] = 0.f;
+    auto gate = [&](const VT &a, VT b, int r) {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+            if (!(ew_f32(a[e]) > 0.f)) b[e] = (T)0.f;
+            acc[e] += ew_f32(b[e]);
+        }
+        T *o = dpre + (long)r * C + col;
+        if (!ANY || skip == 0) {
+            *(MT *)o = b;
+        } else {
+#pragma unroll
+            for (int e = 0; e < VEC; ++e)
+                if (e >= skip) o[e] = b[e];
+        }
+    };
     if (live) {
         const int r1 = min(R, (chunk + 1) * rows_per_chunk);
-        const long col = (long)cv * VEC;
         int r = chunk * rows_per_chunk + ty;
         for (; r + 3 * lanes < r1; r += 4 * lanes) {
             VT a[4], b[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                a[u] = *(const VT *)(z + (long)(r + u * lanes) * C + col);
-                b[u] = *(const VT *)(dz + (long)(r + u * lanes) * C + col);
+                a[u] = *(const MT *)(z + (long)(r + u * lanes) * C + col);
+                b[u] = *(const MT *)(dz + (long)(r + u * lanes) * C + col);
             }
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-#pragma unroll
-                for (int e = 0; e < VEC; ++e) {
-                    if (!(ew_f32(a[u][e]) > 0.f)) b[u][e] = (T)0.f;
-                    acc[e] += ew_f32(b[u][e]);
-                }
-                *(VT *)(dpre + (long)(r + u * lanes) * C + col) = b[u];
-            }
+            for (int u = 0; u < 4; ++u) gate(a[u], b[u], r + u * lanes);
         }
         for (; r < r1; r += lanes) {
-            const VT a = *(const VT *)(z + (long)r * C + col);
-            VT b = *(const VT *)(dz + (long)r * C + col);
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) {
-                if (!(ew_f32(a[e]) > 0.f)) b[e] = (T)0.f;
-                acc[e] += ew_f32(b[e]);
-            }
-            *(VT *)(dpre + (long)r * C + col) = b;
+            const VT a = *(const MT *)(z + (long)r * C + col);
+            const VT b = *(const MT *)(dz + (long)r * C + col);
+            gate(a, b, r);
         }
     }
 #pragma unroll
@@ -249,13 +258,15 @@ __global__ __launch_bounds__(256) void relu_gate_column_sum_kernel(const T *__re
 #pragma unroll
             for (int e = 0; e < VEC; ++e) acc[e] += part[k * TX + tx][e];
         if (chunks == 1) {
-            T *o = g + (long)cv * VEC;
+            T *o = g + col;
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) o[e] = (T)((keep != 0.f ? ew_f32(o[e]) : 0.f) + acc[e]);
+            for (int e = 0; e < VEC; ++e)
+                if (e >= skip) o[e] = (T)((keep != 0.f ? ew_f32(o[e]) : 0.f) + acc[e]);
         } else {
-            float *o = partial + (long)chunk * C + (long)cv * VEC;
+            float *o = partial + (long)chunk * C + col;
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) o[e] = acc[e];
+            for (int e = 0; e < VEC; ++e)
+                if (e >= skip) o[e] = acc[e];
         }
     }
 }
@@ -605,14 +616,20 @@ static int relu_gate_sum_t(const T *z, const T *dz, T *dpre, T *g, long rows, in
     const size_t need = (size_t)chunks * cols * sizeof(float);
     if (chunks > 1 && (!scratch || scratch_bytes < need || !al16(scratch))) chunks = 1, rpc = (int)rows;
     const bool wide = cols % WIDE == 0 && al16(g) && al16(dz) && al16(z) && al16(dpre);
-    const long cvs = cols / (wide ? WIDE : 1);
+    // rows that start at any element: 16-byte accesses too where a row is more than sixteen of them, so that 32 threads lie
+    // across the columns as they do in d8_add_grad's single-element pass over such a tensor and the sums stay its own
+    const bool any = !wide && cols > 16 * WIDE;
+    const int vec = wide || any ? WIDE : 1;
+    const long cvs = ((long)cols + vec - 1) / vec;
     int TX = 1;
     while (TX < 32 && TX < cvs) TX *= 2;
     dim3 grid((unsigned)((cvs + TX - 1) / TX), (unsigned)chunks, 1);
-    if (wide)
-        hipLaunchKernelGGL((relu_gate_column_sum_kernel<T, WIDE>), grid, dim3(256), 0, s, z, dz, dpre, g, (float *)scratch, (int)rows, cols, TX, rpc, chunks, keep);
+    if (any)
+        hipLaunchKernelGGL((relu_gate_column_sum_kernel<T, WIDE, true>), grid, dim3(256), 0, s, z, dz, dpre, g, (float *)scratch, (int)rows, cols, TX, rpc, chunks, keep);
+    else if (wide)
+        hipLaunchKernelGGL((relu_gate_column_sum_kernel<T, WIDE, false>), grid, dim3(256), 0, s, z, dz, dpre, g, (float *)scratch, (int)rows, cols, TX, rpc, chunks, keep);
     else
-        hipLaunchKernelGGL((relu_gate_column_sum_kernel<T, 1>), grid, dim3(256), 0, s, z, dz, dpre, g, (float *)scratch, (int)rows, cols, TX, rpc, chunks, keep);
+        hipLaunchKernelGGL((relu_gate_column_sum_kernel<T, 1, false>), grid, dim3(256), 0, s, z, dz, dpre, g, (float *)scratch, (int)rows, cols, TX, rpc, chunks, keep);
     D8_LAUNCH_CHECK();
     if (chunks > 1) {
         hipLaunchKernelGGL((column_sum_finish_kernel<T>), dim3((unsigned)((cols + 15) / 16)), dim3(256), 0, s,
