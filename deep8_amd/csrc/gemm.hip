@@ -680,11 +680,14 @@ static double tile_cost(bool half_elems, int bm, int bn, const GemmArgs &g, long
     return n * len * area * (n == 1 ? 1.1 : area < 0.3 ? 1.08 : 1.0) + 0.5 + 2.0 * sqrt(area) + 0.3 * (n - 1) + (s > 1 ? 2.0 + s * (mn / 2e6) : 0.0);
 }
 
-static void few_tiles_small(int dtype, GemmArgs &g, size_t usable) {
+static void few_tiles_small(int dtype, GemmArgs &g, int transA, int transB, size_t usable) {
     // (a filter gradient's pieces stay those of the launch it may share with the input's: one sum, one result)
     if (g.virt == VIRT_A_CLASSES || g.virt == VIRT_B_KROWS || gemm_is_small(g.M, g.N, g.K, g.batch, g.red)) return;
     if ((long)ceil_div(g.M, 128) * ceil_div(g.N, 128) * g.batch >= cu_count()) return;
     const bool half_elems = dtype == D8_FLOAT16;
+    // (half rows that start anywhere: a 64 x 64 tile's step takes 0.6 us of the 0.9 of a 128 x 128 one's, so the pieces stay:
+    // 1024 x 4096 x 1001 TN 38.9 us whole on small tiles, 21.7 + 5.4 in four pieces)
+    if (half_elems && gemm_tiled_loose(dtype, g, transA, transB)) return;
     const int BK = gemm_tiled_k_step(dtype);
     const long total = (long)g.red * ceil_div(g.K, BK);
     const bool half = g.splits == 1 && gemm_tiled_half_tiles(g.M, g.N, g.batch, total, BK);
@@ -716,7 +719,7 @@ static int gemm_tiled_run_whole(int dtype, GemmArgs &g, int transA, int transB, 
     g.ws = (float *)workspace;
     const size_t usable = (workspace && ((size_t)workspace & 15) == 0) ? workspace_bytes : 0;
     g.splits = plan_splits(gemm_tiled_k_step(dtype), g.M, g.N, g.K, g.batch, g.red, usable, &g.tiles_per_split, g.virt);
-    few_tiles_small(dtype, g, usable);
+    few_tiles_small(dtype, g, transA, transB, usable);
     return dtype == D8_FLOAT16 ? launch<f16>(g, transA, transB, true, stream) : launch<float>(g, transA, transB, true, stream);
 }
 
@@ -846,7 +849,7 @@ bool gemm_tiled_run_plain_pair(int dtype, GemmArgs &g0, int ta0, int tb0, GemmAr
     // (in half the two products fill the chip together on larger tiles, which sum an unsplit reduction in the same order)
     for (GemmArgs *g : {&g0, &g1}) {
         const int whole = g->splits == 1 && dtype == D8_FLOAT16;
-        few_tiles_small(dtype, *g, usable);
+        few_tiles_small(dtype, *g, g == &g1, g == &g0, usable);
         if (whole) g->tile_hint = HINT_NONE;
     }
     const size_t need0 = g0.splits > 1 ? ((size_t)g0.splits * g0.batch * g0.M * g0.N * sizeof(float) + 255) & ~(size_t)255 : 0;

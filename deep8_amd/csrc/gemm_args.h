@@ -121,6 +121,7 @@ int gemm_tiled_k_step(int dtype);  // K elements per step: 64 (fp16) or 32 (fp32
 bool gemm_tiled_eligible(int dtype, const GemmArgs &g, int transA, int transB, TiledRule rule = TILED_ANY);
 // Launch; with g.splits > 1 the fp32 partial sums go to g.ws for the caller to reduce.
 int gemm_tiled_launch(int dtype, const GemmArgs &g, int transA, int transB, hipStream_t stream);
+bool gemm_tiled_loose(int dtype, const GemmArgs &g, int transA, int transB);  // runs on the variant for rows that start anywhere
 // Two patch-matrix products as ONE launch: gx with patch rows as A (NN: a convolution's gradient of its input), gy with
 // patch k-rows as B (TN: its filter gradient; g.splits / tiles_per_split set, the caller reduces).  Workgroups of
 // both are resident side by side.  gemm_tiled_pair_workgroups: how many workgroups the launch would have, 0 when the

@@ -49,6 +49,11 @@ bool gemm_tiled_eligible(int dtype, const GemmArgs &g, int transA, int transB, T
     return dtype == D8_FLOAT16 ? eligible<f16>(g, transA, transB, rule) : eligible<float>(g, transA, transB, rule);
 }
 
+bool gemm_tiled_loose(int dtype, const GemmArgs &g, int transA, int transB) {
+    if (g.virt != VIRT_NONE) return false;
+    return dtype == D8_FLOAT16 ? !in_pieces<f16>(g, !transA, transB) : !in_pieces<float>(g, !transA, transB);
+}
+
 int gemm_tiled_launch(int dtype, const GemmArgs &g, int transA, int transB, hipStream_t stream) {
     if (g.virt == VIRT_NONE)
         return dtype == D8_FLOAT16 ? gemm_tiled_plain_f16(g, transA, transB, stream) : gemm_tiled_plain_f32(g, transA, transB, stream);
