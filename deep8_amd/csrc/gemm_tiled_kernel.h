@@ -65,7 +65,7 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 //                LDS; what a piece of a row stored along K brings in from past K is cut off there as well.  Rows
 //                keep their parity from step to step (K steps and passes are even numbers of rows), so shift and extra
 //                dword are constants of a thread.  Half 4096 x 1024 by 1024 x 1001, which a kernel that moved single elements
-//                served before: product with bias and ReLu 68 -> 29 us, its gradients 50 and 68 -> 21 and 22 us.  Bound by
+//                served before: product with bias and ReLu 68 -> 24 us, its gradients 50 and 68 -> 21 and 22 us.  Bound by
 //                the K loop's latency as the other variants, plus 60 vector instructions a step.
 enum { EDGE_NONE = 0, EDGE_PIECES = 1, EDGE_ANY = 2 };
 
@@ -315,16 +315,21 @@ struct RowMap {
     }
 };
 
-template <typename T, typename O>
+// LOOSE (the kernels for rows that start anywhere): the same with 16-byte accesses at the alignment of an element, and
+// element by element only where the eight columns of a lane cross the edge of what is this workgroup's.  Half 4096 x 1024 by
+// 1024 x 1001 with bias and ReLu: 28.2 -> 23.8 us; the element-wise store below asks for beta, bias and ReLu at
+// every one of its 64 elements a thread.
+template <typename T, typename O, bool LOOSE = false>
 __device__ __forceinline__ void store_tile(f32x16 (&acc)[T::TM][T::TN], float *lds0, float *lds1, O *C, int ldc, float beta,
                                            bool aligned, int N, const Origin &o, const RowMap &crow,
                                            const O *bias = nullptr, bool relu = false, bool round_first = false) {
     constexpr int TM = T::TM, TN = T::TN, OPV = 16 / sizeof(O);
     typedef O OV __attribute__((ext_vector_type(OPV)));
+    typedef OV MV __attribute__((aligned(LOOSE ? sizeof(O) : sizeof(OV))));  // as it lies in memory
     constexpr int HALF_WAVES = T::NT / 128;
     static_assert((size_t)T::PATCH_SZ * T::ES >= (size_t)HALF_WAVES * 32 * 36 * sizeof(float), "patch space");
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, lhi = lane >> 5;
-    if (aligned && N % 8 == 0 && !crow.perm_OC && ((size_t)bias & 15) == 0) {
+    if (!crow.perm_OC && (LOOSE || (aligned && N % 8 == 0 && ((size_t)bias & 15) == 0))) {
         float *patch = (wave < HALF_WAVES ? lds0 + wave * (32 * 36) : lds1 + (wave - HALF_WAVES) * (32 * 36));
 #pragma unroll
         for (int i = 0; i < TM; ++i)
@@ -339,25 +344,35 @@ __device__ __forceinline__ void store_tile(f32x16 (&acc)[T::TM][T::TN], float *l
                     float v[8];
                     *(f32x4 *)&v[0] = *(const f32x4 *)(patch + row * 36 + cc);
                     *(f32x4 *)&v[4] = *(const f32x4 *)(patch + row * 36 + cc + 4);
-                    if (m >= o.m_own && n >= o.n_own && m < o.m_end && n < o.n_end) {
+                    const bool in_m = m >= o.m_own && m < o.m_end, whole = !LOOSE || n + 8 <= o.n_end;
+                    if (in_m && n >= o.n_own && n < o.n_end && whole) {
                         O *c = C + crow(m) * ldc + n;
 #pragma unroll
                         for (int h = 0; h < 8 / OPV; ++h) {
                             OV out;
                             if (beta != 0.f) {
-                                const OV old = *(const OV *)(c + h * OPV);
+                                const OV old = *(const MV *)(c + h * OPV);
 #pragma unroll
                                 for (int e = 0; e < OPV; ++e) v[h * OPV + e] += as_f32(old[e]);
                             }
                             if (bias) {
-                                const OV bv = *(const OV *)(bias + n + h * OPV);
+                                const OV bv = *(const MV *)(bias + n + h * OPV);
 #pragma unroll
                                 for (int e = 0; e < OPV; ++e) v[h * OPV + e] = (round_first ? as_f32((O)v[h * OPV + e]) : v[h * OPV + e]) + as_f32(bv[e]);
                             }
 #pragma unroll
                             for (int e = 0; e < OPV; ++e) out[e] = (O)(relu && !(v[h * OPV + e] > 0.f) ? 0.f : v[h * OPV + e]);
-                            *(OV *)(c + h * OPV) = out;
+                            *(MV *)(c + h * OPV) = out;
                         }
+                    } else if (LOOSE && in_m) {
+                        O *c = C + crow(m) * ldc + n;
+                        for (int e = 0; e < 8; ++e)
+                            if (n + e >= o.n_own && n + e < o.n_end) {
+                                float w = patch[row * 36 + cc + e];
+                                if (beta != 0.f) w += as_f32(c[e]);
+                                if (bias) w = (round_first ? as_f32((O)w) : w) + as_f32(bias[n + e]);
+                                c[e] = (O)(relu && !(w > 0.f) ? 0.f : w);
+                            }
                     }
                 }
             }
@@ -729,11 +744,11 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     if (in_tail) {  // partial sums of the band, rows counted from its first
         const int tail_M = M - g.tail_m0;
         const Origin ot = {m0 - g.tail_m0, n0, m_own - g.tail_m0, n_own, tail_M, g.N, (wm * TM) * 32, (wn * TN) * 32};
-        store_tile<T, float>(acc, patches, patches1, g.ws + ((long)split * tail_M) * g.N, g.N, 0.f, true, g.N, ot, plain);
+        store_tile<T, float, EDGE == EDGE_ANY>(acc, patches, patches1, g.ws + ((long)split * tail_M) * g.N, g.N, 0.f, true, g.N, ot, plain);
     } else if (g.splits > 1)
-        store_tile<T, float>(acc, patches, patches1, g.ws + ((long)(b * g.splits + split) * g.M) * g.N, g.N, 0.f, true, g.N, o, plain);
+        store_tile<T, float, EDGE == EDGE_ANY>(acc, patches, patches1, g.ws + ((long)(b * g.splits + split) * g.M) * g.N, g.N, 0.f, true, g.N, o, plain);
     else
-        store_tile<T, E>(acc, patches, patches1, (E *)g.C + (long)b * g.sC, g.ldc, g.beta,
+        store_tile<T, E, EDGE == EDGE_ANY>(acc, patches, patches1, (E *)g.C + (long)b * g.sC, g.ldc, g.beta,
                          g.ldc % EPV == 0 && g.sC % EPV == 0 && ((size_t)g.C & 15) == 0, g.N, o, crow, (const E *)g.bias, g.relu != 0,
                          ES == 2 && g.round_first != 0);
     if (g.phase_rec) {
