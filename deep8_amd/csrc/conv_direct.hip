@@ -509,13 +509,17 @@ bool plan_grad(int dtype, const DirectShape &s, const void *x, const void *gz, D
 
 bool conv_direct_eligible(int dtype, const DirectShape &s) {
     if (dtype != D8_FLOAT16 && dtype != D8_FLOAT32) return false;
+    // More than 192 output channels: the image's fragments are built again for every block of channels, which costs more than
+    // the patch matrix saves (forward, gate and filter gradient, before and with these kernels: fp32 8 x 116x116x3 -> 320 5x5
+    // 339 / 462 us, half 30 x 47x47x3 -> 320 5x5 126 / 127; fp32 148x148x1 -> 152 5x5 75 / 49, half 33 x 85x85x1 -> 128 3x3 74 / 45)
+    if (s.OC > 192) return false;
     if (s.dx != 1 || (long)s.FH * s.FW * s.C >= 4096 || pieces_of(dtype, s) > 2 * most_groups(dtype)) return false;
     DirectArgs a;
     size_t lds;
     return plan_forward(dtype, s, nullptr, a, lds) && plan_grad(dtype, s, nullptr, nullptr, a, lds);
 }
 
-// Every layer of the shape qualifies: on these sizes the interim matrix lost everywhere it was measured.  Half 16 x
+// Up to 192 channels the interim matrix lost everywhere it was measured.  Half 16 x
 // 224x224x3 -> 64, 7x7 stride 2 (K = 147): patch matrix + padded filter + product 81 -> 23 us (26 MB are stored: 5 us at a
 // copy's rate; what the rest goes on is the way of a tile's rows from memory to the first fragment); fp32 64 x 28x28x1 -> 32,
 // 5x5: patch matrix + product 18 -> 11 us.
