@@ -771,8 +771,11 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
 
 // (EDGE: instantiations of their own, so that the per-piece offsets of the ordinary case stay constants; patch k-rows as B
 // need none)
+// (classes on 128 x 128 tiles: left to itself the compiler takes 280 registers for the addresses of the element-wise store,
+// which leaves room for one workgroup per compute unit; told to make room for two it takes 186 and spills none.  Half DeConv2d
+// 32 x 20x20x128 -> 128, 2x2 stride 2, 15.7 -> 11.0 us; 24 x 26x26x448 -> 288, 4x4 stride 2, 150 -> 119 us)
 template <typename T, int EDGE = EDGE_NONE>
-__global__ __launch_bounds__(T::NT) void gemm_tiled_kernel(GemmArgs g, int tilesM, int tilesN) {
+__global__ __launch_bounds__(T::NT, T::VIRT == VIRT_A_CLASSES && T::BN == 128 ? 2 : 1) void gemm_tiled_kernel(GemmArgs g, int tilesM, int tilesN) {
     typedef typename T::E E;
     // four separate arrays, so that reads of one half are known not to touch the other
     __shared__ __attribute__((aligned(16))) E As0[T::A_SZ];
