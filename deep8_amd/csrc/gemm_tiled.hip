@@ -20,6 +20,9 @@ static bool eligible(const GemmArgs &g, int transA, int transB, TiledRule rule) 
     if (va && (transA || g.K != g.pg.C)) return false;                       // a K step stays inside one tap
     if (vb && (!transA || transB || g.red != 1 || g.pg.C % EPV || g.N % g.pg.C)) return false;  // a piece stays inside one tap
     if ((va || vb) && (g.pg.bytes >= (1u << 31) || g.batch != 1)) return false;
+    // (pixels past the last, in a last partial step, are told from the image by their 32-bit byte offset, which must not come
+    // round to its start: one output pixel per image of 64 MiB, say)
+    if (vb && ((g.K + BK - 1) / BK * BK - 1) / ((long)g.pg.OH * g.pg.OW) + 1 > (1L << 32) / (ES * g.pg.H * g.pg.W * g.pg.C)) return false;
     // byte offsets inside one operand (all summed products of it included) are 32-bit
     if (!va && ((g.red - 1) * g.sA + (long)(transA ? g.K : g.M) * g.lda) * ES >= (1L << 31)) return false;
     if (!vb && ((g.red - 1) * g.sB + (long)(transB ? g.N : g.K) * g.ldb) * ES >= (1L << 31)) return false;

@@ -63,3 +63,24 @@ def test_partial_steps_without_interim_matrix(oracle_port, op, cfg, dtype):
         for scratch in (0, asked):
             got = _call(lib, name, dt, bufs, shape, filt, g, nan, scratch)
             assert np.array_equal(got, want[which]), (which, scratch)
+
+
+def test_pixels_past_the_last_of_a_large_image():
+    """one output pixel on an image of 77 MB: the 63 pixels that fill the K step up lie up to 4.9 GB past the image, whose other
+    elements (NaN) they must not meet"""
+    from deep8_amd import capi
+    from deep8_amd.capi import DeviceArray, check
+    lib = capi.init()
+    size, IC, OC, F = 2200, 8, 64, 3
+    geo = (0, size, size, 1, 1)
+    x = np.full((1, size, size, IC), np.nan, np.float16)
+    r = rng(5)
+    x[0, :F, :F] = ints(r, (F, F, IC), 5)
+    gz = ints(r, (1, 1, 1, OC), 5)
+    want = gz.reshape(OC, 1, 1, 1) * f(x[:, :F, :F])
+    shape, filt = (1, size, size, IC), (OC, F, F)
+    need = lib.d8_conv2d_scratch_bytes(capi.FLOAT16, 2, *shape, *filt, *geo)
+    dx, dg, out = DeviceArray.from_numpy(x), DeviceArray.from_numpy(h(gz)), DeviceArray.from_numpy(np.full(want.shape, np.nan, np.float16))
+    ws = DeviceArray((need,), np.uint8)
+    check(lib.d8_conv2d_grad_y_overwrite(capi.FLOAT16, dx.ptr, *shape, out.ptr, *filt, dg.ptr, *geo, ws.ptr, need, None))
+    assert np.array_equal(f(out.numpy()), want)
