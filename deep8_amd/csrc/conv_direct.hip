@@ -548,7 +548,8 @@ int conv_direct_forward(int dtype, const DirectShape &s, const void *x, const vo
 }
 
 // One workgroup per compute unit (10 waves for 147 columns): the partial sums are OC * K floats each, and a second workgroup
-// would double what is written and read again.  The layers above: 82 -> 28 us, 29 -> 13 us, both with the reduction.
+// would double what is written and read again.  In all, rounded down: with one workgroup more a compute unit holds two, and the
+// others wait for it (half 18 x 221x173x3 -> 192, 7x7, three groups of channels: 3 x 86 workgroups 486 us, 3 x 85 258).  The layers above: 82 -> 28 us, 29 -> 13 us, both with the reduction.
 bool conv_direct_grad_y(int dtype, const DirectShape &s, const void *x, void *gw, const void *gz, float beta, void *ws,
                         size_t ws_bytes, hipStream_t stream, int *rc) {
     DirectArgs a;
@@ -556,7 +557,7 @@ bool conv_direct_grad_y(int dtype, const DirectShape &s, const void *x, void *gw
     if (!plan_grad(dtype, s, x, gz, a, lds)) return false;
     const int nb = s.OC > 32 ? 2 : 1, oc_tiles = ceil_div(s.OC, nb * 32);
     const size_t one = (size_t)s.OC * a.K * sizeof(float);
-    long wgs = ceil_div(cu_count(), oc_tiles);
+    long wgs = oc_tiles < cu_count() ? cu_count() / oc_tiles : 1;
     if (wgs > a.ntiles) wgs = a.ntiles;
     if (wgs > (long)(ws_bytes / one)) wgs = (long)(ws_bytes / one);
     if (wgs < 1 || ((size_t)ws & 3)) return false;
