@@ -13,6 +13,12 @@ struct DirectShape {
 // Whether the kernels take this layer: Float32 / Float16, dilation 1 along x, and a patch row that, with each of its FH
 // runs of FW * C elements filled up to 16-byte pieces, fits the registers a wave keeps the filter in.
 bool conv_direct_eligible(int dtype, const DirectShape &s);
+// Microseconds that an eligible layer is expected to take on them (the gradient: infinite where ws_bytes do not hold the partial
+// sums of one workgroup per 64 output channels).
+double conv_direct_forward_us(int dtype, const DirectShape &s, const void *x);
+double conv_direct_grad_us(int dtype, const DirectShape &s, const void *x, const void *gz, size_t ws_bytes);
+// Partial sums of all the workgroups that the gradient would have.
+size_t conv_direct_grad_bytes(int dtype, const DirectShape &s);
 // z = conv(x, w) [+ bias] [relu]; round_first as GemmArgs::round_first.
 int conv_direct_forward(int dtype, const DirectShape &s, const void *x, const void *w, void *z, const void *bias, int relu,
                         int round_first, hipStream_t stream);

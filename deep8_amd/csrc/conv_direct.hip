@@ -14,6 +14,8 @@
 //             in fp32) consecutive pixels of a row, i.e. strided single elements; dz is staged beside the image and read
 //             transposed.  Waves beyond the n blocks take every other group of pixels and meet in LDS, workgroups leave
 //             partial sums that conv_direct_reduce_kernel adds in a fixed order.
+#include <cmath>
+
 #include "conv_direct.h"
 #include "gemm_tiled_kernel.h"
 
@@ -509,17 +511,63 @@ bool plan_grad(int dtype, const DirectShape &s, const void *x, const void *gz, D
 
 bool conv_direct_eligible(int dtype, const DirectShape &s) {
     if (dtype != D8_FLOAT16 && dtype != D8_FLOAT32) return false;
-    // More than 192 output channels: the image's fragments are built again for every block of channels, which costs more than
-    // the patch matrix saves (forward, gate and filter gradient, before and with these kernels: fp32 8 x 116x116x3 -> 320 5x5
-    // 339 / 462 us, half 30 x 47x47x3 -> 320 5x5 126 / 127; fp32 148x148x1 -> 152 5x5 75 / 49, half 33 x 85x85x1 -> 128 3x3 74 / 45)
-    if (s.OC > 192) return false;
     if (s.dx != 1 || (long)s.FH * s.FW * s.C >= 4096 || pieces_of(dtype, s) > 2 * most_groups(dtype)) return false;
     DirectArgs a;
     size_t lds;
     return plan_forward(dtype, s, nullptr, a, lds) && plan_grad(dtype, s, nullptr, nullptr, a, lds);
 }
 
-// Up to 192 channels the interim matrix lost everywhere it was measured.  Half 16 x
+// What the kernels take, fitted to 4776 calls on 2500 drawn layers (1 - 170 channels to 8 - 512, both types; half of the calls
+// within 7 % of the estimate, nine tenths of the forward ones within 20 %).  Forward: the filter's way into registers, a
+// tile's accesses to the image, a wave's blocks of 32 pixels (products and stores); the image's fragments are built again for
+// every 64 (fp32: 32) output channels.
+double conv_direct_forward_us(int dtype, const DirectShape &s, const void *x) {
+    DirectArgs a;
+    size_t lds;
+    if (!plan_forward(dtype, s, x, a, lds)) return INFINITY;
+    const bool half = dtype == D8_FLOAT16;
+    const int es = half ? 2 : 4, ch = forward_channels(dtype, s), groups = ceil_div(pieces_of(dtype, s), 2), cus = cu_count();
+    const int kept = half ? (groups <= 3 ? 3 : groups <= 5 ? 5 : 11) : (groups <= 5 ? 5 : groups <= 10 ? 10 : 21);
+    const long wide = a.ntiles < 2 * cus ? a.ntiles : 2 * cus, wgs = wide * ceil_div(s.OC, ch), per_cu = (wgs + cus - 1) / cus;
+    const double rounds = (double)((wgs + 2 * cus - 1) / (2 * cus)), tiles = (double)((a.ntiles + wide - 1) / wide);
+    const double blocks = per_cu * tiles * ceil_div(ceil_div(a.TR * a.TC, 32), 4), accesses = rounds * tiles * ceil_div(a.rows * (a.pitch / a.vec_x), 256);
+    const double filter = rounds * ch * a.K / 1000.0, single = s.OC % (16 / es) ? blocks * (ch / 32) : 0.0;
+    if (half) return 4.2 + 0.04 * blocks * kept + 0.57 * blocks * (ch / 32) + 0.55 * single + 0.14 * accesses + 0.31 * filter;
+    return 4.4 + 0.185 * blocks * kept + 0.5 * single + 0.15 * accesses + 0.48 * filter + 0.105e-6 * es * s.B * s.OH * s.OW * (double)s.OC;
+}
+
+static long grad_workgroups(const DirectArgs &a, const DirectShape &s) {
+    const int oc_tiles = ceil_div(s.OC, s.OC > 32 ? 64 : 32);
+    const long most = oc_tiles < cu_count() ? cu_count() / oc_tiles : 1;
+    return most < a.ntiles ? most : a.ntiles;
+}
+
+size_t conv_direct_grad_bytes(int dtype, const DirectShape &s) {
+    DirectArgs a;
+    size_t lds;
+    return plan_grad(dtype, s, nullptr, nullptr, a, lds) ? (size_t)grad_workgroups(a, s) * s.OC * a.K * sizeof(float) : 0;
+}
+
+// Gradient: per tile a wave's groups of pixels, and the accesses to dz and the image (single ones where a row or a pixel's
+// channels are no multiple of 16 bytes, which do not overlap the products); then the partial sums.
+double conv_direct_grad_us(int dtype, const DirectShape &s, const void *x, const void *gz, size_t ws_bytes) {
+    DirectArgs a;
+    size_t lds;
+    if (!plan_grad(dtype, s, x, gz, a, lds)) return INFINITY;
+    const bool half = dtype == D8_FLOAT16;
+    const int epv = half ? 8 : 4, nb = s.OC > 32 ? 2 : 1, waves = grad_waves(a.kb), nt = 64 * waves;
+    const size_t one = (size_t)s.OC * a.K * sizeof(float);
+    long wgs = grad_workgroups(a, s);
+    if (wgs > (long)(ws_bytes / one)) wgs = (long)(ws_bytes / one);
+    if (wgs < 1) return INFINITY;
+    const double tiles = (double)((a.ntiles + wgs - 1) / wgs), groups = ceil_div(a.pixels_p / (2 * epv), waves / a.kb) * nb;
+    const double image = ceil_div(a.rows * (a.pitch / a.vec_x), nt), dz = ceil_div((long)a.pixels_p * nb * 32 / a.vec_z, nt);
+    const bool ahead = a.vec_x == epv && a.vec_z == epv && a.rows * (a.pitch / epv) <= 3 * nt && a.pixels_p * (nb * 32 / epv) <= 4 * nt;
+    const double staging = ahead ? (half ? 0.04 : 0.15) * (image + dz) : 0.115 * image + 0.225 * dz + (half ? 0.0 : 0.45);
+    return 6.7 + tiles * ((half ? 1.2 + 0.147 * groups : 0.44 + 0.33 * groups) + staging) + 0.77e-6 * wgs * one;
+}
+
+// Half 16 x
 // 224x224x3 -> 64, 7x7 stride 2 (K = 147): patch matrix + padded filter + product 81 -> 23 us (26 MB are stored: 5 us at a
 // copy's rate; what the rest goes on is the way of a tile's rows from memory to the first fragment); fp32 64 x 28x28x1 -> 32,
 // 5x5: patch matrix + product 18 -> 11 us.
@@ -557,8 +605,7 @@ bool conv_direct_grad_y(int dtype, const DirectShape &s, const void *x, void *gw
     if (!plan_grad(dtype, s, x, gz, a, lds)) return false;
     const int nb = s.OC > 32 ? 2 : 1, oc_tiles = ceil_div(s.OC, nb * 32);
     const size_t one = (size_t)s.OC * a.K * sizeof(float);
-    long wgs = oc_tiles < cu_count() ? cu_count() / oc_tiles : 1;
-    if (wgs > a.ntiles) wgs = a.ntiles;
+    long wgs = grad_workgroups(a, s);
     if (wgs > (long)(ws_bytes / one)) wgs = (long)(ws_bytes / one);
     if (wgs < 1 || ((size_t)ws & 3)) return false;
     a.w = gz, a.ws = (float *)ws;

@@ -173,6 +173,8 @@ bool gemm_tiled_run_pair(int dtype, GemmArgs &gx, GemmArgs &gy, void *workspace,
 // The workspace holds both products' partial sums side by side.
 bool gemm_tiled_run_plain_pair(int dtype, GemmArgs &g0, int ta0, int tb0, GemmArgs &g1, int ta1, int tb1, void *workspace,
                                size_t workspace_bytes, hipStream_t stream, int *rc);
+// Microseconds that a product is expected to take with all the workspace it asks for (which of two ways a convolution goes).
+double gemm_estimate_us(int dtype, const GemmArgs &g, int transA, int transB);
 // Workspace gemm_tiled_run may use for this shape.
 size_t gemm_tiled_workspace(int dtype, int M, int N, int K, int red, int virt = VIRT_NONE);
 // Whether a product whose B is a patch matrix (VIRT_B_KROWS) runs on 64 x 64 tiles: fewer than 128 rows, and the last

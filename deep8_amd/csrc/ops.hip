@@ -161,6 +161,43 @@ static int implicit_run(int dtype, GemmArgs &g, int ta, int tb, void *scratch, s
     return gemm_tiled_run(dtype, g, ta, tb, scratch, scratch_bytes, stream);
 }
 
+// How many convolution calls (a gradient is one) have gone which way: d8_conv_route_calls.
+enum { ROUTE_INTERIM = 0, ROUTE_PATCH = 1, ROUTE_DIRECT = 2 };
+static std::atomic<unsigned long> route_calls[3];
+
+// Microseconds of a product and of the map that writes (reads) its interim matrix.  What a map takes per byte of the matrix
+// depends on what it can move at once: 16 bytes of a pixel's channels, 16 bytes of a padded row gathered from single elements, or
+// single elements.  (2500 drawn layers, forward and filter gradient: half within 7 %, nine tenths within 30 % of this.)
+static double interim_us(int dtype, const Gemm &product, double elements, int channels, bool padded) {
+    const bool half = dtype == D8_FLOAT16;
+    const GemmArgs g = to_args(product);
+    const double bytes = elements * (half ? 2 : 4);
+    const double rate = padded ? (half ? 1.0 : 0.63) : channels % (half ? 8 : 4) == 0 ? 0.42 : half ? 2.1 : 1.22;  // us per MB
+    const double slower = half && gemm_tiled_loose(dtype, g, product.ta, product.tb) ? 1.5 : 1.0;
+    return 3.0 + (padded ? 2.5 : 0.0) + 1e-6 * rate * bytes + slower * gemm_estimate_us(dtype, g, product.ta, product.tb);
+}
+
+// Whether a layer whose patches the tile loader can read runs on the interim matrix all the same.  Layers of whole K steps and
+// whole tiles never do.  For the others either way can win: a K step ends with its tap, so that few channels multiply mostly
+// padding (fp32 17 x 104x104x8 -> 128, 3x3: 125 us in the loader, 82 on the matrix), classes of output pixels are not cut into
+// pieces (fp32 DeConv2d 3 x 6x6x480 -> 352, 3x3 stride 2: 116 and 17), filter gradients have no 64 x 64 tiles beside wider
+// outputs (fp32 Conv2d 29 x 13x13 -> 128, 464 pixels, N = 360: 35 and 11); while the matrix moves
+// FH * FW / stride^2 times the image (half 72 x 41x41x480 -> 64, 3x3: 145 and 583 us).  What both are expected to take decides.
+// Without room for the matrix the loader serves.  Over 3578 calls on drawn layers: 115 ms on the matrix, 76 in the loader, 72.5 with
+// the better of the two, 73.2 with this choice.
+// (col2im: the matrix is the gradient of the patches, and what it is added up in may have to be cleared first.  Counted whether
+// or not it has to be: a call that adds takes the same way as one that overwrites.)
+static bool prefer_interim(int dtype, const GemmArgs &patch, int ta, int tb, const Gemm &product, double elements, int channels, bool col2im,
+                           const void *scratch, size_t scratch_bytes) {
+    if (dtype == D8_FLOAT64 || !scratch || (double)scratch_bytes < elements * dtype_bytes(dtype)) return false;
+    GemmArgs g = patch;
+    if (g.virt == VIRT_A_CLASSES)  // (g.M is the largest one's)
+        for (int i = 0; i < g.ncls; ++i)
+            if (g.cls[i].M < g.M) g.M = g.cls[i].M;
+    if (gemm_tiled_eligible(dtype, g, ta, tb, TILED_WHOLE)) return false;
+    return interim_us(dtype, product, elements, channels, false) + (col2im ? 3.0 : 0.0) < gemm_estimate_us(dtype, patch, ta, tb);
+}
+
 // Float64 gradient of x: the product's N is the input channel count, and under 128 channels the fp64 kernel is
 // left with its 64 x 64 tiles, half the flops per operand byte of the 128 x 128 tiles that the staged product
 // ([patch rows] x [taps x channels]) runs on -- measured at B32 56x56x64 3x3: 0.53 ms against 0.42 ms staged,
@@ -336,6 +373,8 @@ int d8_matmul_grad_y_overwrite(int dtype, const void *x, int xb, int xr, int xc,
     return run(dtype, mm_plan(2, x, xb, xr, xc, dy, yb, yr, yc, dz, 0.f), scratch, scratch_bytes, stream);
 }
 
+unsigned long d8_conv_route_calls(int route) { return route >= 0 && route < 3 ? route_calls[route].load() : 0; }
+
 static std::atomic<unsigned long> matmul_pair_launches{0};
 unsigned long d8_matmul_grad_pair_launches(void) { return matmul_pair_launches.load(); }
 
@@ -455,10 +494,20 @@ static PaddedScratch conv_padded_scratch(int dtype, int which, int M, int OC, in
     return s;
 }
 
-// Layers that stage a patch matrix only because the tile loader cannot read their image (1 or 3 channels) run on the
-// kernels that read it from LDS.
-static bool conv_direct(int dtype, const DirectShape &s) {
-    return getenv("D8_CONV_EXPLICIT") == nullptr && conv_direct_eligible(dtype, s);
+// Layers of few channels (1 or 3, an image's) that would stage a patch matrix have kernels that read the image from LDS
+// (conv_direct.hip).  They take the layer where they are expected to be faster than the matrix: many output channels build the
+// image's fragments again and again, rows or channels that cannot be moved 16 bytes at a time are staged element by element
+// (filter gradient of half 17 x 137x137x3 -> 142, 3x3: 430 us, 73 on the matrix; 16 x 224x224x3 -> 64, 7x7 stride 2: 28 and 82).
+// 2479 forward calls on drawn layers: 42.3 ms on those kernels, 56.6 on the matrix, 40.8 by this rule, 39.3 at best; 2297 filter
+// gradients: 60.4, 54.0, 44.5 and 43.0.
+static bool prefer_direct(int dtype, int which, const DirectShape &s, const void *x, const void *gz, const void *scratch, size_t scratch_bytes) {
+    if (getenv("D8_CONV_EXPLICIT") != nullptr || !conv_direct_eligible(dtype, s)) return false;
+    if (getenv("D8_CONV_DIRECT") != nullptr) return true;  // test aid: wherever they can
+    const int M = s.B * s.OH * s.OW, K = s.FH * s.FW * s.C, pitch = conv_padded_pitch(dtype, K, s.OC), columns = pitch ? pitch : K;
+    const bool padded = pitch && (scratch_bytes >= conv_padded_scratch(dtype, which, M, s.OC, pitch).total);
+    const double interim = interim_us(dtype, conv_plan(which, M, columns, s.OC, nullptr, nullptr, nullptr), (double)M * columns, s.C, padded);
+    if (which == 0) return conv_direct_forward_us(dtype, s, x) < interim + 0.25e-6 * M * (double)s.OC * dtype_bytes(dtype);
+    return ((size_t)scratch & 3) == 0 && conv_direct_grad_us(dtype, s, x, gz, scratch_bytes) < interim;
 }
 
 size_t d8_conv2d_scratch_bytes(int dtype, int which, int B, int IH, int IW, int IC,
@@ -478,12 +527,18 @@ size_t d8_conv2d_scratch_bytes(int dtype, int which, int B, int IH, int IW, int 
     bool untouched = false;
     if (which == 1 && conv_classes_grad_x(dtype, cs, nullptr, nullptr, nullptr, ga, &untouched)) return 0;
     const size_t col = align256((size_t)M * K * dtype_bytes(dtype));
-    const size_t plain = col + gemm_ws(dtype, conv_plan(which, M, K, OC, nullptr, nullptr, nullptr));
+    size_t most = col + gemm_ws(dtype, conv_plan(which, M, K, OC, nullptr, nullptr, nullptr));
     if (const int pitch = conv_padded_pitch(dtype, K, OC)) {
         const size_t padded = conv_padded_scratch(dtype, which, M, OC, pitch).total;
-        return padded > plain ? padded : plain;
+        if (padded > most) most = padded;
     }
-    return plain;
+    // (few pixels: the partial sums of the kernels that read the image from LDS are more than the patch matrix)
+    const DirectShape ds = {B, IH, IW, IC, OC, FH, FW, g[0], g[1], sy, sx, dy, dx, g[2], g[3]};
+    if (which == 2 && prefer_direct(dtype, 2, ds, nullptr, nullptr, nullptr, (size_t)-1)) {
+        const size_t sums = conv_direct_grad_bytes(dtype, ds);
+        if (sums > most) most = sums;
+    }
+    return most;
 }
 
 static int conv2d_impl(int dtype, const void *x, int B, int IH, int IW, int IC,
@@ -500,7 +555,9 @@ static int conv2d_impl(int dtype, const void *x, int B, int IH, int IW, int IC,
         const ConvShape cs = {B, IH, IW, IC, OC, FH, FW, g[0], g[1], sy, sx, dy, dx, g[2], g[3]};
         GemmArgs ga;
         int ta, tb;
-        if (conv_implicit_plan(dtype, 0, cs, x, w, z, ga, ta, tb)) {
+        if (conv_implicit_plan(dtype, 0, cs, x, w, z, ga, ta, tb) &&
+            !prefer_interim(dtype, ga, ta, tb, conv_plan(0, M, K, OC, scratch, w, z), (double)M * K, IC, false, scratch, scratch_bytes)) {
+            ++route_calls[ROUTE_PATCH];
             ga.bias = bias, ga.relu = relu;  // applied in the tile store (and in the remainder band's reduction)
             ga.round_first = !gemm_tiled_eligible(dtype, ga, ta, tb, TILED_WHOLE) &&
                              !gemm_fuses_store(dtype, to_args(conv_plan(0, M, K, OC, nullptr, w, z)), 0, 1, TILED_PIECES);
@@ -510,13 +567,15 @@ static int conv2d_impl(int dtype, const void *x, int B, int IH, int IW, int IC,
     if (int rc = need_scratch("d8_conv2d", scratch, scratch_bytes, (size_t)M * K * dtype_bytes(dtype), x, w, z)) return rc;
     {
         const DirectShape ds = {B, IH, IW, IC, OC, FH, FW, g[0], g[1], sy, sx, dy, dx, g[2], g[3]};
-        if (conv_direct(dtype, ds)) {
+        if (prefer_direct(dtype, 0, ds, x, nullptr, scratch, scratch_bytes)) {
             // (in half the layers whose bias used to be added by a pass of its own find the product rounded)
             const int pitch = conv_padded_pitch(dtype, K, OC);
             const int round_first = !gemm_fuses_store(dtype, to_args(conv_plan(0, M, pitch ? pitch : K, OC, nullptr, pitch ? nullptr : w, z)), 0, 1, TILED_PIECES);
+            ++route_calls[ROUTE_DIRECT];
             return conv_direct_forward(dtype, ds, x, w, z, bias, relu, round_first, as_stream(stream));
         }
     }
+    ++route_calls[ROUTE_INTERIM];
     if (const int pitch = conv_padded_pitch(dtype, K, OC)) {
         const PaddedScratch ps = conv_padded_scratch(dtype, 0, M, OC, pitch);
         if (scratch_bytes >= ps.total && ((size_t)scratch & 15) == 0) {  // a smaller scratch still serves the plain route
@@ -563,12 +622,17 @@ static int d8_conv2d_grad_x_impl(int dtype, void *gx, int B, int IH, int IW, int
         const ConvShape cs = {B, IH, IW, IC, OC, FH, FW, g[0], g[1], sy, sx, dy, dx, g[2], g[3]};
         GemmArgs ga;
         int ta, tb;
-        if (conv_implicit_plan(dtype, 1, cs, gx, w, gz, ga, ta, tb)) {
+        const Gemm product = conv_plan(1, M, K, OC, scratch, w, gz);
+        if (conv_implicit_plan(dtype, 1, cs, gx, w, gz, ga, ta, tb) &&
+            !prefer_interim(dtype, ga, ta, tb, product, (double)M * K, IC, true, scratch, scratch_bytes)) {
+            ++route_calls[ROUTE_PATCH];
             ga.beta = beta;
             return implicit_run(dtype, ga, ta, tb, scratch, scratch_bytes, as_stream(stream));
         }
         bool untouched = false;
-        if (conv_classes_grad_x(dtype, cs, gx, w, gz, ga, &untouched)) {
+        if (conv_classes_grad_x(dtype, cs, gx, w, gz, ga, &untouched) &&
+            !prefer_interim(dtype, ga, 0, 0, product, (double)M * K, IC, true, scratch, scratch_bytes)) {
+            ++route_calls[ROUTE_PATCH];
             if (untouched && beta == 0.f) {  // pixels of dx that no tap reaches: zero, and the classes add to that
                 if (int rc = d8_fill(dtype, gx, (size_t)B * IH * IW * IC, 0.f, stream)) return rc;
                 beta = 1.f;
@@ -578,6 +642,7 @@ static int d8_conv2d_grad_x_impl(int dtype, void *gx, int B, int IH, int IW, int
         }
     }
     if (int rc = need_scratch("d8_conv2d_grad_x", scratch, scratch_bytes, (size_t)M * K * dtype_bytes(dtype), gx, w, gz)) return rc;
+    ++route_calls[ROUTE_INTERIM];
     if (const int pitch = conv_padded_pitch(dtype, K, OC)) {
         const PaddedScratch ps = conv_padded_scratch(dtype, 1, M, OC, pitch);
         if (scratch_bytes >= ps.total && ((size_t)scratch & 15) == 0) {
@@ -613,7 +678,9 @@ static int d8_conv2d_grad_y_impl(int dtype, const void *x, int B, int IH, int IW
         const ConvShape cs = {B, IH, IW, IC, OC, FH, FW, g[0], g[1], sy, sx, dy, dx, g[2], g[3]};
         GemmArgs ga;
         int ta, tb;
-        if (conv_implicit_plan(dtype, 2, cs, x, gw, gz, ga, ta, tb)) {
+        if (conv_implicit_plan(dtype, 2, cs, x, gw, gz, ga, ta, tb) &&
+            !prefer_interim(dtype, ga, ta, tb, conv_plan(2, M, K, OC, scratch, gw, gz), (double)M * K, IC, false, scratch, scratch_bytes)) {
+            ++route_calls[ROUTE_PATCH];
             ga.beta = beta;
             return implicit_run(dtype, ga, ta, tb, scratch, scratch_bytes, as_stream(stream));
         }
@@ -622,8 +689,12 @@ static int d8_conv2d_grad_y_impl(int dtype, const void *x, int B, int IH, int IW
     {
         const DirectShape ds = {B, IH, IW, IC, OC, FH, FW, g[0], g[1], sy, sx, dy, dx, g[2], g[3]};
         int rc = 0;
-        if (conv_direct(dtype, ds) && conv_direct_grad_y(dtype, ds, x, gw, gz, beta, scratch, scratch_bytes, as_stream(stream), &rc)) return rc;
+        if (prefer_direct(dtype, 2, ds, x, gz, scratch, scratch_bytes) && conv_direct_grad_y(dtype, ds, x, gw, gz, beta, scratch, scratch_bytes, as_stream(stream), &rc)) {
+            ++route_calls[ROUTE_DIRECT];
+            return rc;
+        }
     }
+    ++route_calls[ROUTE_INTERIM];
     if (const int pitch = conv_padded_pitch(dtype, K, OC)) {
         const PaddedScratch ps = conv_padded_scratch(dtype, 2, M, OC, pitch);
         if (scratch_bytes >= ps.total && ((size_t)scratch & 15) == 0) {
@@ -804,13 +875,16 @@ static int deconv2d_impl(int dtype, const void *x, int B, int IH, int IW, int IC
     {
         GemmArgs ga;
         bool untouched = false;
-        if (deconv_implicit_fwd(dtype, B, IH, IW, IC, OC, FH, FW, sy, sx, g, x, w, z, ga, &untouched)) {
+        if (deconv_implicit_fwd(dtype, B, IH, IW, IC, OC, FH, FW, sy, sx, g, x, w, z, ga, &untouched) &&
+            !prefer_interim(dtype, ga, 0, 1, deconv_plan(0, M, T, OC, IC, scratch, w, x), (double)M * T * OC, OC, false, scratch, scratch_bytes)) {
+            ++route_calls[ROUTE_PATCH];
             if (untouched)  // the pixels between the filter's footprints stay zero
                 if (int rc = d8_fill(dtype, z, (size_t)B * g[0] * g[1] * OC, 0.f, stream)) return rc;
             return implicit_run(dtype, ga, 0, 1, nullptr, 0, as_stream(stream));
         }
     }
     if (int rc = need_scratch("d8_deconv2d", scratch, scratch_bytes, (size_t)M * T * OC * dtype_bytes(dtype), x, w, z)) return rc;
+    ++route_calls[ROUTE_INTERIM];
     const size_t ws = scratch_bytes > mat ? scratch_bytes - mat : 0;
     if (int rc = run(dtype, deconv_plan(0, M, T, OC, IC, scratch, w, x), ws ? (char *)scratch + mat : nullptr, ws, stream))
         return rc;
@@ -847,12 +921,15 @@ static int deconv2d_grad_x_geo(int dtype, void *gx, int B, int IH, int IW, int I
     if (int rc = check_deconv_out("d8_deconv2d_grad_x", B, g)) return rc;
     {
         GemmArgs ga;
-        if (deconv_implicit_grad_x(dtype, B, IH, IW, IC, OC, FH, FW, sy, sx, g, gx, w, gz, ga)) {
+        if (deconv_implicit_grad_x(dtype, B, IH, IW, IC, OC, FH, FW, sy, sx, g, gx, w, gz, ga) &&
+            !prefer_interim(dtype, ga, 0, 0, deconv_plan(1, M, T, OC, IC, scratch, w, gx), (double)M * T * OC, OC, false, scratch, scratch_bytes)) {
+            ++route_calls[ROUTE_PATCH];
             ga.beta = beta;
             return implicit_run(dtype, ga, 0, 0, scratch, scratch_bytes, as_stream(stream));
         }
     }
     if (int rc = need_scratch("d8_deconv2d_grad_x", scratch, scratch_bytes, (size_t)M * T * OC * dtype_bytes(dtype), gx, w, gz)) return rc;
+    ++route_calls[ROUTE_INTERIM];
     if (int rc = launch_im2col(dtype, gz, scratch, deconv_mirror(B, IH, IW, OC, FH, FW, sy, sx, g), as_stream(stream)))
         return rc;
     const size_t ws = scratch_bytes > mat ? scratch_bytes - mat : 0;
@@ -891,12 +968,15 @@ static int deconv2d_grad_y_geo(int dtype, const void *x, int B, int IH, int IW, 
     if (int rc = check_deconv_out("d8_deconv2d_grad_y", B, g)) return rc;
     {
         GemmArgs ga;
-        if (deconv_implicit_grad_y(dtype, B, IH, IW, IC, OC, FH, FW, sy, sx, g, x, gw, gz, ga)) {
+        if (deconv_implicit_grad_y(dtype, B, IH, IW, IC, OC, FH, FW, sy, sx, g, x, gw, gz, ga) &&
+            !prefer_interim(dtype, ga, 1, 0, deconv_plan(2, M, T, OC, IC, scratch, gw, x), (double)M * T * OC, OC, false, scratch, scratch_bytes)) {
+            ++route_calls[ROUTE_PATCH];
             ga.beta = beta;
             return implicit_run(dtype, ga, 1, 0, scratch, scratch_bytes, as_stream(stream));
         }
     }
     if (int rc = need_scratch("d8_deconv2d_grad_y", scratch, scratch_bytes, (size_t)M * T * OC * dtype_bytes(dtype), x, gw, gz)) return rc;
+    ++route_calls[ROUTE_INTERIM];
     if (int rc = launch_im2col(dtype, gz, scratch, deconv_mirror(B, IH, IW, OC, FH, FW, sy, sx, g), as_stream(stream)))
         return rc;
     const size_t ws = scratch_bytes > mat ? scratch_bytes - mat : 0;
@@ -976,7 +1056,10 @@ int d8_conv2d_grad_xy(int dtype, const void *x, void *gx, int B, int IH, int IW,
         if (conv_implicit_plan(dtype, 1, cs, gx, w, gz, px, ta, tb) && conv_implicit_plan(dtype, 2, cs, x, gw, gz, pw, ta, tb)) {
             px.beta = bx, pw.beta = bw;
             int rc = 0;
-            if (gemm_tiled_run_pair(dtype, px, pw, scratch, scratch_bytes, as_stream(stream), &rc)) return rc;
+            if (gemm_tiled_run_pair(dtype, px, pw, scratch, scratch_bytes, as_stream(stream), &rc)) {
+                route_calls[ROUTE_PATCH] += 2;
+                return rc;
+            }
         }
     }
     if (int rc = d8_conv2d_grad_x_impl(dtype, gx, B, IH, IW, IC, w, OC, FH, FW, gz, covered, sy, sx, dy, dx, scratch, scratch_bytes, stream, bx))
@@ -997,7 +1080,10 @@ static int deconv2d_grad_xy_geo(int dtype, const void *x, void *gx, int B, int I
             deconv_implicit_grad_y(dtype, B, IH, IW, IC, OC, FH, FW, sy, sx, g, x, gw, gz, pw)) {
             px.beta = bx, pw.beta = bw;
             int rc = 0;
-            if (gemm_tiled_run_pair(dtype, px, pw, scratch, scratch_bytes, as_stream(stream), &rc)) return rc;
+            if (gemm_tiled_run_pair(dtype, px, pw, scratch, scratch_bytes, as_stream(stream), &rc)) {
+                route_calls[ROUTE_PATCH] += 2;
+                return rc;
+            }
         }
     }
     if (int rc = deconv2d_grad_x_geo(dtype, gx, B, IH, IW, IC, w, OC, FH, FW, gz, g, sy, sx, scratch, scratch_bytes, stream, bx)) return rc;

@@ -1,6 +1,6 @@
-"""Conv2d forward and filter gradient on images of few channels, which are read from LDS instead of through a patch matrix:
-whole numbers bit for bit against the oracle, an infinity in the image (what fills a run or a row up must not meet it), and
-tensors that start at any element."""
+"""Conv2d forward and filter gradient on images of few channels, which are read from LDS instead of through a patch matrix
+(D8_CONV_DIRECT: also where the matrix is expected to be faster): whole numbers bit for bit against the oracle, an infinity in the
+image (what fills a run or a row up must not meet it), and tensors that start at any element."""
 import numpy as np
 import pytest
 
@@ -20,6 +20,9 @@ CASES = [
     (1, 40, 36, 2, 96, 5, 5, True, 2, 1, 1, 1),     # two groups of output channels
     (2, 13, 13, 1, 130, 7, 7, True, 1, 2, 1, 1),
     (600, 6, 8, 1, 8, 3, 3, True, 1, 1, 1, 1),      # more tiles than workgroups
+    (3, 20, 20, 3, 192, 3, 3, True, 2, 2, 1, 1),    # whole groups of 64 output channels
+    (3, 20, 20, 3, 193, 3, 3, True, 2, 2, 2, 1),    # ... and one channel more; the image rows two apart
+    (2, 9, 9, 3, 321, 5, 5, True, 1, 1, 1, 1),      # six groups
     (2, 12, 12, 6, 24, 3, 4, False, 1, 3, 1, 1),
 ]
 
@@ -35,7 +38,8 @@ def _shifted(a, elements):
 @pytest.mark.parametrize("cfg", CASES)
 @pytest.mark.parametrize("dtype", [np.float32, np.float16])
 @pytest.mark.parametrize("start,infinite", [(0, False), (1, False), (0, True)])
-def test_few_channels(oracle_port, cfg, dtype, start, infinite):
+def test_few_channels(oracle_port, cfg, dtype, start, infinite, monkeypatch):
+    monkeypatch.setenv("D8_CONV_DIRECT", "1")
     from deep8_amd import capi, ops
     from deep8_amd.capi import DeviceArray, check
     lib = capi.init()
@@ -61,6 +65,7 @@ def test_few_channels(oracle_port, cfg, dtype, start, infinite):
     nan = lambda shape: np.full(shape, np.nan, dtype)
     need = [lib.d8_conv2d_scratch_bytes(dt, k, *shape, *filt, *g) for k in (0, 2)]
     ws = DeviceArray((max(need),), np.uint8)
+    before = lib.d8_conv_route_calls(2)
     out, po = _shifted(nan(want_z.shape), start)
     if infinite:
         check(lib.d8_conv2d(dt, px, *shape, pw, *filt, po, *g, ws.ptr, need[0], None))
@@ -71,9 +76,10 @@ def test_few_channels(oracle_port, cfg, dtype, start, infinite):
     assert np.array_equal(got[start:start + n].reshape(want_z.shape), want_z, equal_nan=True)
     assert np.isnan(got[:start]).all() and np.isnan(got[start + n:]).all()
     n = want_gw.size
-    for name, before, want in (("d8_conv2d_grad_y_overwrite", nan(w.shape), want_gw), ("d8_conv2d_grad_y", c(old), want_gw + old)):
-        out, po = _shifted(before, start)
+    for name, there, want in (("d8_conv2d_grad_y_overwrite", nan(w.shape), want_gw), ("d8_conv2d_grad_y", c(old), want_gw + old)):
+        out, po = _shifted(there, start)
         check(getattr(lib, name)(dt, px, *shape, po, *filt, pg, *g, ws.ptr, need[1], None))
         got = f(out.numpy())
         assert np.array_equal(got[start:start + n].reshape(w.shape), want, equal_nan=True), name
         assert np.isnan(got[:start]).all() and np.isnan(got[start + n:]).all()
+    assert lib.d8_conv_route_calls(2) == before + 3

@@ -1,7 +1,7 @@
 """Convolutions whose channel counts leave a partial K step in every filter tap, whose pixel count is no multiple of the K
-step, or whose output is smaller than a tile: all of them read their patch matrix in the GEMM's loader.  Called without
-scratch (the staged route would refuse) and with it (the reduction may then be split); integers bit for bit against the
-oracle."""
+step, or whose output is smaller than a tile: all of them can read their patch matrix in the GEMM's loader.  Called without
+scratch and with less than the interim matrix needs (the reduction may then be split), where they do, and with what is asked for,
+where they take the way that is expected to be faster; integers bit for bit against the oracle."""
 import numpy as np
 import pytest
 
@@ -60,9 +60,50 @@ def test_partial_steps_without_interim_matrix(oracle_port, op, cfg, dtype):
         bufs = [DeviceArray.from_numpy(c(x)), DeviceArray.from_numpy(c(w)), DeviceArray.from_numpy(c(gz))]
         bufs[(2, 0, 1)[which]] = nan
         asked = getattr(lib, "d8_%s_scratch_bytes" % op)(dt, which, *shape, *filt, *g)
-        for scratch in (0, asked):
+        interim = (B * OH * OW * IC if op == "conv2d" else B * IH * IW * OC) * FH * FW * np.dtype(dtype).itemsize
+        for scratch in (0, interim - 16, asked):
+            before = lib.d8_conv_route_calls(1)
             got = _call(lib, name, dt, bufs, shape, filt, g, nan, scratch)
             assert np.array_equal(got, want[which]), (which, scratch)
+            assert scratch == asked or lib.d8_conv_route_calls(1) == before + 1
+
+
+# op, which, element type, layer, the way it has to go with all the scratch it asks for (0 interim matrix, 1 loader, 2 LDS): both
+# sides were measured, in us, on the matrix / in the loader / from LDS
+ROUTES = [
+    ("conv2d", 0, np.float32, (3, 15, 15, 48, 140, 3, 3, True, 2, 2, 1, 1), 0),      # 10 / 46
+    ("conv2d", 0, np.float32, (2, 46, 46, 8, 128, 3, 3, True, 1, 1, 1, 1), 0),       # a quarter of every K step is not padding
+    ("conv2d", 0, np.float16, (3, 15, 15, 96, 136, 3, 3, True, 2, 2, 1, 1), 1),
+    ("conv2d", 1, np.float32, (5, 10, 7, 152, 512, 5, 5, True, 2, 2, 1, 1), 0),      # 23 / 275
+    ("conv2d", 1, np.float32, (10, 20, 20, 32, 96, 3, 3, True, 2, 2, 1, 1), 1),
+    ("conv2d", 2, np.float32, (29, 13, 13, 40, 128, 3, 3, True, 2, 2, 1, 1), 0),     # 10 / 35
+    ("conv2d", 2, np.float16, (9, 30, 30, 96, 160, 3, 3, True, 2, 2, 1, 1), 1),
+    ("conv2d", 2, np.float16, (6, 137, 137, 3, 142, 3, 3, True, 1, 1, 1, 1), 0),     # (17 images) 73 / - / 430
+    ("conv2d", 2, np.float16, (4, 56, 56, 3, 64, 7, 7, True, 2, 2, 1, 1), 2),
+    ("conv2d", 0, np.float32, (64, 28, 28, 1, 32, 5, 5, True, 1, 1, 1, 1), 2),       # 18 / - / 8
+    ("deconv2d", 0, np.float32, (1, 7, 7, 128, 448, 3, 3, False, 1, 1), 0),          # 14 / 74
+    ("deconv2d", 0, np.float16, (6, 12, 12, 96, 40, 4, 4, False, 2, 2), 1),
+    ("deconv2d", 1, np.float32, (6, 5, 5, 160, 8, 4, 4, False, 2, 2), 0),            # 7 / 37
+    ("deconv2d", 2, np.float16, (6, 11, 11, 160, 32, 4, 4, False, 2, 2), 0),         # 12 / 19
+]
+
+
+@pytest.mark.parametrize("op,which,dtype,cfg,route", ROUTES)
+def test_the_way_a_layer_goes(op, which, dtype, cfg, route):
+    from deep8_amd import capi, ops
+    from deep8_amd.capi import DeviceArray, check
+    lib = capi.init()
+    B, IH, IW, IC, OC, FH, FW = cfg[:7]
+    geo = (int(cfg[7]),) + cfg[8:]
+    OH, OW, _, _ = getattr(ops, op + "_geometry")(IH, IW, FH, FW, *cfg[7:])
+    dt, shape, filt = capi.dtype_id(np.dtype(dtype)), (B, IH, IW, IC), (OC, FH, FW)
+    x, w, z = (DeviceArray(s, dtype, zero=True) for s in (shape, (OC, FH, FW, IC), (B, OH, OW, OC)))
+    name = ("d8_" + op, "d8_%s_grad_x_overwrite" % op, "d8_%s_grad_y_overwrite" % op)[which]
+    asked = getattr(lib, "d8_%s_scratch_bytes" % op)(dt, which, *shape, *filt, *geo)
+    ws = DeviceArray((max(asked, 16),), np.uint8)
+    before = [lib.d8_conv_route_calls(k) for k in range(3)]
+    check(getattr(lib, name)(dt, x.ptr, *shape, w.ptr, *filt, z.ptr, *geo, ws.ptr, asked, None))
+    assert [lib.d8_conv_route_calls(k) - before[k] for k in range(3)] == [int(k == route) for k in range(3)]
 
 
 def test_pixels_past_the_last_of_a_large_image():
