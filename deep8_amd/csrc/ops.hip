@@ -185,9 +185,9 @@ static double interim_us(int dtype, const Gemm &product, double elements, int ch
 // FH * FW / stride^2 times the image (half 72 x 41x41x480 -> 64, 3x3: 145 and 583 us).  What both are expected to take decides.
 // Without room for the matrix the loader serves.  Over 3578 calls on drawn layers: 115 ms on the matrix, 76 in the loader, 72.5 with
 // the better of the two, 73.2 with this choice.
-// (col2im: the matrix is the gradient of the patches, and what it is added up in may have to be cleared first.  Counted whether
-// or not it has to be: a call that adds takes the same way as one that overwrites.)
-static bool prefer_interim(int dtype, const GemmArgs &patch, int ta, int tb, const Gemm &product, double elements, int channels, bool col2im,
+// (clears: how many tensors more the way over the matrix clears before it adds into them.  Counted whether or not the caller's
+// has to be cleared: a call that adds takes the same way as one that overwrites.)
+static bool prefer_interim(int dtype, const GemmArgs &patch, int ta, int tb, const Gemm &product, double elements, int channels, int clears,
                            const void *scratch, size_t scratch_bytes) {
     if (dtype == D8_FLOAT64 || !scratch || (double)scratch_bytes < elements * dtype_bytes(dtype)) return false;
     GemmArgs g = patch;
@@ -195,7 +195,7 @@ static bool prefer_interim(int dtype, const GemmArgs &patch, int ta, int tb, con
         for (int i = 0; i < g.ncls; ++i)
             if (g.cls[i].M < g.M) g.M = g.cls[i].M;
     if (gemm_tiled_eligible(dtype, g, ta, tb, TILED_WHOLE)) return false;
-    return interim_us(dtype, product, elements, channels, false) + (col2im ? 3.0 : 0.0) < gemm_estimate_us(dtype, patch, ta, tb);
+    return interim_us(dtype, product, elements, channels, false) + 3.0 * clears < gemm_estimate_us(dtype, patch, ta, tb);
 }
 
 // Float64 gradient of x: the product's N is the input channel count, and under 128 channels the fp64 kernel is
@@ -556,7 +556,7 @@ static int conv2d_impl(int dtype, const void *x, int B, int IH, int IW, int IC,
         GemmArgs ga;
         int ta, tb;
         if (conv_implicit_plan(dtype, 0, cs, x, w, z, ga, ta, tb) &&
-            !prefer_interim(dtype, ga, ta, tb, conv_plan(0, M, K, OC, scratch, w, z), (double)M * K, IC, false, scratch, scratch_bytes)) {
+            !prefer_interim(dtype, ga, ta, tb, conv_plan(0, M, K, OC, scratch, w, z), (double)M * K, IC, 0, scratch, scratch_bytes)) {
             ++route_calls[ROUTE_PATCH];
             ga.bias = bias, ga.relu = relu;  // applied in the tile store (and in the remainder band's reduction)
             ga.round_first = !gemm_tiled_eligible(dtype, ga, ta, tb, TILED_WHOLE) &&
@@ -624,14 +624,14 @@ static int d8_conv2d_grad_x_impl(int dtype, void *gx, int B, int IH, int IW, int
         int ta, tb;
         const Gemm product = conv_plan(1, M, K, OC, scratch, w, gz);
         if (conv_implicit_plan(dtype, 1, cs, gx, w, gz, ga, ta, tb) &&
-            !prefer_interim(dtype, ga, ta, tb, product, (double)M * K, IC, true, scratch, scratch_bytes)) {
+            !prefer_interim(dtype, ga, ta, tb, product, (double)M * K, IC, 1, scratch, scratch_bytes)) {
             ++route_calls[ROUTE_PATCH];
             ga.beta = beta;
             return implicit_run(dtype, ga, ta, tb, scratch, scratch_bytes, as_stream(stream));
         }
         bool untouched = false;
         if (conv_classes_grad_x(dtype, cs, gx, w, gz, ga, &untouched) &&
-            !prefer_interim(dtype, ga, 0, 0, product, (double)M * K, IC, true, scratch, scratch_bytes)) {
+            !prefer_interim(dtype, ga, 0, 0, product, (double)M * K, IC, untouched ? 0 : 1, scratch, scratch_bytes)) {
             ++route_calls[ROUTE_PATCH];
             if (untouched && beta == 0.f) {  // pixels of dx that no tap reaches: zero, and the classes add to that
                 if (int rc = d8_fill(dtype, gx, (size_t)B * IH * IW * IC, 0.f, stream)) return rc;
@@ -679,7 +679,7 @@ static int d8_conv2d_grad_y_impl(int dtype, const void *x, int B, int IH, int IW
         GemmArgs ga;
         int ta, tb;
         if (conv_implicit_plan(dtype, 2, cs, x, gw, gz, ga, ta, tb) &&
-            !prefer_interim(dtype, ga, ta, tb, conv_plan(2, M, K, OC, scratch, gw, gz), (double)M * K, IC, false, scratch, scratch_bytes)) {
+            !prefer_interim(dtype, ga, ta, tb, conv_plan(2, M, K, OC, scratch, gw, gz), (double)M * K, IC, 0, scratch, scratch_bytes)) {
             ++route_calls[ROUTE_PATCH];
             ga.beta = beta;
             return implicit_run(dtype, ga, ta, tb, scratch, scratch_bytes, as_stream(stream));
@@ -876,7 +876,7 @@ static int deconv2d_impl(int dtype, const void *x, int B, int IH, int IW, int IC
         GemmArgs ga;
         bool untouched = false;
         if (deconv_implicit_fwd(dtype, B, IH, IW, IC, OC, FH, FW, sy, sx, g, x, w, z, ga, &untouched) &&
-            !prefer_interim(dtype, ga, 0, 1, deconv_plan(0, M, T, OC, IC, scratch, w, x), (double)M * T * OC, OC, false, scratch, scratch_bytes)) {
+            !prefer_interim(dtype, ga, 0, 1, deconv_plan(0, M, T, OC, IC, scratch, w, x), (double)M * T * OC, OC, untouched ? -1 : 0, scratch, scratch_bytes)) {
             ++route_calls[ROUTE_PATCH];
             if (untouched)  // the pixels between the filter's footprints stay zero
                 if (int rc = d8_fill(dtype, z, (size_t)B * g[0] * g[1] * OC, 0.f, stream)) return rc;
@@ -922,7 +922,7 @@ static int deconv2d_grad_x_geo(int dtype, void *gx, int B, int IH, int IW, int I
     {
         GemmArgs ga;
         if (deconv_implicit_grad_x(dtype, B, IH, IW, IC, OC, FH, FW, sy, sx, g, gx, w, gz, ga) &&
-            !prefer_interim(dtype, ga, 0, 0, deconv_plan(1, M, T, OC, IC, scratch, w, gx), (double)M * T * OC, OC, false, scratch, scratch_bytes)) {
+            !prefer_interim(dtype, ga, 0, 0, deconv_plan(1, M, T, OC, IC, scratch, w, gx), (double)M * T * OC, OC, 0, scratch, scratch_bytes)) {
             ++route_calls[ROUTE_PATCH];
             ga.beta = beta;
             return implicit_run(dtype, ga, 0, 0, scratch, scratch_bytes, as_stream(stream));
@@ -969,7 +969,7 @@ static int deconv2d_grad_y_geo(int dtype, const void *x, int B, int IH, int IW, 
     {
         GemmArgs ga;
         if (deconv_implicit_grad_y(dtype, B, IH, IW, IC, OC, FH, FW, sy, sx, g, x, gw, gz, ga) &&
-            !prefer_interim(dtype, ga, 1, 0, deconv_plan(2, M, T, OC, IC, scratch, gw, x), (double)M * T * OC, OC, false, scratch, scratch_bytes)) {
+            !prefer_interim(dtype, ga, 1, 0, deconv_plan(2, M, T, OC, IC, scratch, gw, x), (double)M * T * OC, OC, 0, scratch, scratch_bytes)) {
             ++route_calls[ROUTE_PATCH];
             ga.beta = beta;
             return implicit_run(dtype, ga, 1, 0, scratch, scratch_bytes, as_stream(stream));

@@ -76,6 +76,7 @@ ROUTES = [
     ("conv2d", 0, np.float16, (3, 15, 15, 96, 136, 3, 3, True, 2, 2, 1, 1), 1),
     ("conv2d", 1, np.float32, (5, 10, 7, 152, 512, 5, 5, True, 2, 2, 1, 1), 0),      # 23 / 275
     ("conv2d", 1, np.float32, (10, 20, 20, 32, 96, 3, 3, True, 2, 2, 1, 1), 1),
+    ("conv2d", 1, np.float32, (14, 8, 8, 224, 24, 1, 1, False, 2, 2, 1, 1), 0),      # 9 / 14: three of four pixels have no tap
     ("conv2d", 2, np.float32, (29, 13, 13, 40, 128, 3, 3, True, 2, 2, 1, 1), 0),     # 10 / 35
     ("conv2d", 2, np.float16, (9, 30, 30, 96, 160, 3, 3, True, 2, 2, 1, 1), 1),
     ("conv2d", 2, np.float16, (6, 137, 137, 3, 142, 3, 3, True, 1, 1, 1, 1), 0),     # (17 images) 73 / - / 430
