@@ -28,9 +28,17 @@ static bool eligible(const GemmArgs &g, int transA, int transB, TiledRule rule) 
     if (!vb && ((g.red - 1) * g.sB + (long)(transB ? g.N : g.K) * g.ldb) * ES >= (1L << 31)) return false;
     if (g.K < 1) return false;  // (a K below one K step is a lone partial step)
     if ((long)ceil_div(g.M, 128) * ceil_div(g.N, 128) > 0x7fffffffL || (long)g.batch * 128 > 65535) return false;
-    if (g.virt == VIRT_NONE && rule == TILED_ANY)
-        // rows may start at any element (EDGE_ANY); a thread's shift must hold for all products of a sum
-        return in_pieces<E>(g, !transA, transB) || g.red == 1 || ((g.sA | g.sB) * ES) % 4 == 0;
+    if (g.virt == VIRT_NONE && rule == TILED_ANY) {
+        if (in_pieces<E>(g, !transA, transB)) return true;
+        // Rows may start at any element (EDGE_ANY).  But products of at most half a K step that give every compute unit a tile are
+        // left to the any-shape kernel, whose K step is half as long (fp32 4032 x 2 x 2672, 9 summed: 43 us against 63, 2624 x 13 x
+        // 3207 14.5 against 21.8; with fewer tiles, 8583 x 8 x 296, 9.0 against 7.5); in half, whose steps wait longer than they
+        // multiply, only A^T . B over many tiles (57 x 1480 x 8 x 139 19.5 against 25.3; 9728 x 17 x 1300 level).
+        const long tiles = (long)ceil_div(g.M, 128) * ceil_div(g.N, 128) * g.batch;
+        if (g.K <= 16 && (ES == 4 ? g.M > 64 && g.N > 64 && tiles >= cu_count() : transA && tiles >= 4L * cu_count())) return false;
+        // a thread's shift must hold for all products of a sum
+        return g.red == 1 || ((g.sA | g.sB) * ES) % 4 == 0;
+    }
     // one side may be shorter than any tile (a few rows against a wide matrix: the 64 x 128 / 128 x 64 tile
     // then reaches past it) when the other side fills a tile; a patch-matrix product may have both short
     if (g.M < 128 && g.N < 128 && (g.virt == VIRT_NONE || rule == TILED_WHOLE)) return false;

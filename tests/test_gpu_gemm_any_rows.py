@@ -55,6 +55,33 @@ def test_rows_that_start_anywhere(oracle_port, M, N, K, ta, tb, dtype):
         assert np.array_equal(f(dC.numpy()), f(wantbuf), equal_nan=True), (batch, pad, first, gap)
 
 
+@pytest.mark.parametrize("M,N,K", [(2310, 1930, 7), (2310, 1930, 16), (2310, 1930, 17), (4230, 65, 3)])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0)])
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+def test_short_products_over_many_tiles(oracle_port, M, N, K, ta, tb, dtype):
+    """either side of the reductions and outputs that are left to the any-shape kernel; a sum of products too"""
+    from deep8_amd import capi
+    from deep8_amd.capi import DeviceArray, check
+    lib = capi.init()
+    dt = capi.dtype_id(np.dtype(dtype))
+    r = rng(M + N + K)
+    batch = 8 if N == 65 else 4 if (ta, dtype) == (1, np.float16) else 1
+    A, B = ints(r, (batch,) + ((K, M) if ta else (M, K)), 9), ints(r, (batch,) + ((N, K) if tb else (K, N)), 9)
+    (bufA, sA), (bufB, sB) = _embed(A, A.shape[2], 0, 0, dtype), _embed(B, B.shape[2], 0, 0, dtype)
+    dA, dB = DeviceArray.from_numpy(bufA), DeviceArray.from_numpy(bufB)
+    each = [oracle_port.gemm(ta, tb, A[i], B[i]) for i in range(batch)]
+    for summed in (False, True) if N == 65 and K % 2 else (False,):
+        want = sum(each) if summed else np.stack(each)
+        assert want.max() < 2048
+        dC = DeviceArray.from_numpy(np.full(want.shape, np.nan, dtype))
+        sC = 0 if summed else M * N
+        nb = lib.d8_gemm_workspace_bytes(dt, ta, tb, M, N, K, batch, sC)
+        ws = DeviceArray((max(nb, 16),), np.uint8)
+        check(lib.d8_gemm(dt, ta, tb, M, N, K, dA.ptr, A.shape[2], sA, dB.ptr, B.shape[2], sB, 0.0, dC.ptr, N, sC, batch, ws.ptr if nb else None,
+                          nb, None))
+        assert np.array_equal(f(dC.numpy()), want)
+
+
 @pytest.mark.parametrize("batch,stride_odd", [(5, False), (4, True)])
 @pytest.mark.parametrize("dtype", [np.float32, np.float16])
 def test_summed_batch_of_odd_matrices(oracle_port, batch, stride_odd, dtype):
