@@ -676,7 +676,11 @@ size_t gemm_tiled_workspace(int dtype, int M, int N, int K, int red, int virt) {
 static double tile_cost(bool half_elems, int bm, int bn, const GemmArgs &g, long total, long s) {
     const long cus = cu_count(), n = (ceil_div(g.M, bm) * (long)ceil_div(g.N, bn) * g.batch * s + cus - 1) / cus, len = (total + s - 1) / s;
     const double area = bm * bn / 16384.0, mn = (double)g.M * g.N * g.batch;
-    if (half_elems) return n * len * (area < 0.3 ? 0.5 : area < 0.6 ? 0.76 : 1.0) + 7.0 + 0.5 * (n - 1) + (s > 1 ? 6.5 + s * (mn / 0.25e6) : 0.0);
+    // (operands of 16 MB and more come from beyond the L2: a 64 x 64 half step then takes 0.4 us.  It counts as 0.3, because the
+    // larger tiles' steps take longer as well.  3264 x 4416 x 256 NT 31.4 us whole on 64 x 64 tiles, 22.6 in four pieces on
+    // 128 x 128; 16288 x 4672 x 64 TN 42.1 and 33.8.)
+    const bool far = 2.0 * g.red * g.K * g.batch * ((double)g.M + g.N) >= 16e6;
+    if (half_elems) return n * len * (area < 0.3 ? (far ? 0.6 : 0.5) : area < 0.6 ? 0.76 : 1.0) + 7.0 + 0.5 * (n - 1) + (s > 1 ? 6.5 + s * (mn / 0.25e6) : 0.0);
     return n * len * area * (n == 1 ? 1.1 : area < 0.3 ? 1.08 : 1.0) + 0.5 + 2.0 * sqrt(area) + 0.3 * (n - 1) + (s > 1 ? 2.0 + s * (mn / 2e6) : 0.0);
 }
 
