@@ -348,8 +348,8 @@ static bool gemm_is_small(int M, int N, int K, int batch, int red) {
 }
 
 // C[b][m][n] = beta * C + sum_s ws[b][s][m][n].  A workgroup covers groups of 4 consecutive outputs.
-// Few pieces (LANES = 1): 256 groups, a thread adds all pieces of its group in order, four loads in
-// flight.  Many (LANES = 8): 32 groups, 8 thread rows each add every 8th piece, and the 8 sums meet in
+// Few pieces of many groups (LANES = 1): 256 groups, a thread adds all pieces of its group in order, four loads in
+// flight.  Else (LANES = 8): 32 groups, 8 thread rows each add every 8th piece, and the 8 sums meet in
 // LDS in a fixed order.  Either way the result does not depend on scheduling, and up to 8 pieces
 // it is the same.  Five pieces of 12544 x 32: 4.9 -> 4.0 us, four of 1024 x 1001 in half: 7.1 -> 5.4 us (3 us of which is
 // what any launch behind one that wrote a lot takes).  The groups count through an output's elements
@@ -357,7 +357,13 @@ static bool gemm_is_small(int M, int N, int K, int batch, int red) {
 // a 16-byte load needs) and may go on in the next row.  An output a thread, as rows of an odd length had it first, took
 // 17.3 us for four partial sums of 1024 x 1001, this takes 8.0 us.
 typedef f32x4 f32x4_any __attribute__((aligned(4)));
-__host__ __device__ static inline int reduce_lanes(const GemmArgs &g) { return g.splits <= 8 ? 1 : 8; }
+// Which of the two: a thread per group only where that alone gives every compute unit more than a workgroup, and two where
+// the output is stored transposed per tap (four scattered stores a thread).  Whole calls, a thread per group and eight: half
+// 512 x 3136 x 1024 NT 14.7 and 16.2 us, 160 x 2048 x 1024 TN 8.9 and 8.2; filter gradient of half DeConv2d
+// 32 x 7x7x256 -> 64, 4x4 stride 2 15.4 and 12.9, of fp32 16 x 8x8x256 -> 64, 4x4 23.5 and 21.3.
+__host__ __device__ static inline int reduce_lanes(const GemmArgs &g) {
+    return g.splits <= 8 && (long)g.M * g.N * g.batch > (g.perm_OC ? 2 : 1) * 4 * 256 * 256L ? 1 : 8;
+}
 
 // (ROWS: the rows are multiples of 4, so a group lies in one row and may be stored at once)
 template <typename T, bool ROWS, int LANES>
