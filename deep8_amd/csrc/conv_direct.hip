@@ -511,6 +511,8 @@ bool plan_grad(int dtype, const DirectShape &s, const void *x, const void *gz, D
 
 bool conv_direct_eligible(int dtype, const DirectShape &s) {
     if (dtype != D8_FLOAT16 && dtype != D8_FLOAT32) return false;
+    // (the groups of output channels are the grid's second dimension)
+    if (ceil_div(s.OC, 32) > 65535 || (long)s.OC * s.FH * s.FW * s.C > 0x7fffffffL) return false;
     if (s.dx != 1 || (long)s.FH * s.FW * s.C >= 4096 || pieces_of(dtype, s) > 2 * most_groups(dtype)) return false;
     DirectArgs a;
     size_t lds;

@@ -83,3 +83,23 @@ def test_few_channels(oracle_port, cfg, dtype, start, infinite, monkeypatch):
         assert np.array_equal(got[start:start + n].reshape(w.shape), want, equal_nan=True), name
         assert np.isnan(got[:start]).all() and np.isnan(got[start + n:]).all()
     assert lib.d8_conv_route_calls(2) == before + 3
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+def test_more_groups_of_channels_than_a_grid_takes(dtype, monkeypatch):
+    """groups of 32 output channels beyond the grid's second dimension: the layer keeps the patch matrix"""
+    monkeypatch.setenv("D8_CONV_DIRECT", "1")
+    from deep8_amd import capi, ops
+    lib = capi.init()
+    OC = 65536 * 32
+    r = rng(7)
+    x, w = ints(r, (1, 4, 4, 1), 3), r.integers(0, 3, size=(OC, 3, 3, 1), dtype=np.int8)
+    gz = np.zeros((1, 2, 2, OC), dtype)
+    gz[0, 1, 0, ::1000] = 1
+    patches = np.stack([x[0, i:i + 3, j:j + 3, 0].ravel() for i in range(2) for j in range(2)])
+    before = lib.d8_conv_route_calls(0), lib.d8_conv_route_calls(2)
+    z = ops.conv2d(x.astype(dtype), w.astype(dtype), False)
+    assert np.array_equal(z.reshape(4, OC), (patches @ w.reshape(OC, 9).T.astype(np.float32)).astype(dtype))
+    gw = ops.conv2d_grad_y(x.astype(dtype), w.astype(dtype), gz, False)
+    assert np.array_equal(gw.reshape(OC, 9), gz[0, 1, 0][:, None] * patches[2].astype(dtype))
+    assert (lib.d8_conv_route_calls(0), lib.d8_conv_route_calls(2)) == (before[0] + 2, before[1])
