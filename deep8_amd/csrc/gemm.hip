@@ -357,12 +357,13 @@ static bool gemm_is_small(int M, int N, int K, int batch, int red) {
 // a 16-byte load needs) and may go on in the next row.  An output a thread, as rows of an odd length had it first, took
 // 17.3 us for four partial sums of 1024 x 1001, this takes 8.0 us.
 typedef f32x4 f32x4_any __attribute__((aligned(4)));
-// Which of the two: a thread per group only where that alone gives every compute unit more than a workgroup, and two where
-// the output is stored transposed per tap (four scattered stores a thread).  Whole calls, a thread per group and eight: half
-// 512 x 3136 x 1024 NT 14.7 and 16.2 us, 160 x 2048 x 1024 TN 8.9 and 8.2; filter gradient of half DeConv2d
-// 32 x 7x7x256 -> 64, 4x4 stride 2 15.4 and 12.9, of fp32 16 x 8x8x256 -> 64, 4x4 23.5 and 21.3.
+// Which of the two: a thread per group only where that alone gives three of four compute units a workgroup, and never where the
+// output is stored transposed per tap (four scattered stores a thread).  Whole calls, a thread per group and eight, two to
+// eight pieces: up to 147456 outputs level with two or four pieces and 0.1 - 0.8 us slower with others, 235520 level,
+// 327680 0.3 - 0.5 us faster, 512512 up to 1.5; transposed 0 - 2.6 us slower from 65536 outputs to 1048576 (filter gradient of
+// half DeConv2d 32 x 7x7x256 -> 64, 4x4 stride 2 15.4 and 12.9, of fp32 16 x 8x8x256 -> 64, 4x4 23.5 and 21.3).
 __host__ __device__ static inline int reduce_lanes(const GemmArgs &g) {
-    return g.splits <= 8 && (long)g.M * g.N * g.batch > (g.perm_OC ? 2 : 1) * 4 * 256 * 256L ? 1 : 8;
+    return g.splits <= 8 && !g.perm_OC && (long)g.M * g.N * g.batch > 3 * 256 * 256L ? 1 : 8;
 }
 
 // (ROWS: the rows are multiples of 4, so a group lies in one row and may be stored at once)

@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 # M, N, K: either side of a tile, of a band of rows beyond whole rounds of the chip, reductions with and without a rest
 SHAPES = [(784, 128, 1152), (130, 191, 608), (65, 260, 999), (1000, 64, 32), (320, 320, 36), (129, 32, 200), (33000, 32, 96),
           (34100, 20, 40), (513, 1, 1000), (128, 31, 2048),
-          (512, 512, 700), (512, 513, 700)]  # (either side of where a few pieces are added by a thread per group of outputs)
+          (384, 512, 700), (384, 513, 700)]  # (either side of where a few pieces are added by a thread per group of outputs)
 
 
 @pytest.mark.parametrize("M,N,K", SHAPES)
@@ -41,7 +41,7 @@ def test_products(oracle_port, M, N, K, ta, tb, dtype):
 CONV = [(2, 28, 28, 32, 64, 5, 5, True, 1, 1, 1, 1), (3, 15, 17, 24, 20, 3, 3, True, 1, 1, 1, 1), (1, 28, 28, 128, 128, 3, 3, True, 1, 1, 1, 1),
         (4, 19, 19, 20, 96, 3, 3, True, 2, 2, 1, 1), (64, 26, 26, 32, 32, 3, 3, False, 1, 1, 1, 1)]
 DECONV = [(2, 14, 14, 64, 32, 4, 4, False, 2, 2), (2, 12, 12, 32, 20, 3, 3, False, 1, 1),
-          (8, 8, 8, 512, 64, 4, 4, False, 2, 2), (8, 8, 8, 512, 68, 4, 4, False, 2, 2)]  # (as above, stored transposed per tap)
+          (8, 8, 8, 512, 68, 4, 4, False, 2, 2)]  # (many outputs, stored transposed per tap)
 
 
 @pytest.mark.parametrize("op,cfg", [("conv2d", c) for c in CONV] + [("deconv2d", c) for c in DECONV])
