@@ -3,7 +3,8 @@ against the unfused HIP sequence (d8_matmul / d8_conv2d, d8_add, d8_relu; d8_rel
 
 Integers: bit for bit in both precisions.  Float32 reals: bit for bit against the unfused sequence wherever the
 product itself runs the same way, and within 1e-5 of the oracle.  Float16 reals: the fused store rounds once
-where the sequence rounds three times, so they are compared with the oracle within 2e-3."""
+where the sequence rounds three times, so they are compared with the oracle within 2e-3; which products are rounded
+before the bias is added is checked on whole numbers that half does not hold."""
 import numpy as np
 import pytest
 
@@ -114,6 +115,79 @@ def test_conv2d_bias_relu_float32_reals_bit_for_bit_with_the_sequence():
     x, w, b = nrm(r, (4, 20, 20, 64)), nrm(r, (64, 3, 3, 64), 0.1), nrm(r, (64,))
     seq = ops.relu(ops.add(ops.conv2d(x, w), b.reshape(1, 64)))
     assert np.array_equal(ops.conv2d_bias_relu(x, w, b, True), seq)
+
+
+def _whole_numbers(r, shape, K):
+    """whole numbers whose sums of K products are mostly between 2048 and 32768: exact in fp32, rounded by half"""
+    hi = max(2, int(np.sqrt(18000 / np.sqrt(K))))
+    return r.integers(-hi, hi + 1, size=shape).astype(np.float32)
+
+
+def _half_rounding(product, bias, first):
+    """half(product + bias), or half(half(product) + bias), then ReLu; both sums are exact in fp32"""
+    once, twice = h(product + bias), h(f(h(product)) + bias)
+    assert np.abs(product).max() < 60000 and not np.array_equal(np.maximum(once, 0), np.maximum(twice, 0))
+    return np.maximum(twice if first else once, 0)
+
+
+@pytest.mark.parametrize("rows,inner,cols,first", [
+    (64, 128, 256, True),       # the small-product kernel
+    (200, 72, 77, True),        # rows that start anywhere
+    (1030, 64, 72, False),
+    (300, 3136, 256, False),    # in pieces
+    (300, 3137, 255, True),
+    (33068, 520, 80, False),    # a remainder band
+    (33068, 520, 77, True),
+])
+def test_where_half_products_are_rounded(rows, inner, cols, first):
+    """Half: products that always had the bias added in their own store round the sum once; the others round the product
+    first, as a pass of its own finds it (a layer keeps the gates of its ReLu)."""
+    from deep8_amd import ops
+    r = rng(rows + inner + cols)
+    x, w = _whole_numbers(r, (1, rows, inner), inner), _whole_numbers(r, (1, inner, cols), inner)
+    bias = r.integers(-9, 10, size=cols).astype(np.float32)
+    got = ops.matmul_bias_relu(h(x), h(w), h(bias))
+    assert np.array_equal(got.reshape(rows, cols), _half_rounding(x[0] @ w[0], bias, first))
+
+
+# B, IH, IW, IC, OC, FH, FW, covered, sy, sx, dy, dx; scratch (all that is asked for, none, or less than the interim matrix: the
+# product may then be cut into pieces); the route; whether the product is rounded before the bias is added
+HALF_CONV = [
+    ((2, 20, 20, 3, 64, 3, 3, True, 1, 1, 1, 1), "asked", 2, True),      # the image read from LDS
+    ((4, 30, 30, 3, 64, 7, 7, True, 2, 2, 1, 1), "asked", 2, False),     # ... in the place of padded patch rows
+    ((1, 11, 11, 72, 40, 3, 3, True, 1, 1, 1, 1), "none", 1, True),      # partial K steps, an output smaller than a tile
+    ((1, 11, 11, 72, 40, 3, 3, True, 1, 1, 1, 1), "less", 1, True),
+    ((1, 12, 12, 72, 40, 3, 3, True, 1, 1, 1, 1), "none", 1, False),     # ... and no smaller
+    ((1, 12, 12, 72, 40, 3, 3, True, 1, 1, 1, 1), "less", 1, False),
+    ((33, 32, 32, 72, 40, 1, 1, True, 1, 1, 1, 1), "none", 1, False),
+    ((33, 32, 32, 72, 8, 3, 3, True, 1, 1, 1, 1), "less", 1, False),     # a remainder band
+    ((1, 11, 11, 72, 40, 3, 3, True, 1, 1, 1, 1), "asked", None, True),  # whichever way is expected to be faster
+    ((1, 12, 12, 72, 40, 3, 3, True, 1, 1, 1, 1), "asked", None, False),
+]
+
+
+@pytest.mark.parametrize("cfg,scratch,route,first", HALF_CONV)
+def test_where_half_convolutions_are_rounded(oracle_port, cfg, scratch, route, first, monkeypatch):
+    from deep8_amd import capi
+    from deep8_amd.capi import DeviceArray, check
+    lib = capi.init()
+    if route == 2:
+        monkeypatch.setenv("D8_CONV_DIRECT", "1")
+    B, IH, IW, IC, OC, FH, FW = cfg[:7]
+    geo, K = (int(cfg[7]),) + cfg[8:], FH * FW * IC
+    r = rng(sum(cfg[:7]))
+    x, w = _whole_numbers(r, (B, IH, IW, IC), K), _whole_numbers(r, (OC, FH, FW, IC), K)
+    bias = r.integers(-9, 10, size=OC).astype(np.float32)
+    product = oracle_port.conv2d(x, w, *cfg[7:])
+    dt, shape, filt = capi.dtype_id(np.dtype(np.float16)), (B, IH, IW, IC), (OC, FH, FW)
+    asked = lib.d8_conv2d_scratch_bytes(dt, 0, *shape, *filt, *geo)
+    given = {"asked": asked, "none": 0, "less": 2 * product[..., 0].size * K - 16}[scratch]
+    dx, dw, db, dz = (DeviceArray.from_numpy(h(a)) for a in (x, w, bias, np.full(product.shape, np.nan)))
+    ws = DeviceArray((max(given, 16),), np.uint8)
+    before = lib.d8_conv_route_calls(route or 0)
+    check(lib.d8_conv2d_bias_relu(dt, dx.ptr, *shape, dw.ptr, *filt, db.ptr, 1, dz.ptr, *geo, ws.ptr if given else None, given, None))
+    assert route is None or lib.d8_conv_route_calls(route) == before + 1
+    assert np.array_equal(dz.numpy(), _half_rounding(product, bias, first))
 
 
 GRAD = [(1, 7), (5, 1), (33, 12), (1000, 64), (100352, 64), (4096, 200), (3, 5000), (777, 3)]
