@@ -79,7 +79,7 @@ __device__ inline void wave_mma(const float *As, const float *Bs, int arow, int 
 
 // ------------------------------------------------------------------------------------------
 // General kernel: what the tiled kernels refuse -- operands of 2 GiB and more, sums over half matrices that lie an odd
-// number of elements apart.  128 x 128 tile, 4 waves in a
+// number of elements apart, reductions of at most 16 over many tiles of rows that start anywhere.  128 x 128 tile, 4 waves in a
 // 2 x 2 arrangement, 64 x 64 per wave; element-wise, bounds-checked tile loads.
 // ------------------------------------------------------------------------------------------
 template <typename T, bool TA, bool TB>
@@ -672,8 +672,10 @@ size_t gemm_tiled_workspace(int dtype, int M, int N, int K, int red, int virt) {
 // 64 x 64 tiles where the 128-wide ones leave compute units idle.  In fp32, whose K step is bound by the matrix pipe, a step of
 // theirs is a quarter of the work; in half, whose step waits longer than it multiplies, half of it (0.25 us against 0.38 for a
 // 64 x 128 tile and 0.46 for 128 x 128).  The same pieces -- or none, and no second pass -- spread over four times as many
-// workgroups.  The estimate counts as plan_few_tiles does, in steps of a 128 x 128 tile (about 2 us of a CU in fp32, 0.5 us in
-// half), for the plan that g holds (splits set) and for 64 x 64 tiles in 1 .. as many pieces as that plan; 7 % or more decide.
+// workgroups.  The estimate counts steps of a 128 x 128 tile (about 2 us of a CU in fp32, 0.5 us in half), for the plan that g
+// holds (splits set) and for 64 x 64 tiles in 1 .. as many pieces as that plan; 7 % or more decide.  It was fitted anew, to the
+// kernels as they are: a 64 x 128 half step is 0.76 here and 0.65 in plan_few_tiles, a half product's second pass 6.5 steps + 1
+// per 0.25e6 outputs and piece here, 14 + 1 per 0.5e6 there, which only chooses among 128-wide tiles.
 // A narrow output (128 x 32 tiles, below) counts its pieces the same way.
 // NN, us before and after (M x K x N; NT and TN alike): fp32 512 x 512 x 512 16.4 -> 10.2, 784 x 1152 x 128 16.0 -> 10.3,
 // 1024 x 1024 x 1024 33.6 -> 23.5, 12544 x 800 x 64 24.0 -> 17.0, 3136 x 576 x 256 24.5 -> 12.7, 1536 x 1536 x 1536

@@ -71,7 +71,7 @@ struct GemmArgs {
     // is given): every workgroup records when its prologue, K loop and epilogue ended into ws
     int stamps;
     size_t ws_bytes;  // size of ws as d8_gemm received it (0 where a planner filled the block in)
-    // Fused store (the tiled kernels, the large-output fp16 kernel and the split reduction): after the product
+    // Fused store (the tiled kernels, the large-output fp16 kernel, the small-product kernel and the split reduction): after the product
     // (and beta * C), column n of the result gets bias[n] added (bias: N elements of C's type, may be null),
     // then negative values become 0 when relu is set.  What Add (a per-column bias broadcast over the rows) and
     // ReLu do as separate passes over C in the reference (deep8/src/math/Add.cu:21-52, ReLu.cu:20-59).
@@ -81,7 +81,8 @@ struct GemmArgs {
     // product and bias + ReLu used to be two passes: a gate decided by the sum that is rounded once opens for other
     // elements (about one in five thousand), and a layer keeps the gates it had.
     int round_first;
-    // a smaller tile than the shape's own (128 x 32: fp32 only), chosen by gemm_tiled_run (few_tiles_small, narrow_output)
+    // a smaller tile than the shape's own (128 x 32: fp32 only), chosen by gemm_tiled_run and gemm_tiled_run_plain_pair
+    // (few_tiles_small, narrow_output)
     int tile_hint;
     // Remainder band in the same launch (tail_splits > 0; unsplit, unbatched products only): rows tail_m0 .. M - 1
     // are not tiled by the launch's first tiles(tail_m0) x tiles(N) workgroups but by further ones, tail_splits per
@@ -108,11 +109,12 @@ int gemm_run_fused(int dtype, GemmArgs &g, int transA, int transB, void *workspa
 // z[r][c] = relu?(z[r][c] + bias[c]) in place, one pass (bias may be null): the fallback for shapes the fused store does not take.
 int launch_bias_relu(int dtype, void *z, const void *bias, long rows, int cols, int relu, hipStream_t stream);
 
-// Tiled kernels (fp16 and fp32) for shapes whose operands can be moved in 16-byte pieces.
+// Tiled kernels (fp16 and fp32): operands that can be moved in 16-byte pieces, and real matrices whose rows start at any element.
 int gemm_tiled_k_step(int dtype);  // K elements per step: 64 (fp16) or 32 (fp32)
 // Whether the shape qualifies (g.splits / g.tiles_per_split need not be set yet).
-//   TILED_ANY     whatever a single launch takes: real matrices of any shape and alignment, patch matrices whose channels
-//                 can be moved in 16-byte pieces
+//   TILED_ANY     whatever a single launch takes: real matrices of any shape and alignment (but sums of half matrices an odd
+//                 number of elements apart, and short reductions over many tiles of rows that start anywhere, which the
+//                 any-shape kernel has), patch matrices whose channels can be moved in 16-byte pieces
 //   TILED_PIECES  ... real matrices too only in 16-byte pieces, and at least one side of the output as long as a tile (what
 //                 a launch of two products takes)
 //   TILED_WHOLE   ... and patch matrices only where all K steps are whole and the output is no smaller than a tile (what

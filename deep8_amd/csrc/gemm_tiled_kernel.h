@@ -378,11 +378,11 @@ __device__ __forceinline__ void store_tile(f32x16 (&acc)[T::TM][T::TN], float *l
             }
         return;
     }
-    // element by element: 32 lanes store 32 consecutive columns of a row.  (A row's address is formed once per row, the
-    // bias read once per column.)
-    // (Where an element of column n goes is a start and a step per row of the tile, but for the pixels of a class: divided
-    // out at every element, a filter gradient stored transposed per tap lost some 5 us to divisions: half DeConv2d
-    // 33 x 4x4x320 -> 64, 3x3 stride 2, forward and both gradients 41.5 -> 37.1 us.)
+    // element by element: 32 lanes store 32 consecutive columns of a row.  The outer loop runs over a thread's columns, the
+    // bias of a column being read once; an element of it lies at a start of the column plus a step per row of the tile, but
+    // for the pixels of a class, whose rows are looked up one by one.  (Divided out at every element, a filter gradient
+    // stored transposed per tap lost some 5 us to divisions: half DeConv2d 33 x 4x4x320 -> 64, 3x3 stride 2, forward and
+    // both gradients 41.5 -> 37.1 us.)
     const bool lines = !crow.plane || crow.perm_OC;
     const long step = crow.perm_OC ? 1 : ldc;
 #pragma unroll

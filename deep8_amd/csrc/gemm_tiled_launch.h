@@ -64,7 +64,7 @@ static int launch_plain(const GemmArgs &g, int transA, int transB, hipStream_t s
 // A patch matrix as one of them.
 template <typename E>
 static int launch_patch(const GemmArgs &g, int transB, hipStream_t stream) {
-    if (g.virt == VIRT_A_CLASSES) {  // every class has at least 128 rows (checked by eligible)
+    if (g.virt == VIRT_A_CLASSES) {  // (the last tile of a class, or its only one, may reach past it)
         if constexpr (sizeof(E) == 4)
             if (g.N <= 32)  // (see narrow_output in gemm.hip)
                 return transB ? launch_tiled<E, 128, 32, 4, 1, true, true, VIRT_A_CLASSES>(g, stream)
