@@ -11,7 +11,7 @@
 //   * AvgPooling2dGrad (AvgPooling2d.cpp:199-245): every in-image element of the window receives
 //     dy / (FH * FW).
 // The reference's GPU path calls cuDNN for max pooling (deep8/src/math/MaxPooling2d.cu:41-147),
-// whose padding behaves differently; the CPU path is the one the checker restates.
+// whose padding behaves differently; the CPU path is the one that is matched here.
 #include "common.h"
 
 namespace d8 {

@@ -1,9 +1,9 @@
-"""CPU checkers for the Deep8 dense-contraction hot path.  TEST INFRASTRUCTURE ONLY.
+"""CPU oracles for the Deep8 dense-contraction hot path.  TEST INFRASTRUCTURE ONLY.
 
 Only tests/, ``__graft_entry__.smoke()`` and ``bench.py``'s ``cpu_baseline`` leg may import this
 package; the product (``deep8_amd``) never does.
 
-Two checkers with the same numpy-level interface:
+Two of them with the same numpy-level interface:
 
 * ``port``  -- ``libdeep8_oracle.so``, the plain-C restatement in ``deep8_oracle.c``.
 * ``ref``   -- ``_ref/libdeep8_ref.so``, Deep8's own CPU (Eigen) sources compiled unmodified and
@@ -30,7 +30,7 @@ _i = ctypes.c_int
 
 
 def build(with_ref=True):
-    """Compile the checkers (the reference build only where /root/reference exists)."""
+    """Compile the oracles (the reference build only where /root/reference exists)."""
     subprocess.check_call(["make", "-s", "-C", _HERE, "oracle"])
     if with_ref:
         subprocess.check_call(["make", "-s", "-j8", "-C", _HERE, "ref"])
@@ -104,8 +104,8 @@ def _filt(w):
     return w
 
 
-# The working precision of the MatrixMultiply / gemm / Conv2d / DeConv2d checkers: float32, or
-# float64 inside ``with oracle.float64():`` (every other checker is float32 only).
+# The working precision of the MatrixMultiply / gemm / Conv2d / DeConv2d oracles: float32, or
+# float64 inside ``with oracle.float64():`` (every other oracle is float32 only).
 _WORK = [np.float32]
 
 

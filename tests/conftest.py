@@ -24,7 +24,7 @@ def oracle_port():
 
 @pytest.fixture(scope="session")
 def oracle(oracle_port):
-    """The checker package itself (for its float64() switch)."""
+    """The oracle package itself (for its float64() switch)."""
     import oracle
     return oracle
 

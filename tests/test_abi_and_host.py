@@ -37,7 +37,7 @@ def test_missing_library_fails_loudly(monkeypatch):
 
 
 def test_product_never_imports_the_oracle():
-    """Nothing under deep8_amd/ or include/ may refer to the CPU checkers."""
+    """Nothing under deep8_amd/ or include/ may refer to the CPU oracles."""
     for base, _, files in os.walk(os.path.join(ROOT, "deep8_amd")):
         for f in files:
             if f.endswith((".py", ".hip", ".h", ".cpp")) or f == "Makefile":

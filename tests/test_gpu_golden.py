@@ -1,6 +1,6 @@
 """The HIP path against the vectors Deep8's own CPU (Eigen) build wrote (tests/golden/deep8_cpu_reference.npz,
 made by tests/golden/make_golden.py from deep8/src/math/{MatrixMultiply,Conv2d,DeConv2d,...}.cpp), with no
-checker in between: inputs from the file go through the C ABI, results are compared with the stored outputs.
+oracle in between: inputs from the file go through the C ABI, results are compared with the stored outputs.
 
 fp32 results within a relative Frobenius error of 1e-5; the patch matrices bit for bit (the uint32 views are
 compared), which is the sentence "im2col bit-exact against Deep8's own CPU Eigen path" taken literally.

@@ -54,7 +54,7 @@ def test_two_calls_in_a_row_match_the_scratch_taking_entry_point(dtype, integers
         want = _grad_y("d8_matmul_grad_y", x, dy0, dz, True)
         got = _grad_y("d8_matmul_grad_y_static", x, dy0, dz, False)
         assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), (i, dtype)
-        # and the existing entry point itself agrees with the CPU checker
+        # and the existing entry point itself agrees with the CPU oracle
         ref = oracle_port.matmul_grad_y(x.astype(np.float32), dy0.astype(np.float32), dz.astype(np.float32),
                                         dy0.astype(np.float32))
         err = np.linalg.norm(got.astype(np.float64) - ref) / max(np.linalg.norm(ref), 1e-30)
