@@ -183,13 +183,13 @@ static double interim_us(int dtype, const Gemm &product, double elements, int ch
 // pieces (fp32 DeConv2d 3 x 6x6x480 -> 352, 3x3 stride 2: 116 and 17), filter gradients have no 64 x 64 tiles beside wider
 // outputs (fp32 Conv2d 29 x 13x13 -> 128, 464 pixels, N = 360: 35 and 11); while the matrix moves
 // FH * FW / stride^2 times the image (half 72 x 41x41x480 -> 64, 3x3: 145 and 583 us).  What both are expected to take decides.
-// Without room for the matrix the loader serves.  Over 3578 calls on drawn layers: 115 ms on the matrix, 76 in the loader, 72.5 with
+// Without room for the matrix, aligned as the maps' 16-byte accesses want it, the loader serves.  Over 3578 calls on drawn layers: 115 ms on the matrix, 76 in the loader, 72.5 with
 // the better of the two, 73.2 with this choice.
 // (clears: how many tensors more the way over the matrix clears before it adds into them.  Counted whether or not the caller's
 // has to be cleared: a call that adds takes the same way as one that overwrites.)
 static bool prefer_interim(int dtype, const GemmArgs &patch, int ta, int tb, const Gemm &product, double elements, int channels, int clears,
                            const void *scratch, size_t scratch_bytes) {
-    if (dtype == D8_FLOAT64 || !scratch || (double)scratch_bytes < elements * dtype_bytes(dtype)) return false;
+    if (dtype == D8_FLOAT64 || !scratch || ((size_t)scratch & 15) || (double)scratch_bytes < elements * dtype_bytes(dtype)) return false;
     GemmArgs g = patch;
     if (g.virt == VIRT_A_CLASSES)  // (g.M is the largest one's)
         for (int i = 0; i < g.ncls; ++i)

@@ -107,6 +107,24 @@ def test_the_way_a_layer_goes(op, which, dtype, cfg, route):
     assert [lib.d8_conv_route_calls(k) - before[k] for k in range(3)] == [int(k == route) for k in range(3)]
 
 
+def test_scratch_that_starts_anywhere_is_no_room_for_the_matrix(oracle_port):
+    """a layer that goes over the matrix with the scratch it asks for reads its patches in the loader when that is not aligned"""
+    from deep8_amd import capi
+    from deep8_amd.capi import DeviceArray, check
+    lib = capi.init()
+    r = rng(5)
+    x, w = ints(r, (3, 15, 15, 48), 4), ints(r, (140, 3, 3, 48), 4)
+    want = oracle_port.conv2d(x, w, True, 2, 2, 1, 1)
+    args = (3, 15, 15, 48), (140, 3, 3), (1, 2, 2, 1, 1)
+    asked = lib.d8_conv2d_scratch_bytes(capi.FLOAT32, 0, *args[0], *args[1], *args[2])
+    dx, dw, ws = DeviceArray.from_numpy(x), DeviceArray.from_numpy(w), DeviceArray((asked + 16,), np.uint8)
+    for shift, route in ((0, 0), (4, 1)):
+        dz = DeviceArray.from_numpy(np.full(want.shape, np.nan, np.float32))
+        before = lib.d8_conv_route_calls(route)
+        check(lib.d8_conv2d(capi.FLOAT32, dx.ptr, *args[0], dw.ptr, *args[1], dz.ptr, *args[2], ws.ptr + shift, asked, None))
+        assert lib.d8_conv_route_calls(route) == before + 1 and np.array_equal(dz.numpy(), want)
+
+
 def test_pixels_past_the_last_of_a_large_image():
     """one output pixel on an image of 77 MB: the 63 pixels that fill the K step up lie up to 4.9 GB past the image, whose other
     elements (NaN) they must not meet"""
