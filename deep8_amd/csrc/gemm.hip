@@ -685,11 +685,13 @@ size_t gemm_tiled_workspace(int dtype, int M, int N, int K, int red, int virt) {
 static double tile_cost(bool half_elems, int bm, int bn, const GemmArgs &g, long total, long s) {
     const long cus = cu_count(), n = (ceil_div(g.M, bm) * (long)ceil_div(g.N, bn) * g.batch * s + cus - 1) / cus, len = (total + s - 1) / s;
     const double area = bm * bn / 16384.0, mn = (double)g.M * g.N * g.batch;
-    // (operands of 16 MB and more come from beyond the L2: a 64 x 64 half step then takes 0.4 us.  It counts as 0.3, because the
-    // larger tiles' steps take longer as well.  3264 x 4416 x 256 NT 31.4 us whole on 64 x 64 tiles, 22.6 in four pieces on
-    // 128 x 128; 16288 x 4672 x 64 TN 42.1 and 33.8.)
-    const bool far = 2.0 * g.red * g.K * g.batch * ((double)g.M + g.N) >= 16e6;
-    if (half_elems) return n * len * (area < 0.3 ? (far ? 0.6 : 0.5) : area < 0.6 ? 0.76 : 1.0) + 7.0 + 0.5 * (n - 1) + (s > 1 ? 6.5 + s * (mn / 0.25e6) : 0.0);
+    // (a 64 x 64 half step takes 0.25 us on operands that its XCD's L2 holds and 0.41 on others; of products of 4 MB none had the
+    // longer step, of 7 MB half of them, from 14 MB on all.  The longer one counts as 0.36, because the larger tiles' steps take
+    // longer as well.  3264 x 4416 x 256 NT 31.4 us whole on 64 x 64 tiles, 22.6 in four pieces on 128 x 128; 256 x 3136 x 2200 TN
+    // 25.3 and 18.9; 1472 x 3368 x 416 25.3 and 19.1.  700 drawn products, the same operands again / others each time: 9964 / 10556 us
+    // with 0.3 from 16 MB on, 9900 / 10494 so, 9702 / 10290 at best.)
+    const double far = (2.0 * g.red * g.K * g.batch * ((double)g.M + g.N) - 4e6) / 8e6;
+    if (half_elems) return n * len * (area < 0.3 ? 0.5 + 0.22 * (far < 0.0 ? 0.0 : far > 1.0 ? 1.0 : far) : area < 0.6 ? 0.76 : 1.0) + 7.0 + 0.5 * (n - 1) + (s > 1 ? 6.5 + s * (mn / 0.25e6) : 0.0);
     return n * len * area * (n == 1 ? 1.1 : area < 0.3 ? 1.08 : 1.0) + 0.5 + 2.0 * sqrt(area) + 0.3 * (n - 1) + (s > 1 ? 2.0 + s * (mn / 2e6) : 0.0);
 }
 
