@@ -380,21 +380,29 @@ __device__ __forceinline__ void gemm_split_reduce_body(const GemmArgs &g, const 
     const int n_out = ROWS || mn - r >= 4 ? 4 : (int)(mn - r);
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
     if (live) {
-        const float *p = g.ws + (long)b * g.splits * mn + r;
-        if (n_out == 4) {
-            int s = row;
-            for (; s + 3 * LANES < g.splits; s += 4 * LANES) {
-                f32x4 t[4];
+        // (a last group of fewer than 4 is loaded with the outputs before it and moved down; an output of fewer than 4 in all
+        // is loaded one by one)
+        const bool tiny = !ROWS && mn < 4;
+        const int back = ROWS || tiny ? 0 : 4 - n_out;
+        const float *p = g.ws + (long)b * g.splits * mn + r - back;
+        auto piece = [&](int s) -> f32x4 {
+            const float *q = p + (long)s * mn;
+            if (!tiny) return *(const f32x4_any *)q;
+            f32x4 t = {q[0], 0.f, 0.f, 0.f};
+            if (n_out > 1) t[1] = q[1];
+            if (n_out > 2) t[2] = q[2];
+            return t;
+        };
+        int s = row;
+        for (; s + 3 * LANES < g.splits; s += 4 * LANES) {
+            f32x4 t[4];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) t[u] = *(const f32x4_any *)(p + (long)(s + u * LANES) * mn);
+            for (int u = 0; u < 4; ++u) t[u] = piece(s + u * LANES);
 #pragma unroll
-                for (int u = 0; u < 4; ++u) v += t[u];
-            }
-            for (; s < g.splits; s += LANES) v += *(const f32x4_any *)(p + (long)s * mn);
-        } else {
-            for (int s = row; s < g.splits; s += LANES)
-                for (int k = 0; k < n_out; ++k) v[k] += p[(long)s * mn + k];
+            for (int u = 0; u < 4; ++u) v += t[u];
         }
+        for (; s < g.splits; s += LANES) v += piece(s);
+        for (int k = 0; k < back; ++k) v = (f32x4){v[1], v[2], v[3], 0.f};
     }
     if constexpr (LANES > 1) {
         part[row][lane] = v;

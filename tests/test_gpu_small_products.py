@@ -38,3 +38,25 @@ def test_bias_and_relu_round_as_passes_of_their_own(rows, inner, cols, dtype):
     want = ops.relu(ops.add(ops.matmul(x, y), b.reshape(1, cols)))
     got = ops.matmul_bias_relu(x, y, b)
     assert np.array_equal(got, want.reshape(got.shape))
+
+
+@pytest.mark.parametrize("M,N", [(1, 1), (2, 1), (1, 3), (2, 2), (5, 1), (34, 103), (19, 111), (37, 175)])
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+def test_long_reductions_of_few_outputs(oracle_port, M, N, dtype):
+    """cut into many pieces: groups of four outputs with one, two and three left over, and fewer than four outputs in all;
+    summed products that lie an odd number of elements apart (the any-shape kernel) and a single one"""
+    from deep8_amd import capi
+    from deep8_amd.capi import DeviceArray, check
+    lib = capi.init()
+    dt, r = capi.dtype_id(np.dtype(dtype)), rng(M + N)
+    for batch, K in ((1, 9000), (51, 339)):
+        A, B = ints(r, (batch, M, K), 3), ints(r, (batch, K, N), 3)
+        A *= r.random(A.shape) < 0.05  # (thinned: half holds the sums)
+        want = sum(oracle_port.gemm(0, 0, A[i], B[i]) for i in range(batch))
+        assert 0 < want.max() < 2048
+        dA, dB = DeviceArray.from_numpy(A.astype(dtype)), DeviceArray.from_numpy(B.astype(dtype))
+        sC = 0 if batch > 1 else M * N
+        nb = lib.d8_gemm_workspace_bytes(dt, 0, 0, M, N, K, batch, sC)
+        dC, ws = DeviceArray.from_numpy(np.full((M, N), np.nan, dtype)), DeviceArray.from_numpy(np.full(nb + 64, 255, np.uint8))
+        check(lib.d8_gemm(dt, 0, 0, M, N, K, dA.ptr, K, M * K, dB.ptr, N, K * N, 0.0, dC.ptr, N, sC, batch, ws.ptr, nb, None))
+        assert np.array_equal(dC.numpy().astype(np.float32), want), batch
