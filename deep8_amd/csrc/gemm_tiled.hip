@@ -30,12 +30,20 @@ static bool eligible(const GemmArgs &g, int transA, int transB, TiledRule rule) 
     if ((long)ceil_div(g.M, 128) * ceil_div(g.N, 128) > 0x7fffffffL || (long)g.batch * 128 > 65535) return false;
     if (g.virt == VIRT_NONE && rule == TILED_ANY) {
         if (in_pieces<E>(g, !transA, transB)) return true;
-        // Rows may start at any element (EDGE_ANY).  But products of at most half a K step that give every compute unit a tile are
-        // left to the any-shape kernel, whose K step is half as long (fp32 4032 x 2 x 2672, 9 summed: 43 us against 63, 2624 x 13 x
-        // 3207 14.5 against 21.8; with fewer tiles, 8583 x 8 x 296, 9.0 against 7.5); in half, whose steps wait longer than they
-        // multiply, only A^T . B over many tiles (57 x 1480 x 8 x 139 19.5 against 25.3; 9728 x 17 x 1300 level).
-        const long tiles = (long)ceil_div(g.M, 128) * ceil_div(g.N, 128) * g.batch;
-        if (g.K <= 16 && (ES == 4 ? g.M > 64 && g.N > 64 && tiles >= cu_count() : transA && tiles >= 4L * cu_count())) return false;
+        // Rows may start at any element (EDGE_ANY).  But short products over many tiles are left to the any-shape kernel.  Its K step
+        // is half as long, so it has half of the padding of a reduction of at most half a step (fp32 4032 x 2 x 2672, 9 summed:
+        // 43 us against 63, 2624 x 13 x 3207 14.5 against 21.8; with fewer tiles, 8583 x 8 x 296, 9.0 against 7.5); and four of its
+        // workgroups fit a compute unit, where two of the tiled kernels' do, which a third of a tile's time away from the last round
+        // shows (fp32 4141 x 35 x 2349, 627 tiles, 21.9 and 27.6; 15 products of K <= 32 and 513 to 768 tiles 0.78 to 0.98 of the
+        // tiled time, 32 of K <= 80 0.79 to 1.04, with up to 512 or 769 to 1024 tiles 0.95 to 1.2 at the median).  In half, whose
+        // steps wait longer than they multiply, only A^T . B, whose tiles are turned on the way to the matrix instructions
+        // (57 x 1480 x 8 x 139 19.5 against 25.3; 6 of K <= 32 with more than 1024 tiles 0.90 to 0.95, 13 of K <= 64 with 513 to 768 0.78
+        // to 0.94).  A product that adds a bias or cuts at zero stays: the any-shape kernel does neither, and a pass over that
+        // much output takes longer than the difference.
+        const long tiles = (long)ceil_div(g.M, 128) * ceil_div(g.N, 128) * g.batch, cus = cu_count();
+        const bool third_round = tiles > 2 * cus && tiles <= 3 * cus;
+        if (!g.bias && !g.relu && (ES == 4 ? g.M > 64 && g.N > 64 && ((g.K <= 16 && 4 * tiles >= 3 * cus) || (g.K <= 80 && third_round))
+                                           : transA && ((g.K <= 32 && tiles >= 4 * cus) || (g.K <= 64 && third_round)))) return false;
         // a thread's shift must hold for all products of a sum
         return g.red == 1 || ((g.sA | g.sB) * ES) % 4 == 0;
     }

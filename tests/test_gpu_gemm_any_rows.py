@@ -55,7 +55,7 @@ def test_rows_that_start_anywhere(oracle_port, M, N, K, ta, tb, dtype):
         assert np.array_equal(f(dC.numpy()), f(wantbuf), equal_nan=True), (batch, pad, first, gap)
 
 
-@pytest.mark.parametrize("M,N,K", [(2310, 1930, 7), (2310, 1930, 16), (2310, 1930, 17), (4230, 65, 3)])
+@pytest.mark.parametrize("M,N,K", [(2310, 1930, 7), (2310, 1930, 16), (2310, 1930, 17), (2310, 1930, 33), (2310, 1930, 65), (2310, 1930, 81), (4230, 65, 3)])
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0)])
 @pytest.mark.parametrize("dtype", [np.float32, np.float16])
 def test_short_products_over_many_tiles(oracle_port, M, N, K, ta, tb, dtype):
@@ -65,8 +65,9 @@ def test_short_products_over_many_tiles(oracle_port, M, N, K, ta, tb, dtype):
     lib = capi.init()
     dt = capi.dtype_id(np.dtype(dtype))
     r = rng(M + N + K)
-    batch = 8 if N == 65 else 4 if (ta, dtype) == (1, np.float16) else 1
-    A, B = ints(r, (batch,) + ((K, M) if ta else (M, K)), 9), ints(r, (batch,) + ((N, K) if tb else (K, N)), 9)
+    batch = 8 if N == 65 else 2 if K > 17 else 4 if (ta, dtype) == (1, np.float16) else 1
+    hi = 5 if K > 17 else 9
+    A, B = ints(r, (batch,) + ((K, M) if ta else (M, K)), hi), ints(r, (batch,) + ((N, K) if tb else (K, N)), hi)
     (bufA, sA), (bufB, sB) = _embed(A, A.shape[2], 0, 0, dtype), _embed(B, B.shape[2], 0, 0, dtype)
     dA, dB = DeviceArray.from_numpy(bufA), DeviceArray.from_numpy(bufB)
     each = [oracle_port.gemm(ta, tb, A[i], B[i]) for i in range(batch)]
@@ -106,7 +107,7 @@ def test_summed_batch_of_odd_matrices(oracle_port, batch, stride_odd, dtype):
     assert want.max() < 2048 and np.array_equal(f(dC.numpy()), want)
 
 
-@pytest.mark.parametrize("rows,inner,cols", [(200, 72, 77), (1030, 64, 130), (96, 1000, 333)])
+@pytest.mark.parametrize("rows,inner,cols", [(200, 72, 77), (1030, 64, 130), (96, 1000, 333), (2310, 13, 1931)])
 @pytest.mark.parametrize("dtype", [np.float32, np.float16])
 def test_bias_and_relu_of_odd_columns_round_as_passes_of_their_own(rows, inner, cols, dtype):
     """matmul_bias_relu on rows that start anywhere: bit for bit matmul, add, relu -- in half too, where the product is
