@@ -79,7 +79,7 @@ __device__ inline void wave_mma(const float *As, const float *Bs, int arow, int 
 
 // ------------------------------------------------------------------------------------------
 // General kernel: what the tiled kernels refuse -- operands of 2 GiB and more, sums over half matrices that lie an odd
-// number of elements apart, reductions of at most 16 over many tiles of rows that start anywhere.  128 x 128 tile, 4 waves in a
+// number of elements apart, short reductions over many tiles of rows that start anywhere (see gemm_tiled.hip).  128 x 128 tile, 4 waves in a
 // 2 x 2 arrangement, 64 x 64 per wave; element-wise, bounds-checked tile loads.
 // ------------------------------------------------------------------------------------------
 template <typename T, bool TA, bool TB>
