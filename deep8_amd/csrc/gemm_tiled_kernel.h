@@ -27,6 +27,9 @@
 // a compact block of tiles and share A / B panels in that XCD's L2.  The epilogue turns each
 // 32 x 32 accumulator block around through LDS so that C is read and written 16 bytes per lane.
 //
+// That is Tile: fp32, half products on 256 x 256 tiles and half operands whose rows start anywhere.  Half operands that can be
+// moved in 16-byte pieces go straight into LDS (DmaTile, dma_loop); everything around the K loop is shared.
+//
 // An operand may be a patch matrix that is never written out (GemmArgs::virt): its loader turns
 // row / column numbers into image offsets, and an offset outside the image makes the buffer load
 // return zeros, which is the padding.  That carries the convolutions: Conv2d forward and its two
@@ -40,6 +43,8 @@
 // its loads bring in from there only enters results that are not stored.
 #ifndef DEEP8_AMD_GEMM_TILED_KERNEL_H
 #define DEEP8_AMD_GEMM_TILED_KERNEL_H
+
+#include <type_traits>
 
 #include "gemm_args.h"
 
@@ -128,6 +133,8 @@ struct Tile {
     static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_;
     static constexpr bool A_KC = A_KC_, B_KC = B_KC_;
     static constexpr int VIRT = VIRT_;  // which operand, if any, is a patch matrix read from its image
+    static constexpr bool TWO_FIT = false;  // (the compiler is not told to make room for two workgroups per compute unit)
+    static constexpr bool DMA = false;  // pieces go through registers (DmaTile: straight into LDS)
     static_assert((VIRT != VIRT_A_ROWS && VIRT != VIRT_A_CLASSES) || A_KC, "patch rows are K-contiguous");
     static_assert(VIRT != VIRT_B_KROWS || !B_KC, "patch k-rows are N-contiguous");
     static constexpr int ES = sizeof(E), EPV = 16 / ES;  // element size, elements per 16-byte piece
@@ -165,6 +172,78 @@ struct Tile {
     static constexpr bool PATCH_IN_A = A_SZ >= B_SZ;
     static constexpr int PATCH_SZ = PATCH_IN_A ? A_SZ : B_SZ;
 };
+
+// fp16 tile whose operand pieces go from global memory straight into LDS (buffer_load_dwordx4 ... lds), STAGES K steps ahead: no
+// registers between the two, no LDS writes, and operands that have to come from memory are asked for early enough.  Against
+// tiles that pass through registers, one step ahead: 1024^3 8.4 -> 7.4 us and, with operands that no cache holds, 12.6 -> 8.2;
+// 6272 x 256 x 2304 19.8 -> 16.0, cold 32.3 -> 24.
+//
+// A lane's 16 bytes land at a wave-uniform base + 16 x lane, so rows cannot be padded; bank conflicts are avoided by choosing
+// WHICH 16 bytes a lane fetches.  The LDS reads serve 256 bytes (64 banks) at a time:
+//   * [row][64 k], 128 bytes a row: chunk c of row r lies at position c ^ (r >> 1 & 7), so that the 16 rows of a 16-byte read
+//     cover all banks;
+//   * [k][row], 2 * BM (2 * BN) bytes a k-row: 32 lanes of a transposing read touch 64 bytes of each of 4 k-rows.  Rows of 256
+//     bytes keep their 64-byte groups at g ^ (k & 3), rows of 128 bytes at g ^ (k >> 1 & 1).
+template <int BM_, int BN_, int WGM_, int WGN_, int STAGES_, bool A_KC_, bool B_KC_, int VIRT_ = VIRT_NONE>
+struct DmaTile {
+    typedef f16 E;
+    typedef Elem<f16> EL;
+    static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, STAGES = STAGES_;
+    static constexpr bool A_KC = A_KC_, B_KC = B_KC_;
+    static constexpr int VIRT = VIRT_;
+    static constexpr bool DMA = true, B_COLS = false;
+    static constexpr int ES = 2, EPV = 8, BK = 64, QUARTERS = 4, KQ = 16;
+    static constexpr int NT = WGM * WGN * 64;
+    static constexpr int TM = BM / WGM / 32, TN = BN / WGN / 32;
+    static constexpr int A_IT = BM * 8 / NT, B_IT = BN * 8 / NT, NP = A_IT + B_IT;
+    static_assert(A_IT * NT == BM * 8 && B_IT * NT == BN * 8, "every thread moves whole pieces of either operand");
+    static constexpr int A_ROWS = A_KC ? NT / 8 : NT / (BM / EPV), B_ROWS = B_KC ? NT / 8 : NT / (BN / EPV);
+    static_assert(A_ROWS % 16 == 0 && B_ROWS % 16 == 0, "a thread's swizzle is the same in every pass");
+    __device__ __host__ static constexpr int kc_row(int r) { return r * BK; }
+    static constexpr int A_LD = BM, B_LD = BN;
+    static constexpr int A_BYTES = BM * 128, STAGE_BYTES = (BM + BN) * 128, LDS_BYTES = STAGES * STAGE_BYTES;
+    static constexpr int HALF_PATCHES = NT / 128 * 32 * 36;  // floats: the epilogue's patches, in the stages
+    static constexpr int PATCH_SZ = HALF_PATCHES * 4 / ES;
+    static constexpr bool TWO_FIT = LDS_BYTES <= 80 * 1024;  // two workgroups per compute unit
+    static_assert(LDS_BYTES >= 2 * HALF_PATCHES * 4, "the patches fit the stages");
+    static constexpr bool PATCH_IN_A = true;
+    // position of a thread's piece in its row -> which piece of the row it fetches
+    template <bool KC, int SIDE>
+    __device__ __forceinline__ static int chunk_of(int row, int pos) {
+        if (KC) return pos ^ ((row >> 1) & 7);
+        return SIDE == 128 ? pos ^ ((row & 3) << 2) : pos ^ (((row >> 1) & 1) << 2);
+    }
+    // byte offset in an operand area of what this lane reads of 32-row block `blk` at k group 0
+    template <bool KC, int SIDE>
+    __device__ __forceinline__ static int frag_of(int lane, int blk) {
+        if (KC) return (blk * 32 + (lane & 31)) * 128 + (((lane >> 5) ^ ((lane >> 1) & 7)) << 4);
+        const int k = (lane >> 5) * 8 + ((lane & 15) >> 2), s = SIDE == 128 ? k & 3 : (k >> 1) & 1;
+        return k * SIDE * 2 + ((blk ^ s) << 6) + ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
+    }
+    template <bool KC, int SIDE>
+    __device__ __forceinline__ static f16x8 read(const char *area, int frag, int kg) {
+        if (KC) return *(const f16x8 *)(area + (frag ^ (kg << 5)));
+        const char *p = area + frag + kg * 16 * SIDE * 2;
+        const f16x4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4f16(LDS_PTR(f16x4v, p));
+        const f16x4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4f16(LDS_PTR(f16x4v, p + 4 * SIDE * 2));
+        const f16x8v both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        return __builtin_bit_cast(f16x8, both);
+    }
+};
+
+// One 16-byte piece per lane from global memory into LDS: lane i's lands at `target` + 16 * i (target, soffset and the descriptor
+// are uniform).  Written as asm so that the compiler does not hold every later LDS read until the load has landed; the waits and
+// the barrier of each K step order the two.  (m0 is written a wait state before the load that uses it.)
+__device__ __forceinline__ void dma_piece(unsigned target, const u32x4 &desc, unsigned voffset, unsigned soffset) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 : : "s"(target), "v"(voffset), "s"(desc), "s"(soffset) : "memory");
+}
+// s_waitcnt vmcnt(n) lgkmcnt(0): the builtin, so that the compiler knows that its own LDS reads have arrived
+template <int N>
+__device__ __forceinline__ void wait_loads_and_lds() {
+    static_assert(N >= 0 && N < 64, "vmcnt has six bits");
+    __builtin_amdgcn_s_waitcnt((N & 15) | 0x70 | ((N >> 4) << 14));
+}
 
 // Pieces [lo(q), lo(q+1)) are written to LDS during quarter q = 0, 1, 2 of a step and re-fetched
 // from global memory during quarter q + 1.
@@ -407,6 +486,83 @@ __device__ __forceinline__ void store_tile(f32x16 (&acc)[T::TM][T::TN], float *l
     }
 }
 
+// body(std::integral_constant<int, 0>) ... body(std::integral_constant<int, N - 1>), in order
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void each(F &&body) {
+    if constexpr (I < N) {
+        body(std::integral_constant<int, I>());
+        each<N, I + 1>(body);
+    }
+}
+
+// The K loop of a DmaTile.  In step t a wave's fragments of the whole step are in registers: the stage they came from is free,
+// and the fragments of step t + 1 are read while step t is multiplied, so neither the way from memory (STAGES - 1 steps) nor
+// that from LDS (one step) is waited for, and a step needs one barrier.
+// A load into LDS holds its wave until the address path (16 cycles a load, one path a compute unit) has taken it: issued in one
+// go behind the barrier the loads of all waves keep every matrix instruction waiting for 256 to 512 cycles (a 64 x 128 step
+// then takes 836 cycles instead of 620).  They are issued one at a time between the matrix instructions.
+// Bound by the loads: without them a 64 x 64 / 64 x 128 step takes 245 / 369 cycles, the loads alone 326 / 606, both 454 / 620 (about
+// 40 bytes a cycle and compute unit; free-running waves reach 64, waves that meet at a barrier do not, whatever the number of
+// stages, the pitch of the rows or the order of the steps).
+//   aim()                   turns to the next step; fetch(piece, target) puts a piece of it on its way
+//   started()               is called when the first operands have arrived
+template <typename T, class Aim, class Fetch, class Started>
+__device__ __forceinline__ void dma_loop(f16 *lds, int wave, int lane, int wm, int wn, int nsteps, f32x16 (&acc)[T::TM][T::TN],
+                                         Aim &&aim, Fetch &&fetch, Started &&started) {
+    constexpr int TM = T::TM, TN = T::TN, KG = T::QUARTERS, S = T::STAGES, NP = T::NP, NF = KG * (TM + TN), NM = KG * TM * TN;
+    const char *const base = (const char *)lds;
+    const unsigned wave_base = (unsigned)(unsigned long)LDS_PTR(char, lds) + (unsigned)wave * 1024u;
+    f16x8 fa[2][KG][TM], fb[2][KG][TN];
+    int a_at[TM], b_at[TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) a_at[i] = T::template frag_of<T::A_KC, T::BM>(lane, wm * TM + i);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) b_at[j] = T::template frag_of<T::B_KC, T::BN>(lane, wn * TN + j);
+    // fragment f of a step: k group by k group, in the order of their first use
+    auto read = [&](auto f, int set, int stage) {
+        constexpr int q = decltype(f)::value / (TM + TN), e = decltype(f)::value % (TM + TN);
+        const char *const as = base + stage * T::STAGE_BYTES, *const bs = as + T::A_BYTES;
+        if constexpr (e < TN) fb[set][q][e] = T::template read<T::B_KC, T::BN>(bs, b_at[e], q);
+        else fa[set][q][e - TN] = T::template read<T::A_KC, T::BM>(as, a_at[e - TN], q);
+    };
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        aim();
+        each<NP>([&](auto p) { fetch(p, wave_base + s * T::STAGE_BYTES); });
+    }
+    wait_loads_and_lds<(S - 1) * NP>();
+    __syncthreads();
+    each<NF>([&](auto f) { read(f, 0, 0); });
+    started();
+    int stage = 0;  // of step t
+    auto step = [&](auto set_tag) {
+        constexpr int set = decltype(set_tag)::value;
+        const int next = stage + 1 == S ? 0 : stage + 1;
+        const unsigned target = wave_base + stage * T::STAGE_BYTES;
+        aim();
+        // this wave's fragments of step t have been read and its pieces of step t + 1 have landed; behind the barrier that
+        // holds for all waves
+        wait_loads_and_lds<(S - 2) * NP>();
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
+        each<NM>([&](auto m_tag) {
+            constexpr int m = decltype(m_tag)::value, q = m / (TM * TN), i = m % (TM * TN) / TN, j = m % TN;
+            each<NF>([&](auto f) { if constexpr (slot_of(decltype(f)::value, NF, NM) == m) read(f, set ^ 1, next); });
+            acc[i][j] = Elem<f16>::mfma(fa[set][q][i], fb[set][q][j], acc[i][j], 0);
+            __builtin_amdgcn_sched_barrier(0);
+            each<NP>([&](auto p) { if constexpr (slot_of(decltype(p)::value, NP, NM) == m) fetch(p, target); });
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        stage = next;
+    };
+    for (int t = 0; t + 1 < nsteps; t += 2) {
+        step(std::integral_constant<int, 0>());
+        step(std::integral_constant<int, 1>());
+    }
+    if (nsteps & 1) step(std::integral_constant<int, 0>());
+    wait_loads_and_lds<0>();  // (nothing lands in LDS any more: the epilogue uses it)
+}
+
 // The work of one workgroup: workgroup (bx, bz) of a grid of nbx x layers (the launch's own blockIdx / gridDim, or what a
 // launch of two products makes of them).  As0 .. Bs1: the two halves of both operand areas in LDS.
 template <typename T, int EDGE>
@@ -419,7 +575,7 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     constexpr int A_IT = T::A_IT, NP = T::NP, ES = T::ES, EPV = T::EPV;
     constexpr bool A_KC = T::A_KC, B_KC = T::B_KC;
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = T::DMA ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
     const int wm = wave / T::WGN, wn = wave % T::WGN;
     unsigned long long st_w[4] = {0, 0, 0, 0}, st_c[2] = {0, 0};  // phase record (GemmArgs::phase_rec), a measurement aid
     if (g.phase_rec) st_w[0] = wall_clock64();
@@ -469,8 +625,8 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
             const int j = linear >> 3, piece = j / total;
             layer = (piece << 3) + (linear & 7);
             id = j - piece * total;
-        } else if ((total & 7) == 0) {
-            id = (id & 7) * (total >> 3) + (id >> 3);
+        } else if (T::DMA || (total & 7) == 0) {  // (the first total % 8 runs are one tile longer)
+            id = (id & 7) * (total >> 3) + min(id & 7, total & 7) + (id >> 3);
         }
         if (by_batch) b = layer;
         else split = layer;
@@ -503,15 +659,15 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     const long a_len = ANY ? (g.red - 1) * g.sA + (a_rows - 1) * g.lda + (A_KC ? g.K : g.M) + a_odd : (g.red - 1) * g.sA + a_rows * g.lda;
     // (the taps of a filter interleave inside its rows: the filter ends with its last row)
     const long b_len = ANY ? (g.red - 1) * g.sB + (b_rows - 1) * g.ldb + (B_KC ? g.K : g.N) + b_odd : (VA ? 0 : (g.red - 1) * g.sB) + b_rows * g.ldb;
-    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(Ab - a_odd), 0, VA ? (int)pg.bytes : (int)((ES * a_len + 3) & ~3L), 0x00020000);
-    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(Bb - b_odd), 0, VIRT == VIRT_B_KROWS ? (int)pg.bytes : (int)((ES * b_len + 3) & ~3L), 0x00020000);
+    const int a_bytes = VA ? (int)pg.bytes : (int)((ES * a_len + 3) & ~3L), b_bytes = VIRT == VIRT_B_KROWS ? (int)pg.bytes : (int)((ES * b_len + 3) & ~3L);
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void *)(Ab - a_odd), 0, a_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void *)(Bb - b_odd), 0, b_bytes, 0x00020000);
     // where the tile starts, in elements: uniform, but for half rows at any element only the dword part of it is
     const unsigned a_tile = (A_KC ? (unsigned)m0 * g.lda : (unsigned)m0) + a_odd, b_tile = (B_KC ? (unsigned)n0 * g.ldb : (unsigned)n0) + b_odd;
     const unsigned Au = (unsigned)ES * (ODD ? a_tile & ~1u : a_tile), Bu = (unsigned)ES * (ODD ? b_tile & ~1u : b_tile);
-    const int a_r = A_KC ? tid >> 3 : tid / (BM / EPV), a_c = A_KC ? tid & 7 : tid % (BM / EPV);
-    const int b_r = (B_KC || T::B_COLS) ? tid >> 3 : tid / (BN / EPV), b_c = (B_KC || T::B_COLS) ? tid & 7 : tid % (BN / EPV);
+    const int a_r = A_KC ? tid >> 3 : tid / (BM / EPV), b_r = (B_KC || T::B_COLS) ? tid >> 3 : tid / (BN / EPV);
+    int a_c = A_KC ? tid & 7 : tid % (BM / EPV), b_c = (B_KC || T::B_COLS) ? tid & 7 : tid % (BN / EPV);
+    if constexpr (T::DMA) a_c = T::template chunk_of<A_KC, BM>(a_r, a_c), b_c = T::template chunk_of<B_KC, BN>(b_r, b_c);
     const int a_dst = (A_KC ? T::kc_row(a_r) : a_r * A_LD) + a_c * EPV, b_dst = (B_KC ? T::kc_row(b_r) : b_r * B_LD) + b_c * EPV;
     const unsigned a_pass = VA ? 0u : (unsigned)ES * T::A_ROWS * g.lda;  // bytes
     const unsigned b_pass = VIRT == VIRT_B_KROWS ? 0u : (unsigned)ES * T::B_ROWS * g.ldb;
@@ -583,12 +739,6 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
         }
     }
 
-    // ---- per-lane LDS offsets of its MFMA operands
-    const int a_frag = A_KC ? T::kc_row(wm * TM * 32 + (lane & 31)) + (lane >> 5) * EL::KC_HALF : EL::tr_offset(lane, A_LD, wm * TM * 32);
-    const int b_frag = B_KC ? T::kc_row(wn * TN * 32 + (lane & 31)) + (lane >> 5) * EL::KC_HALF : EL::tr_offset(lane, B_LD, wn * TN * 32);
-
-    u32x4 R[NP];
-    typename EL::Frag fa[2][TM], fb[2][TN];
     f32x16 acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -596,6 +746,10 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
         for (int j = 0; j < TN; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+
+    // ---- per-lane LDS offsets of its MFMA operands
+    const int a_frag = A_KC ? T::kc_row(wm * TM * 32 + (lane & 31)) + (lane >> 5) * EL::KC_HALF : EL::tr_offset(lane, A_LD, wm * TM * 32);
+    const int b_frag = B_KC ? T::kc_row(wn * TN * 32 + (lane & 31)) + (lane >> 5) * EL::KC_HALF : EL::tr_offset(lane, B_LD, wn * TN * 32);
 
     // ---- this workgroup's steps x0 .. x0 + nsteps - 1 of the extended reduction; step x reads
     // product x / ktiles at K offset (x % ktiles) * BK (all uniform: scalar arithmetic, counted on from step to step)
@@ -609,8 +763,9 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     // The step that is fetched next: its product, K step and filter tap are counted on from step to step (every step is
     // fetched once, in order), because four divisions by runtime numbers at the head of each step -- some 35 dependent
     // scalar instructions that no matrix instruction covers -- were a fifth of a short half step's time.
-    int ld_i = 0, ld_r = x0 / ktiles, ld_kx = x0 - ld_r * ktiles;
-    int ld_fy = VA ? ld_r / pg.FW : 0, ld_fx = VA ? ld_r - ld_fy * pg.FW : 0;
+    // (uniform, and said to be: the compiler keeps the quotients of an integer division in vector registers otherwise)
+    int ld_i = 0, ld_r = T::DMA ? __builtin_amdgcn_readfirstlane(x0 / ktiles) : x0 / ktiles, ld_kx = x0 - ld_r * ktiles;
+    int ld_fy = !VA ? 0 : T::DMA ? __builtin_amdgcn_readfirstlane(ld_r / pg.FW) : ld_r / pg.FW, ld_fx = VA ? ld_r - ld_fy * pg.FW : 0;
     // patch k-rows: what BK more pixels add, and the corrections when a row or an image is complete
     int vb_dy = 0, vb_dx = 0, vb_d = 0, vb_d_row = 0, vb_d_img = 0;
     if constexpr (VIRT == VIRT_B_KROWS) {
@@ -702,42 +857,64 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
         pa = step_a(), pb = step_b();
         step_on();
     };
-    auto fetch_all = [&](unsigned pa, unsigned pb) {
-#pragma unroll
-        for (int p = 0; p < NP; ++p) {
-            R[p] = p < A_IT ? __builtin_amdgcn_raw_buffer_load_b128(ra, av[p < A_IT ? p : 0], pa + p * a_pass, 0)
-                            : __builtin_amdgcn_raw_buffer_load_b128(rb, bv[p < A_IT ? 0 : p - A_IT], pb + (p - A_IT) * b_pass, 0);
-            L.fetch(p, p < A_IT ? ra : rb, p < A_IT ? av[p < A_IT ? p : 0] : bv[p < A_IT ? 0 : p - A_IT], p < A_IT ? pa + p * a_pass : pb + (p - A_IT) * b_pass);
-        }
-    };
-
-    // ---- prologue: step 0 into LDS half 0, step 1 into registers, first operands of step 0
     unsigned pa, pb;
-    next_step(pa, pb);
-    fetch_all(pa, pb);
-    next_step(pa, pb);
-#pragma unroll
-    for (int p = 0; p < NP; ++p)
-        *(u32x4 *)(p < A_IT ? As0 + a_dst + p * T::A_PASS : Bs0 + b_dst + (p - A_IT) * T::B_PASS) = L.place(p, R[p]);
-    fetch_all(pa, pb);
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-        fa[0][i] = A_KC ? EL::read_kc(As0 + a_frag + i * T::A_BLK) : EL::read_tr(As0 + a_frag + i * 32, A_LD);
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-        fb[0][j] = B_KC ? EL::read_kc(Bs0 + b_frag + j * T::B_BLK) : EL::read_tr(Bs0 + b_frag + j * 32, B_LD);
-
-    if (g.phase_rec) st_w[1] = wall_clock64(), st_c[0] = __builtin_readcyclecounter();
-    // ---- main loop, two steps per trip so that the LDS half of every access is known statically;
-    for (int i = 0; i < nsteps; i += 2) {
-        next_step(pa, pb);
-        k_step<T, EDGE>(As0 + a_frag, Bs0 + b_frag, As1 + a_frag, Bs1 + b_frag, As1 + a_dst, Bs1 + b_dst, ra, rb, pa, pb,
-                        a_pass, b_pass, av, bv, R, L, fa, fb, acc);
-        if (i + 1 < nsteps) {
+    if constexpr (T::DMA) {
+        // the next step: where it lies (past the last one nothing is fetched), then its pieces one by one
+        u32x4 da, db;
+        unsigned sa, sb;
+        auto aim = [&]() {
+            const bool live = ld_i < nsteps;
             next_step(pa, pb);
-            k_step<T, EDGE>(As1 + a_frag, Bs1 + b_frag, As0 + a_frag, Bs0 + b_frag, As0 + a_dst, Bs0 + b_dst, ra, rb, pa, pb,
+            sa = __builtin_amdgcn_readfirstlane(pa), sb = __builtin_amdgcn_readfirstlane(pb);  // (uniform already)
+            const unsigned long at_a = (unsigned long)Ab, at_b = (unsigned long)Bb;
+            da = (u32x4){(unsigned)at_a, (unsigned)(at_a >> 32) & 0xffffu, live ? (unsigned)a_bytes : 0u, 0x00020000u};
+            db = (u32x4){(unsigned)at_b, (unsigned)(at_b >> 32) & 0xffffu, live ? (unsigned)b_bytes : 0u, 0x00020000u};
+        };
+        auto fetch = [&](auto piece, unsigned target) {
+            constexpr int p = decltype(piece)::value;
+            if constexpr (p < A_IT) dma_piece(target + p * T::NT * 16, da, av[p], sa + p * a_pass);
+            else dma_piece(target + T::A_BYTES + (p - A_IT) * T::NT * 16, db, bv[p - A_IT], sb + (p - A_IT) * b_pass);
+        };
+        dma_loop<T>(As0, wave, lane, wm, wn, nsteps, acc, aim, fetch, [&]() { if (g.phase_rec) st_w[1] = wall_clock64(), st_c[0] = __builtin_readcyclecounter(); });
+    } else {
+        u32x4 R[NP];
+        typename EL::Frag fa[2][TM], fb[2][TN];
+        auto fetch_all = [&](unsigned pa, unsigned pb) {
+#pragma unroll
+            for (int p = 0; p < NP; ++p) {
+                R[p] = p < A_IT ? __builtin_amdgcn_raw_buffer_load_b128(ra, av[p < A_IT ? p : 0], pa + p * a_pass, 0)
+                                : __builtin_amdgcn_raw_buffer_load_b128(rb, bv[p < A_IT ? 0 : p - A_IT], pb + (p - A_IT) * b_pass, 0);
+                L.fetch(p, p < A_IT ? ra : rb, p < A_IT ? av[p < A_IT ? p : 0] : bv[p < A_IT ? 0 : p - A_IT], p < A_IT ? pa + p * a_pass : pb + (p - A_IT) * b_pass);
+            }
+        };
+
+        // ---- prologue: step 0 into LDS half 0, step 1 into registers, first operands of step 0
+        next_step(pa, pb);
+        fetch_all(pa, pb);
+        next_step(pa, pb);
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+            *(u32x4 *)(p < A_IT ? As0 + a_dst + p * T::A_PASS : Bs0 + b_dst + (p - A_IT) * T::B_PASS) = L.place(p, R[p]);
+        fetch_all(pa, pb);
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+            fa[0][i] = A_KC ? EL::read_kc(As0 + a_frag + i * T::A_BLK) : EL::read_tr(As0 + a_frag + i * 32, A_LD);
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+            fb[0][j] = B_KC ? EL::read_kc(Bs0 + b_frag + j * T::B_BLK) : EL::read_tr(Bs0 + b_frag + j * 32, B_LD);
+
+        if (g.phase_rec) st_w[1] = wall_clock64(), st_c[0] = __builtin_readcyclecounter();
+        // ---- main loop, two steps per trip so that the LDS half of every access is known statically;
+        for (int i = 0; i < nsteps; i += 2) {
+            next_step(pa, pb);
+            k_step<T, EDGE>(As0 + a_frag, Bs0 + b_frag, As1 + a_frag, Bs1 + b_frag, As1 + a_dst, Bs1 + b_dst, ra, rb, pa, pb,
                             a_pass, b_pass, av, bv, R, L, fa, fb, acc);
+            if (i + 1 < nsteps) {
+                next_step(pa, pb);
+                k_step<T, EDGE>(As1 + a_frag, Bs1 + b_frag, As0 + a_frag, Bs0 + b_frag, As0 + a_dst, Bs0 + b_dst, ra, rb, pa, pb,
+                                a_pass, b_pass, av, bv, R, L, fa, fb, acc);
+            }
         }
     }
 
@@ -746,6 +923,7 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     __syncthreads();  // every wave is past the last step: the operand areas are free
     const Origin o = {m0, n0, m_own, n_own, M, g.N, (wm * TM) * 32, (wn * TN) * 32};
     float *patches = (float *)(T::PATCH_IN_A ? As0 : Bs0), *patches1 = (float *)(T::PATCH_IN_A ? As1 : Bs1);
+    if constexpr (T::DMA) patches1 = patches + T::HALF_PATCHES;
     if (in_tail) {  // partial sums of the band, rows counted from its first
         const int tail_M = M - g.tail_m0;
         const Origin ot = {m0 - g.tail_m0, n0, m_own - g.tail_m0, n_own, tail_M, g.N, (wm * TM) * 32, (wn * TN) * 32};
@@ -775,14 +953,19 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
 // which leaves room for one workgroup per compute unit; told to make room for two it takes 186 and spills none.  Half DeConv2d
 // 32 x 20x20x128 -> 128, 2x2 stride 2, 15.7 -> 11.0 us; 24 x 26x26x448 -> 288, 4x4 stride 2, 150 -> 119 us)
 template <typename T, int EDGE = EDGE_NONE>
-__global__ __launch_bounds__(T::NT, T::VIRT == VIRT_A_CLASSES && T::BN == 128 ? 2 : 1) void gemm_tiled_kernel(GemmArgs g, int tilesM, int tilesN) {
+__global__ __launch_bounds__(T::NT, T::VIRT == VIRT_A_CLASSES && T::BN == 128 || T::TWO_FIT ? 2 : 1) void gemm_tiled_kernel(GemmArgs g, int tilesM, int tilesN) {
     typedef typename T::E E;
-    // four separate arrays, so that reads of one half are known not to touch the other
-    __shared__ __attribute__((aligned(16))) E As0[T::A_SZ];
-    __shared__ __attribute__((aligned(16))) E As1[T::A_SZ];
-    __shared__ __attribute__((aligned(16))) E Bs0[T::B_SZ];
-    __shared__ __attribute__((aligned(16))) E Bs1[T::B_SZ];
-    gemm_tiled_body<T, EDGE>(g, tilesM, tilesN, (int)blockIdx.x, (int)blockIdx.z, (int)gridDim.x, As0, As1, Bs0, Bs1);
+    if constexpr (T::DMA) {
+        __shared__ __attribute__((aligned(1024))) E stages[T::LDS_BYTES / T::ES];
+        gemm_tiled_body<T, EDGE>(g, tilesM, tilesN, (int)blockIdx.x, (int)blockIdx.z, (int)gridDim.x, stages, nullptr, nullptr, nullptr);
+    } else {
+        // four separate arrays, so that reads of one half are known not to touch the other
+        __shared__ __attribute__((aligned(16))) E As0[T::A_SZ];
+        __shared__ __attribute__((aligned(16))) E As1[T::A_SZ];
+        __shared__ __attribute__((aligned(16))) E Bs0[T::B_SZ];
+        __shared__ __attribute__((aligned(16))) E Bs1[T::B_SZ];
+        gemm_tiled_body<T, EDGE>(g, tilesM, tilesN, (int)blockIdx.x, (int)blockIdx.z, (int)gridDim.x, As0, As1, Bs0, Bs1);
+    }
 }
 
 // Two products in one launch: the first nx0 * nz0 workgroups are the first product's grid (x fastest), the rest the
@@ -791,23 +974,57 @@ __global__ __launch_bounds__(T::NT, T::VIRT == VIRT_A_CLASSES && T::BN == 128 ? 
 // that nothing hides when a compute unit holds one workgroup), and side by side on a compute unit one's waits are
 // the other's issue slots.  The operand areas are as large as the larger tile needs.
 template <typename T0, typename T1>
-__global__ __launch_bounds__(T0::NT) void gemm_tiled_pair_kernel(GemmArgs g0, GemmArgs g1, int tilesM0, int tilesN0, int nx0, int nz0,
+__global__ __launch_bounds__(T0::NT, T0::TWO_FIT && T1::TWO_FIT ? 2 : 1) void gemm_tiled_pair_kernel(GemmArgs g0, GemmArgs g1, int tilesM0, int tilesN0, int nx0, int nz0,
                                                                  int tilesM1, int tilesN1, int nx1) {
     typedef typename T0::E E;
-    static_assert(T0::NT == T1::NT && sizeof(typename T0::E) == sizeof(typename T1::E), "one workgroup shape, one element type");
-    constexpr int A_SZ = T0::A_SZ > T1::A_SZ ? T0::A_SZ : T1::A_SZ, B_SZ = T0::B_SZ > T1::B_SZ ? T0::B_SZ : T1::B_SZ;
-    __shared__ __attribute__((aligned(16))) E As0[A_SZ];
-    __shared__ __attribute__((aligned(16))) E As1[A_SZ];
-    __shared__ __attribute__((aligned(16))) E Bs0[B_SZ];
-    __shared__ __attribute__((aligned(16))) E Bs1[B_SZ];
-    const int id = (int)blockIdx.x, first = nx0 * nz0;
-    if (id < first) {
-        gemm_tiled_body<T0, EDGE_NONE>(g0, tilesM0, tilesN0, id % nx0, id / nx0, nx0, As0, As1, Bs0, Bs1);
+    static_assert(T0::NT == T1::NT && sizeof(typename T0::E) == sizeof(typename T1::E) && T0::DMA == T1::DMA, "one workgroup shape, one element type");
+    if constexpr (T0::DMA) {
+        __shared__ __attribute__((aligned(1024))) E stages[(T0::LDS_BYTES > T1::LDS_BYTES ? T0::LDS_BYTES : T1::LDS_BYTES) / T0::ES];
+        const int id = (int)blockIdx.x, first = nx0 * nz0, j = id - first;
+        if (id < first) gemm_tiled_body<T0, EDGE_NONE>(g0, tilesM0, tilesN0, id % nx0, id / nx0, nx0, stages, nullptr, nullptr, nullptr);
+        else gemm_tiled_body<T1, EDGE_NONE>(g1, tilesM1, tilesN1, j % nx1, j / nx1, nx1, stages, nullptr, nullptr, nullptr);
     } else {
-        const int j = id - first;
-        gemm_tiled_body<T1, EDGE_NONE>(g1, tilesM1, tilesN1, j % nx1, j / nx1, nx1, As0, As1, Bs0, Bs1);
+        constexpr int A_SZ = T0::A_SZ > T1::A_SZ ? T0::A_SZ : T1::A_SZ, B_SZ = T0::B_SZ > T1::B_SZ ? T0::B_SZ : T1::B_SZ;
+        __shared__ __attribute__((aligned(16))) E As0[A_SZ];
+        __shared__ __attribute__((aligned(16))) E As1[A_SZ];
+        __shared__ __attribute__((aligned(16))) E Bs0[B_SZ];
+        __shared__ __attribute__((aligned(16))) E Bs1[B_SZ];
+        const int id = (int)blockIdx.x, first = nx0 * nz0;
+        if (id < first) {
+            gemm_tiled_body<T0, EDGE_NONE>(g0, tilesM0, tilesN0, id % nx0, id / nx0, nx0, As0, As1, Bs0, Bs1);
+        } else {
+            const int j = id - first;
+            gemm_tiled_body<T1, EDGE_NONE>(g1, tilesM1, tilesN1, j % nx1, j / nx1, nx1, As0, As1, Bs0, Bs1);
+        }
     }
 }
+
+// The kernel tile of a BM x BN output tile: in half, operands in whole pieces go straight into LDS.  Four waves, and as many
+// stages as let two workgroups share a compute unit.  DEEP: 128 x 128 tiles of a launch of at most one workgroup per compute unit,
+// which may have all of its LDS: two stages fetch one step ahead, less than the way from memory takes (2048^3, a K step of 128 x
+// 128: 1270 cycles with two stages, 825 - 870 with four; with five the same), and eight waves share out the addresses of
+// patch rows (Conv2d 16 x 57x57x96 -> 160, 3x3 stride 2, forward 17.1 us with four waves, 15.3 with eight).  More stages or
+// eight waves on the smaller tiles gave nothing (64 x 64 with 4, 6, 8 stages 454, 516, 522 cycles a step, with eight waves 520).
+template <typename E, int BM, int BN, bool A_KC, bool B_KC, int VIRT = VIRT_NONE, bool DEEP = false>
+struct TileOf {
+    typedef Tile<E, BM, BN, BM == 256 || BN == 32 ? 4 : 2, BN == 32 ? 1 : 2, A_KC, B_KC, VIRT> type;
+};
+template <bool A_KC, bool B_KC, int VIRT>
+struct TileOf<f16, 64, 64, A_KC, B_KC, VIRT> {
+    typedef DmaTile<64, 64, 2, 2, 4, A_KC, B_KC, VIRT> type;
+};
+template <bool A_KC, bool B_KC, int VIRT>
+struct TileOf<f16, 64, 128, A_KC, B_KC, VIRT> {
+    typedef DmaTile<64, 128, 2, 2, 3, A_KC, B_KC, VIRT> type;
+};
+template <bool A_KC, bool B_KC, int VIRT>
+struct TileOf<f16, 128, 64, A_KC, B_KC, VIRT> {
+    typedef DmaTile<128, 64, 2, 2, 3, A_KC, B_KC, VIRT> type;
+};
+template <bool A_KC, bool B_KC, int VIRT, bool DEEP>
+struct TileOf<f16, 128, 128, A_KC, B_KC, VIRT, DEEP> {
+    typedef DmaTile<128, 128, 2, DEEP ? 4 : 2, DEEP ? 4 : 2, A_KC, B_KC, VIRT> type;
+};
 
 // where d8_gemm_phase_record asked the next launches to write their records (process-wide; null: no records; defined in
 // gemm_tiled.hip)

@@ -19,13 +19,13 @@ static int launch_pair(const GemmArgs &gx, const GemmArgs &gy, hipStream_t strea
     if (!pair_tiles<E>(gx, gy, tx, ty)) return fail(D8_ERR_ARGUMENT, "gemm_tiled_pair_launch: no kernel for this pair of tiles");
 #define D8_PAIR_Y(TXT)                                                                                                  \
     switch (ty) {                                                                                                       \
-        case TILE_128x128: return launch_pair_tiles<TXT, Tile<E, 128, 128, 2, 2, false, false, VIRT_B_KROWS>>(gx, gy, stream); \
-        case TILE_64x128: return launch_pair_tiles<TXT, Tile<E, 64, 128, 2, 2, false, false, VIRT_B_KROWS>>(gx, gy, stream);   \
-        default: return launch_pair_tiles<TXT, Tile<E, 64, 64, 2, 2, false, false, VIRT_B_KROWS>>(gx, gy, stream);            \
+        case TILE_128x128: return launch_pair_tiles<TXT, typename TileOf<E, 128, 128, false, false, VIRT_B_KROWS>::type>(gx, gy, stream); \
+        case TILE_64x128: return launch_pair_tiles<TXT, typename TileOf<E, 64, 128, false, false, VIRT_B_KROWS>::type>(gx, gy, stream);   \
+        default: return launch_pair_tiles<TXT, typename TileOf<E, 64, 64, false, false, VIRT_B_KROWS>::type>(gx, gy, stream);            \
     }
-    typedef Tile<E, 64, 128, 2, 2, true, false, VIRT_A_ROWS> X0;
-    typedef Tile<E, 128, 128, 2, 2, true, false, VIRT_A_ROWS> X1;
-    typedef Tile<E, 128, 64, 2, 2, true, false, VIRT_A_ROWS> X2;
+    typedef typename TileOf<E, 64, 128, true, false, VIRT_A_ROWS>::type X0;
+    typedef typename TileOf<E, 128, 128, true, false, VIRT_A_ROWS>::type X1;
+    typedef typename TileOf<E, 128, 64, true, false, VIRT_A_ROWS>::type X2;
     if (tx == TILE_64x128) { D8_PAIR_Y(X0) }
     if (tx == TILE_128x128) { D8_PAIR_Y(X1) }
     D8_PAIR_Y(X2)

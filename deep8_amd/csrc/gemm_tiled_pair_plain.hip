@@ -20,15 +20,15 @@ static int launch_plain_pair(const GemmArgs &g0, const GemmArgs &g1, hipStream_t
     if (!plain_pair_tiles<E>(g0, g1, t0, t1)) return fail(D8_ERR_ARGUMENT, "gemm_tiled_plain_pair_launch: no kernel for this pair of tiles");
 #define D8_PAIR_1(T0T)                                                                                              \
     switch (t1) {                                                                                                   \
-        case TILE_128x128: return launch_pair_tiles<T0T, Tile<E, 128, 128, 2, 2, false, false>>(g0, g1, stream);    \
-        case TILE_64x128: return launch_pair_tiles<T0T, Tile<E, 64, 128, 2, 2, false, false>>(g0, g1, stream);      \
-        case TILE_64x64: return launch_pair_tiles<T0T, Tile<E, 64, 64, 2, 2, false, false>>(g0, g1, stream);        \
-        default: return launch_pair_tiles<T0T, Tile<E, 128, 64, 2, 2, false, false>>(g0, g1, stream);               \
+        case TILE_128x128: return launch_pair_tiles<T0T, typename TileOf<E, 128, 128, false, false>::type>(g0, g1, stream);    \
+        case TILE_64x128: return launch_pair_tiles<T0T, typename TileOf<E, 64, 128, false, false>::type>(g0, g1, stream);      \
+        case TILE_64x64: return launch_pair_tiles<T0T, typename TileOf<E, 64, 64, false, false>::type>(g0, g1, stream);        \
+        default: return launch_pair_tiles<T0T, typename TileOf<E, 128, 64, false, false>::type>(g0, g1, stream);               \
     }
-    typedef Tile<E, 64, 128, 2, 2, true, true> A0;
-    typedef Tile<E, 128, 128, 2, 2, true, true> A1;
-    typedef Tile<E, 128, 64, 2, 2, true, true> A2;
-    typedef Tile<E, 64, 64, 2, 2, true, true> A3;
+    typedef typename TileOf<E, 64, 128, true, true>::type A0;
+    typedef typename TileOf<E, 128, 128, true, true>::type A1;
+    typedef typename TileOf<E, 128, 64, true, true>::type A2;
+    typedef typename TileOf<E, 64, 64, true, true>::type A3;
     if (t0 == TILE_64x64) { D8_PAIR_1(A3) }
     if (t0 == TILE_64x128) { D8_PAIR_1(A0) }
     if (t0 == TILE_128x128) { D8_PAIR_1(A1) }
