@@ -564,6 +564,168 @@ static int plan_splits(int BK, int M, int N, int K, int batch, int red, size_t w
     return tps > 0 ? (int)((total + tps - 1) / tps) : 1;
 }
 
+// ---- rows that start anywhere, copied to rows of whole pieces -------------------------------------------------
+struct PackArgs {
+    const f16 *src;
+    f16 *dst;
+    int rows, cols, ld, pitch;  // rows of all matrices that follow each other, `per` of them `stride` elements from the next
+    int per;
+    long stride;
+    int across;
+    unsigned first;  // workgroup
+};
+struct PackList {
+    PackArgs m[3];
+    int n;
+};
+
+// Bound by memory.  `across` threads (a power of two, at most 256) lie along a row, a thread copies 16 bytes of four rows before it
+// goes on along them, read at the alignment of an element.  Copied rows start at multiples of 128 bytes, as the K steps of
+// the product want them (pitch 1008 instead of 1024: 4096 x 1001 x 1024 loop of the product 9.7 us instead of 8.3).
+constexpr int PACK_ROWS = 4;
+__global__ __launch_bounds__(256) void pack_rows_kernel(PackList L) {
+    typedef f16x8 f16x8_any __attribute__((aligned(2)));
+    const int i = L.n > 2 && blockIdx.x >= L.m[2].first ? 2 : L.n > 1 && blockIdx.x >= L.m[1].first ? 1 : 0;
+    const PackArgs &a = L.m[i];
+    const int down = 256 / a.across, row0 = (int)(blockIdx.x - a.first) * PACK_ROWS * down + (int)threadIdx.x / a.across;
+    const f16 *src[PACK_ROWS];
+    f16 *const dst = a.dst + (long)row0 * a.pitch;
+#pragma unroll
+    for (int u = 0; u < PACK_ROWS; ++u) {
+        const int row = row0 + u * down, m = a.per < a.rows ? row / a.per : 0;
+        src[u] = row < a.rows ? a.src + (long)m * a.stride + (long)(row - m * a.per) * a.ld : nullptr;
+    }
+    for (int c = ((int)threadIdx.x & (a.across - 1)) * 8; c < a.pitch; c += a.across * 8) {
+        f16x8 v[PACK_ROWS];
+#pragma unroll
+        for (int u = 0; u < PACK_ROWS; ++u) {
+            v[u] = (f16x8)(f16)0.f;
+            if (!src[u]) continue;
+            if (c + 8 <= a.cols) v[u] = *(const f16x8_any *)(src[u] + c);
+            else
+                for (int e = 0; e < 8; ++e)
+                    if (c + e < a.cols) v[u][e] = src[u][c + e];
+        }
+#pragma unroll
+        for (int u = 0; u < PACK_ROWS; ++u)
+            if (src[u]) *(f16x8 *)(dst + (long)u * down * a.pitch + c) = v[u];
+    }
+}
+
+// Which operands of a product have to be copied (bit 0: A, bit 1: B): those that cannot be moved in whole pieces, and if K is no
+// multiple of a piece all that are stored along K, whose copies end in zeros.
+static int pack_operands(const GemmArgs &g, int ta, int tb) {
+    auto odd = [](const void *p, int ld, long s, int extent) { return (((size_t)p & 15) || ld % 8 || s % 8 || extent % 8) ? 1 : 0; };
+    return odd(g.A, g.lda, g.sA, ta ? g.M : g.K) | odd(g.B, g.ldb, g.sB, tb ? g.K : g.N) << 1;
+}
+
+struct PackShape {
+    const void *p;
+    long rows;
+    int cols, ld, per;
+    long stride;
+};
+static PackShape pack_shape(const GemmArgs &g, int ta, int tb, int op) {
+    const int count = (op ? g.sB : g.sA) ? g.batch * g.red : 1;
+    PackShape s;
+    s.p = op ? g.B : g.A;
+    s.per = op ? (tb ? g.N : g.K) : (ta ? g.K : g.M), s.cols = op ? (tb ? g.K : g.N) : (ta ? g.M : g.K);
+    s.rows = (long)s.per * count, s.ld = op ? g.ldb : g.lda, s.stride = op ? g.sB : g.sA;
+    return s;
+}
+static int pack_pitch(const PackShape &s) { return (s.cols + 63) & ~63; }
+static size_t pack_bytes(const PackShape &s) { return (size_t)s.rows * pack_pitch(s) * 2; }  // (a multiple of 128)
+
+// What is to be copied for two products: a matrix that both read is copied once.
+struct PackPlan {
+    PackShape shapes[4];
+    int n, slot[2][2];
+    size_t bytes;
+};
+
+// Whether copies pay: a product then saves some 0.13 us per K step of a 128 x 128 tile and round of the chip where one of its
+// operands is odd and 0.33 where both are, and the two share a launch; the copies take 3 us and 0.4 a MB.  Calls with odd sizes,
+// 500 drawn: 10822 us on the kernels for rows that start anywhere, 9892 on copies always, 10017 with this rule (and fewer that
+// lose: small products, and large matrices copied for few rows or columns); 400 others 8686 and 8037, the better of the two
+// 8008.  4096 rows, 1024 -> 1001: 44.6 -> 38.2 us.  (A product by itself gains too seldom: 600 drawn 6593 us without copies, 7927
+// with, 6442 the better of the two.)
+static bool pack_pays(const PackedProduct (&p)[2], const PackPlan &plan) {
+    const char *force = getenv("D8_GEMM_PACK");  // tuning and test aid (read at every call): 0 never, 1 always
+    if (force) return atoi(force) != 0;
+    double saved = 0.0;
+    for (int i = 0; i < 2; ++i) {
+        const GemmArgs &g = *p[i].g;
+        const int odd = (plan.slot[i][0] >= 0) + (plan.slot[i][1] >= 0), shortest = g.M < g.N ? (g.M < g.K ? g.M : g.K) : (g.N < g.K ? g.N : g.K);
+        if (shortest < 64 || (double)g.M * g.N * g.K < (1 << 25)) return false;
+        const double steps = (double)ceil_div(g.M, 128) * ceil_div(g.N, 128) * g.batch * g.red * ceil_div(g.K, 64) / cu_count();
+        saved += (odd == 2 ? 0.33 : odd == 1 ? 0.13 : 0.0) * (steps < 1.0 ? 1.0 : steps);
+    }
+    return saved > 0.2e-6 * plan.bytes;
+}
+
+// (products of one launch, on the tiled kernels)
+static bool pack_plan(int dtype, const PackedProduct (&p)[2], PackPlan &plan) {
+    plan.n = 0, plan.bytes = 0;
+    if (dtype != D8_FLOAT16) return false;
+    for (int i = 0; i < 2; ++i) {
+        const GemmArgs &g = *p[i].g;
+        if (g.virt != VIRT_NONE || g.K < 1 || g.batch > 448 || g.M > 65535 * 128 || gemm_is_small(g.M, g.N, g.K, g.batch, g.red) ||
+            !gemm_tiled_eligible(dtype, g, p[i].ta, p[i].tb)) return false;
+        const int ops = pack_operands(g, p[i].ta, p[i].tb);
+        for (int op = 0; op < 2; ++op) {
+            plan.slot[i][op] = -1;
+            if (!(ops >> op & 1)) continue;
+            const PackShape s = pack_shape(g, p[i].ta, p[i].tb, op);
+            if (pack_bytes(s) >= (1u << 31)) return false;  // (byte offsets inside an operand are 32-bit)
+            int k = 0;
+            while (k < plan.n && !(plan.shapes[k].p == s.p && plan.shapes[k].rows == s.rows && plan.shapes[k].cols == s.cols &&
+                                   plan.shapes[k].ld == s.ld && plan.shapes[k].per == s.per && plan.shapes[k].stride == s.stride)) ++k;
+            if (k == plan.n) plan.shapes[plan.n++] = s, plan.bytes += pack_bytes(s);
+            plan.slot[i][op] = k;
+        }
+    }
+    return plan.n > 0 && plan.n <= 3 && pack_pays(p, plan);
+}
+
+size_t gemm_pack_bytes(int dtype, const PackedProduct (&p)[2]) {
+    PackPlan plan;
+    return pack_plan(dtype, p, plan) ? plan.bytes : 0;
+}
+
+bool gemm_pack(int dtype, const PackedProduct (&p)[2], void *workspace, size_t workspace_bytes, size_t *used, hipStream_t stream, int *rc) {
+    PackPlan plan;
+    if (!workspace || ((size_t)workspace & 15) || !pack_plan(dtype, p, plan) || plan.bytes > workspace_bytes) return false;
+    PackList L;
+    L.n = plan.n;
+    unsigned blocks = 0;
+    char *to = (char *)workspace;
+    for (int k = 0; k < plan.n; ++k) {
+        const PackShape &s = plan.shapes[k];
+        int across = 8;
+        while (across < 256 && across * 8 < pack_pitch(s)) across *= 2;
+        L.m[k] = {(const f16 *)s.p, (f16 *)to, (int)s.rows, s.cols, s.ld, pack_pitch(s), s.per, s.stride, across, blocks};
+        blocks += (unsigned)ceil_div(s.rows, PACK_ROWS * (256 / across));
+        to += pack_bytes(s);
+    }
+    *used = plan.bytes;
+    hipLaunchKernelGGL(pack_rows_kernel, dim3(blocks), dim3(256), 0, stream, L);
+    const hipError_t e = hipGetLastError();
+    *rc = e == hipSuccess ? 0 : fail((int)e, "kernel launch: %s", hipGetErrorString(e));
+    for (int i = 0; i < 2; ++i) {
+        GemmArgs &g = *p[i].g;
+        if (plan.slot[i][0] >= 0) {
+            const PackArgs &a = L.m[plan.slot[i][0]];
+            g.A = a.dst, g.lda = a.pitch, g.sA = g.sA ? (long)a.per * a.pitch : 0;
+        }
+        if (plan.slot[i][1] >= 0) {
+            const PackArgs &b = L.m[plan.slot[i][1]];
+            g.B = b.dst, g.ldb = b.pitch, g.sB = g.sB ? (long)b.per * b.pitch : 0;
+        }
+        g.packed = 1, g.padM = (g.M + 7) & ~7, g.padN = (g.N + 7) & ~7;
+    }
+    return true;
+}
+
 // C = beta * C + the g.splits partial sums in g.ws (+ bias, ReLu)
 static long reduce_blocks(const GemmArgs &g, int lanes) {
     const int groups = 256 / lanes;
@@ -897,7 +1059,7 @@ bool gemm_tiled_run_plain_pair(int dtype, GemmArgs &g0, int ta0, int tb0, GemmAr
     const bool off = getenv("D8_MATMUL_GRADS_APART") != nullptr;  // tuning and test aid (read at every call)
     if (off || dtype == D8_FLOAT64 || ta0 || !tb0 || !ta1 || tb1) return false;
     if (g0.virt != VIRT_NONE || g1.virt != VIRT_NONE || g0.K < 1 || g1.K < 1) return false;
-    if (!gemm_tiled_eligible(dtype, g0, ta0, tb0, TILED_PIECES) || !gemm_tiled_eligible(dtype, g1, ta1, tb1, TILED_PIECES)) return false;
+    if (!g0.packed && !g1.packed && (!gemm_tiled_eligible(dtype, g0, ta0, tb0, TILED_PIECES) || !gemm_tiled_eligible(dtype, g1, ta1, tb1, TILED_PIECES))) return false;
     if (gemm_is_small(g0.M, g0.N, g0.K, g0.batch, g0.red) || gemm_is_small(g1.M, g1.N, g1.K, g1.batch, g1.red)) return false;
     if (balanced_rows(g0) || balanced_rows(g1)) return false;
     const size_t usable = (workspace && ((size_t)workspace & 15) == 0) ? workspace_bytes : 0;

@@ -81,6 +81,10 @@ struct GemmArgs {
     // product and bias + ReLu used to be two passes: a gate decided by the sum that is rounded once opens for other
     // elements (about one in five thousand), and a layer keeps the gates it had.
     int round_first;
+    // Half, rows that started anywhere, copied to rows of whole 16-byte pieces (gemm_pack): the operands may be moved in pieces
+    // though M, N or K is no multiple of one; what the loads may reach along M and N (operands not stored along K) is padM,
+    // padN; what follows K in a row is zero.  C is stored at the alignment of an element.
+    int packed, padM, padN;
     // a smaller tile than the shape's own (128 x 32: fp32 only), chosen by gemm_tiled_run and gemm_tiled_run_plain_pair
     // (few_tiles_small, narrow_output)
     int tile_hint;
@@ -162,6 +166,17 @@ int gemm_f64_splits(int M, int N, int K, int batch, int red, size_t workspace_by
 // for the chip, enough half-height ones, and a reduction (k_steps K steps in all) too short to
 // be worth splitting.
 bool gemm_tiled_half_tiles(int M, int N, int batch, long k_steps, int BK);
+
+// The two gradients of a MatrixMultiply in half whose rows start anywhere: the operands that cannot be moved in 16-byte pieces are
+// copied to rows that can, into the workspace, where that is expected to pay (one launch, a matrix that both read once).
+// On success the products read the copies and *used bytes of the workspace are taken; false, with nothing launched and the
+// products untouched, where it does not pay or the copies do not fit.
+struct PackedProduct {
+    GemmArgs *g;
+    int ta, tb;
+};
+bool gemm_pack(int dtype, const PackedProduct (&p)[2], void *workspace, size_t workspace_bytes, size_t *used, hipStream_t stream, int *rc);
+size_t gemm_pack_bytes(int dtype, const PackedProduct (&p)[2]);  // what it takes of the workspace (0: it does not pay)
 
 // Plan the split of the reduction, launch the tiled kernel (which must be eligible) and reduce.
 int gemm_tiled_run(int dtype, GemmArgs &g, int transA, int transB, void *workspace, size_t workspace_bytes,

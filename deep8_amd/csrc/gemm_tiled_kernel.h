@@ -72,6 +72,8 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 //                dword are constants of a thread.  Half 4096 x 1024 by 1024 x 1001, which a kernel that moved single elements
 //                served before: product with bias and ReLu 68 -> 24 us, its gradients 50 and 68 -> 21 and 22 us.  Bound by
 //                the K loop's latency as the other variants, plus 60 vector instructions a step.
+//                A DmaTile cannot shift its pieces: it takes copies of such operands (GemmArgs::packed), and EDGE_ANY there means
+//                a partial last step and a C whose rows start anywhere.
 enum { EDGE_NONE = 0, EDGE_PIECES = 1, EDGE_ANY = 2 };
 
 // ---- per element type: operand fragments and how to multiply one k group --------------------
@@ -255,7 +257,7 @@ __device__ __host__ constexpr int slot_of(int t, int n, int MQ) { return t * MQ 
 // EDGE_ANY: what a thread needs to put its pieces into place
 template <typename T, int EDGE>
 struct Loose {
-    static constexpr bool ANY = EDGE == EDGE_ANY, ODD = ANY && T::ES == 2;
+    static constexpr bool ANY = EDGE == EDGE_ANY && !T::DMA, ODD = ANY && T::ES == 2;
     unsigned X[ODD ? T::NP : 1];  // the dword after each piece
     unsigned shift[2], next[2];   // per operand: bits to shift by, byte offset of that dword (outside the buffer where it is not needed)
     u32x4 keep[2];                // ... and which bits of a piece are within K (operands stored along K)
@@ -644,7 +646,9 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     // (a matrix with fewer rows or columns than the tile: the tile starts at 0 and reaches past it; what the loads
     // bring in from there -- zeros past the end of the buffer, otherwise whatever follows -- only ever enters
     // results of rows / columns past the matrix, which are not stored)
-    const int m0 = max(0, min(m_own, M - BM)), n0 = max(0, min(n_own, g.N - BN));
+    // (copies in whole pieces, GemmArgs::packed: the tile is moved back by whole pieces)
+    const int M_in = T::DMA && EDGE == EDGE_ANY && !A_KC ? g.padM : M, N_in = T::DMA && EDGE == EDGE_ANY && !B_KC ? g.padN : g.N;
+    const int m0 = max(0, min(m_own, M_in - BM)), n0 = max(0, min(n_own, N_in - BN));
 
     // ---- the 16-byte pieces this thread moves each K step: piece `it` of an operand lies a fixed
     // number of rows below piece 0, in global memory and in LDS alike.  Global memory is read
@@ -652,7 +656,7 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     // registers) + per-thread part (one VGPR per operand).
     // EDGE_ANY: the buffers start at the dword that holds the operand's first element and end with the one that holds its
     // last (a dword at a multiple of 4 never reaches into another page); at the elements before and after sit no results.
-    constexpr bool ANY = EDGE == EDGE_ANY, ODD = Loose<T, EDGE>::ODD;
+    constexpr bool ANY = Loose<T, EDGE>::ANY, ODD = Loose<T, EDGE>::ODD;
     const long a_rows = A_KC ? g.M : g.K, b_rows = B_KC ? g.N : g.K;
     const E *Ab = (const E *)g.A + (long)b * g.sA, *Bb = (const E *)g.B + (long)b * g.sB;
     const unsigned a_odd = ODD ? (unsigned)((size_t)Ab & 2) >> 1 : 0u, b_odd = ODD ? (unsigned)((size_t)Bb & 2) >> 1 : 0u;
@@ -973,7 +977,7 @@ __global__ __launch_bounds__(T::NT, T::VIRT == VIRT_A_CLASSES && T::BN == 128 ||
 // each leave the chip half empty: their workgroups are short (a dozen K steps between a prologue and an epilogue
 // that nothing hides when a compute unit holds one workgroup), and side by side on a compute unit one's waits are
 // the other's issue slots.  The operand areas are as large as the larger tile needs.
-template <typename T0, typename T1>
+template <typename T0, typename T1, int EDGE = EDGE_NONE>
 __global__ __launch_bounds__(T0::NT, T0::TWO_FIT && T1::TWO_FIT ? 2 : 1) void gemm_tiled_pair_kernel(GemmArgs g0, GemmArgs g1, int tilesM0, int tilesN0, int nx0, int nz0,
                                                                  int tilesM1, int tilesN1, int nx1) {
     typedef typename T0::E E;
@@ -981,8 +985,8 @@ __global__ __launch_bounds__(T0::NT, T0::TWO_FIT && T1::TWO_FIT ? 2 : 1) void ge
     if constexpr (T0::DMA) {
         __shared__ __attribute__((aligned(1024))) E stages[(T0::LDS_BYTES > T1::LDS_BYTES ? T0::LDS_BYTES : T1::LDS_BYTES) / T0::ES];
         const int id = (int)blockIdx.x, first = nx0 * nz0, j = id - first;
-        if (id < first) gemm_tiled_body<T0, EDGE_NONE>(g0, tilesM0, tilesN0, id % nx0, id / nx0, nx0, stages, nullptr, nullptr, nullptr);
-        else gemm_tiled_body<T1, EDGE_NONE>(g1, tilesM1, tilesN1, j % nx1, j / nx1, nx1, stages, nullptr, nullptr, nullptr);
+        if (id < first) gemm_tiled_body<T0, EDGE>(g0, tilesM0, tilesN0, id % nx0, id / nx0, nx0, stages, nullptr, nullptr, nullptr);
+        else gemm_tiled_body<T1, EDGE>(g1, tilesM1, tilesN1, j % nx1, j / nx1, nx1, stages, nullptr, nullptr, nullptr);
     } else {
         constexpr int A_SZ = T0::A_SZ > T1::A_SZ ? T0::A_SZ : T1::A_SZ, B_SZ = T0::B_SZ > T1::B_SZ ? T0::B_SZ : T1::B_SZ;
         __shared__ __attribute__((aligned(16))) E As0[A_SZ];
@@ -991,10 +995,10 @@ __global__ __launch_bounds__(T0::NT, T0::TWO_FIT && T1::TWO_FIT ? 2 : 1) void ge
         __shared__ __attribute__((aligned(16))) E Bs1[B_SZ];
         const int id = (int)blockIdx.x, first = nx0 * nz0;
         if (id < first) {
-            gemm_tiled_body<T0, EDGE_NONE>(g0, tilesM0, tilesN0, id % nx0, id / nx0, nx0, As0, As1, Bs0, Bs1);
+            gemm_tiled_body<T0, EDGE>(g0, tilesM0, tilesN0, id % nx0, id / nx0, nx0, As0, As1, Bs0, Bs1);
         } else {
             const int j = id - first;
-            gemm_tiled_body<T1, EDGE_NONE>(g1, tilesM1, tilesN1, j % nx1, j / nx1, nx1, As0, As1, Bs0, Bs1);
+            gemm_tiled_body<T1, EDGE>(g1, tilesM1, tilesN1, j % nx1, j / nx1, nx1, As0, As1, Bs0, Bs1);
         }
     }
 }
@@ -1044,6 +1048,7 @@ enum TileId { TILE_WIDE, TILE_256, TILE_128x64, TILE_64x64, TILE_64x128, TILE_12
 template <typename E>
 static bool in_pieces(const GemmArgs &g, bool a_kc, bool b_kc) {
     constexpr int EPV = 16 / (int)sizeof(E), BK = 128 / (int)sizeof(E);
+    if (g.packed) return true;
     if ((g.lda | g.ldb) % EPV || (g.sA | g.sB) % EPV || (((size_t)g.A | (size_t)g.B) & 15)) return false;
     if ((a_kc || b_kc) && g.K % BK && g.K % EPV) return false;
     return (a_kc || g.M % EPV == 0) && (b_kc || g.N % EPV == 0);
@@ -1058,7 +1063,7 @@ static TileId choose_tile(const GemmArgs &g, bool any = false) {
     if (force && g.M >= 256 && g.N >= 256) big = atoi(force) != 128;
     // fp32 runs 64-cycle MFMAs on a quarter of the bytes per flop: the 128 x 128 tile already
     // keeps the matrix pipe fed, and the compiler cannot hold the 256 x 256 variant in registers
-    if (any) big = false;  // (and rows that start anywhere have no kernel of 256 x 256 tiles)
+    if (any || g.packed) big = false;  // (and rows that start anywhere have no kernel of 256 x 256 tiles)
     if constexpr (sizeof(E) == 2) {
         static const char *wide = getenv("D8_GEMM_WIDE");  // tuning aid: 0 keeps the 32x32x16 kernel
         if (big && VIRT == VIRT_NONE && !(wide && atoi(wide) == 0) && gemm_wide_eligible(g, !A_KC, B_KC)) return TILE_WIDE;
@@ -1084,7 +1089,7 @@ static void grid_of(TileId t, const GemmArgs &g, int &tilesM, int &tilesN) {
     tilesM = ceil_div(g.M, bm), tilesN = ceil_div(g.N, bn);
 }
 
-template <typename TX, typename TY>
+template <typename TX, typename TY, int EDGE = EDGE_NONE>
 static int launch_pair_tiles(const GemmArgs &gx0, const GemmArgs &gy0, hipStream_t stream) {
     GemmArgs gx = gx0, gy = gy0;
     // (gx may carry its remainder band as pieces of the same launch: GemmArgs::tail_m0; then it has one layer)
@@ -1097,7 +1102,7 @@ static int launch_pair_tiles(const GemmArgs &gx0, const GemmArgs &gy0, hipStream
     const bool rec = (size_t)(ny * nzy + nx * nzx) * 64 <= phase_rec_bytes;
     gy.phase_rec = rec ? phase_rec_buf : nullptr, gy.stamps = 0;
     gx.phase_rec = rec && phase_rec_buf ? phase_rec_buf + 8L * ny * nzy : nullptr, gx.stamps = 1;
-    hipLaunchKernelGGL((gemm_tiled_pair_kernel<TY, TX>), dim3(ny * nzy + nx * nzx), dim3(TX::NT), 0, stream, gy, gx, tMy, tNy, ny, nzy, tMx, tNx, nx);
+    hipLaunchKernelGGL((gemm_tiled_pair_kernel<TY, TX, EDGE>), dim3(ny * nzy + nx * nzx), dim3(TX::NT), 0, stream, gy, gx, tMy, tNy, ny, nzy, tMx, tNx, nx);
     D8_LAUNCH_CHECK();
     return 0;
 }

@@ -36,6 +36,8 @@ static int launch_edge(const GemmArgs &g0, hipStream_t stream) {
 
 template <typename T>
 static int launch_whole(const GemmArgs &g, hipStream_t stream) {
+    if constexpr (T::DMA && T::VIRT == VIRT_NONE)
+        if (g.packed) return launch_edge<T, EDGE_ANY>(g, stream);
     if constexpr (T::VIRT != VIRT_B_KROWS)
         if (g.K % T::BK) return launch_edge<T, EDGE_PIECES>(g, stream);
     return launch_edge<T, EDGE_NONE>(g, stream);

@@ -318,8 +318,14 @@ extern "C" {
 // ---------------------------------------------------------------------------------------------
 size_t d8_matmul_scratch_bytes(int dtype, int which, int xb, int xr, int xc, int yb, int yr, int yc) {
     if (check_mm("d8_matmul_scratch_bytes", dtype, xb, xr, xc, yb, yr, yc)) return 0;
-    if (which == 3)  // for d8_matmul_grad_xy: both gradients' scratch side by side (they may share a launch)
-        return align256(d8_matmul_scratch_bytes(dtype, 1, xb, xr, xc, yb, yr, yc)) + d8_matmul_scratch_bytes(dtype, 2, xb, xr, xc, yb, yr, yc);
+    if (which == 3) {  // for d8_matmul_grad_xy: both gradients' scratch side by side (they may share a launch), and their copies
+        const char *const base = (const char *)4096;  // (three matrices, none of them the same)
+        const Gemm px = mm_plan(1, nullptr, xb, xr, xc, base, yb, yr, yc, base + 4096), py = mm_plan(2, base + 8192, xb, xr, xc, nullptr, yb, yr, yc, base + 4096);
+        GemmArgs gx = to_args(px), gy = to_args(py);
+        const PackedProduct both[2] = {{&gx, px.ta, px.tb}, {&gy, py.ta, py.tb}};
+        return align256(d8_matmul_scratch_bytes(dtype, 1, xb, xr, xc, yb, yr, yc)) + d8_matmul_scratch_bytes(dtype, 2, xb, xr, xc, yb, yr, yc) +
+               gemm_pack_bytes(dtype, both);
+    }
     return gemm_ws(dtype, mm_plan(which, nullptr, xb, xr, xc, nullptr, yb, yr, yc, nullptr));
 }
 
@@ -411,9 +417,18 @@ int d8_matmul_grad_xy(int dtype, const void *x, void *dx, int xb, int xr, int xc
     {  // both on the tiled kernels with all their workgroups resident at once: one launch, then their split reductions
         int rc = 0;
         GemmArgs gx = to_args(px), gy = to_args(py);
-        if (gemm_tiled_run_plain_pair(dtype, gx, px.ta, px.tb, gy, py.ta, py.tb, scratch, scratch_bytes, as_stream(stream), &rc)) {
+        const PackedProduct both[2] = {{&gx, px.ta, px.tb}, {&gy, py.ta, py.tb}};
+        size_t used = 0;
+        const bool packed = gemm_pack(dtype, both, scratch, scratch_bytes, &used, as_stream(stream), &rc);
+        if (packed && rc) return rc;
+        char *const rest = (char *)scratch + used;
+        if (gemm_tiled_run_plain_pair(dtype, gx, px.ta, px.tb, gy, py.ta, py.tb, rest, scratch_bytes - used, as_stream(stream), &rc)) {
             ++matmul_pair_launches;
             return rc;
+        }
+        if (packed) {
+            if (int e = gemm_tiled_run(dtype, gx, px.ta, px.tb, rest, scratch_bytes - used, as_stream(stream))) return e;
+            return gemm_tiled_run(dtype, gy, py.ta, py.tb, rest, scratch_bytes - used, as_stream(stream));
         }
     }
     if (int rc = run(dtype, px, scratch, scratch_bytes, stream)) return rc;
