@@ -84,6 +84,9 @@ __global__ __launch_bounds__(256) void add_kernel(const T *x, const T *__restric
 enum { LOAD_ID = 0, LOAD_ABS = 1, LOAD_SQUARE = 2 };
 template <int OP>
 __device__ inline float ew_load(float v) { return OP == LOAD_ABS ? fabsf(v) : (OP == LOAD_SQUARE ? v * v : v); }
+// ... and to its result: the root of a sum of squares (an L2 norm), taken of the sum as T holds it
+template <typename T, int OP>
+__device__ inline T ew_result(float v) { return OP == LOAD_SQUARE ? (T)sqrtf(ew_f32((T)v)) : (T)v; }
 
 // g = keep * g + scale * op(dz), same shape.  keep is 1 (the reference's accumulate) or 0 (g's old contents are
 // not read: the overwrite forms).  The same convention holds for every kernel below that takes `keep`.
@@ -99,7 +102,7 @@ __global__ __launch_bounds__(256) void accumulate_kernel(T *__restrict__ g, cons
         const VT b = *(const VT *)(dz + idx * VEC);
         VT o;
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) o[e] = (T)(ew_f32(a[e]) + scale * ew_load<OP>(ew_f32(b[e])));
+        for (int e = 0; e < VEC; ++e) o[e] = ew_result<T, OP>(ew_f32(a[e]) + scale * ew_load<OP>(ew_f32(b[e])));
         *(VT *)(g + idx * VEC) = o;
     }
 }
@@ -145,13 +148,15 @@ __global__ __launch_bounds__(256) void column_sum_kernel(const T *__restrict__ d
     for (int e = 0; e < VEC; ++e) part[threadIdx.x][e] = acc[e];
     __syncthreads();
     if (ty == 0 && live) {
-        for (int k = 1; k < lanes; ++k)
+        // (lanes that had no row hold zeros: 64 sums of ten values each waited 3 us for 246 of them)
+        const int met = min(lanes, min(R - chunk * rows_per_chunk, rows_per_chunk));
+        for (int k = 1; k < met; ++k)
 #pragma unroll
             for (int e = 0; e < VEC; ++e) acc[e] += part[k * TX + tx][e];
         if (chunks == 1) {
             T *o = g + (long)k0 * C + (long)cv * VEC;
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) o[e] = (T)((keep != 0.f ? ew_f32(o[e]) : 0.f) + scale * acc[e]);
+            for (int e = 0; e < VEC; ++e) o[e] = ew_result<T, OP>((keep != 0.f ? ew_f32(o[e]) : 0.f) + scale * acc[e]);
         } else {
             float *o = partial + ((long)k0 * chunks + chunk) * C + (long)cv * VEC;
 #pragma unroll
@@ -162,7 +167,7 @@ __global__ __launch_bounds__(256) void column_sum_kernel(const T *__restrict__ d
 
 // g[k0][c] += sum over chunks of partial[k0][chunk][c].  A block covers 16 outputs; 16 lanes per
 // output each add every 16th chunk (eight loads in flight) and meet in LDS in a fixed order.
-template <typename T>
+template <typename T, int OP = LOAD_ID>
 __global__ __launch_bounds__(256) void column_sum_finish_kernel(const float *__restrict__ partial, T *__restrict__ g,
                                                                 int C, int chunks, long total, float scale, float keep) {
     __shared__ float part[16][16];
@@ -188,7 +193,7 @@ __global__ __launch_bounds__(256) void column_sum_finish_kernel(const float *__r
     if (ty == 0 && idx < total) {
 #pragma unroll
         for (int k = 1; k < 16; ++k) v += part[k][tx];
-        g[idx] = (T)((keep != 0.f ? ew_f32(g[idx]) : 0.f) + scale * v);
+        g[idx] = ew_result<T, OP>((keep != 0.f ? ew_f32(g[idx]) : 0.f) + scale * v);
     }
 }
 
@@ -254,7 +259,9 @@ __global__ __launch_bounds__(256) void relu_gate_column_sum_kernel(const T *__re
     for (int e = 0; e < VEC; ++e) part[threadIdx.x][e] = acc[e];
     __syncthreads();
     if (ty == 0 && live) {
-        for (int k = 1; k < lanes; ++k)
+        // (lanes that had no row hold zeros: 64 sums of ten values each waited 3 us for 246 of them)
+        const int met = min(lanes, min(R - chunk * rows_per_chunk, rows_per_chunk));
+        for (int k = 1; k < met; ++k)
 #pragma unroll
             for (int e = 0; e < VEC; ++e) acc[e] += part[k * TX + tx][e];
         if (chunks == 1) {
@@ -375,16 +382,6 @@ __global__ __launch_bounds__(256) void norm_grad_kernel(const T *__restrict__ x,
         }
         *(VT *)(dx + idx * VEC) = o;
     }
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void sqrt_kernel(T *p, long n) {
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) p[i] = (T)sqrtf(ew_f32(p[i]));
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void ew_zero_kernel(T *p, long n) {
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) p[i] = (T)0;
 }
 
 // z = alpha * x + beta * y (z may be x or y)
@@ -514,7 +511,7 @@ static int reduce_t(T *g, const int *d, const T *dz, const int *zd, void *scratc
                                TX, rpc, chunks, scale, keep);
         if (chunks > 1) {
             D8_LAUNCH_CHECK();
-            hipLaunchKernelGGL((column_sum_finish_kernel<T>), dim3((unsigned)((ng + 15) / 16)), dim3(256), 0, s,
+            hipLaunchKernelGGL((column_sum_finish_kernel<T, OP>), dim3((unsigned)((ng + 15) / 16)), dim3(256), 0, s,
                                (const float *)scratch, g, (int)p.C, chunks, ng, scale, keep);
         }
     } else {
@@ -555,18 +552,12 @@ static int add_t(const T *x, const int *xd, const T *y, const int *yd, T *z, con
     return 0;
 }
 
-// y[b] = sum over i of op(x[b][i]) (then the square root for L2): zero, reduce, finish.
+// y[b] = sum over i of op(x[b][i]) (then the square root for L2), written by the reduction itself.  A launch each to clear y and
+// to take the roots were what a small batch waited for: 64 x 10 in fp32 8.4 -> 3.4 us.
 template <typename T, int WIDE, int OP>
 static int norm_t(const T *x, T *y, int batch, long size, void *scratch, size_t scratch_bytes, hipStream_t s) {
     const int yd[5] = {batch, 1, 1, 1, 1}, xd[5] = {batch, 1, 1, 1, (int)size};
-    hipLaunchKernelGGL((ew_zero_kernel<T>), dim3(ew_grid(batch, 256)), dim3(256), 0, s, y, (long)batch);
-    D8_LAUNCH_CHECK();
-    if (int rc = reduce_t<T, WIDE, OP>(y, yd, x, xd, scratch, scratch_bytes, s)) return rc;
-    if (OP == LOAD_SQUARE) {
-        hipLaunchKernelGGL((sqrt_kernel<T>), dim3(ew_grid(batch, 256)), dim3(256), 0, s, y, (long)batch);
-        D8_LAUNCH_CHECK();
-    }
-    return 0;
+    return reduce_t<T, WIDE, OP>(y, yd, x, xd, scratch, scratch_bytes, s, 1.f, 0.f);
 }
 
 template <typename T, int WIDE, bool L2>
@@ -818,16 +809,10 @@ int d8_reduce_mean(int dtype, const void *x, const int *xdims, void *y, const in
     double count = 1;
     if (int rc = mean_count("d8_reduce_mean", xdims, ydims, &count)) return rc;
     hipStream_t s = as_stream(stream);
-    const long ny = prod5(ydims);
-    const float scale = (float)(1.0 / count);
-    if (dtype == D8_FLOAT32) {
-        hipLaunchKernelGGL((ew_zero_kernel<float>), dim3(ew_grid(ny, 256)), dim3(256), 0, s, (float *)y, ny);
-        D8_LAUNCH_CHECK();
-        return reduce_t<float, 4>((float *)y, ydims, (const float *)x, xdims, scratch, scratch_bytes, s, scale);
-    }
-    hipLaunchKernelGGL((ew_zero_kernel<f16>), dim3(ew_grid(ny, 256)), dim3(256), 0, s, (f16 *)y, ny);
-    D8_LAUNCH_CHECK();
-    return reduce_t<f16, 8>((f16 *)y, ydims, (const f16 *)x, xdims, scratch, scratch_bytes, s, scale);
+    const float scale = (float)(1.0 / count);  // (y is written, not added to)
+    return dtype == D8_FLOAT32
+               ? reduce_t<float, 4>((float *)y, ydims, (const float *)x, xdims, scratch, scratch_bytes, s, scale, 0.f)
+               : reduce_t<f16, 8>((f16 *)y, ydims, (const f16 *)x, xdims, scratch, scratch_bytes, s, scale, 0.f);
 }
 
 int d8_reduce_mean_grad(int dtype, void *dx, const int *xdims, const void *dy, const int *ydims, void *stream) {
