@@ -565,6 +565,22 @@ __device__ __forceinline__ void dma_loop(f16 *lds, int wave, int lane, int wm, i
     wait_loads_and_lds<0>();  // (nothing lands in LDS any more: the epilogue uses it)
 }
 
+// Division of many 0 <= n < 2^31 by one uniform d: floor((2^32 - 1) / d) is taken once, and n times that over 2^32 is the quotient
+// or one less.  Half a dozen instructions instead of some 35 each for the patch operands' eight divisions a thread: Conv2d
+// 32 x 14x14x256 3x3 half, forward and gradients, 54.4 -> 54.2 us, fp32 1 x 28x28x128 forward 10.50 -> 10.45.
+struct Divisor {
+    int d;
+    unsigned m;
+    __device__ __forceinline__ explicit Divisor(int by) : d(by), m(0xffffffffu / (unsigned)by) {}
+    __device__ __forceinline__ int div(int n, int &rem) const {
+        int q = (int)__umulhi((unsigned)n, m);
+        rem = n - q * d;
+        const bool more = rem >= d;
+        rem -= more ? d : 0;
+        return q + (more ? 1 : 0);
+    }
+};
+
 // The work of one workgroup: workgroup (bx, bz) of a grid of nbx x layers (the launch's own blockIdx / gridDim, or what a
 // launch of two products makes of them).  As0 .. Bs1: the two halves of both operand areas in LDS.
 template <typename T, int EDGE>
@@ -696,11 +712,11 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     // patch rows as A: this thread's rows never change; a step selects the tap
     int va_base[A_IT], va_iy[A_IT], va_ix[A_IT];
     if constexpr (VA) {
-        const int plane = pg.OH * pg.OW;
+        const Divisor plane(pg.OH * pg.OW), width(pg.OW);
 #pragma unroll
         for (int p = 0; p < A_IT; ++p) {
-            const int m = g.m_base + m0 + a_r + p * T::A_ROWS, img = m / plane, rem = m - img * plane;
-            const int oy = rem / pg.OW, ox = rem - oy * pg.OW;
+            int rem, ox;
+            const int m = g.m_base + m0 + a_r + p * T::A_ROWS, img = plane.div(m, rem), oy = width.div(rem, ox);
             va_iy[p] = oy * pg.sy - pg.pt;
             va_ix[p] = ox * pg.sx - pg.pl;
             va_base[p] = (((img * pg.H + va_iy[p]) * pg.W + va_ix[p]) * pg.C + a_c * EPV) * ES;
@@ -719,12 +735,14 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     if constexpr (VIRT == VIRT_B_KROWS) {
         int cy = -pg.pt, cx = -pg.pl, cc = 0;  // what the tap and channel add to an output pixel's source coordinates
         if constexpr (T::B_COLS) {
+            const Divisor channels(pg.C), taps(pg.FW);
 #pragma unroll
             for (int p = 0; p < B_IT; ++p) {
-                const int n = n0 + p * T::B_PASS + b_c * EPV, t = n / pg.C, fy = t / pg.FW, fx = t - fy * pg.FW;
+                int c, fx;
+                const int t = channels.div(n0 + p * T::B_PASS + b_c * EPV, c), fy = taps.div(t, fx);
                 vb_ty[p] = fy * pg.dy;
                 vb_tx[p] = fx * pg.dx;
-                vb_toff[p] = ((vb_ty[p] * pg.W + vb_tx[p]) * pg.C + (n - t * pg.C)) * ES;
+                vb_toff[p] = ((vb_ty[p] * pg.W + vb_tx[p]) * pg.C + c) * ES;
             }
         } else {
             const int n = n0 + b_c * EPV, t = n / pg.C, fy = t / pg.FW, fx = t - fy * pg.FW;
@@ -733,12 +751,13 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
             cx += fx * pg.dx;
         }
         vb_y_end = pg.OH * pg.sy + cy, vb_x_end = pg.OW * pg.sx + cx;
-        const int plane = pg.OH * pg.OW;
+        const Divisor plane(pg.OH * pg.OW), width(pg.OW);
 #pragma unroll
         for (int p = 0; p < VB_N; ++p) {
-            const int m = split * tps * BK + b_r + p * T::B_ROWS, img = m / plane, rem = m - img * plane, oy = rem / pg.OW;
+            int rem, ox;
+            const int m = split * tps * BK + b_r + p * T::B_ROWS, img = plane.div(m, rem), oy = width.div(rem, ox);
             vb_y[p] = oy * pg.sy + cy;
-            vb_x[p] = (rem - oy * pg.OW) * pg.sx + cx;
+            vb_x[p] = ox * pg.sx + cx;
             vb_off[p] = (((img * pg.H + vb_y[p]) * pg.W + vb_x[p]) * pg.C + cc) * ES;
         }
     }
