@@ -1116,7 +1116,8 @@ static int launch_pair_tiles(const GemmArgs &gx0, const GemmArgs &gy0, hipStream
     const int tMx = ceil_div(tail ? gx.tail_m0 : gx.M, TX::BM), tNx = ceil_div(gx.N, TX::BN), tMy = ceil_div(gy.M, TY::BM), tNy = ceil_div(gy.N, TY::BN);
     const int extra = tail ? ceil_div(gx.M - gx.tail_m0, TX::BM) * tNx * gx.tail_splits : 0;
     // the longer-running product first: gy's pieces, then gx's tiles
-    const int ny = tMy * tNy, nzy = gy.batch * gy.splits, nx = tMx * tNx + extra, nzx = tail ? 1 : gx.batch * gx.splits;
+    const int ny = tMy * tNy, nzy = gy.batch * gy.splits, nx = tMx * tNx + extra;
+    const int nzx = TX::VIRT == VIRT_A_CLASSES ? gx.ncls : tail ? 1 : gx.batch * gx.splits;
     // phase records (a measurement aid): gy's workgroups first, then gx's, tagged 0 and 1
     const bool rec = (size_t)(ny * nzy + nx * nzx) * 64 <= phase_rec_bytes;
     gy.phase_rec = rec ? phase_rec_buf : nullptr, gy.stamps = 0;

@@ -5,6 +5,7 @@
 //   MatrixMultiply   deep8/src/math/MatrixMultiply.cu:21-57 (fwd), :193-232 (GradX), :381-420 (GradY)
 //   Conv2d           deep8/src/math/Conv2d.cu:145-196, :440-492, :750-802, pads :332-336
 //   DeConv2d         deep8/src/math/DeConv2d.cu:76-131, :371-429, :642-700, pads :99-100
+#include <algorithm>
 #include <atomic>
 
 #include "conv_direct.h"
@@ -256,6 +257,12 @@ static bool conv_implicit_plan(int dtype, int which, const ConvShape &c, const v
 // product: *untouched tells the caller, who zero-fills dx before an overwriting call.
 static int gcd_of(int a, int b) { return b ? gcd_of(b, a % b) : a; }
 
+// The classes with the most taps first: launched last, their workgroups would be the chip's last wave (3x3 stride 2: 1, 2, 2 and 4
+// taps in the order of the pixels).
+static void longest_first(GemmArgs &g) {
+    std::stable_sort(g.cls, g.cls + g.ncls, [](const OutClass &a, const OutClass &b) { return a.red > b.red; });
+}
+
 static bool conv_classes_grad_x(int dtype, const ConvShape &c, const void *gx, const void *w, const void *gz, GemmArgs &g, bool *untouched) {
     *untouched = false;
     if (getenv("D8_CONV_EXPLICIT") != nullptr) return false;
@@ -302,6 +309,7 @@ static bool conv_classes_grad_x(int dtype, const ConvShape &c, const void *gx, c
             most_taps = k.red > most_taps ? k.red : most_taps;
         }
     if (g.ncls == 0) return false;
+    longest_first(g);
     g.tiles_per_split = most_taps * (c.OC / (dtype == D8_FLOAT64 ? 16 : gemm_tiled_k_step(dtype)) + 1);
     g.M = smallest;
     const bool ok = implicit_eligible(dtype, g, 0, 0);
@@ -807,6 +815,7 @@ static bool deconv_implicit_fwd(int dtype, int B, int IH, int IW, int IC, int OC
             most_taps = c.red > most_taps ? c.red : most_taps;
         }
     if (g.ncls == 0) return false;
+    longest_first(g);
     g.tiles_per_split = most_taps * (IC / (dtype == D8_FLOAT64 ? 16 : gemm_tiled_k_step(dtype)) + 1);  // never the limit: a class walks all its taps
     g.M = smallest;
     const bool ok = implicit_eligible(dtype, g, 0, 1);
@@ -1075,6 +1084,24 @@ int d8_conv2d_grad_xy(int dtype, const void *x, void *gx, int B, int IH, int IW,
                 route_calls[ROUTE_PATCH] += 2;
                 return rc;
             }
+        }
+    }
+    {  // (strides above 1: both gradients where the two calls would have them in the loader)
+        const ConvShape cs = {B, IH, IW, IC, OC, FH, FW, g[0], g[1], sy, sx, dy, dx, g[2], g[3]};
+        const int M = B * g[0] * g[1], K = FH * FW * IC;
+        GemmArgs px, pw;
+        int ta, tb;
+        bool untouched = false;
+        if (dtype == D8_FLOAT16 && conv_classes_grad_x(dtype, cs, gx, w, gz, px, &untouched) && conv_implicit_plan(dtype, 2, cs, x, gw, gz, pw, ta, tb) &&
+            gemm_tiled_class_pair_plan(dtype, px, pw, scratch, scratch_bytes) &&
+            !prefer_interim(dtype, px, 0, 0, conv_plan(1, M, K, OC, scratch, w, gz), (double)M * K, IC, untouched ? 0 : 1, scratch, scratch_bytes) &&
+            !prefer_interim(dtype, pw, ta, tb, conv_plan(2, M, K, OC, scratch, gw, gz), (double)M * K, IC, 0, scratch, scratch_bytes)) {
+            const bool clear = untouched && bx == 0.f;  // as d8_conv2d_grad_x_impl
+            if (clear)
+                if (int rc = d8_fill(dtype, gx, (size_t)B * IH * IW * IC, 0.f, stream)) return rc;
+            px.beta = clear ? 1.f : bx, pw.beta = bw;
+            route_calls[ROUTE_PATCH] += 2;
+            return gemm_tiled_class_pair_run(dtype, px, pw, as_stream(stream));
         }
     }
     if (int rc = d8_conv2d_grad_x_impl(dtype, gx, B, IH, IW, IC, w, OC, FH, FW, gz, covered, sy, sx, dy, dx, scratch, scratch_bytes, stream, bx))

@@ -1,0 +1,67 @@
+"""Conv2d with a stride in half, both gradients from one call: classes of output pixels beside the filter gradient in one launch.
+Channels that cut the last K step short, outputs narrower and wider than a tile, classes that no tap reaches, one-pixel classes,
+dilation, every combination of written and added gradients, scratch for no pieces of the filter gradient.  Integers, against the
+oracle, bit for bit; reals, bit for bit what two launches leave."""
+import numpy as np
+import pytest
+
+from util import f, h, ints, nrm, rng
+
+pytestmark = pytest.mark.gpu
+
+# B, IH, IW, IC, OC, FH, FW, covered, sy, sx, dy, dx
+LAYERS = [
+    (4, 17, 15, 64, 64, 3, 3, True, 2, 2, 1, 1),      # 128 x 64 tiles, whole K steps
+    (3, 19, 21, 96, 160, 3, 3, True, 2, 2, 1, 1),     # K steps cut short
+    (8, 16, 16, 136, 72, 3, 3, False, 2, 2, 1, 1),    # 128 x 128 tiles, columns past a tile
+    (16, 18, 18, 64, 64, 1, 1, True, 2, 2, 1, 1),     # three classes that no tap reaches
+    (12, 20, 20, 128, 128, 2, 2, False, 3, 3, 1, 1),  # five of nine
+    (6, 16, 18, 64, 128, 3, 3, True, 2, 1, 1, 2),     # one stride, dilation along the other axis
+    (4, 17, 17, 72, 64, 5, 5, True, 2, 2, 1, 1),
+    (32, 3, 4, 64, 64, 3, 3, True, 2, 2, 1, 1),       # classes of one row and column
+    (2, 40, 40, 256, 192, 3, 3, True, 2, 2, 1, 1),    # filter gradient on 128 x 128 tiles
+]
+
+
+@pytest.mark.parametrize("cfg", LAYERS)
+def test_integers_against_the_oracle(oracle_port, cfg):
+    from deep8_amd import ops
+    B, IH, IW, IC, OC, FH, FW = cfg[:7]
+    geo = cfg[7:]
+    OH, OW, _, _ = ops.conv2d_geometry(IH, IW, FH, FW, *geo)
+    r = rng(sum(cfg[:7]))
+    x, w, gz = ints(r, (B, IH, IW, IC), 2), ints(r, (OC, FH, FW, IC), 2), ints(r, (B, OH, OW, OC), 2)
+    gz = gz * (r.random(gz.shape) < min(1.0, 400.0 / (B * OH * OW)))  # thinned: sums that half holds
+    gx0, gw0 = ints(r, x.shape, 2), ints(r, w.shape, 2)
+    want_x, want_w = oracle_port.conv2d_grad_x(x, w, gz, *geo), oracle_port.conv2d_grad_y(x, w, gz, *geo)
+    assert max(np.abs(want_x).max(), np.abs(want_w).max()) < 2000
+    for ox, ow in ((True, True), (False, True), (True, False), (False, False)):
+        gx, gw = ops.conv2d_grad_xy(h(x), h(w), h(gz), *geo, h(gx0), h(gw0), ox, ow)
+        assert np.array_equal(f(gx), want_x + (0 if ox else gx0)), (ox, ow)
+        assert np.array_equal(f(gw), want_w + (0 if ow else gw0)), (ox, ow)
+
+
+@pytest.mark.parametrize("cfg", LAYERS)
+def test_one_launch_leaves_what_two_leave(cfg, monkeypatch):
+    from deep8_amd import capi, ops
+    from deep8_amd.capi import DeviceArray, check
+    lib = capi.init()
+    B, IH, IW, IC, OC, FH, FW = cfg[:7]
+    geo = cfg[7:]
+    OH, OW, _, _ = ops.conv2d_geometry(IH, IW, FH, FW, *geo)
+    r = rng(sum(cfg[:7]) + 1)
+    x, w, gz = (DeviceArray.from_numpy(h(nrm(r, s))) for s in ((B, IH, IW, IC), (OC, FH, FW, IC), (B, OH, OW, OC)))
+    asked = lib.d8_conv2d_scratch_bytes(capi.FLOAT16, 3, B, IH, IW, IC, OC, FH, FW, *(int(v) for v in geo))
+    for nb in (0, asked):
+        got = []
+        for apart in (False, True):
+            if apart:
+                monkeypatch.setenv("D8_CONV_GRADS_APART", "1")
+            else:
+                monkeypatch.delenv("D8_CONV_GRADS_APART", raising=False)
+            gx, gw = (DeviceArray.from_numpy(np.full(s, np.nan, np.float16)) for s in ((B, IH, IW, IC), (OC, FH, FW, IC)))
+            ws = DeviceArray((max(nb, 16),), np.uint8)
+            check(lib.d8_conv2d_grad_xy(capi.FLOAT16, x.ptr, gx.ptr, B, IH, IW, IC, w.ptr, gw.ptr, OC, FH, FW, gz.ptr,
+                                        *(int(v) for v in geo), 3, ws.ptr if nb else None, nb, None))
+            got.append((gx.numpy().view(np.uint16), gw.numpy().view(np.uint16)))
+        assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1]), nb
