@@ -1,7 +1,7 @@
-"""Conv2d with a stride in half, both gradients from one call: classes of output pixels beside the filter gradient in one launch.
-Channels that cut the last K step short, outputs narrower and wider than a tile, classes that no tap reaches, one-pixel classes,
-dilation, every combination of written and added gradients, scratch for no pieces of the filter gradient.  Integers, against the
-oracle, bit for bit; reals, bit for bit what two launches leave."""
+"""Convolutions in half, both gradients from one call, on layers whose two products are tiled and cut as they would be alone and
+share a launch: classes of output pixels (strides above 1), last K steps that are cut short, gradients of x in pieces.  Channels
+narrower and wider than a tile, classes that no tap reaches, one-pixel classes, dilation, every combination of written and added
+gradients, scratch for no pieces.  Integers, against the oracle, bit for bit; reals, bit for bit what two launches leave."""
 import numpy as np
 import pytest
 
@@ -20,6 +20,10 @@ LAYERS = [
     (4, 17, 17, 72, 64, 5, 5, True, 2, 2, 1, 1),
     (32, 3, 4, 64, 64, 3, 3, True, 2, 2, 1, 1),       # classes of one row and column
     (2, 40, 40, 256, 192, 3, 3, True, 2, 2, 1, 1),    # filter gradient on 128 x 128 tiles
+    (3, 19, 21, 96, 160, 3, 3, True, 1, 1, 1, 1),     # stride 1, K steps cut short
+    (6, 13, 13, 56, 72, 3, 3, False, 1, 1, 2, 1),     # 64 x 64 tiles of few columns
+    (8, 11, 11, 256, 128, 5, 5, True, 1, 1, 1, 1),    # gradient of x in pieces
+    (16, 28, 28, 136, 88, 3, 3, True, 1, 1, 1, 1),    # 128 x 128 tiles, columns past a tile
 ]
 
 
@@ -65,3 +69,41 @@ def test_one_launch_leaves_what_two_leave(cfg, monkeypatch):
                                         *(int(v) for v in geo), 3, ws.ptr if nb else None, nb, None))
             got.append((gx.numpy().view(np.uint16), gw.numpy().view(np.uint16)))
         assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1]), nb
+
+
+# B, IH, IW, IC, OC, FH, FW, covered, sy, sx
+TRANSPOSED = [
+    (4, 14, 13, 64, 72, 4, 4, False, 2, 2),
+    (2, 9, 11, 136, 40, 3, 3, True, 2, 2),
+    (18, 6, 6, 72, 16, 5, 5, False, 2, 2),
+    (6, 16, 16, 64, 200, 3, 3, False, 1, 1),
+    (8, 20, 20, 128, 88, 2, 2, False, 2, 2),
+]
+
+
+@pytest.mark.parametrize("cfg", TRANSPOSED)
+def test_transposed_convolutions(oracle_port, cfg, monkeypatch):
+    from deep8_amd import ops
+    B, IH, IW, IC, OC, FH, FW = cfg[:7]
+    geo = cfg[7:]
+    OH, OW, _, _ = ops.deconv2d_geometry(IH, IW, FH, FW, *geo)
+    r = rng(sum(cfg[:7]) + 2)
+    for whole in (True, False):
+        if whole:
+            x, w, gz = ints(r, (B, IH, IW, IC), 2), ints(r, (OC, FH, FW, IC), 2), ints(r, (B, OH, OW, OC), 2)
+            x = x * (r.random(x.shape) < min(1.0, 400.0 / (B * IH * IW)))  # thinned: sums that half holds
+            gz = gz * (r.random(gz.shape) < 0.3)
+        else:
+            x, w, gz = nrm(r, (B, IH, IW, IC)), nrm(r, (OC, FH, FW, IC)), nrm(r, (B, OH, OW, OC))
+        gx0, gw0 = ints(r, x.shape, 2), ints(r, w.shape, 2)
+        for ox, ow in ((True, True), (False, False)):
+            monkeypatch.delenv("D8_CONV_GRADS_APART", raising=False)
+            one = ops.deconv2d_grad_xy(h(x), h(w), h(gz), *geo, h(gx0), h(gw0), ox, ow)
+            monkeypatch.setenv("D8_CONV_GRADS_APART", "1")
+            two = ops.deconv2d_grad_xy(h(x), h(w), h(gz), *geo, h(gx0), h(gw0), ox, ow)
+            assert all(np.array_equal(a.view(np.uint16), b.view(np.uint16)) for a, b in zip(one, two))
+            if whole:
+                want_x, want_w = oracle_port.deconv2d_grad_x(x, w, gz, *geo), oracle_port.deconv2d_grad_y(x, w, gz, *geo)
+                assert max(np.abs(want_x).max(), np.abs(want_w).max()) < 2000
+                assert np.array_equal(f(one[0]), want_x + (0 if ox else gx0))
+                assert np.array_equal(f(one[1]), want_w + (0 if ow else gw0))
