@@ -1059,15 +1059,18 @@ bool gemm_tiled_run_pair(int dtype, GemmArgs &gx, GemmArgs &gy, void *workspace,
 // 16 x 57x57x96 -> 160, 3x3 stride 2: both gradients 38.4 -> 31.8 us; 60 drawn layers 1810 -> 1539 us, none slower.
 // Patch rows whose last K step is cut short, or that are cut into pieces: a launch or two fewer, and no half empty chip behind the
 // pieces of either.  98 drawn layers 3642 -> 3312 us, 9 x 33x33x64 -> 64 3x3 18.5 -> 12.4, 15 x 18x18x192 -> 272 5x5 67.1 -> 49.7,
-// DeConv2d 1 x 33x33x56 -> 320 2x2 stride 2 19.2 -> 11.7; none slower by more than 1 %.
+// DeConv2d 1 x 33x33x56 -> 320 2x2 stride 2 19.2 -> 11.7; none slower by more than 1 %.  fp32
+// (where kept_tiles takes it): 340 drawn layers 15179 -> 14044 us, 6 x 8x8x64 -> 64 3x3 17.8 -> 9.9.
 bool gemm_tiled_kept_pair_plan(int dtype, GemmArgs &gx, GemmArgs &gy, void *workspace, size_t workspace_bytes) {
-    if (getenv("D8_CONV_GRADS_APART") != nullptr || dtype != D8_FLOAT16) return false;
+    if (getenv("D8_CONV_GRADS_APART") != nullptr || dtype == D8_FLOAT64) return false;
     const size_t usable = (workspace && ((size_t)workspace & 15) == 0) ? workspace_bytes : 0;
     const int BK = gemm_tiled_k_step(dtype);
     if (!gemm_tiled_eligible(dtype, gy, 1, 0) || gemm_is_small(gy.M, gy.N, gy.K, gy.batch, gy.red)) return false;
     gy.ws = (float *)workspace;
     gy.splits = plan_splits(BK, gy.M, gy.N, gy.K, 1, gy.red, usable, &gy.tiles_per_split, gy.virt);
-    if (gx.virt == VIRT_A_CLASSES) return gemm_tiled_class_pair_tiles(gx, gy);
+    const auto tiles = dtype == D8_FLOAT16 ? gemm_tiled_kept_pair_tiles_f16 : gemm_tiled_kept_pair_tiles_f32;
+    if (gx.virt == VIRT_A_CLASSES) return tiles(gx, gy);
+    if (narrow_output(dtype, gx)) gx.tile_hint = HINT_128x32;
     if (gx.virt != VIRT_A_ROWS || balanced_rows(gx) || !gemm_tiled_eligible(dtype, gx, 0, 0) || gemm_is_small(gx.M, gx.N, gx.K, gx.batch, gx.red)) return false;
     gx.splits = plan_splits(BK, gx.M, gx.N, gx.K, 1, gx.red, usable, &gx.tiles_per_split, gx.virt);
     few_tiles_small(dtype, gx, 0, 0, usable);
@@ -1076,11 +1079,13 @@ bool gemm_tiled_kept_pair_plan(int dtype, GemmArgs &gx, GemmArgs &gy, void *work
     const size_t gx_bytes = gx.splits > 1 ? (size_t)gx.splits * gx.M * gx.N * sizeof(float) : 0;
     if (gy_bytes + gx_bytes > usable) return false;
     gx.ws = (float *)((char *)workspace + gy_bytes);
-    return gemm_tiled_rows_pair_tiles(gx, gy);
+    return tiles(gx, gy);
 }
 
 int gemm_tiled_kept_pair_run(int dtype, const GemmArgs &gx, const GemmArgs &gy, hipStream_t stream) {
-    if (int rc = gx.virt == VIRT_A_CLASSES ? gemm_tiled_class_pair_launch(gx, gy, stream) : gemm_tiled_rows_pair_launch(gx, gy, stream)) return rc;
+    const bool classes = gx.virt == VIRT_A_CLASSES;
+    const auto pair = dtype == D8_FLOAT16 ? (classes ? gemm_tiled_pair_classes_f16 : gemm_tiled_pair_rows_f16) : (classes ? gemm_tiled_pair_classes_f32 : gemm_tiled_pair_rows_f32);
+    if (int rc = pair(gx, gy, stream)) return rc;
     return launch_reduce_pair(dtype, gx, gy, stream);
 }
 

@@ -134,15 +134,17 @@ bool gemm_tiled_loose(int dtype, const GemmArgs &g, int transA, int transB);  //
 // pair cannot run this way (the tiles the two products would choose have no common kernel, or one is cut into a band).
 long gemm_tiled_pair_workgroups(int dtype, const GemmArgs &gx, const GemmArgs &gy);
 int gemm_tiled_pair_launch(int dtype, const GemmArgs &gx, const GemmArgs &gy, hipStream_t stream);
-// The same in half with both products tiled and cut as they would be alone, also where K cuts the last step of gx short and where
+// The same with both products tiled and cut as they would be alone, also where K cuts the last step of gx short and where
 // gx runs over classes of output pixels (VIRT_A_CLASSES: strides above 1).  _plan decides and sets how the reductions are
 // cut; _run launches and reduces.
 bool gemm_tiled_kept_pair_plan(int dtype, GemmArgs &gx, GemmArgs &gy, void *workspace, size_t workspace_bytes);
 int gemm_tiled_kept_pair_run(int dtype, const GemmArgs &gx, const GemmArgs &gy, hipStream_t stream);
-bool gemm_tiled_rows_pair_tiles(const GemmArgs &gx, const GemmArgs &gy);
-int gemm_tiled_rows_pair_launch(const GemmArgs &gx, const GemmArgs &gy, hipStream_t stream);
-bool gemm_tiled_class_pair_tiles(const GemmArgs &gx, const GemmArgs &gy);
-int gemm_tiled_class_pair_launch(const GemmArgs &gx, const GemmArgs &gy, hipStream_t stream);
+bool gemm_tiled_kept_pair_tiles_f16(const GemmArgs &gx, const GemmArgs &gy);
+bool gemm_tiled_kept_pair_tiles_f32(const GemmArgs &gx, const GemmArgs &gy);
+int gemm_tiled_pair_rows_f16(const GemmArgs &gx, const GemmArgs &gy, hipStream_t stream);
+int gemm_tiled_pair_rows_f32(const GemmArgs &gx, const GemmArgs &gy, hipStream_t stream);
+int gemm_tiled_pair_classes_f16(const GemmArgs &gx, const GemmArgs &gy, hipStream_t stream);
+int gemm_tiled_pair_classes_f32(const GemmArgs &gx, const GemmArgs &gy, hipStream_t stream);
 // The same for two real products: g0 NT, g1 TN (the two gradients of a MatrixMultiply), each batched or split as planned
 // (g.splits / tiles_per_split / ws set; the caller reduces).
 long gemm_tiled_plain_pair_workgroups(int dtype, const GemmArgs &g0, const GemmArgs &g1);

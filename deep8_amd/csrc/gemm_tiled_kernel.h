@@ -1122,7 +1122,14 @@ static int launch_pair_tiles(const GemmArgs &gx0, const GemmArgs &gy0, hipStream
     const bool rec = (size_t)(ny * nzy + nx * nzx) * 64 <= phase_rec_bytes;
     gy.phase_rec = rec ? phase_rec_buf : nullptr, gy.stamps = 0;
     gx.phase_rec = rec && phase_rec_buf ? phase_rec_buf + 8L * ny * nzy : nullptr, gx.stamps = 1;
-    hipLaunchKernelGGL((gemm_tiled_pair_kernel<TY, TX, EDGE>), dim3(ny * nzy + nx * nzx), dim3(TX::NT), 0, stream, gy, gx, tMy, tNy, ny, nzy, tMx, tNx, nx);
+    // (at most two workgroups per compute unit: none takes a third, as in launch_edge)
+    constexpr long third = 160 * 1024 / 3;
+    long lds;
+    if constexpr (TX::DMA) lds = TX::LDS_BYTES > TY::LDS_BYTES ? TX::LDS_BYTES : TY::LDS_BYTES;
+    else lds = 2L * ((TX::A_SZ > TY::A_SZ ? TX::A_SZ : TY::A_SZ) + (TX::B_SZ > TY::B_SZ ? TX::B_SZ : TY::B_SZ)) * TX::ES;
+    const long wgs = (long)ny * nzy + (long)nx * nzx, cus = cu_count();
+    const unsigned pad = lds <= third && wgs > cus && wgs <= 2 * cus ? (unsigned)(third + 512 - lds) : 0u;
+    hipLaunchKernelGGL((gemm_tiled_pair_kernel<TY, TX, EDGE>), dim3(ny * nzy + nx * nzx), dim3(TX::NT), pad, stream, gy, gx, tMy, tNy, ny, nzy, tMx, tNx, nx);
     D8_LAUNCH_CHECK();
     return 0;
 }

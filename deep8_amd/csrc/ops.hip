@@ -1086,13 +1086,13 @@ int d8_conv2d_grad_xy(int dtype, const void *x, void *gx, int B, int IH, int IW,
             }
         }
     }
-    {  // one launch in half too where the two calls would have both in the loader (strides above 1, channels that cut a K step short)
+    {  // one launch too where the two calls would have both in the loader (strides above 1, channels that cut a K step short)
         const ConvShape cs = {B, IH, IW, IC, OC, FH, FW, g[0], g[1], sy, sx, dy, dx, g[2], g[3]};
         const int M = B * g[0] * g[1], K = FH * FW * IC;
         GemmArgs px, pw;
         int ta, tb;
         bool untouched = false;
-        if (dtype == D8_FLOAT16 && (conv_implicit_plan(dtype, 1, cs, gx, w, gz, px, ta, tb) || conv_classes_grad_x(dtype, cs, gx, w, gz, px, &untouched)) &&
+        if (dtype != D8_FLOAT64 && (conv_implicit_plan(dtype, 1, cs, gx, w, gz, px, ta, tb) || conv_classes_grad_x(dtype, cs, gx, w, gz, px, &untouched)) &&
             conv_implicit_plan(dtype, 2, cs, x, gw, gz, pw, ta, tb) &&
             !prefer_interim(dtype, px, 0, 0, conv_plan(1, M, K, OC, scratch, w, gz), (double)M * K, IC, untouched ? 0 : 1, scratch, scratch_bytes) &&
             !prefer_interim(dtype, pw, ta, tb, conv_plan(2, M, K, OC, scratch, gw, gz), (double)M * K, IC, 0, scratch, scratch_bytes) &&
@@ -1132,7 +1132,7 @@ static int deconv2d_grad_xy_geo(int dtype, const void *x, void *gx, int B, int I
     {  // as d8_conv2d_grad_xy
         const int M = B * IH * IW, T = FH * FW;
         GemmArgs px, pw;
-        if (dtype == D8_FLOAT16 && deconv_implicit_grad_x(dtype, B, IH, IW, IC, OC, FH, FW, sy, sx, g, gx, w, gz, px) &&
+        if (dtype != D8_FLOAT64 && deconv_implicit_grad_x(dtype, B, IH, IW, IC, OC, FH, FW, sy, sx, g, gx, w, gz, px) &&
             deconv_implicit_grad_y(dtype, B, IH, IW, IC, OC, FH, FW, sy, sx, g, x, gw, gz, pw) &&
             !prefer_interim(dtype, px, 0, 0, deconv_plan(1, M, T, OC, IC, scratch, w, gx), (double)M * T * OC, OC, 0, scratch, scratch_bytes) &&
             !prefer_interim(dtype, pw, 1, 0, deconv_plan(2, M, T, OC, IC, scratch, gw, x), (double)M * T * OC, OC, 0, scratch, scratch_bytes) &&

@@ -1,4 +1,4 @@
-"""Convolutions in half, both gradients from one call, on layers whose two products are tiled and cut as they would be alone and
+"""Convolutions, both gradients from one call, on layers whose two products are tiled and cut as they would be alone and
 share a launch: classes of output pixels (strides above 1), last K steps that are cut short, gradients of x in pieces.  Channels
 narrower and wider than a tile, classes that no tap reaches, one-pixel classes, dilation, every combination of written and added
 gradients, scratch for no pieces.  Integers, against the oracle, bit for bit; reals, bit for bit what two launches leave."""
@@ -45,17 +45,18 @@ def test_integers_against_the_oracle(oracle_port, cfg):
         assert np.array_equal(f(gw), want_w + (0 if ow else gw0)), (ox, ow)
 
 
-@pytest.mark.parametrize("cfg", LAYERS)
-def test_one_launch_leaves_what_two_leave(cfg, monkeypatch):
+@pytest.mark.parametrize("cfg", LAYERS + [(16, 14, 14, 32, 64, 5, 5, True, 1, 1, 1, 1), (7, 28, 28, 40, 16, 3, 3, True, 2, 2, 1, 1)])
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+def test_one_launch_leaves_what_two_leave(cfg, dtype, monkeypatch):
     from deep8_amd import capi, ops
     from deep8_amd.capi import DeviceArray, check
     lib = capi.init()
     B, IH, IW, IC, OC, FH, FW = cfg[:7]
     geo = cfg[7:]
     OH, OW, _, _ = ops.conv2d_geometry(IH, IW, FH, FW, *geo)
-    r = rng(sum(cfg[:7]) + 1)
-    x, w, gz = (DeviceArray.from_numpy(h(nrm(r, s))) for s in ((B, IH, IW, IC), (OC, FH, FW, IC), (B, OH, OW, OC)))
-    asked = lib.d8_conv2d_scratch_bytes(capi.FLOAT16, 3, B, IH, IW, IC, OC, FH, FW, *(int(v) for v in geo))
+    r, dt = rng(sum(cfg[:7]) + 1), capi.FLOAT16 if dtype == np.float16 else capi.FLOAT32
+    x, w, gz = (DeviceArray.from_numpy(nrm(r, s).astype(dtype)) for s in ((B, IH, IW, IC), (OC, FH, FW, IC), (B, OH, OW, OC)))
+    asked = lib.d8_conv2d_scratch_bytes(dt, 3, B, IH, IW, IC, OC, FH, FW, *(int(v) for v in geo))
     for nb in (0, asked):
         got = []
         for apart in (False, True):
@@ -63,11 +64,11 @@ def test_one_launch_leaves_what_two_leave(cfg, monkeypatch):
                 monkeypatch.setenv("D8_CONV_GRADS_APART", "1")
             else:
                 monkeypatch.delenv("D8_CONV_GRADS_APART", raising=False)
-            gx, gw = (DeviceArray.from_numpy(np.full(s, np.nan, np.float16)) for s in ((B, IH, IW, IC), (OC, FH, FW, IC)))
+            gx, gw = (DeviceArray.from_numpy(np.full(s, np.nan, dtype)) for s in ((B, IH, IW, IC), (OC, FH, FW, IC)))
             ws = DeviceArray((max(nb, 16),), np.uint8)
-            check(lib.d8_conv2d_grad_xy(capi.FLOAT16, x.ptr, gx.ptr, B, IH, IW, IC, w.ptr, gw.ptr, OC, FH, FW, gz.ptr,
+            check(lib.d8_conv2d_grad_xy(dt, x.ptr, gx.ptr, B, IH, IW, IC, w.ptr, gw.ptr, OC, FH, FW, gz.ptr,
                                         *(int(v) for v in geo), 3, ws.ptr if nb else None, nb, None))
-            got.append((gx.numpy().view(np.uint16), gw.numpy().view(np.uint16)))
+            got.append((gx.numpy().view(np.uint8), gw.numpy().view(np.uint8)))
         assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1]), nb
 
 
