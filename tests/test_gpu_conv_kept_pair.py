@@ -45,8 +45,11 @@ def test_integers_against_the_oracle(oracle_port, cfg):
         assert np.array_equal(f(gw), want_w + (0 if ow else gw0)), (ox, ow)
 
 
-@pytest.mark.parametrize("cfg", LAYERS + [(16, 14, 14, 32, 64, 5, 5, True, 1, 1, 1, 1), (7, 28, 28, 40, 16, 3, 3, True, 2, 2, 1, 1)])
-@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+# (fp32: 128 x 32 tiles; in half the first would run whole in company, in pieces alone)
+NARROW = [(16, 14, 14, 32, 64, 5, 5, True, 1, 1, 1, 1), (7, 28, 28, 32, 40, 3, 3, True, 2, 2, 1, 1)]
+
+
+@pytest.mark.parametrize("cfg,dtype", [(c, t) for c in LAYERS for t in (np.float32, np.float16)] + [(c, np.float32) for c in NARROW])
 def test_one_launch_leaves_what_two_leave(cfg, dtype, monkeypatch):
     from deep8_amd import capi, ops
     from deep8_amd.capi import DeviceArray, check
