@@ -330,7 +330,7 @@ __global__ __launch_bounds__(256) void broadcast_sum_kernel(const T *__restrict_
             }
             if (a < 0) break;
         }
-        g[idx] = (T)((keep != 0.f ? ew_f32(g[idx]) : 0.f) + scale * acc);
+        g[idx] = ew_result<T, OP>((keep != 0.f ? ew_f32(g[idx]) : 0.f) + scale * acc);
     }
 }
 

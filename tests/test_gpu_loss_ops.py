@@ -69,6 +69,28 @@ def test_l1_and_l2_norm(oracle_port, shape, dtype):
     assert rel_fro(f(ops.l2norm_grad(x, c(y2), c(dyr), c(dx0))), oracle_port.l2norm_grad(f(x), f(c(y2)), f(c(dyr)), dx0)) <= tol
 
 
+@pytest.mark.parametrize("batch", [65535, 65536, 70001])
+@pytest.mark.parametrize("size", [1, 3, 8])
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+def test_norms_of_more_rows_than_a_grid_is_deep(batch, size, dtype):
+    """integers, whose sums of absolute values and of squares are exact in both types; the root of a sum within a unit in the last
+    place of the type"""
+    from deep8_amd import capi
+    from deep8_amd.capi import DeviceArray, check
+    lib = capi.init()
+    dt = capi.FLOAT16 if dtype == np.float16 else capi.FLOAT32
+    x = (ints(rng(batch + size), (batch, size), 7) - 3).astype(dtype)
+    dx = DeviceArray.from_numpy(x)
+    want1 = np.abs(x.astype(np.float64)).sum(1)
+    want2 = np.sqrt((x.astype(np.float64) ** 2).sum(1)).astype(np.float32).astype(dtype)
+    for nb in (0, 1 << 20):
+        ws = DeviceArray((max(nb, 16),), np.uint8)
+        for call, want in ((lib.d8_l1norm, want1), (lib.d8_l2norm, want2)):
+            y = DeviceArray.from_numpy(np.full(batch, np.nan, dtype))
+            check(call(dt, dx.ptr, y.ptr, batch, size, ws.ptr if nb else None, nb, None))
+            assert np.allclose(f(y.numpy()), f(want), rtol=np.finfo(dtype).eps, atol=0), (call.__name__, nb)
+
+
 @pytest.mark.parametrize("shape,axes", [((3, 8), ()), ((3, 8), (0,)), ((3, 8), (1,)), ((2, 4, 5, 8), (1, 3)), ((2, 4, 5, 6), (-1,)),
                                         ((2, 3, 4, 5, 6), (0, 2, 4)), ((1, 12), (0, 1)), ((16, 1), ()), ((32, 56, 56, 64), (0, 1, 2)),
                                         ((4, 4096), ())])
