@@ -581,6 +581,18 @@ struct Divisor {
     }
 };
 
+// A value that is the same for all lanes, in a scalar register (DmaTile).  The compiler keeps the quotients of integer divisions
+// and what it computes from them in vector registers, and would read a load's offset from there right before dma_piece: a load wants
+// five wait states behind a vector instruction that writes a scalar it takes, which the compiler keeps before loads of its own
+// only.  Whatever an offset is made of is therefore made scalar well before the loads (tests/test_kernel_wait_states.py looks
+// for any that is not).  Five wait states before every step's loads instead: a dense layer of 4096 x 1024 x 1024 with its gradients
+// 23.0 -> 23.8 us; so, 23.2, and Conv2d 32 x 14x14x256 3x3 with its 56.5 -> 56.9.
+template <typename T>
+__device__ __forceinline__ int uniform(int v) {
+    if constexpr (T::DMA) return __builtin_amdgcn_readfirstlane(v);
+    else return v;
+}
+
 // The work of one workgroup: workgroup (bx, bz) of a grid of nbx x layers (the launch's own blockIdx / gridDim, or what a
 // launch of two products makes of them).  As0 .. Bs1: the two halves of both operand areas in LDS.
 template <typename T, int EDGE>
@@ -658,7 +670,7 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     const int tn = in_tail ? id / tail_tilesM : in_band / rows_in_band;
     // A tile that would stick out of the matrix is moved back inside; the rows / columns it then
     // shares with its neighbour are computed twice but stored only by the neighbour.
-    const int m_own = (in_tail ? g.tail_m0 : 0) + tm * BM, n_own = tn * BN;
+    const int m_own = uniform<T>((in_tail ? g.tail_m0 : 0) + tm * BM), n_own = uniform<T>(tn * BN);
     // (a matrix with fewer rows or columns than the tile: the tile starts at 0 and reaches past it; what the loads
     // bring in from there -- zeros past the end of the buffer, otherwise whatever follows -- only ever enters
     // results of rows / columns past the matrix, which are not stored)
@@ -673,6 +685,7 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     // EDGE_ANY: the buffers start at the dword that holds the operand's first element and end with the one that holds its
     // last (a dword at a multiple of 4 never reaches into another page); at the elements before and after sit no results.
     constexpr bool ANY = Loose<T, EDGE>::ANY, ODD = Loose<T, EDGE>::ODD;
+    b = uniform<T>(b);
     const long a_rows = A_KC ? g.M : g.K, b_rows = B_KC ? g.N : g.K;
     const E *Ab = (const E *)g.A + (long)b * g.sA, *Bb = (const E *)g.B + (long)b * g.sB;
     const unsigned a_odd = ODD ? (unsigned)((size_t)Ab & 2) >> 1 : 0u, b_odd = ODD ? (unsigned)((size_t)Bb & 2) >> 1 : 0u;
@@ -780,15 +793,14 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     // partly past K, and the pieces that lie past it are fetched at an offset beyond the buffer, i.e. as zeros.  Where the
     // reduction runs over patch rows or over the rows of a real matrix, rows past the last lie outside the buffer anyway.
     const int ktiles = (g.K + BK - 1) / BK, last_len = g.K - (ktiles - 1) * BK;
-    const int x0 = split * tps, nsteps = min(red * ktiles, x0 + tps) - x0;
+    const int x0 = uniform<T>(split * tps), nsteps = min(red * ktiles, x0 + tps) - x0;
     const unsigned a_prod = (unsigned)ES * (unsigned)g.sA, b_prod = (unsigned)ES * (unsigned)g.sB;
     const unsigned b_prod_row = (unsigned)ES * (unsigned)g.sB_row, b_first = (unsigned)ES * b_cls;
     // The step that is fetched next: its product, K step and filter tap are counted on from step to step (every step is
     // fetched once, in order), because four divisions by runtime numbers at the head of each step -- some 35 dependent
     // scalar instructions that no matrix instruction covers -- were a fifth of a short half step's time.
-    // (uniform, and said to be: the compiler keeps the quotients of an integer division in vector registers otherwise)
-    int ld_i = 0, ld_r = T::DMA ? __builtin_amdgcn_readfirstlane(x0 / ktiles) : x0 / ktiles, ld_kx = x0 - ld_r * ktiles;
-    int ld_fy = !VA ? 0 : T::DMA ? __builtin_amdgcn_readfirstlane(ld_r / pg.FW) : ld_r / pg.FW, ld_fx = VA ? ld_r - ld_fy * pg.FW : 0;
+    int ld_i = 0, ld_r = uniform<T>(x0 / ktiles), ld_kx = x0 - ld_r * ktiles;
+    int ld_fy = !VA ? 0 : uniform<T>(ld_r / pg.FW), ld_fx = VA ? ld_r - ld_fy * pg.FW : 0;
     // patch k-rows: what BK more pixels add, and the corrections when a row or an image is complete
     int vb_dy = 0, vb_dx = 0, vb_d = 0, vb_d_row = 0, vb_d_img = 0;
     if constexpr (VIRT == VIRT_B_KROWS) {
@@ -847,13 +859,13 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     auto step_on = [&]() {
         ld_kx += ++ld_i < nsteps ? 1 : 0;
         const int done = ld_kx == ktiles ? 1 : 0;
-        ld_kx = done ? 0 : ld_kx;
-        ld_r += done;
+        ld_kx = uniform<T>(done ? 0 : ld_kx);
+        ld_r = uniform<T>(ld_r + done);
         if constexpr (VA) {
             ld_fx += done;
             const int row = ld_fx == pg.FW ? 1 : 0;
-            ld_fx = row ? 0 : ld_fx;
-            ld_fy += row;
+            ld_fx = uniform<T>(row ? 0 : ld_fx);
+            ld_fy = uniform<T>(ld_fy + row);
         }
         if constexpr (VIRT == VIRT_B_KROWS) {
 #pragma unroll
@@ -888,7 +900,7 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
         auto aim = [&]() {
             const bool live = ld_i < nsteps;
             next_step(pa, pb);
-            sa = __builtin_amdgcn_readfirstlane(pa), sb = __builtin_amdgcn_readfirstlane(pb);  // (uniform already)
+            sa = __builtin_amdgcn_readfirstlane(pa), sb = __builtin_amdgcn_readfirstlane(pb);  // (scalars already: see uniform)
             const unsigned long at_a = (unsigned long)Ab, at_b = (unsigned long)Bb;
             da = (u32x4){(unsigned)at_a, (unsigned)(at_a >> 32) & 0xffffu, live ? (unsigned)a_bytes : 0u, 0x00020000u};
             db = (u32x4){(unsigned)at_b, (unsigned)(at_b >> 32) & 0xffffu, live ? (unsigned)b_bytes : 0u, 0x00020000u};
