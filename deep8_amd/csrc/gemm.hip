@@ -999,7 +999,8 @@ bool gemm_small_pair_run(int dtype, const GemmArgs &g0, int ta0, int tb0, const 
     return true;
 }
 
-static std::atomic<unsigned long> pair_launches{0};  // d8_conv_grad_pair_launches
+// d8_conv_grad_pair_launches, d8_conv_grad_kept_pair_launches
+static std::atomic<unsigned long> pair_launches{0}, kept_pair_launches{0};
 
 // Both gradients of a convolution as one launch (gemm_tiled_pair_launch) when that fills compute units the two
 // products would each leave idle: gx is not cut into a band and not split, the workgroups of both fit the chip
@@ -1085,6 +1086,7 @@ bool gemm_tiled_kept_pair_plan(int dtype, GemmArgs &gx, GemmArgs &gy, void *work
 int gemm_tiled_kept_pair_run(int dtype, const GemmArgs &gx, const GemmArgs &gy, hipStream_t stream) {
     const bool classes = gx.virt == VIRT_A_CLASSES;
     const auto pair = dtype == D8_FLOAT16 ? (classes ? gemm_tiled_pair_classes_f16 : gemm_tiled_pair_rows_f16) : (classes ? gemm_tiled_pair_classes_f32 : gemm_tiled_pair_rows_f32);
+    ++kept_pair_launches;
     if (int rc = pair(gx, gy, stream)) return rc;
     return launch_reduce_pair(dtype, gx, gy, stream);
 }
@@ -1203,6 +1205,7 @@ static int gemm_one(int dtype, int transA, int transB, int M, int N, int K,
 }
 
 unsigned long d8_conv_grad_pair_launches(void) { return pair_launches.load(); }
+unsigned long d8_conv_grad_kept_pair_launches(void) { return kept_pair_launches.load(); }
 
 int d8_gemm_phase_record(void *records, size_t bytes) {
     D8_REQUIRE(((size_t)records & 7) == 0, "d8_gemm_phase_record: the record buffer is not 8-byte aligned");

@@ -296,8 +296,10 @@ int d8_deconv2d_grad_xy_ex(int dtype, const void *x, void *gx, int B, int IH, in
                            void *scratch, size_t scratch_bytes, void *stream);
 
 /* Test and measurement aid: how many of the _grad_xy calls above have run as one launch since the library was
- * loaded (no counterpart in the reference).                                                                       */
+ * loaded (no counterpart in the reference): those whose gradient of x runs whole, or with its remainder band, and
+ * those whose two products are tiled and cut as they would be alone.  A call counts in one of them at most.        */
 unsigned long d8_conv_grad_pair_launches(void);
+unsigned long d8_conv_grad_kept_pair_launches(void);
 unsigned long d8_matmul_grad_pair_launches(void);  /* ... and of the d8_matmul_grad_xy calls */
 /* How many Conv2d / DeConv2d calls have run (each gradient is one; both gradients from one call are two), by route: 0 on an
  * interim matrix in scratch, 1 with the patches read by the GEMM's loader, 2 on the kernels for images of few channels. */

@@ -1,11 +1,12 @@
 """Convolutions, both gradients from one call, on layers whose two products are tiled and cut as they would be alone and
 share a launch: classes of output pixels (strides above 1), last K steps that are cut short, gradients of x in pieces.  Channels
 narrower and wider than a tile, classes that no tap reaches, one-pixel classes, dilation, every combination of written and added
-gradients, scratch for no pieces.  Integers, against the oracle, bit for bit; reals, bit for bit what two launches leave."""
+gradients, scratch for no pieces.  Integers, against the oracle, bit for bit; reals, bit for bit what two launches leave; and which
+calls share one is counted."""
 import numpy as np
 import pytest
 
-from util import f, h, ints, nrm, rng
+from util import f, ints, nrm, rng
 
 pytestmark = pytest.mark.gpu
 
@@ -25,10 +26,50 @@ LAYERS = [
     (8, 11, 11, 256, 128, 5, 5, True, 1, 1, 1, 1),    # gradient of x in pieces
     (16, 28, 28, 136, 88, 3, 3, True, 1, 1, 1, 1),    # 128 x 128 tiles, columns past a tile
 ]
+# (fp32: 128 x 32 tiles; in half the first would run whole in company, in pieces alone)
+NARROW = [(16, 14, 14, 32, 64, 5, 5, True, 1, 1, 1, 1), (7, 28, 28, 32, 40, 3, 3, True, 2, 2, 1, 1)]
+# With the scratch that is asked for these run apart: their patch matrix is expected to be faster
+APART = [(LAYERS[i], np.float32) for i in (1, 2, 4, 7, 9, 10, 11)] + [(LAYERS[5], np.float16)]
+# ... and this without scratch: shared whole by the older rule
+APART_WHOLE = [(NARROW[0], np.float32)]
+
+# B, IH, IW, IC, OC, FH, FW, covered, sy, sx
+TRANSPOSED = [
+    (4, 14, 13, 64, 72, 4, 4, False, 2, 2),
+    (2, 9, 11, 136, 40, 3, 3, True, 2, 2),            # too small for tiles
+    (18, 6, 6, 72, 16, 5, 5, False, 2, 2),
+    (6, 16, 16, 64, 200, 3, 3, False, 1, 1),
+    (8, 20, 20, 128, 88, 2, 2, False, 2, 2),
+]
+APART_TRANSPOSED = [(TRANSPOSED[0], np.float16), (TRANSPOSED[1], np.float32), (TRANSPOSED[1], np.float16)]
+APART_TRANSPOSED_WHOLE = APART_TRANSPOSED[1:]
+
+
+def _layer(name, cfg, dtype, x, w, gz):
+    """call(gx0, gw0, overwrite, scratch bytes) -> both gradients and how many launches were shared; the scratch asked for"""
+    from deep8_amd import capi
+    from deep8_amd.capi import DeviceArray, check
+    lib = capi.init()
+    dt, (B, IH, IW, IC, OC, FH, FW), geo = capi.FLOAT16 if dtype == np.float16 else capi.FLOAT32, cfg[:7], tuple(int(v) for v in cfg[7:])
+    dx, dw, dgz = (DeviceArray.from_numpy(np.asarray(t, dtype)) for t in (x, w, gz))
+
+    def call(gx0, gw0, overwrite, nb):
+        gx, gw, ws = DeviceArray.from_numpy(np.asarray(gx0, dtype)), DeviceArray.from_numpy(np.asarray(gw0, dtype)), DeviceArray((max(nb, 16),), np.uint8)
+        before = lib.d8_conv_grad_kept_pair_launches()
+        check(getattr(lib, f"d8_{name}_grad_xy")(dt, dx.ptr, gx.ptr, B, IH, IW, IC, dw.ptr, gw.ptr, OC, FH, FW, dgz.ptr, *geo, overwrite,
+                                                 ws.ptr if nb else None, nb, None))
+        return gx.numpy(), gw.numpy(), lib.d8_conv_grad_kept_pair_launches() - before
+
+    return call, getattr(lib, f"d8_{name}_scratch_bytes")(dt, 3, B, IH, IW, IC, OC, FH, FW, *geo)
+
+
+def _shares(cfg, dtype, nb, apart, apart_whole):
+    return int((cfg, dtype) not in (apart if nb else apart_whole))
 
 
 @pytest.mark.parametrize("cfg", LAYERS)
-def test_integers_against_the_oracle(oracle_port, cfg):
+@pytest.mark.parametrize("dtype", [np.float16])
+def test_integers_against_the_oracle(oracle_port, cfg, dtype):
     from deep8_amd import ops
     B, IH, IW, IC, OC, FH, FW = cfg[:7]
     geo = cfg[7:]
@@ -39,54 +80,36 @@ def test_integers_against_the_oracle(oracle_port, cfg):
     gx0, gw0 = ints(r, x.shape, 2), ints(r, w.shape, 2)
     want_x, want_w = oracle_port.conv2d_grad_x(x, w, gz, *geo), oracle_port.conv2d_grad_y(x, w, gz, *geo)
     assert max(np.abs(want_x).max(), np.abs(want_w).max()) < 2000
-    for ox, ow in ((True, True), (False, True), (True, False), (False, False)):
-        gx, gw = ops.conv2d_grad_xy(h(x), h(w), h(gz), *geo, h(gx0), h(gw0), ox, ow)
-        assert np.array_equal(f(gx), want_x + (0 if ox else gx0)), (ox, ow)
-        assert np.array_equal(f(gw), want_w + (0 if ow else gw0)), (ox, ow)
-
-
-# (fp32: 128 x 32 tiles; in half the first would run whole in company, in pieces alone)
-NARROW = [(16, 14, 14, 32, 64, 5, 5, True, 1, 1, 1, 1), (7, 28, 28, 32, 40, 3, 3, True, 2, 2, 1, 1)]
+    call, asked = _layer("conv2d", cfg, dtype, x, w, gz)
+    for nb in (0, asked):
+        for overwrite in (3, 2, 1, 0):
+            gx, gw, shared = call(gx0, gw0, overwrite, nb)
+            assert shared == _shares(cfg, dtype, nb, APART, APART_WHOLE), nb
+            assert np.array_equal(f(gx), want_x + (0 if overwrite & 1 else gx0)), (nb, overwrite)
+            assert np.array_equal(f(gw), want_w + (0 if overwrite & 2 else gw0)), (nb, overwrite)
 
 
 @pytest.mark.parametrize("cfg,dtype", [(c, t) for c in LAYERS for t in (np.float32, np.float16)] + [(c, np.float32) for c in NARROW])
 def test_one_launch_leaves_what_two_leave(cfg, dtype, monkeypatch):
-    from deep8_amd import capi, ops
-    from deep8_amd.capi import DeviceArray, check
-    lib = capi.init()
+    from deep8_amd import ops
     B, IH, IW, IC, OC, FH, FW = cfg[:7]
     geo = cfg[7:]
     OH, OW, _, _ = ops.conv2d_geometry(IH, IW, FH, FW, *geo)
-    r, dt = rng(sum(cfg[:7]) + 1), capi.FLOAT16 if dtype == np.float16 else capi.FLOAT32
-    x, w, gz = (DeviceArray.from_numpy(nrm(r, s).astype(dtype)) for s in ((B, IH, IW, IC), (OC, FH, FW, IC), (B, OH, OW, OC)))
-    asked = lib.d8_conv2d_scratch_bytes(dt, 3, B, IH, IW, IC, OC, FH, FW, *(int(v) for v in geo))
+    r = rng(sum(cfg[:7]) + 1)
+    x, w, gz = (nrm(r, s) for s in ((B, IH, IW, IC), (OC, FH, FW, IC), (B, OH, OW, OC)))
+    call, asked = _layer("conv2d", cfg, dtype, x, w, gz)
     for nb in (0, asked):
-        got = []
-        for apart in (False, True):
-            if apart:
-                monkeypatch.setenv("D8_CONV_GRADS_APART", "1")
-            else:
-                monkeypatch.delenv("D8_CONV_GRADS_APART", raising=False)
-            gx, gw = (DeviceArray.from_numpy(np.full(s, np.nan, dtype)) for s in ((B, IH, IW, IC), (OC, FH, FW, IC)))
-            ws = DeviceArray((max(nb, 16),), np.uint8)
-            check(lib.d8_conv2d_grad_xy(dt, x.ptr, gx.ptr, B, IH, IW, IC, w.ptr, gw.ptr, OC, FH, FW, gz.ptr,
-                                        *(int(v) for v in geo), 3, ws.ptr if nb else None, nb, None))
-            got.append((gx.numpy().view(np.uint8), gw.numpy().view(np.uint8)))
-        assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1]), nb
-
-
-# B, IH, IW, IC, OC, FH, FW, covered, sy, sx
-TRANSPOSED = [
-    (4, 14, 13, 64, 72, 4, 4, False, 2, 2),
-    (2, 9, 11, 136, 40, 3, 3, True, 2, 2),
-    (18, 6, 6, 72, 16, 5, 5, False, 2, 2),
-    (6, 16, 16, 64, 200, 3, 3, False, 1, 1),
-    (8, 20, 20, 128, 88, 2, 2, False, 2, 2),
-]
+        monkeypatch.delenv("D8_CONV_GRADS_APART", raising=False)
+        one = call(np.full(x.shape, np.nan), np.full(w.shape, np.nan), 3, nb)
+        monkeypatch.setenv("D8_CONV_GRADS_APART", "1")
+        two = call(np.full(x.shape, np.nan), np.full(w.shape, np.nan), 3, nb)
+        assert (one[2], two[2]) == (_shares(cfg, dtype, nb, APART, APART_WHOLE), 0), nb
+        assert all(np.array_equal(a.view(np.uint8), b.view(np.uint8)) for a, b in zip(one[:2], two[:2])), nb
 
 
 @pytest.mark.parametrize("cfg", TRANSPOSED)
-def test_transposed_convolutions(oracle_port, cfg, monkeypatch):
+@pytest.mark.parametrize("dtype", [np.float16])
+def test_transposed_convolutions(oracle_port, cfg, dtype, monkeypatch):
     from deep8_amd import ops
     B, IH, IW, IC, OC, FH, FW = cfg[:7]
     geo = cfg[7:]
@@ -100,14 +123,17 @@ def test_transposed_convolutions(oracle_port, cfg, monkeypatch):
         else:
             x, w, gz = nrm(r, (B, IH, IW, IC)), nrm(r, (OC, FH, FW, IC)), nrm(r, (B, OH, OW, OC))
         gx0, gw0 = ints(r, x.shape, 2), ints(r, w.shape, 2)
-        for ox, ow in ((True, True), (False, False)):
-            monkeypatch.delenv("D8_CONV_GRADS_APART", raising=False)
-            one = ops.deconv2d_grad_xy(h(x), h(w), h(gz), *geo, h(gx0), h(gw0), ox, ow)
-            monkeypatch.setenv("D8_CONV_GRADS_APART", "1")
-            two = ops.deconv2d_grad_xy(h(x), h(w), h(gz), *geo, h(gx0), h(gw0), ox, ow)
-            assert all(np.array_equal(a.view(np.uint16), b.view(np.uint16)) for a, b in zip(one, two))
-            if whole:
-                want_x, want_w = oracle_port.deconv2d_grad_x(x, w, gz, *geo), oracle_port.deconv2d_grad_y(x, w, gz, *geo)
-                assert max(np.abs(want_x).max(), np.abs(want_w).max()) < 2000
-                assert np.array_equal(f(one[0]), want_x + (0 if ox else gx0))
-                assert np.array_equal(f(one[1]), want_w + (0 if ow else gw0))
+        call, asked = _layer("deconv2d", cfg, dtype, x, w, gz)
+        for nb in (0, asked):
+            for overwrite in (3, 0):
+                monkeypatch.delenv("D8_CONV_GRADS_APART", raising=False)
+                one = call(gx0, gw0, overwrite, nb)
+                monkeypatch.setenv("D8_CONV_GRADS_APART", "1")
+                two = call(gx0, gw0, overwrite, nb)
+                assert (one[2], two[2]) == (_shares(cfg, dtype, nb, APART_TRANSPOSED, APART_TRANSPOSED_WHOLE), 0), nb
+                assert all(np.array_equal(a.view(np.uint8), b.view(np.uint8)) for a, b in zip(one[:2], two[:2])), nb
+                if whole:
+                    want_x, want_w = oracle_port.deconv2d_grad_x(x, w, gz, *geo), oracle_port.deconv2d_grad_y(x, w, gz, *geo)
+                    assert max(np.abs(want_x).max(), np.abs(want_w).max()) < 2000
+                    assert np.array_equal(f(one[0]), want_x + (0 if overwrite else gx0))
+                    assert np.array_equal(f(one[1]), want_w + (0 if overwrite else gw0))
