@@ -28,10 +28,20 @@ LAYERS = [
 ]
 # (fp32: 128 x 32 tiles; in half the first would run whole in company, in pieces alone)
 NARROW = [(16, 14, 14, 32, 64, 5, 5, True, 1, 1, 1, 1), (7, 28, 28, 32, 40, 3, 3, True, 2, 2, 1, 1)]
-# With the scratch that is asked for these run apart: their patch matrix is expected to be faster
-APART = [(LAYERS[i], np.float32) for i in (1, 2, 4, 7, 9, 10, 11)] + [(LAYERS[5], np.float16)]
-# ... and this without scratch: shared whole by the older rule
-APART_WHOLE = [(NARROW[0], np.float32)]
+# fp32, on either side of the limit of workgroups, with and without pieces
+CROWDED = [
+    (64, 14, 14, 32, 64, 5, 5, True, 1, 1, 1, 1),     # 128 x 32 tiles beside 64 x 128: any number
+    (64, 14, 14, 28, 40, 3, 3, True, 1, 1, 1, 1),
+    (12, 28, 28, 136, 168, 3, 3, True, 1, 1, 1, 1),   # filter gradient on 128 x 128 tiles: two a compute unit
+    (24, 28, 28, 136, 88, 3, 3, True, 1, 1, 1, 1),
+    (6, 67, 67, 64, 64, 3, 3, True, 1, 1, 1, 1),      # 128 x 64 tiles: two a compute unit
+    (8, 40, 40, 136, 136, 3, 3, True, 1, 1, 1, 1),    # 128 x 128 tiles in both: never
+]
+# With the scratch that is asked for these run apart: their patch matrix is expected to be faster, or (fp32) pieces make more
+# workgroups than a compute unit holds two of.
+APART = [(LAYERS[i], np.float32) for i in (1, 2, 4, 7, 9, 10, 11)] + [(LAYERS[5], np.float16)] + [(CROWDED[i], np.float32) for i in (2, 3, 4, 5)]
+# ... and these without scratch: shared whole by the older rule, or never
+APART_WHOLE = [(NARROW[0], np.float32), (CROWDED[0], np.float32), (CROWDED[5], np.float32)]
 
 # B, IH, IW, IC, OC, FH, FW, covered, sy, sx
 TRANSPOSED = [
@@ -40,6 +50,7 @@ TRANSPOSED = [
     (18, 6, 6, 72, 16, 5, 5, False, 2, 2),
     (6, 16, 16, 64, 200, 3, 3, False, 1, 1),
     (8, 20, 20, 128, 88, 2, 2, False, 2, 2),
+    (4, 12, 12, 136, 136, 3, 3, False, 2, 2),
 ]
 APART_TRANSPOSED = [(TRANSPOSED[0], np.float16), (TRANSPOSED[1], np.float32), (TRANSPOSED[1], np.float16)]
 APART_TRANSPOSED_WHOLE = APART_TRANSPOSED[1:]
@@ -68,7 +79,7 @@ def _shares(cfg, dtype, nb, apart, apart_whole):
 
 
 @pytest.mark.parametrize("cfg", LAYERS)
-@pytest.mark.parametrize("dtype", [np.float16])
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
 def test_integers_against_the_oracle(oracle_port, cfg, dtype):
     from deep8_amd import ops
     B, IH, IW, IC, OC, FH, FW = cfg[:7]
@@ -89,7 +100,7 @@ def test_integers_against_the_oracle(oracle_port, cfg, dtype):
             assert np.array_equal(f(gw), want_w + (0 if overwrite & 2 else gw0)), (nb, overwrite)
 
 
-@pytest.mark.parametrize("cfg,dtype", [(c, t) for c in LAYERS for t in (np.float32, np.float16)] + [(c, np.float32) for c in NARROW])
+@pytest.mark.parametrize("cfg,dtype", [(c, t) for c in LAYERS for t in (np.float32, np.float16)] + [(c, np.float32) for c in NARROW + CROWDED])
 def test_one_launch_leaves_what_two_leave(cfg, dtype, monkeypatch):
     from deep8_amd import ops
     B, IH, IW, IC, OC, FH, FW = cfg[:7]
@@ -108,7 +119,7 @@ def test_one_launch_leaves_what_two_leave(cfg, dtype, monkeypatch):
 
 
 @pytest.mark.parametrize("cfg", TRANSPOSED)
-@pytest.mark.parametrize("dtype", [np.float16])
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
 def test_transposed_convolutions(oracle_port, cfg, dtype, monkeypatch):
     from deep8_amd import ops
     B, IH, IW, IC, OC, FH, FW = cfg[:7]
