@@ -389,7 +389,8 @@ int d8_matmul_grad_y_overwrite(int dtype, const void *x, int xb, int xr, int xc,
 
 unsigned long d8_conv_route_calls(int route) { return route >= 0 && route < 3 ? route_calls[route].load() : 0; }
 
-static std::atomic<unsigned long> matmul_pair_launches{0};
+static std::atomic<unsigned long> matmul_pair_launches{0}, matmul_copied_calls{0};
+unsigned long d8_matmul_grad_copied_calls(void) { return matmul_copied_calls.load(); }
 unsigned long d8_matmul_grad_pair_launches(void) { return matmul_pair_launches.load(); }
 
 int d8_matmul_grad_xy(int dtype, const void *x, void *dx, int xb, int xr, int xc, const void *y, void *dy, int yb, int yr,
@@ -428,6 +429,7 @@ int d8_matmul_grad_xy(int dtype, const void *x, void *dx, int xb, int xr, int xc
         const PackedProduct both[2] = {{&gx, px.ta, px.tb}, {&gy, py.ta, py.tb}};
         size_t used = 0;
         const bool packed = gemm_pack(dtype, both, scratch, scratch_bytes, &used, as_stream(stream), &rc);
+        if (packed) ++matmul_copied_calls;
         if (packed && rc) return rc;
         char *const rest = (char *)scratch + used;
         if (gemm_tiled_run_plain_pair(dtype, gx, px.ta, px.tb, gy, py.ta, py.tb, rest, scratch_bytes - used, as_stream(stream), &rc)) {

@@ -301,6 +301,7 @@ int d8_deconv2d_grad_xy_ex(int dtype, const void *x, void *gx, int B, int IH, in
 unsigned long d8_conv_grad_pair_launches(void);
 unsigned long d8_conv_grad_kept_pair_launches(void);
 unsigned long d8_matmul_grad_pair_launches(void);  /* ... and of the d8_matmul_grad_xy calls */
+unsigned long d8_matmul_grad_copied_calls(void);   /* d8_matmul_grad_xy calls that ran on copies of their odd operands */
 /* How many Conv2d / DeConv2d calls have run (each gradient is one; both gradients from one call are two), by route: 0 on an
  * interim matrix in scratch, 1 with the patches read by the GEMM's loader, 2 on the kernels for images of few channels. */
 unsigned long d8_conv_route_calls(int route);
