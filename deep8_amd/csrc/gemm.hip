@@ -644,12 +644,12 @@ struct PackPlan {
 };
 
 // Whether copies pay: a product then saves some 0.13 us per K step of a 128 x 128 tile and round of the chip where one of its
-// operands is odd and 0.33 where both are, and the two share a launch; the copies take 3 us and 0.4 a MB.  Calls with odd sizes,
-// 500 drawn: 10822 us on the kernels for rows that start anywhere, 9892 on copies always, 10017 with this rule (and fewer that
-// lose: small products, and large matrices copied for few rows or columns); 400 others 8686 and 8037, the better of the two
-// 8008.  4096 rows, 1024 -> 1001: 44.6 -> 38.2 us.  (A product by itself gains too seldom: 600 drawn 6593 us without copies, 7927
-// with, 6442 the better of the two.)
-static bool pack_pays(const PackedProduct (&p)[2], const PackPlan &plan) {
+// operands is odd and 0.33 where both are; the copies take 3 us and 0.4 a MB, of which products that share a launch, which they would not
+// without copies, get the launch back.  600 drawn calls with odd sizes.  401 that share: 11517 us on the kernels for rows that
+// start anywhere, 10253 on copies always, 10268 with this rule, 10132 the better of the two.  199 that do not: 29622, 26101, 25915
+// and 25657; of these and 166 others one lost more than 3 % (4; with the rule of the others 35 of 199, up to 28 %: 913 x 6859 x 177
+// 26.4 -> 36.9).  4096 rows, 1024 -> 1001: 44.6 -> 38.2 us.
+static bool pack_pays(const PackedProduct (&p)[2], const PackPlan &plan, bool shared) {
     const char *force = getenv("D8_GEMM_PACK");  // tuning and test aid (read at every call): 0 never, 1 always
     if (force) return atoi(force) != 0;
     double saved = 0.0;
@@ -660,10 +660,11 @@ static bool pack_pays(const PackedProduct (&p)[2], const PackPlan &plan) {
         const double steps = (double)ceil_div(g.M, 128) * ceil_div(g.N, 128) * g.batch * g.red * ceil_div(g.K, 64) / cu_count();
         saved += (odd == 2 ? 0.33 : odd == 1 ? 0.13 : 0.0) * (steps < 1.0 ? 1.0 : steps);
     }
+    if (!shared) return saved > 3.0 + 0.5e-6 * plan.bytes;
     return saved > 0.2e-6 * plan.bytes;
 }
 
-// (products of one launch, on the tiled kernels)
+// (products on the tiled kernels; false: nothing to copy, or not with these)
 static bool pack_plan(int dtype, const PackedProduct (&p)[2], PackPlan &plan) {
     plan.n = 0, plan.bytes = 0;
     if (dtype != D8_FLOAT16) return false;
@@ -684,46 +685,7 @@ static bool pack_plan(int dtype, const PackedProduct (&p)[2], PackPlan &plan) {
             plan.slot[i][op] = k;
         }
     }
-    return plan.n > 0 && plan.n <= 3 && pack_pays(p, plan);
-}
-
-size_t gemm_pack_bytes(int dtype, const PackedProduct (&p)[2]) {
-    PackPlan plan;
-    return pack_plan(dtype, p, plan) ? plan.bytes : 0;
-}
-
-bool gemm_pack(int dtype, const PackedProduct (&p)[2], void *workspace, size_t workspace_bytes, size_t *used, hipStream_t stream, int *rc) {
-    PackPlan plan;
-    if (!workspace || ((size_t)workspace & 15) || !pack_plan(dtype, p, plan) || plan.bytes > workspace_bytes) return false;
-    PackList L;
-    L.n = plan.n;
-    unsigned blocks = 0;
-    char *to = (char *)workspace;
-    for (int k = 0; k < plan.n; ++k) {
-        const PackShape &s = plan.shapes[k];
-        int across = 8;
-        while (across < 256 && across * 8 < pack_pitch(s)) across *= 2;
-        L.m[k] = {(const f16 *)s.p, (f16 *)to, (int)s.rows, s.cols, s.ld, pack_pitch(s), s.per, s.stride, across, blocks};
-        blocks += (unsigned)ceil_div(s.rows, PACK_ROWS * (256 / across));
-        to += pack_bytes(s);
-    }
-    *used = plan.bytes;
-    hipLaunchKernelGGL(pack_rows_kernel, dim3(blocks), dim3(256), 0, stream, L);
-    const hipError_t e = hipGetLastError();
-    *rc = e == hipSuccess ? 0 : fail((int)e, "kernel launch: %s", hipGetErrorString(e));
-    for (int i = 0; i < 2; ++i) {
-        GemmArgs &g = *p[i].g;
-        if (plan.slot[i][0] >= 0) {
-            const PackArgs &a = L.m[plan.slot[i][0]];
-            g.A = a.dst, g.lda = a.pitch, g.sA = g.sA ? (long)a.per * a.pitch : 0;
-        }
-        if (plan.slot[i][1] >= 0) {
-            const PackArgs &b = L.m[plan.slot[i][1]];
-            g.B = b.dst, g.ldb = b.pitch, g.sB = g.sB ? (long)b.per * b.pitch : 0;
-        }
-        g.packed = 1, g.padM = (g.M + 7) & ~7, g.padN = (g.N + 7) & ~7;
-    }
-    return true;
+    return plan.n > 0 && plan.n <= 3;
 }
 
 // C = beta * C + the g.splits partial sums in g.ws (+ bias, ReLu)
@@ -1091,8 +1053,7 @@ int gemm_tiled_kept_pair_run(int dtype, const GemmArgs &gx, const GemmArgs &gy, 
     return launch_reduce_pair(dtype, gx, gy, stream);
 }
 
-bool gemm_tiled_run_plain_pair(int dtype, GemmArgs &g0, int ta0, int tb0, GemmArgs &g1, int ta1, int tb1, void *workspace,
-                               size_t workspace_bytes, hipStream_t stream, int *rc) {
+static bool plain_pair_plan(int dtype, GemmArgs &g0, int ta0, int tb0, GemmArgs &g1, int ta1, int tb1, void *workspace, size_t workspace_bytes) {
     const bool off = getenv("D8_MATMUL_GRADS_APART") != nullptr;  // tuning and test aid (read at every call)
     if (off || dtype == D8_FLOAT64 || ta0 || !tb0 || !ta1 || tb1) return false;
     if (g0.virt != VIRT_NONE || g1.virt != VIRT_NONE || g0.K < 1 || g1.K < 1) return false;
@@ -1116,11 +1077,85 @@ bool gemm_tiled_run_plain_pair(int dtype, GemmArgs &g0, int ta0, int tb0, GemmAr
     g0.ws = (float *)workspace, g1.ws = (float *)((char *)workspace + need0);
     g0.tail_splits = g1.tail_splits = 0;
     const long wgs = gemm_tiled_plain_pair_workgroups(dtype, g0, g1);
-    if (wgs <= 0 || wgs > 2L * cu_count()) return false;
-    *rc = gemm_tiled_plain_pair_launch(dtype, g0, g1, stream);
-    if (*rc == 0) *rc = launch_reduce_pair(dtype, g0, g1, stream);
+    return wgs > 0 && wgs <= 2L * cu_count();
+}
+
+static int plain_pair_run(int dtype, const GemmArgs &g0, const GemmArgs &g1, hipStream_t stream) {
+    if (int rc = gemm_tiled_plain_pair_launch(dtype, g0, g1, stream)) return rc;
+    return launch_reduce_pair(dtype, g0, g1, stream);
+}
+
+bool gemm_tiled_run_plain_pair(int dtype, GemmArgs &g0, int ta0, int tb0, GemmArgs &g1, int ta1, int tb1, void *workspace,
+                               size_t workspace_bytes, hipStream_t stream, int *rc) {
+    if (!plain_pair_plan(dtype, g0, ta0, tb0, g1, ta1, tb1, workspace, workspace_bytes)) return false;
+    *rc = plain_pair_run(dtype, g0, g1, stream);
     return true;
 }
+
+// The two products on copies, and how: whether they share a launch is known before anything is copied, because copies for products
+// that run one after the other have to save more (pack_pays), and then only those products read them that have something to copy.
+struct PackRun {
+    PackPlan plan;
+    PackList list;
+    unsigned blocks;
+    GemmArgs g[2];
+    bool shared;
+};
+static bool pack_run_plan(int dtype, const PackedProduct (&p)[2], void *workspace, size_t workspace_bytes, PackRun &r) {
+    if (!workspace || ((size_t)workspace & 15) || !pack_plan(dtype, p, r.plan) || r.plan.bytes > workspace_bytes) return false;
+    r.list.n = r.plan.n, r.blocks = 0;
+    char *to = (char *)workspace;
+    for (int k = 0; k < r.plan.n; ++k) {
+        const PackShape &s = r.plan.shapes[k];
+        int across = 8;
+        while (across < 256 && across * 8 < pack_pitch(s)) across *= 2;
+        r.list.m[k] = {(const f16 *)s.p, (f16 *)to, (int)s.rows, s.cols, s.ld, pack_pitch(s), s.per, s.stride, across, r.blocks};
+        r.blocks += (unsigned)ceil_div(s.rows, PACK_ROWS * (256 / across));
+        to += pack_bytes(s);
+    }
+    auto packed = [&](int i) {
+        GemmArgs g = *p[i].g;
+        if (r.plan.slot[i][0] >= 0) {
+            const PackArgs &a = r.list.m[r.plan.slot[i][0]];
+            g.A = a.dst, g.lda = a.pitch, g.sA = g.sA ? (long)a.per * a.pitch : 0;
+        }
+        if (r.plan.slot[i][1] >= 0) {
+            const PackArgs &b = r.list.m[r.plan.slot[i][1]];
+            g.B = b.dst, g.ldb = b.pitch, g.sB = g.sB ? (long)b.per * b.pitch : 0;
+        }
+        g.packed = 1, g.padM = (g.M + 7) & ~7, g.padN = (g.N + 7) & ~7;
+        return g;
+    };
+    r.g[0] = packed(0), r.g[1] = packed(1);
+    const size_t rest = workspace_bytes - r.plan.bytes;
+    r.shared = plain_pair_plan(dtype, r.g[0], p[0].ta, p[0].tb, r.g[1], p[1].ta, p[1].tb, to, rest);
+    if (!pack_pays(p, r.plan, r.shared)) return false;
+    for (int i = 0; i < 2; ++i) {
+        const GemmArgs &g = *p[i].g;  // (not at the cost of the pieces that it would run in without copies)
+        if (d8_gemm_workspace_bytes(dtype, p[i].ta, p[i].tb, g.M, g.N, g.K, g.red > 1 ? g.red : g.batch, g.red > 1 ? 0 : 1) > rest) return false;
+        if (!r.shared) r.g[i] = r.plan.slot[i][0] >= 0 || r.plan.slot[i][1] >= 0 ? packed(i) : g;
+    }
+    return true;
+}
+
+size_t gemm_pack_bytes(int dtype, const PackedProduct (&p)[2]) {
+    PackRun r;
+    return pack_run_plan(dtype, p, (void *)4096, (size_t)1 << 62, r) ? r.plan.bytes : 0;
+}
+
+bool gemm_pack_run(int dtype, const PackedProduct (&p)[2], void *workspace, size_t workspace_bytes, hipStream_t stream, bool *shared, int *rc) {
+    PackRun r;
+    if (!pack_run_plan(dtype, p, workspace, workspace_bytes, r)) return false;
+    *shared = r.shared;
+    hipLaunchKernelGGL(pack_rows_kernel, dim3(r.blocks), dim3(256), 0, stream, r.list);
+    const hipError_t e = hipGetLastError();
+    *rc = e == hipSuccess ? 0 : fail((int)e, "kernel launch: %s", hipGetErrorString(e));
+    if (*rc == 0 && r.shared) *rc = plain_pair_run(dtype, r.g[0], r.g[1], stream);
+    for (int i = 0; i < 2 && !r.shared && *rc == 0; ++i)
+        *rc = gemm_tiled_run(dtype, r.g[i], p[i].ta, p[i].tb, (char *)workspace + r.plan.bytes, workspace_bytes - r.plan.bytes, stream);
+    return true;
+}
+
 
 bool gemm_fuses_store(int dtype, const GemmArgs &g, int transA, int transB, TiledRule rule) {
     // (a product beyond one launch's limits -- more than 448 outputs, more than 65535 * 128 rows -- is cut into several

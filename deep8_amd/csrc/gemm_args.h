@@ -179,14 +179,14 @@ int gemm_f64_splits(int M, int N, int K, int batch, int red, size_t workspace_by
 bool gemm_tiled_half_tiles(int M, int N, int batch, long k_steps, int BK);
 
 // The two gradients of a MatrixMultiply in half whose rows start anywhere: the operands that cannot be moved in 16-byte pieces are
-// copied to rows that can, into the workspace, where that is expected to pay (one launch, a matrix that both read once).
-// On success the products read the copies and *used bytes of the workspace are taken; false, with nothing launched and the
-// products untouched, where it does not pay or the copies do not fit.
+// copied to rows that can, into the workspace, where that is expected to pay (one launch, a matrix that both read once), and
+// the products run on the copies, in one launch (*shared) or one after the other.  False, with nothing launched, where it does not
+// pay or the copies do not fit beside the partial sums.
 struct PackedProduct {
     GemmArgs *g;
     int ta, tb;
 };
-bool gemm_pack(int dtype, const PackedProduct (&p)[2], void *workspace, size_t workspace_bytes, size_t *used, hipStream_t stream, int *rc);
+bool gemm_pack_run(int dtype, const PackedProduct (&p)[2], void *workspace, size_t workspace_bytes, hipStream_t stream, bool *shared, int *rc);
 size_t gemm_pack_bytes(int dtype, const PackedProduct (&p)[2]);  // what it takes of the workspace (0: it does not pay)
 
 // Plan the split of the reduction, launch the tiled kernel (which must be eligible) and reduce.

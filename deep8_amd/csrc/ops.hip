@@ -427,18 +427,15 @@ int d8_matmul_grad_xy(int dtype, const void *x, void *dx, int xb, int xr, int xc
         int rc = 0;
         GemmArgs gx = to_args(px), gy = to_args(py);
         const PackedProduct both[2] = {{&gx, px.ta, px.tb}, {&gy, py.ta, py.tb}};
-        size_t used = 0;
-        const bool packed = gemm_pack(dtype, both, scratch, scratch_bytes, &used, as_stream(stream), &rc);
-        if (packed) ++matmul_copied_calls;
-        if (packed && rc) return rc;
-        char *const rest = (char *)scratch + used;
-        if (gemm_tiled_run_plain_pair(dtype, gx, px.ta, px.tb, gy, py.ta, py.tb, rest, scratch_bytes - used, as_stream(stream), &rc)) {
-            ++matmul_pair_launches;
+        bool shared = false;
+        if (gemm_pack_run(dtype, both, scratch, scratch_bytes, as_stream(stream), &shared, &rc)) {
+            ++matmul_copied_calls;
+            if (shared) ++matmul_pair_launches;
             return rc;
         }
-        if (packed) {
-            if (int e = gemm_tiled_run(dtype, gx, px.ta, px.tb, rest, scratch_bytes - used, as_stream(stream))) return e;
-            return gemm_tiled_run(dtype, gy, py.ta, py.tb, rest, scratch_bytes - used, as_stream(stream));
+        if (gemm_tiled_run_plain_pair(dtype, gx, px.ta, px.tb, gy, py.ta, py.tb, scratch, scratch_bytes, as_stream(stream), &rc)) {
+            ++matmul_pair_launches;
+            return rc;
         }
     }
     if (int rc = run(dtype, px, scratch, scratch_bytes, stream)) return rc;

@@ -61,3 +61,49 @@ def test_gradients(oracle_port, copies, xb, R, I, yb, O, overwrite, before):
             got = f(bufs[i][0].numpy())
             assert np.array_equal(got[before[i]:before[i] + want.size].reshape(want.shape), want), (nb, i)
             assert np.isnan(got[:before[i]]).all() and np.isnan(got[before[i] + want.size:]).all()
+
+
+# R, I, O, forced, copied: products that do not share a launch
+@pytest.mark.parametrize("R,I,O,forced,copied", [(913, 6859, 177, False, 0),    # (copies took it from 26 to 37 us)
+                                                 (6539, 1674, 785, False, 1),
+                                                 (5200, 1301, 1304, True, 1)])  # only the second gradient has an operand to copy
+def test_products_one_after_the_other(monkeypatch, R, I, O, forced, copied):
+    from deep8_amd import capi
+    from deep8_amd.capi import DeviceArray, check
+    lib = capi.init()
+    r = rng(R + I + O)
+    dx, dy, dz = (DeviceArray.from_numpy(t.astype(np.float16)) for t in (ints(r, (R, I), 2), ints(r, (I, O), 2), ints(r, (R, O), 2) * (r.random((R, O)) < 0.25)))
+    left = []
+    for switch in ("1" if forced else None, "0"):
+        if switch is None:
+            monkeypatch.delenv("D8_GEMM_PACK", raising=False)
+        else:
+            monkeypatch.setenv("D8_GEMM_PACK", switch)
+        nb = lib.d8_matmul_scratch_bytes(capi.FLOAT16, 3, 1, R, I, 1, I, O)
+        gx, gy, ws = DeviceArray.from_numpy(np.full((R, I), np.nan, np.float16)), DeviceArray.from_numpy(np.full((I, O), np.nan, np.float16)), DeviceArray((max(nb, 16),), np.uint8)
+        before = lib.d8_matmul_grad_copied_calls(), lib.d8_matmul_grad_pair_launches()
+        check(lib.d8_matmul_grad_xy(capi.FLOAT16, dx.ptr, gx.ptr, 1, R, I, dy.ptr, gy.ptr, 1, I, O, dz.ptr, 3, ws.ptr if nb else None, nb, None))
+        assert (lib.d8_matmul_grad_copied_calls(), lib.d8_matmul_grad_pair_launches()) == (before[0] + (copied if switch != "0" else 0), before[1])
+        left.append((f(gx.numpy()), f(gy.numpy())))
+    assert max(left[1][0].max(), left[1][1].max()) < 2048
+    assert np.array_equal(left[0][0], left[1][0]) and np.array_equal(left[0][1], left[1][1])
+
+
+def test_copies_leave_room_for_the_pieces(monkeypatch):
+    """scratch for the copies alone: the products keep it for their partial sums"""
+    from deep8_amd import capi
+    from deep8_amd.capi import DeviceArray, check
+    lib = capi.init()
+    R, I, O = 2048, 520, 501
+    q = lambda which: lib.d8_matmul_scratch_bytes(capi.FLOAT16, which, 1, R, I, 1, I, O)
+    monkeypatch.setenv("D8_GEMM_PACK", "1")
+    asked, largest = q(3), max(q(1), q(2))
+    monkeypatch.setenv("D8_GEMM_PACK", "0")
+    copies = asked - q(3)
+    assert copies > 0 and largest > 0
+    monkeypatch.setenv("D8_GEMM_PACK", "1")
+    dx, gx, dy, gy, dz, ws = (DeviceArray((n,), np.uint8) for n in (2 * R * I, 2 * R * I, 2 * I * O, 2 * I * O, 2 * R * O, asked))
+    for nb, copied in ((copies, 0), (copies + largest - 16, 0), (copies + largest, 1), (asked, 1)):
+        before = lib.d8_matmul_grad_copied_calls()
+        check(lib.d8_matmul_grad_xy(capi.FLOAT16, dx.ptr, gx.ptr, 1, R, I, dy.ptr, gy.ptr, 1, I, O, dz.ptr, 3, ws.ptr, nb, None))
+        assert lib.d8_matmul_grad_copied_calls() - before == copied, nb
