@@ -645,23 +645,27 @@ struct PackPlan {
 
 // Whether copies pay: a product then saves some 0.13 us per K step of a 128 x 128 tile and round of the chip where one of its
 // operands is odd and 0.33 where both are; the copies take 3 us and 0.4 a MB, of which products that share a launch, which they would not
-// without copies, get the launch back.  600 drawn calls with odd sizes.  401 that share: 11517 us on the kernels for rows that
-// start anywhere, 10253 on copies always, 10268 with this rule, 10132 the better of the two.  199 that do not: 29622, 26101, 25915
-// and 25657; of these and 166 others one lost more than 3 % (4; with the rule of the others 35 of 199, up to 28 %: 913 x 6859 x 177
-// 26.4 -> 36.9).  4096 rows, 1024 -> 1001: 44.6 -> 38.2 us.
+// without copies, get the launch back.  1100 drawn calls with odd sizes, us on the kernels for rows that start anywhere / on copies
+// always / with this rule / with the better of the two, and how many lose more than 3 %:
+//   shared, both have operands to copy   15392 / 13464 / 13648 / 13314, 7 of 509 (with 0.2 a MB 13448, 16; with 0.3 13960, 2)
+//   shared, one has                       5657 /  5245 /  5326 /  5167, none of 226 (by the other line 5267, 22: 66 x 3167 x 528 12.7 -> 16.4)
+//   one after the other                  54096 / 47163 / 46767 / 46322, at most 1 of 365 (0.2 a MB and no launch: 35 of 199, 913 x 6859 x 177 26.4 -> 36.9)
+// 4096 rows, 1024 -> 1001: 44.6 -> 38.2 us.
 static bool pack_pays(const PackedProduct (&p)[2], const PackPlan &plan, bool shared) {
     const char *force = getenv("D8_GEMM_PACK");  // tuning and test aid (read at every call): 0 never, 1 always
     if (force) return atoi(force) != 0;
     double saved = 0.0;
+    bool both = true;
     for (int i = 0; i < 2; ++i) {
         const GemmArgs &g = *p[i].g;
         const int odd = (plan.slot[i][0] >= 0) + (plan.slot[i][1] >= 0), shortest = g.M < g.N ? (g.M < g.K ? g.M : g.K) : (g.N < g.K ? g.N : g.K);
         if (shortest < 64 || (double)g.M * g.N * g.K < (1 << 25)) return false;
         const double steps = (double)ceil_div(g.M, 128) * ceil_div(g.N, 128) * g.batch * g.red * ceil_div(g.K, 64) / cu_count();
+        both = both && odd;
         saved += (odd == 2 ? 0.33 : odd == 1 ? 0.13 : 0.0) * (steps < 1.0 ? 1.0 : steps);
     }
     if (!shared) return saved > 3.0 + 0.5e-6 * plan.bytes;
-    return saved > 0.2e-6 * plan.bytes;
+    return both ? saved > 0.25e-6 * plan.bytes : saved > 0.3 + 0.15e-6 * plan.bytes;
 }
 
 // (products on the tiled kernels; false: nothing to copy, or not with these)

@@ -66,7 +66,8 @@ def test_gradients(oracle_port, copies, xb, R, I, yb, O, overwrite, before):
 # R, I, O, forced, copied: products that do not share a launch
 @pytest.mark.parametrize("R,I,O,forced,copied", [(913, 6859, 177, False, 0),    # (copies took it from 26 to 37 us)
                                                  (6539, 1674, 785, False, 1),
-                                                 (5200, 1301, 1304, True, 1)])  # only the second gradient has an operand to copy
+                                                 (5200, 1301, 1304, True, 1),   # only the second gradient has an operand to copy
+                                                 (66, 3167, 528, False, 0)])    # (likewise; copies in one launch: from 13 to 16 us)
 def test_products_one_after_the_other(monkeypatch, R, I, O, forced, copied):
     from deep8_amd import capi
     from deep8_amd.capi import DeviceArray, check
