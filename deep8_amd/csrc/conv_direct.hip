@@ -125,33 +125,18 @@ __device__ __forceinline__ unsigned first_mask(int n, int d) {
 
 // G: k groups (pairs of pieces) a wave keeps of the filter; NB: blocks of 32 channels per workgroup; ODD: half patches may
 // start in the middle of a dword.  A workgroup walks every gridDim.x-th tile, its four waves every fourth block of 32 pixels.
-// The next tile's image rows (the first's: while the filter is laid out) are fetched into registers while the present one is
-// multiplied, where they move in 16-byte pieces and fit.  A block of z is turned around through a patch of LDS of the wave's
-// own, so that consecutive lanes store the consecutive 16-byte chunks of a pixel: whole lines of 128 bytes for 64 channels in
-// half.  Figures at conv_direct_forward.
+// Bound by the store of z and the latency of a tile's image rows, which two workgroups and more per compute unit hide from each
+// other; figures at conv_direct_forward.
 template <typename E, int G, int NB, bool ODD>
 __global__ __launch_bounds__(256, 2) void conv_direct_forward_kernel(DirectArgs a) {
     typedef Elem<E> EL;
     typedef typename EL::Frag Frag;
-    constexpr int EPV = 16 / sizeof(E), IMG_AHEAD = 4, CP = NB * 32 / EPV;  // CP: 16-byte chunks a pixel's channels take
+    constexpr int EPV = 16 / sizeof(E);
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_bytes[];
     __shared__ __attribute__((aligned(16))) float bias_s[NB * 32];
-    __shared__ __attribute__((aligned(16))) u32x4 turned[4][32 * CP];  // chunk c of pixel p at p * CP + (c ^ p % CP)
     E *lds = (E *)lds_bytes;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, half = lane >> 5;
     const int oc0 = blockIdx.y * (NB * 32), ocs = min(NB * 32, a.s.OC - oc0);
-    const int img_total = a.rows * (a.pitch / EPV);
-    const bool ahead = a.vec_x == EPV && img_total <= IMG_AHEAD * 256;
-    u32x4 ri[IMG_AHEAD];
-    auto fetch = [&](const TileAt &t) {
-#pragma unroll
-        for (int u = 0; u < IMG_AHEAD; ++u) {
-            int dst;
-            ri[u] = image_piece<E, u32x4>(a, t, threadIdx.x + u * 256, img_total, dst);
-        }
-    };
-    TileAt at = tile_at(a, blockIdx.x);  // (the grid has no more workgroups than there are tiles)
-    if (ahead) fetch(at);
 
     // ---- the filter: through LDS (rows of K elements, as they lie in memory) into fragments; rows past OC and pieces past
     // the last run are zeros
@@ -159,7 +144,7 @@ __global__ __launch_bounds__(256, 2) void conv_direct_forward_kernel(DirectArgs 
         const E *w = (const E *)a.w + (long)oc0 * a.K;
         const int n = ocs * a.K;
         if (((size_t)w & 15) == 0) {
-            constexpr int LOADS = 5;  // in flight at a time
+            constexpr int LOADS = 5;  // in flight at a time: all that a thread loads of 64 x 7x7x3 in half
             for (int i = threadIdx.x * EPV; i + EPV <= n; i += LOADS * 256 * EPV) {
                 u32x4 v[LOADS];
 #pragma unroll
@@ -211,34 +196,22 @@ __global__ __launch_bounds__(256, 2) void conv_direct_forward_kernel(DirectArgs 
     const int blocks = (a.TR * a.TC + 31) / 32;
     const bool vec = a.s.OC % EPV == 0 && ((size_t)a.z & 15) == 0;
     for (int t = blockIdx.x; t < a.ntiles; t += gridDim.x) {
+        const TileAt at = tile_at(a, t);
         __syncthreads();  // the filter's fragments have been read; every wave is done with the tile before
-        if (ahead) {
-#pragma unroll
-            for (int u = 0; u < IMG_AHEAD; ++u) {
-                const int i = threadIdx.x + u * 256, per_row = a.pitch / EPV, r = quotient(i, a.mg_chunks, per_row);
-                if (i < img_total) *(u32x4 *)(lds + r * a.pitch + (i - r * per_row) * EPV) = ri[u];
-            }
-        } else {
-            stage_image<E>(a, at, lds);
-        }
+        stage_image<E>(a, at, lds);
         __syncthreads();
-        const TileAt here = at;
-        if (t + (int)gridDim.x < a.ntiles) {
-            at = tile_at(a, t + gridDim.x);
-            if (ahead) fetch(at);
-        }
-        E *const z0 = (E *)a.z + (((long)here.b * a.s.OH + here.oy0) * a.s.OW + here.ox0) * a.s.OC + oc0;
-        const int rows_here = min(a.TR, a.s.OH - here.oy0), cols_here = min(a.TC, a.s.OW - here.ox0);
+        E *const z0 = (E *)a.z + (((long)at.b * a.s.OH + at.oy0) * a.s.OW + at.ox0) * a.s.OC + oc0;
+        const int rows_here = min(a.TR, a.s.OH - at.oy0), cols_here = min(a.TC, a.s.OW - at.ox0);
         for (int blk = wave; blk < blocks; blk += 4) {
             const int q = blk * 32 + l32, qc = min(q, a.TR * a.TC - 1), r = quotient(qc, a.mg_tc, a.TC), c = qc - r * a.TC;
-            const int base = r * a.s.sy * a.pitch + c * a.s.sx * a.s.C + here.skip;
+            const int base = r * a.s.sy * a.pitch + c * a.s.sx * a.s.C + at.skip;
             f32x16 acc[NB];
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) acc[nb][i] = 0.f;
-            // (masks built again for every block: hoisted, the four of each group take more registers than the filter leaves)
-            asm volatile("" : "+v"(some), "+v"(all));
+            // (masks built again for every block: hoisted, the four of each group take more registers than a long filter leaves)
+            if constexpr (G * NB > 11) asm volatile("" : "+v"(some), "+v"(all));
 #pragma unroll
             for (int g = 0; g < G; ++g) {
                 u32x4 v = piece_at<E, ODD>(lds, base + koff[g]);
@@ -252,13 +225,15 @@ __global__ __launch_bounds__(256, 2) void conv_direct_forward_kernel(DirectArgs 
             }
             // this lane's pixel, counted from the tile's first; -1: not one of z
             const int px = q < a.TR * a.TC && r < rows_here && c < cols_here ? r * a.s.OW + c : -1;
+            E *const z = z0 + (long)px * a.s.OC;
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
                 // register i of the block is channel 8 * (i / 4) + 4 * half + i % 4 of this lane's pixel
                 E o[16];
                 f32x4 bias[4];
+                if (a.bias)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) bias[i] = *(const f32x4 *)(bias_s + nb * 32 + 8 * i + 4 * half);
+                    for (int i = 0; i < 4; ++i) bias[i] = *(const f32x4 *)(bias_s + nb * 32 + 8 * i + 4 * half);
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
                     float v = acc[nb][i];
@@ -269,8 +244,8 @@ __global__ __launch_bounds__(256, 2) void conv_direct_forward_kernel(DirectArgs 
                     if constexpr (sizeof(E) == 4) {
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
-                            const f32x4 out = {(float)o[4 * i], (float)o[4 * i + 1], (float)o[4 * i + 2], (float)o[4 * i + 3]};
-                            turned[wave][l32 * CP + ((nb * 8 + 2 * i + half) ^ (l32 % CP))] = __builtin_bit_cast(u32x4, out);
+                            const int n = nb * 32 + 8 * i + 4 * half;
+                            if (px >= 0 && n < ocs) *(f32x4 *)(z + n) = (f32x4){(float)o[4 * i], (float)o[4 * i + 1], (float)o[4 * i + 2], (float)o[4 * i + 3]};
                         }
                     } else {
                         // the lower half of the wave takes channels 16 i .. + 7 of its pixel, the upper 16 i + 8 .. + 15
@@ -283,24 +258,16 @@ __global__ __launch_bounds__(256, 2) void conv_direct_forward_kernel(DirectArgs 
                                 const auto s = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, lo), __builtin_bit_cast(unsigned, hi), false, false);
                                 out[d] = s[0], out[d + 2] = s[1];
                             }
-                            turned[wave][l32 * CP + ((nb * 4 + 2 * i + half) ^ (l32 % CP))] = out;
+                            const int n = nb * 32 + 16 * i + 8 * half;
+                            if (px >= 0 && n < ocs) *(u32x4 *)(z + n) = out;
                         }
                     }
                 } else if (px >= 0) {
 #pragma unroll
                     for (int i = 0; i < 16; ++i) {
                         const int n = nb * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
-                        if (n < ocs) z0[(long)px * a.s.OC + n] = o[i];
+                        if (n < ocs) z[n] = o[i];
                     }
-                }
-            }
-            if (vec) {  // (a wave's LDS accesses are in order: its patch needs no barrier)
-#pragma unroll
-                for (int u = 0; u < CP / 2; ++u) {
-                    const int p = (u * 64 + lane) / CP, ch = lane % CP;
-                    const u32x4 out = turned[wave][p * CP + (ch ^ (p % CP))];
-                    const int to = __shfl(px, p, 64);
-                    if (to >= 0 && ch * EPV < ocs) *(u32x4 *)(z0 + (long)to * a.s.OC + ch * EPV) = out;
                 }
             }
         }
@@ -578,7 +545,8 @@ bool conv_direct_eligible(int dtype, const DirectShape &s) {
 }
 
 // What the kernels take, fitted to 4776 calls on 2500 drawn layers (1 - 170 channels to 8 - 512, both types; half of the calls
-// within 7 % of the estimate, nine tenths of the forward ones within 20 %).  Forward: the filter's way into registers, a
+// within 7 % of the estimate, nine tenths of the forward ones within 20 %), before the forward kernel's last changes, which
+// took 4 % off it, 13 % with a bias: the patch matrix keeps a few layers that it would now be faster on.  Forward: the filter's way into registers, a
 // tile's accesses to the image, a wave's blocks of 32 pixels (products and stores); the image's fragments are built again for
 // every 64 (fp32: 32) output channels.
 double conv_direct_forward_us(int dtype, const DirectShape &s, const void *x) {
@@ -630,9 +598,14 @@ double conv_direct_grad_us(int dtype, const DirectShape &s, const void *x, const
 // Half 16 x
 // 224x224x3 -> 64, 7x7 stride 2 (K = 147): patch matrix + padded filter + product 81 -> 23 us (26 MB are stored: 5 us at a
 // copy's rate; what the rest goes on is the filter's fragments and a block's chain of LDS reads, products and stores); fp32 64 x 28x28x1 -> 32,
-// 5x5: patch matrix + product 18 -> 11 us, and
-// 22.1 -> 20.1 and 8.0 -> 7.5 us with image rows fetched ahead, masks that are not kept for every group (two
-// workgroups per compute unit need at most 256 registers; 295 gave 29.8 us) and z stored in whole lines.
+// 5x5: patch matrix + product 18 -> 11 us.
+// Now 19.7 and 7.3 us: the bias is read four values at a time, the filter's loads are in flight together, and masks are not kept for
+// every group where the filter is long (two workgroups per compute unit need at most 256 registers; 295 gave 29.8 us).  A
+// block of z is stored from registers, 16 bytes a lane: turned around through LDS for whole lines it took 21.2 and 7.5 us, and the
+// LDS (8 - 16 KB) and registers kept workgroups off the compute unit (fp32 32 x 311x311x4 -> 64, 5x5 stride 4, 113 us, now 88).  Image
+// rows of the next tile fetched into registers gave nothing beside several workgroups.  248 drawn layers, all three against
+// none: with bias and ReLu 3142 us, now 2901; without 3098 us (125 layers more than 3 % slower than when z was not
+// turned around), now 2853 (one).
 int conv_direct_forward(int dtype, const DirectShape &s, const void *x, const void *w, void *z, const void *bias, int relu,
                         int round_first, hipStream_t stream) {
     DirectArgs a;

@@ -42,3 +42,14 @@ def test_two_workgroups_of_the_tiled_kernels_fit_a_compute_unit():
     assert any("gemm_tiled_pair_kernel" in n for n in found) and len(found) > 100
     over = {n: k[".vgpr_count"] for n, k in found.items() if k[".vgpr_count"] > 256 or k[".vgpr_spill_count"]}
     assert not over
+
+
+def test_two_workgroups_on_images_of_few_channels_fit_a_compute_unit():
+    """up to 64 KB of image rows a tile are asked for at the launch; the kernel's own arrays must leave them to two workgroups"""
+    with open(capi.LIB_PATH, "rb") as f:
+        blob = f.read()
+    found = {k[".name"]: k for at in _code_objects(blob) for k in _kernels(blob, at) if "conv_direct_forward_kernel" in k[".name"]}
+    if not found:
+        pytest.skip("the library's code objects are compressed")
+    assert not {n: k[".group_segment_fixed_size"] for n, k in found.items() if 2 * (k[".group_segment_fixed_size"] + 64 * 1024) > 160 * 1024}
+    assert not {n: k[".vgpr_count"] for n, k in found.items() if k[".vgpr_count"] > 256 or k[".vgpr_spill_count"]}
