@@ -1046,31 +1046,36 @@ __global__ __launch_bounds__(T0::NT, T0::TWO_FIT && T1::TWO_FIT ? 2 : 1) void ge
     }
 }
 
-// The kernel tile of a BM x BN output tile: in half, operands in whole pieces go straight into LDS.  Four waves, and as many
-// stages as let two workgroups share a compute unit.  DEEP: 128 x 128 tiles of a launch of at most one workgroup per compute unit,
+// The kernel tile of a BM x BN output tile: in half, operands in whole pieces go straight into LDS, on four waves and as many
+// stages as let FIT workgroups share a compute unit.
+// FIT 1: 128 x 128 tiles of a launch of at most one workgroup per compute unit,
 // which may have all of its LDS: two stages fetch one step ahead, less than the way from memory takes (2048^3, a K step of 128 x
 // 128: 1270 cycles with two stages, 825 - 870 with four; with five the same), and eight waves share out the addresses of
 // patch rows (Conv2d 16 x 57x57x96 -> 160, 3x3 stride 2, forward 17.1 us with four waves, 15.3 with eight).  More stages or
 // eight waves on the smaller tiles gave nothing (64 x 64 with 4, 6, 8 stages 454, 516, 522 cycles a step, with eight waves 520).
-template <typename E, int BM, int BN, bool A_KC, bool B_KC, int VIRT = VIRT_NONE, bool DEEP = false>
+// FIT 3: smaller tiles of a launch of more than two workgroups per compute unit.  Two stages let three in (64 x 64: four), which
+// hide each other's prologue and store and need no further
+// round.  100 drawn half Conv2d of 8 to 100 channels, forward, 1286 -> 1244 us (1360 on tiles that pass through registers, of which
+// none is lost by 3 % any more): 29 x 55x55x16 -> 42 1x1 12.1 -> 9.3, DeConv2d 23 x 18x18x8 -> 72 4x4 stride 2 12.4 -> 9.8.
+template <typename E, int BM, int BN, bool A_KC, bool B_KC, int VIRT = VIRT_NONE, int FIT = 2>
 struct TileOf {
     typedef Tile<E, BM, BN, BM == 256 || BN == 32 ? 4 : 2, BN == 32 ? 1 : 2, A_KC, B_KC, VIRT> type;
 };
-template <bool A_KC, bool B_KC, int VIRT>
-struct TileOf<f16, 64, 64, A_KC, B_KC, VIRT> {
-    typedef DmaTile<64, 64, 2, 2, 4, A_KC, B_KC, VIRT> type;
+template <bool A_KC, bool B_KC, int VIRT, int FIT>
+struct TileOf<f16, 64, 64, A_KC, B_KC, VIRT, FIT> {
+    typedef DmaTile<64, 64, 2, 2, FIT == 3 ? 2 : 4, A_KC, B_KC, VIRT> type;
 };
-template <bool A_KC, bool B_KC, int VIRT>
-struct TileOf<f16, 64, 128, A_KC, B_KC, VIRT> {
-    typedef DmaTile<64, 128, 2, 2, 3, A_KC, B_KC, VIRT> type;
+template <bool A_KC, bool B_KC, int VIRT, int FIT>
+struct TileOf<f16, 64, 128, A_KC, B_KC, VIRT, FIT> {
+    typedef DmaTile<64, 128, 2, 2, FIT == 3 ? 2 : 3, A_KC, B_KC, VIRT> type;
 };
-template <bool A_KC, bool B_KC, int VIRT>
-struct TileOf<f16, 128, 64, A_KC, B_KC, VIRT> {
-    typedef DmaTile<128, 64, 2, 2, 3, A_KC, B_KC, VIRT> type;
+template <bool A_KC, bool B_KC, int VIRT, int FIT>
+struct TileOf<f16, 128, 64, A_KC, B_KC, VIRT, FIT> {
+    typedef DmaTile<128, 64, 2, 2, FIT == 3 ? 2 : 3, A_KC, B_KC, VIRT> type;
 };
-template <bool A_KC, bool B_KC, int VIRT, bool DEEP>
-struct TileOf<f16, 128, 128, A_KC, B_KC, VIRT, DEEP> {
-    typedef DmaTile<128, 128, 2, DEEP ? 4 : 2, DEEP ? 4 : 2, A_KC, B_KC, VIRT> type;
+template <bool A_KC, bool B_KC, int VIRT, int FIT>
+struct TileOf<f16, 128, 128, A_KC, B_KC, VIRT, FIT> {
+    typedef DmaTile<128, 128, 2, FIT == 1 ? 4 : 2, FIT == 1 ? 4 : 2, A_KC, B_KC, VIRT> type;
 };
 
 // where d8_gemm_phase_record asked the next launches to write their records (process-wide; null: no records; defined in

@@ -47,9 +47,14 @@ template <typename E, int BM, int BN, bool A_KC, bool B_KC, int VIRT>
 static int launch_tiled(const GemmArgs &g, hipStream_t stream, bool any = false) {
     if constexpr (VIRT == VIRT_NONE && BM <= 128)  // rows that start anywhere: shifted into place between memory and LDS
         if (any) return launch_edge<Tile<E, BM, BN, BN == 32 ? 4 : 2, BN == 32 ? 1 : 2, A_KC, B_KC, VIRT>, EDGE_ANY>(g, stream);
-    if constexpr (sizeof(E) == 2 && BM == 128 && BN == 128) {
+    if constexpr (sizeof(E) == 2 && BM <= 128) {
         const long wgs = (long)ceil_div(g.M, BM) * ceil_div(g.N, BN) * (VIRT == VIRT_A_CLASSES ? g.ncls : g.batch * g.splits);
-        if (wgs <= cu_count()) return launch_whole<typename TileOf<E, BM, BN, A_KC, B_KC, VIRT, true>::type>(g, stream);
+        if constexpr (BM == 128 && BN == 128) {
+            if (wgs <= cu_count()) return launch_whole<typename TileOf<E, BM, BN, A_KC, B_KC, VIRT, 1>::type>(g, stream);
+        } else if constexpr (A_KC) {  // (other reductions run over rows or pixels: seldom of few steps, and cut into pieces for the chip)
+            typedef typename TileOf<E, BM, BN, A_KC, B_KC, VIRT, 3>::type T;
+            if (wgs > 2L * cu_count() && !g.packed) return g.K % T::BK ? launch_edge<T, EDGE_PIECES>(g, stream) : launch_edge<T, EDGE_NONE>(g, stream);
+        }
     }
     return launch_whole<typename TileOf<E, BM, BN, A_KC, B_KC, VIRT>::type>(g, stream);
 }
