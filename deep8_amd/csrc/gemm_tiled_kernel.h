@@ -580,11 +580,20 @@ __device__ __forceinline__ void dma_loop(f16 *lds, int wave, int lane, int wm, i
 // Division of many 0 <= n < 2^31 by one uniform d: floor((2^32 - 1) / d) is taken once, and n times that over 2^32 is the quotient
 // or one less.  Half a dozen instructions instead of some 35 each for the patch operands' eight divisions a thread: Conv2d
 // 32 x 14x14x256 3x3 half, forward and gradients, 54.4 -> 54.2 us, fp32 1 x 28x28x128 forward 10.50 -> 10.45.
+// DIVIDE: the quotients are divided out.  DeConv2d's forward kernels are faster so, fp32 25 x 37x37x64 -> 51 3x3 stride 2 54.2
+// us instead of 58.3, half 20 x 4x4x192 -> 69 4x4 stride 2 16.2 instead of 17.4 (found by measuring: both ways have the same
+// workgroups a compute unit, and spill nothing); the gradients on classes, which would hold more than 256 registers, are not.
+template <bool DIVIDE>
 struct Divisor {
     int d;
     unsigned m;
     __device__ __forceinline__ explicit Divisor(int by) : d(by), m(0xffffffffu / (unsigned)by) {}
     __device__ __forceinline__ int div(int n, int &rem) const {
+        if constexpr (DIVIDE) {
+            const int q = n / d;
+            rem = n - q * d;
+            return q;
+        }
         int q = (int)__umulhi((unsigned)n, m);
         rem = n - q * d;
         const bool more = rem >= d;
@@ -737,7 +746,7 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     // patch rows as A: this thread's rows never change; a step selects the tap
     int va_base[A_IT], va_iy[A_IT], va_ix[A_IT];
     if constexpr (VA) {
-        const Divisor plane(pg.OH * pg.OW), width(pg.OW);
+        const Divisor<VIRT == VIRT_A_CLASSES && B_KC> plane(pg.OH * pg.OW), width(pg.OW);
 #pragma unroll
         for (int p = 0; p < A_IT; ++p) {
             int rem, ox;
@@ -760,7 +769,7 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     if constexpr (VIRT == VIRT_B_KROWS) {
         int cy = -pg.pt, cx = -pg.pl, cc = 0;  // what the tap and channel add to an output pixel's source coordinates
         if constexpr (T::B_COLS) {
-            const Divisor channels(pg.C), taps(pg.FW);
+            const Divisor<false> channels(pg.C), taps(pg.FW);
 #pragma unroll
             for (int p = 0; p < B_IT; ++p) {
                 int c, fx;
@@ -776,7 +785,7 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
             cx += fx * pg.dx;
         }
         vb_y_end = pg.OH * pg.sy + cy, vb_x_end = pg.OW * pg.sx + cx;
-        const Divisor plane(pg.OH * pg.OW), width(pg.OW);
+        const Divisor<false> plane(pg.OH * pg.OW), width(pg.OW);
 #pragma unroll
         for (int p = 0; p < VB_N; ++p) {
             int rem, ox;
