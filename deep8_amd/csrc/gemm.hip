@@ -806,11 +806,12 @@ size_t gemm_tiled_workspace(int dtype, int M, int N, int K, int red, int virt) {
 }
 
 // 64 x 64 tiles where the 128-wide ones leave compute units idle.  In fp32, whose K step is bound by the matrix pipe, a step of
-// theirs is a quarter of the work; in half, whose step waits longer than it multiplies, half of it (0.25 us against 0.38 for a
-// 64 x 128 tile and 0.46 for 128 x 128).  The same pieces -- or none, and no second pass -- spread over four times as many
+// theirs is a quarter of the work; in half, whose step waits longer than it multiplies, half of it (through registers 0.25 us against
+// 0.38 for a 64 x 128 tile and 0.46 for 128 x 128).  The same pieces -- or none, and no second pass -- spread over four times as many
 // workgroups.  The estimate counts steps of a 128 x 128 tile (about 2 us of a CU in fp32, 0.5 us in half), for the plan that g
-// holds (splits set) and for 64 x 64 tiles in 1 .. as many pieces as that plan; 7 % or more decide.  It was fitted anew, to the
-// kernels as they are: a 64 x 128 half step is 0.76 here and 0.65 in plan_few_tiles, a half product's second pass 6.5 steps + 1
+// holds (splits set) and for 64 x 64 tiles in 1 .. as many pieces as that plan; 7 % or more decide.  It was fitted to half tiles
+// that pass through registers: straight into LDS the steps take 454, 620 and 1270 cycles (870 with four stages), i.e. 0.36 : 0.49 : 1
+// where 0.5 : 0.76 : 1 is counted, and the plans are still those of then.  A 64 x 128 half step is 0.76 here and 0.65 in plan_few_tiles, a half product's second pass 6.5 steps + 1
 // per 0.25e6 outputs and piece here, 14 + 1 per 0.5e6 there, which only chooses among 128-wide tiles.
 // A narrow output (128 x 32 tiles, below) counts its pieces the same way.
 // NN, us before and after (M x K x N; NT and TN alike): fp32 512 x 512 x 512 16.4 -> 10.2, 784 x 1152 x 128 16.0 -> 10.3,
@@ -866,7 +867,8 @@ static bool narrow_output(int dtype, const GemmArgs &g) {
 }
 
 // What the planners above count for the plan that they make, in microseconds.  (Over 3100 calls on drawn layers the time
-// measured was 1.0 - 1.2 of this at the median in fp32, 1.1 - 1.5 in half, for products and patch products alike.)
+// measured was 1.0 - 1.2 of this at the median in fp32, 1.1 - 1.5 in half, for products and patch products alike, before half
+// tiles went straight into LDS.)
 double gemm_estimate_us(int dtype, const GemmArgs &g0, int transA, int transB) {
     const bool half_elems = dtype == D8_FLOAT16;
     const int BK = gemm_tiled_k_step(dtype);
@@ -1021,7 +1023,8 @@ bool gemm_tiled_run_pair(int dtype, GemmArgs &gx, GemmArgs &gy, void *workspace,
     return true;
 }
 
-// The gradients of a Conv2d with a stride in half: the classes' workgroups are short (1 to 4 taps of a 3 x 3 filter) and rarely a
+// Both gradients of a convolution in one launch, in half and fp32, on classes of output pixels or on patch rows.
+// A Conv2d with a stride in half: the classes' workgroups are short (1 to 4 taps of a 3 x 3 filter) and rarely a
 // whole number of rounds, and the filter gradient's fill the last one.
 // 16 x 57x57x96 -> 160, 3x3 stride 2: both gradients 38.4 -> 31.8 us; 60 drawn layers 1810 -> 1539 us, none slower.
 // Patch rows whose last K step is cut short, or that are cut into pieces: a launch or two fewer, and no half empty chip behind the

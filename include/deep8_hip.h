@@ -173,8 +173,9 @@ int d8_matmul_grad_y_overwrite(int dtype, const void *x, int xb, int xr, int xc,
  * to a tile of dy; everything else is d8_matmul_grad_x followed by d8_matmul_grad_y.  The results are bit for bit
  * those of the two calls.  overwrite: bit 0 -- dx is written instead of added to, bit 1 -- dy likewise (the
  * _overwrite forms above).  scratch: d8_matmul_scratch_bytes(which = 3), room for both gradients' scratch side by
- * side; with less, but at least the larger of which = 1 and which = 2, the call still works (mid-size products
- * then run as two launches).  Two small products (each at most four 128 x 128 tiles over a reduction of at most
+ * side and, in Float16, for copies of the operands whose rows do not start at multiples of 16 bytes, where copies
+ * pay; with less, but at least the larger of which = 1 and which = 2, the call still works (mid-size products
+ * then run as two launches, and such operands are read as they lie, which takes longer).  Two small products (each at most four 128 x 128 tiles over a reduction of at most
  * 512) share a launch as well, and so do two mid-size ones whose workgroups all fit the chip at once.          */
 int d8_matmul_grad_xy(int dtype, const void *x, void *dx, int xb, int xr, int xc,
                       const void *y, void *dy, int yb, int yr, int yc, const void *dz, int overwrite,
