@@ -258,7 +258,8 @@ static bool conv_implicit_plan(int dtype, int which, const ConvShape &c, const v
 static int gcd_of(int a, int b) { return b ? gcd_of(b, a % b) : a; }
 
 // The classes with the most taps first: launched last, their workgroups would be the chip's last wave (3x3 stride 2: 1, 2, 2 and 4
-// taps in the order of the pixels).
+// taps in the order of the pixels).  DeConv2d's forward pass, whose classes are more alike, keeps the order of the pixels: 238 drawn
+// layers 5007 us so, 5008 by taps, with fp32 7 x 23x23x64 -> 112 4x4 stride 3 21.7 and 23.2.
 static void longest_first(GemmArgs &g) {
     std::stable_sort(g.cls, g.cls + g.ncls, [](const OutClass &a, const OutClass &b) { return a.red > b.red; });
 }
@@ -814,7 +815,6 @@ static bool deconv_implicit_fwd(int dtype, int B, int IH, int IW, int IC, int OC
             most_taps = c.red > most_taps ? c.red : most_taps;
         }
     if (g.ncls == 0) return false;
-    longest_first(g);
     g.tiles_per_split = most_taps * (IC / (dtype == D8_FLOAT64 ? 16 : gemm_tiled_k_step(dtype)) + 1);  // never the limit: a class walks all its taps
     g.M = smallest;
     const bool ok = implicit_eligible(dtype, g, 0, 1);
