@@ -645,10 +645,11 @@ struct PackPlan {
 
 // Whether copies pay: a product then saves some 0.13 us per K step of a 128 x 128 tile and round of the chip where one of its
 // operands is odd and 0.33 where both are; the copies take 3 us and 0.4 a MB, of which products that share a launch, which they would not
-// without copies, get the launch back.  1100 drawn calls with odd sizes, us on the kernels for rows that start anywhere / on copies
+// without copies, get the launch back.  1250 drawn calls with odd sizes, us on the kernels for rows that start anywhere / on copies
 // always / with this rule / with the better of the two, and how many lose more than 3 %:
-//   shared, both have operands to copy   15392 / 13464 / 13648 / 13314, 7 of 509 (with 0.2 a MB 13448, 16; with 0.3 13960, 2)
-//   shared, one has                       5657 /  5245 /  5326 /  5167, none of 226 (by the other line 5267, 22: 66 x 3167 x 528 12.7 -> 16.4)
+//   shared, both have operands to copy   15910 / 13579 / 13730 / 13475, 9 of 562 (with 0.25 a MB 14010, 5)
+//   shared, x alone                       7359 /  6896 /  6933 /  6754, 18 of 325 (by the line of the others 6946, 29; with 0.3 and 0.15 a MB throughout
+//                                         7048, 2: of more than 1700 columns x leaves both products many tiles, and less to gain from one launch)
 //   one after the other                  54096 / 47163 / 46767 / 46322, at most 1 of 365 (0.2 a MB and no launch: 35 of 199, 913 x 6859 x 177 26.4 -> 36.9)
 // 4096 rows, 1024 -> 1001: 44.6 -> 38.2 us.
 static bool pack_pays(const PackedProduct (&p)[2], const PackPlan &plan, bool shared) {
@@ -665,7 +666,7 @@ static bool pack_pays(const PackedProduct (&p)[2], const PackPlan &plan, bool sh
         saved += (odd == 2 ? 0.33 : odd == 1 ? 0.13 : 0.0) * (steps < 1.0 ? 1.0 : steps);
     }
     if (!shared) return saved > 3.0 + 0.5e-6 * plan.bytes;
-    return both ? saved > 0.25e-6 * plan.bytes : saved > 0.3 + 0.15e-6 * plan.bytes;
+    return both || p[0].g->N <= 1700 ? saved > 0.2e-6 * plan.bytes : saved > 0.3 + 0.15e-6 * plan.bytes;
 }
 
 // (products on the tiled kernels; false: nothing to copy, or not with these)
