@@ -383,14 +383,17 @@ struct RowMap {
     int plane, OW;                           // 0: identity
     int out_H, out_W, out_sy, out_sx, py, px;
     int perm_T, perm_OC;                     // perm_OC > 0: stored transposed per tap (GemmArgs::perm_OC)
+    unsigned by_plane, by_ow, by_perm;       // reciprocals of plane, OW, perm_OC
     __device__ long operator()(int m) const {
         if (!plane) return m;
-        const int img = m / plane, rem = m - img * plane, y = rem / OW, x = rem - y * OW;
+        int rem, x;
+        const int img = Divisor(plane, by_plane).div(m, rem), y = Divisor(OW, by_ow).div(rem, x);
         return ((long)img * out_H + out_sy * y + py) * out_W + out_sx * x + px;
     }
     __device__ long at(int m, int n, int ldc) const {
         if (perm_OC) {
-            const int t = n / perm_OC, oc = n - t * perm_OC;
+            int oc;
+            const int t = Divisor(perm_OC, by_perm).div(n, oc);
             return ((long)oc * perm_T + t) * ldc + m;
         }
         return (*this)(m) * ldc + n;
@@ -578,31 +581,6 @@ __device__ __forceinline__ void dma_loop(f16 *lds, int wave, int lane, int wm, i
     wait_loads_and_lds<0>();  // (nothing lands in LDS any more: the epilogue uses it)
 }
 
-// Division of many 0 <= n < 2^31 by one uniform d: floor((2^32 - 1) / d) is taken once, and n times that over 2^32 is the quotient
-// or one less.  Half a dozen instructions instead of some 35 each for the patch operands' eight divisions a thread: Conv2d
-// 32 x 14x14x256 3x3 half, forward and gradients, 54.4 -> 54.2 us, fp32 1 x 28x28x128 forward 10.50 -> 10.45.
-// DIVIDE: the quotients are divided out.  DeConv2d's forward kernels are faster so, fp32 25 x 37x37x64 -> 51 3x3 stride 2 54.2
-// us instead of 58.3, half 20 x 4x4x192 -> 69 4x4 stride 2 16.2 instead of 17.4 (found by measuring: both ways have the same
-// workgroups a compute unit, and spill nothing); the gradients on classes, which would hold more than 256 registers, are not.
-template <bool DIVIDE>
-struct Divisor {
-    int d;
-    unsigned m;
-    __device__ __forceinline__ explicit Divisor(int by) : d(by), m(0xffffffffu / (unsigned)by) {}
-    __device__ __forceinline__ int div(int n, int &rem) const {
-        if constexpr (DIVIDE) {
-            const int q = n / d;
-            rem = n - q * d;
-            return q;
-        }
-        int q = (int)__umulhi((unsigned)n, m);
-        rem = n - q * d;
-        const bool more = rem >= d;
-        rem -= more ? d : 0;
-        return q + (more ? 1 : 0);
-    }
-};
-
 // A value that is the same for all lanes, in a scalar register (DmaTile).  The compiler keeps the quotients of integer divisions
 // and what it computes from them in vector registers, and would read a load's offset from there right before dma_piece: a load wants
 // five wait states behind a vector instruction that writes a scalar it takes, which the compiler keeps before loads of its own
@@ -644,28 +622,30 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     PatchGeom pg = g.pg;
     int M = g.M, red = g.red;
     unsigned b_cls = 0;
-    RowMap crow = {0, 0, 0, 0, 0, 0, 0, 0, g.perm_T, g.perm_OC};
-    const RowMap plain = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    RowMap crow = {0, 0, 0, 0, 0, 0, 0, 0, g.perm_T, g.perm_OC, 0, 0, g.by.perm_OC};
+    const RowMap plain = {};
+    unsigned by_plane = g.by.plane, by_ow = g.by.ow;
     if constexpr (VIRT == VIRT_A_CLASSES) {
         const OutClass &c = g.cls[bz];
         M = c.M, red = c.red, b_cls = c.b_off;
         pg.OH = c.OH, pg.OW = c.OW, pg.FW = c.taps_w, pg.pt = c.pt, pg.pl = c.pl;
-        crow = {c.OH * c.OW, c.OW, g.out_H, g.out_W, g.out_sy, g.out_sx, c.py, c.px, 0, 0};
+        by_plane = c.by_plane, by_ow = c.by_ow;
+        crow = {c.OH * c.OW, c.OW, g.out_H, g.out_W, g.out_sy, g.out_sx, c.py, c.px, 0, 0, by_plane, by_ow, 0};
         tilesM = (M + BM - 1) / BM;
         if (bx >= tilesM * tilesN) return;  // the grid is sized for the largest class
     }
     int id = bx;
     const int total = tilesM * tilesN;
-    int b = VIRT == VIRT_A_CLASSES ? 0 : bz / g.splits;
-    int split = VIRT == VIRT_A_CLASSES ? 0 : bz - b * g.splits;
+    int b = 0, split = 0;
+    if constexpr (VIRT != VIRT_A_CLASSES) b = Divisor(g.splits, g.by.layers).div(bz, split);
     // a workgroup past the product's own tiles works on the remainder band (GemmArgs::tail_m0)
     const bool in_tail = VIRT != VIRT_A_CLASSES && g.tail_splits > 0 && id >= total;
     int tps = g.tiles_per_split;
     if (in_tail) {
-        const int t = id - total;
-        split = t % g.tail_splits;
-        id = t / g.tail_splits;  // tile of the band, column by column
+        id = Divisor(g.tail_splits, g.by.tail_splits).div(id - total, split);  // tile of the band, column by column
         tps = g.tail_tps;
+    } else if constexpr (VIRT == VIRT_A_CLASSES) {
+        if (T::DMA || (total & 7) == 0) id = (id & 7) * (total >> 3) + min(id & 7, total & 7) + (id >> 3);
     } else {
         // an unsplit batched product is dealt out the same way over its batch index: one XCD takes all
         // tiles of a batch element, whose A and B it then reads once
@@ -674,9 +654,8 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
         const int layers = by_batch ? g.batch : g.splits;
         const int linear = id + total * layer, whole = total * (layers & ~7);
         if (linear < whole) {
-            const int j = linear >> 3, piece = j / total;
+            const int piece = Divisor(total, g.by.tiles).div(linear >> 3, id);
             layer = (piece << 3) + (linear & 7);
-            id = j - piece * total;
         } else if (T::DMA || (total & 7) == 0) {  // (the first total % 8 runs are one tile longer)
             id = (id & 7) * (total >> 3) + min(id & 7, total & 7) + (id >> 3);
         }
@@ -684,12 +663,15 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
         else split = layer;
     }
     constexpr int GM = 4;
-    const int band = id / (GM * tilesN), first = band * GM;
-    const int rows_in_band = max(1, min(GM, tilesM - first));
-    const int in_band = id - band * GM * tilesN;
-    const int tail_tilesM = in_tail ? (M - g.tail_m0 + BM - 1) / BM : 1;
-    const int tm = in_tail ? id % tail_tilesM : first + in_band % rows_in_band;
-    const int tn = in_tail ? id / tail_tilesM : in_band / rows_in_band;
+    int tm, tn;
+    if (in_tail) {
+        tn = Divisor((M - g.tail_m0 + BM - 1) / BM, g.by.tail_tilesM).div(id, tm);
+    } else {
+        int in_band;
+        const int first = Divisor(GM * tilesN, g.by.band).div(id, in_band) * GM, rows_in_band = max(1, min(GM, tilesM - first));
+        tn = rows_in_band == 3 ? (int)__umulhi((unsigned)in_band, 0x55555556u) : in_band >> (rows_in_band >> 1);  // (four, two or one: a shift)
+        tm = first + in_band - tn * rows_in_band;
+    }
     // A tile that would stick out of the matrix is moved back inside; the rows / columns it then
     // shares with its neighbour are computed twice but stored only by the neighbour.
     const int m_own = uniform<T>((in_tail ? g.tail_m0 : 0) + tm * BM), n_own = uniform<T>(tn * BN);
@@ -747,7 +729,7 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     // patch rows as A: this thread's rows never change; a step selects the tap
     int va_base[A_IT], va_iy[A_IT], va_ix[A_IT];
     if constexpr (VA) {
-        const Divisor<VIRT == VIRT_A_CLASSES && B_KC> plane(pg.OH * pg.OW), width(pg.OW);
+        const Divisor plane(pg.OH * pg.OW, by_plane), width(pg.OW, by_ow);
 #pragma unroll
         for (int p = 0; p < A_IT; ++p) {
             int rem, ox;
@@ -770,7 +752,7 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     if constexpr (VIRT == VIRT_B_KROWS) {
         int cy = -pg.pt, cx = -pg.pl, cc = 0;  // what the tap and channel add to an output pixel's source coordinates
         if constexpr (T::B_COLS) {
-            const Divisor<false> channels(pg.C), taps(pg.FW);
+            const Divisor channels(pg.C, g.by.channels), taps(pg.FW, g.by.taps_w);
 #pragma unroll
             for (int p = 0; p < B_IT; ++p) {
                 int c, fx;
@@ -780,13 +762,13 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
                 vb_toff[p] = ((vb_ty[p] * pg.W + vb_tx[p]) * pg.C + c) * ES;
             }
         } else {
-            const int n = n0 + b_c * EPV, t = n / pg.C, fy = t / pg.FW, fx = t - fy * pg.FW;
-            cc = n - t * pg.C;
+            int fx;
+            const int t = Divisor(pg.C, g.by.channels).div(n0 + b_c * EPV, cc), fy = Divisor(pg.FW, g.by.taps_w).div(t, fx);
             cy += fy * pg.dy;
             cx += fx * pg.dx;
         }
         vb_y_end = pg.OH * pg.sy + cy, vb_x_end = pg.OW * pg.sx + cx;
-        const Divisor<false> plane(pg.OH * pg.OW), width(pg.OW);
+        const Divisor plane(pg.OH * pg.OW, by_plane), width(pg.OW, by_ow);
 #pragma unroll
         for (int p = 0; p < VB_N; ++p) {
             int rem, ox;
@@ -821,13 +803,15 @@ __device__ __forceinline__ void gemm_tiled_body(const GemmArgs &g, int tilesM, c
     // The step that is fetched next: its product, K step and filter tap are counted on from step to step (every step is
     // fetched once, in order), because four divisions by runtime numbers at the head of each step -- some 35 dependent
     // scalar instructions that no matrix instruction covers -- were a fifth of a short half step's time.
-    int ld_i = 0, ld_r = uniform<T>(x0 / ktiles), ld_kx = x0 - ld_r * ktiles;
-    int ld_fy = !VA ? 0 : uniform<T>(ld_r / pg.FW), ld_fx = VA ? ld_r - ld_fy * pg.FW : 0;
+    int ld_i = 0, ld_r = 0, ld_kx = 0, ld_fy = 0, ld_fx = 0;
+    if constexpr (VIRT != VIRT_A_CLASSES) ld_r = uniform<T>(Divisor(ktiles, g.by.ktiles).div(x0, ld_kx));
+    if constexpr (VIRT == VIRT_A_ROWS) ld_fy = uniform<T>(Divisor(pg.FW, g.by.taps_w).div(ld_r, ld_fx));
     // patch k-rows: what BK more pixels add, and the corrections when a row or an image is complete
     int vb_dy = 0, vb_dx = 0, vb_d = 0, vb_d_row = 0, vb_d_img = 0;
     if constexpr (VIRT == VIRT_B_KROWS) {
-        const int plane = pg.OH * pg.OW, img = BK / plane, rem = BK - img * plane, oy = rem / pg.OW;
-        vb_dy = oy * pg.sy, vb_dx = (rem - oy * pg.OW) * pg.sx;
+        int rem, ox;
+        const int img = Divisor(pg.OH * pg.OW, by_plane).div(BK, rem), oy = Divisor(pg.OW, by_ow).div(rem, ox);
+        vb_dy = oy * pg.sy, vb_dx = ox * pg.sx;
         vb_d = ((img * pg.H + vb_dy) * pg.W + vb_dx) * pg.C * ES;
         vb_d_row = (pg.sy * pg.W - pg.OW * pg.sx) * pg.C * ES;
         vb_d_img = (pg.H - pg.OH * pg.sy) * pg.W * pg.C * ES;
@@ -1038,8 +1022,14 @@ __global__ __launch_bounds__(T0::NT, T0::TWO_FIT && T1::TWO_FIT ? 2 : 1) void ge
     if constexpr (T0::DMA) {
         __shared__ __attribute__((aligned(1024))) E stages[(T0::LDS_BYTES > T1::LDS_BYTES ? T0::LDS_BYTES : T1::LDS_BYTES) / T0::ES];
         const int id = (int)blockIdx.x, first = nx0 * nz0, j = id - first;
-        if (id < first) gemm_tiled_body<T0, EDGE>(g0, tilesM0, tilesN0, id % nx0, id / nx0, nx0, stages, nullptr, nullptr, nullptr);
-        else gemm_tiled_body<T1, EDGE>(g1, tilesM1, tilesN1, j % nx1, j / nx1, nx1, stages, nullptr, nullptr, nullptr);
+        int bx;
+        if (id < first) {
+            const int bz = Divisor(nx0, g0.by.nbx).div(id, bx);
+            gemm_tiled_body<T0, EDGE>(g0, tilesM0, tilesN0, bx, bz, nx0, stages, nullptr, nullptr, nullptr);
+        } else {
+            const int bz = Divisor(nx1, g1.by.nbx).div(j, bx);
+            gemm_tiled_body<T1, EDGE>(g1, tilesM1, tilesN1, bx, bz, nx1, stages, nullptr, nullptr, nullptr);
+        }
     } else {
         constexpr int A_SZ = T0::A_SZ > T1::A_SZ ? T0::A_SZ : T1::A_SZ, B_SZ = T0::B_SZ > T1::B_SZ ? T0::B_SZ : T1::B_SZ;
         __shared__ __attribute__((aligned(16))) E As0[A_SZ];
@@ -1047,11 +1037,13 @@ __global__ __launch_bounds__(T0::NT, T0::TWO_FIT && T1::TWO_FIT ? 2 : 1) void ge
         __shared__ __attribute__((aligned(16))) E Bs0[B_SZ];
         __shared__ __attribute__((aligned(16))) E Bs1[B_SZ];
         const int id = (int)blockIdx.x, first = nx0 * nz0;
+        int bx;
         if (id < first) {
-            gemm_tiled_body<T0, EDGE>(g0, tilesM0, tilesN0, id % nx0, id / nx0, nx0, As0, As1, Bs0, Bs1);
+            const int bz = Divisor(nx0, g0.by.nbx).div(id, bx);
+            gemm_tiled_body<T0, EDGE>(g0, tilesM0, tilesN0, bx, bz, nx0, As0, As1, Bs0, Bs1);
         } else {
-            const int j = id - first;
-            gemm_tiled_body<T1, EDGE>(g1, tilesM1, tilesN1, j % nx1, j / nx1, nx1, As0, As1, Bs0, Bs1);
+            const int bz = Divisor(nx1, g1.by.nbx).div(id - first, bx);
+            gemm_tiled_body<T1, EDGE>(g1, tilesM1, tilesN1, bx, bz, nx1, As0, As1, Bs0, Bs1);
         }
     }
 }
@@ -1092,6 +1084,18 @@ struct TileOf<f16, 128, 128, A_KC, B_KC, VIRT, FIT> {
 // gemm_tiled.hip)
 extern unsigned long long *phase_rec_buf;
 extern size_t phase_rec_bytes;
+
+// What the kernel divides by (GemmArgs::by) for a grid of tilesM x tilesN tiles of BM rows and nbx workgroups a layer.
+static inline void set_reciprocals(GemmArgs &g, int tilesM, int tilesN, int BM, int BK, int nbx) {
+    TiledReciprocals &by = g.by;
+    by.layers = reciprocal_of(g.splits), by.tiles = reciprocal_of(tilesM * tilesN), by.band = reciprocal_of(4 * tilesN);
+    by.ktiles = reciprocal_of(ceil_div(g.K, BK)), by.nbx = reciprocal_of(nbx), by.perm_OC = reciprocal_of(g.perm_OC);
+    by.taps_w = reciprocal_of(g.pg.FW), by.channels = reciprocal_of(g.pg.C);
+    by.plane = reciprocal_of(g.pg.OH * g.pg.OW), by.ow = reciprocal_of(g.pg.OW);
+    by.tail_splits = reciprocal_of(g.tail_splits), by.tail_tilesM = reciprocal_of(ceil_div(g.M - g.tail_m0, BM));
+    if (g.virt == VIRT_A_CLASSES)
+        for (int i = 0; i < g.ncls; ++i) g.cls[i].by_plane = reciprocal_of(g.cls[i].OH * g.cls[i].OW), g.cls[i].by_ow = reciprocal_of(g.cls[i].OW);
+}
 
 // Launches of one product, one translation unit each (gemm_tiled_launch.h)
 int gemm_tiled_plain_f16(const GemmArgs &g, int transA, int transB, hipStream_t stream);
@@ -1168,6 +1172,8 @@ static int launch_pair_tiles(const GemmArgs &gx0, const GemmArgs &gy0, hipStream
     else lds = 2L * ((TX::A_SZ > TY::A_SZ ? TX::A_SZ : TY::A_SZ) + (TX::B_SZ > TY::B_SZ ? TX::B_SZ : TY::B_SZ)) * TX::ES;
     const long wgs = (long)ny * nzy + (long)nx * nzx, cus = cu_count();
     const unsigned pad = lds <= third && wgs > cus && wgs <= 2 * cus ? (unsigned)(third + 512 - lds) : 0u;
+    set_reciprocals(gy, tMy, tNy, TY::BM, TY::BK, ny);
+    set_reciprocals(gx, tMx, tNx, TX::BM, TX::BK, nx);
     hipLaunchKernelGGL((gemm_tiled_pair_kernel<TY, TX, EDGE>), dim3(ny * nzy + nx * nzx), dim3(TX::NT), pad, stream, gy, gx, tMy, tNy, ny, nzy, tMx, tNx, nx);
     D8_LAUNCH_CHECK();
     return 0;

@@ -28,6 +28,7 @@ static int launch_edge(const GemmArgs &g0, hipStream_t stream) {
     const unsigned pad = (lds <= third && wgs > cus && wgs <= 2 * cus) ? (unsigned)(third + 512 - lds) : 0u;
     // a launch whose records would not fit the caller's buffer writes none
     g.phase_rec = (size_t)(tilesM * tilesN + extra) * layers * 64 <= phase_rec_bytes ? phase_rec_buf : nullptr;
+    set_reciprocals(g, tilesM, tilesN, BM, T::BK, tilesM * tilesN + extra);
     const dim3 grid(tilesM * tilesN + extra, 1, layers);
     hipLaunchKernelGGL((gemm_tiled_kernel<T, EDGE>), grid, dim3(T::NT), pad, stream, g, tilesM, tilesN);
     D8_LAUNCH_CHECK();
