@@ -422,18 +422,20 @@ __global__ __launch_bounds__(768) void conv_direct_grad_kernel(DirectArgs a) {
 }
 
 // gw[i] = beta * gw[i] + the sum of `parts` partial sums ws[.][i]: 64 outputs per workgroup, 16 waves that take every
-// sixteenth part each (four loads in flight) and meet in LDS in wave order.
+// sixteenth part each (sixteen loads in flight) and meet in LDS in wave order.
 template <typename E>
 __global__ __launch_bounds__(1024) void conv_direct_reduce_kernel(const float *ws, E *gw, int n, int parts, float beta) {
     __shared__ float met[16][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = blockIdx.x * 64 + lane;
     float sum[4] = {0.f, 0.f, 0.f, 0.f};
     if (i < n) {
-        int p = wave;
-        for (; p + 48 < parts; p += 64)
+        for (int p = wave; p < parts; p += 256) {
+            float t[16];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) sum[u] += ws[(long)(p + 16 * u) * n + i];
-        for (; p < parts; p += 16) sum[0] += ws[(long)p * n + i];
+            for (int u = 0; u < 16; ++u) t[u] = p + 16 * u < parts ? ws[(long)(p + 16 * u) * n + i] : 0.f;
+#pragma unroll
+            for (int u = 0; u < 16; ++u) sum[u & 3] += t[u];
+        }
     }
     met[wave][lane] = (sum[0] + sum[1]) + (sum[2] + sum[3]);
     __syncthreads();

@@ -107,6 +107,43 @@ __global__ __launch_bounds__(256) void accumulate_kernel(T *__restrict__ g, cons
     }
 }
 
+// The column sums of a block's 256 / TX row lanes meet in LDS, lane 0's first and the others' in their order, and every column's sum
+// is handed to done(column, sum).  `met` lanes had a row.  A thread adds one column at a time, eight lanes' sums in flight, where one
+// had VEC columns and waited for each lane's sums before it asked for the next's.  With the finishing kernel's loads all in flight,
+// ReLu gate and bias gradient of half 6272 x 256 7.3 -> 5.8 us, 13456 x 160 7.4 -> 5.9 (a launch takes 2.8 of the program's thread).
+// last_start: rows that start at any element, whose last columns' vector was moved back to start there; else 0.
+template <int VEC, class Done>
+__device__ __forceinline__ void meet_in_lds(float *part, const float (&acc)[VEC], int TX, int tx, int ty, int met, int C, int last_start, Done &&done) {
+    const int width = TX * VEC;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) part[ty * width + tx * VEC + e] = acc[e];
+    __syncthreads();
+    for (int i = threadIdx.x; i < width; i += 256) {
+        const long c = (long)blockIdx.x * width + i;
+        if (c >= C) break;
+        // (a vector that was moved back holds column c that much further on)
+        const int at = i + (last_start ? max(0, (int)(blockIdx.x * width + i / VEC * VEC) - last_start) : 0);
+        float v = 0.f;
+        int k = 0;
+        for (; k + 7 < met; k += 8) {
+            float t[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) t[u] = part[(k + u) * width + at];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v += t[u];
+        }
+        if (k < met) {
+            float t[7];
+#pragma unroll
+            for (int u = 0; u < 7; ++u) t[u] = part[min(k + u, met - 1) * width + at];
+#pragma unroll
+            for (int u = 0; u < 7; ++u)
+                if (k + u < met) v += t[u];
+        }
+        done((int)c, v);
+    }
+}
+
 // dz viewed [K0][R][C]; sums over R.  Block (x: column group, y: chunk of R, z: k0); TX threads
 // across column vectors, 256 / TX rows in flight.  The row lanes meet in LDS in a fixed order.
 // With one chunk the sums go straight into g (g += scale * sum); otherwise into
@@ -116,16 +153,15 @@ __global__ __launch_bounds__(256) void column_sum_kernel(const T *__restrict__ d
                                                          float *__restrict__ partial, int R, int C, int TX,
                                                          int rows_per_chunk, int chunks, float scale, float keep) {
     typedef T VT __attribute__((ext_vector_type(VEC)));
-    __shared__ float part[256][VEC];
-    const int tx = threadIdx.x % TX, ty = threadIdx.x / TX, lanes = 256 / TX;
+    __shared__ __attribute__((aligned(16))) float part[256 * VEC];
+    const int tx = threadIdx.x & (TX - 1), ty = threadIdx.x >> __builtin_ctz(TX), lanes = 256 >> __builtin_ctz(TX);
     const int cv = blockIdx.x * TX + tx;
-    const int k0 = blockIdx.z, chunk = blockIdx.y;
+    const int k0 = blockIdx.z, chunk = blockIdx.y, r1 = min(R, (chunk + 1) * rows_per_chunk);
     const bool live = (long)cv * VEC < C;
     float acc[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) acc[e] = 0.f;
     if (live) {
-        const int r1 = min(R, (chunk + 1) * rows_per_chunk);
         const T *p = dz + ((long)k0 * R) * C + (long)cv * VEC;
         int r = chunk * rows_per_chunk + ty;
         // four rows in flight per thread; the adds keep the order of the plain loop
@@ -138,62 +174,54 @@ __global__ __launch_bounds__(256) void column_sum_kernel(const T *__restrict__ d
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) acc[e] += ew_load<OP>(ew_f32(v[u][e]));
         }
-        for (; r < r1; r += lanes) {
-            const VT v = *(const VT *)(p + (long)r * C);
+        if (r < r1) {  // up to three rows more, in flight together
+            VT v[3];
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) acc[e] += ew_load<OP>(ew_f32(v[e]));
+            for (int u = 0; u < 3; ++u) v[u] = *(const VT *)(p + (long)min(r + u * lanes, r1 - 1) * C);
+#pragma unroll
+            for (int u = 0; u < 3; ++u)
+                if (r + u * lanes < r1)
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e) acc[e] += ew_load<OP>(ew_f32(v[u][e]));
         }
     }
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) part[threadIdx.x][e] = acc[e];
-    __syncthreads();
-    if (ty == 0 && live) {
-        // (lanes that had no row hold zeros: 64 sums of ten values each waited 3 us for 246 of them)
-        const int met = min(lanes, min(R - chunk * rows_per_chunk, rows_per_chunk));
-        for (int k = 1; k < met; ++k)
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) acc[e] += part[k * TX + tx][e];
+    const int first_row = chunk * rows_per_chunk;
+    meet_in_lds<VEC>(part, acc, TX, tx, ty, min(lanes, r1 - first_row), C, 0, [&](int c, float v) {
         if (chunks == 1) {
-            T *o = g + (long)k0 * C + (long)cv * VEC;
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) o[e] = ew_result<T, OP>((keep != 0.f ? ew_f32(o[e]) : 0.f) + scale * acc[e]);
+            T *o = g + (long)k0 * C + c;
+            *o = ew_result<T, OP>((keep != 0.f ? ew_f32(*o) : 0.f) + scale * v);
         } else {
-            float *o = partial + ((long)k0 * chunks + chunk) * C + (long)cv * VEC;
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) o[e] = acc[e];
+            partial[((long)k0 * chunks + chunk) * C + c] = v;
         }
-    }
+    });
 }
 
-// g[k0][c] += sum over chunks of partial[k0][chunk][c].  A block covers 16 outputs; 16 lanes per
-// output each add every 16th chunk (eight loads in flight) and meet in LDS in a fixed order.
+// g[k0][c] += sum over chunks of partial[k0][chunk][c], k0 = blockIdx.y.  A block covers 16 outputs; 16 lanes per
+// output each add every 16th chunk, sixteen at a time in flight whatever their number, and meet in LDS in a fixed order.
 template <typename T, int OP = LOAD_ID>
 __global__ __launch_bounds__(256) void column_sum_finish_kernel(const float *__restrict__ partial, T *__restrict__ g,
-                                                                int C, int chunks, long total, float scale, float keep) {
+                                                                int C, int chunks, float scale, float keep) {
     __shared__ float part[16][16];
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    const long idx = (long)blockIdx.x * 16 + tx;
+    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4, c = blockIdx.x * 16 + tx;
     float v = 0.f;
-    if (idx < total) {
-        const long k0 = idx / C;
-        const int c = (int)(idx - k0 * C);
-        const float *p = partial + k0 * chunks * C + c;
-        int k = ty;
-        for (; k + 7 * 16 < chunks; k += 8 * 16) {
-            float t[8];
+    if (c < C) {
+        const float *p = partial + (long)blockIdx.y * chunks * C + c;
+        for (int k = ty; k < chunks; k += 16 * 16) {
+            float t[16];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) t[u] = p[(long)(k + u * 16) * C];
+            for (int u = 0; u < 16; ++u) t[u] = p[(long)min(k + u * 16, chunks - 1) * C];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) v += t[u];
+            for (int u = 0; u < 16; ++u)
+                if (k + u * 16 < chunks) v += t[u];
         }
-        for (; k < chunks; k += 16) v += p[(long)k * C];
     }
     part[ty][tx] = v;
     __syncthreads();
-    if (ty == 0 && idx < total) {
+    if (ty == 0 && c < C) {
 #pragma unroll
         for (int k = 1; k < 16; ++k) v += part[k][tx];
-        g[idx] = ew_result<T, OP>((keep != 0.f ? ew_f32(g[idx]) : 0.f) + scale * v);
+        T *o = g + (long)blockIdx.y * C + c;
+        *o = ew_result<T, OP>((keep != 0.f ? ew_f32(*o) : 0.f) + scale * v);
     }
 }
 
@@ -211,10 +239,10 @@ __global__ __launch_bounds__(256) void relu_gate_column_sum_kernel(const T *__re
                                                                    int TX, int rows_per_chunk, int chunks, float keep) {
     typedef T VT __attribute__((ext_vector_type(VEC)));
     typedef VT MT __attribute__((aligned(ANY ? sizeof(T) : sizeof(VT))));  // a vector as it lies in memory
-    __shared__ float part[256][VEC];
-    const int tx = threadIdx.x % TX, ty = threadIdx.x / TX, lanes = 256 / TX;
+    __shared__ __attribute__((aligned(16))) float part[256 * VEC];
+    const int tx = threadIdx.x & (TX - 1), ty = threadIdx.x >> __builtin_ctz(TX), lanes = 256 >> __builtin_ctz(TX);
     const int cv = blockIdx.x * TX + tx;
-    const int chunk = blockIdx.y;
+    const int chunk = blockIdx.y, r1 = min(R, (chunk + 1) * rows_per_chunk);
     const bool live = (long)cv * VEC < C;
     const long col = ANY ? min((long)cv * VEC, (long)C - VEC) : (long)cv * VEC;
     const int skip = ANY ? (int)((long)cv * VEC - col) : 0;  // leading elements that are the neighbour's
@@ -237,7 +265,6 @@ __global__ __launch_bounds__(256) void relu_gate_column_sum_kernel(const T *__re
         }
     };
     if (live) {
-        const int r1 = min(R, (chunk + 1) * rows_per_chunk);
         int r = chunk * rows_per_chunk + ty;
         for (; r + 3 * lanes < r1; r += 4 * lanes) {
             VT a[4], b[4];
@@ -249,33 +276,24 @@ __global__ __launch_bounds__(256) void relu_gate_column_sum_kernel(const T *__re
 #pragma unroll
             for (int u = 0; u < 4; ++u) gate(a[u], b[u], r + u * lanes);
         }
-        for (; r < r1; r += lanes) {
-            const VT a = *(const MT *)(z + (long)r * C + col);
-            const VT b = *(const MT *)(dz + (long)r * C + col);
-            gate(a, b, r);
+        if (r < r1) {  // up to three rows more, in flight together
+            VT a[3], b[3];
+#pragma unroll
+            for (int u = 0; u < 3; ++u) {
+                const long at = (long)min(r + u * lanes, r1 - 1) * C + col;
+                a[u] = *(const MT *)(z + at);
+                b[u] = *(const MT *)(dz + at);
+            }
+#pragma unroll
+            for (int u = 0; u < 3; ++u)
+                if (r + u * lanes < r1) gate(a[u], b[u], r + u * lanes);
         }
     }
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) part[threadIdx.x][e] = acc[e];
-    __syncthreads();
-    if (ty == 0 && live) {
-        // (lanes that had no row hold zeros: 64 sums of ten values each waited 3 us for 246 of them)
-        const int met = min(lanes, min(R - chunk * rows_per_chunk, rows_per_chunk));
-        for (int k = 1; k < met; ++k)
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) acc[e] += part[k * TX + tx][e];
-        if (chunks == 1) {
-            T *o = g + col;
-#pragma unroll
-            for (int e = 0; e < VEC; ++e)
-                if (e >= skip) o[e] = (T)((keep != 0.f ? ew_f32(o[e]) : 0.f) + acc[e]);
-        } else {
-            float *o = partial + (long)chunk * C + col;
-#pragma unroll
-            for (int e = 0; e < VEC; ++e)
-                if (e >= skip) o[e] = acc[e];
-        }
-    }
+    const int first_row = chunk * rows_per_chunk;
+    meet_in_lds<VEC>(part, acc, TX, tx, ty, min(lanes, r1 - first_row), C, ANY ? C - VEC : 0, [&](int c, float v) {
+        if (chunks == 1) g[c] = (T)((keep != 0.f ? ew_f32(g[c]) : 0.f) + v);
+        else partial[(long)chunk * C + c] = v;
+    });
 }
 
 // z[r][c] = relu?(z[r][c] + bias[c]) in place: the one-pass fallback of the fused GEMM store.
@@ -472,7 +490,7 @@ static ReducePlan plan_reduce(const int *d, const int *zd) {
         }
         const long colblocks = (p.C + 255) / 256;  // upper bound on column groups
         long chunks = (4L * cu_count()) / (colblocks * p.K0);
-        const long max_chunks = (p.R + 63) / 64;
+        const long min_rows = p.C >= 256 && p.R > 64 ? 32 : 64, max_chunks = (p.R + min_rows - 1) / min_rows;
         if (chunks > max_chunks) chunks = max_chunks;
         if (chunks > 512) chunks = 512;
         if (chunks < 1) chunks = 1;
@@ -511,8 +529,8 @@ static int reduce_t(T *g, const int *d, const T *dz, const int *zd, void *scratc
                                TX, rpc, chunks, scale, keep);
         if (chunks > 1) {
             D8_LAUNCH_CHECK();
-            hipLaunchKernelGGL((column_sum_finish_kernel<T, OP>), dim3((unsigned)((ng + 15) / 16)), dim3(256), 0, s,
-                               (const float *)scratch, g, (int)p.C, chunks, ng, scale, keep);
+            hipLaunchKernelGGL((column_sum_finish_kernel<T, OP>), dim3((unsigned)((p.C + 15) / 16), (unsigned)p.K0), dim3(256), 0, s,
+                               (const float *)scratch, g, (int)p.C, chunks, scale, keep);
         }
     } else {
         ReduceGeom q;
@@ -624,7 +642,7 @@ static int relu_gate_sum_t(const T *z, const T *dz, T *dpre, T *g, long rows, in
     D8_LAUNCH_CHECK();
     if (chunks > 1) {
         hipLaunchKernelGGL((column_sum_finish_kernel<T>), dim3((unsigned)((cols + 15) / 16)), dim3(256), 0, s,
-                           (const float *)scratch, g, cols, chunks, (long)cols, 1.f, keep);
+                           (const float *)scratch, g, cols, chunks, 1.f, keep);
         D8_LAUNCH_CHECK();
     }
     return 0;

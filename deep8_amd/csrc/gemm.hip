@@ -14,6 +14,7 @@
 // operand; the transposed-operand cases differ only in how the tile loader walks global memory.
 #include <atomic>
 #include <cmath>
+#include <type_traits>
 
 #include "gemm_args.h"
 
@@ -348,15 +349,14 @@ static bool gemm_is_small(int M, int N, int K, int batch, int red) {
 }
 
 // C[b][m][n] = beta * C + sum_s ws[b][s][m][n].  A workgroup covers groups of 4 consecutive outputs.
-// Few pieces of many groups (LANES = 1): 256 groups, a thread adds all pieces of its group in order, four loads in
-// flight.  Else (LANES = 8): 32 groups, 8 thread rows each add every 8th piece, and the 8 sums meet in
+// Few pieces of many groups (LANES = 1): 256 groups, a thread adds all pieces of its group in order.  Else (LANES = 8): 32 groups, 8 thread rows each add every 8th piece, and the 8 sums meet in
 // LDS in a fixed order.  Either way the result does not depend on scheduling, and up to 8 pieces
 // it is the same.  Five pieces of 12544 x 32: 4.9 -> 4.0 us, four of 1024 x 1001 in half: 7.1 -> 5.4 us (3 us of which is
 // what any launch behind one that wrote a lot takes).  The groups count through an output's elements
 // whatever the length of its rows: with rows of an odd length a group starts at any 4-byte aligned address (which is what
 // a 16-byte load needs) and may go on in the next row.  An output a thread, as rows of an odd length had it first, took
 // 17.3 us for four partial sums of 1024 x 1001, this takes 8.0 us.
-typedef f32x4 f32x4_any __attribute__((aligned(4)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 // Which of the two: a thread per group only where that alone gives three of four compute units a workgroup, and never where the
 // output is stored transposed per tap (four scattered stores a thread).  Whole calls, a thread per group and eight, two to
 // eight pieces: up to 147456 outputs level with two or four pieces and 0.1 - 0.8 us slower with others, 235520 level,
@@ -367,42 +367,61 @@ __host__ __device__ static inline int reduce_lanes(const GemmArgs &g) {
 }
 
 // (ROWS: the rows are multiples of 4, so a group lies in one row and may be stored at once)
+//
+// Bound by latencies: the way of its loads from memory, and what is computed before them.  Up to eight pieces of a thread are in
+// flight at once, with the old C and the bias beside them, and an output is found by 32-bit multiplications (a product that is
+// cut has fewer tiles than the chip has compute units, so outputs and bytes of all pieces are far below 2^31).  Four in flight,
+// the rest one by one, and 64-bit divisions before: filter gradient of half Conv2d 32 x 14x14x256 3x3 5.1 -> 4.1 us, of 16 x
+// 57x57x96 -> 160 4.7 -> 4.1.  The loads are buffer loads because pieces past the last are zeros then without a branch: behind
+// branches of their own they took 88 registers instead of 58 where two products share the pass, and 8.7 us became 23.
 template <typename T, bool ROWS, int LANES>
-__device__ __forceinline__ void gemm_split_reduce_body(const GemmArgs &g, const long block, f32x4 (*part)[32]) {
+__device__ __forceinline__ void gemm_split_reduce_body(const GemmArgs &g, const int block, f32x4 (*part)[32]) {
     typedef T T4 __attribute__((ext_vector_type(4)));
-    const long mn = (long)g.M * g.N, groups = ROWS ? mn / 4 : (mn + 3) / 4;
+    const int mn = g.M * g.N, groups = ROWS ? mn / 4 : (mn + 3) / 4;
     constexpr int GROUPS = 256 / LANES;
     const int lane = threadIdx.x % GROUPS, row = threadIdx.x / GROUPS;
-    const long id = block * GROUPS + lane;  // this thread's group of 4 outputs
+    const int id = block * GROUPS + lane;  // this thread's group of 4 outputs
     const bool live = id < groups * g.batch;
-    const int b = live && g.batch > 1 ? (int)(id / groups) : 0;
-    const long r = (id - (long)b * groups) * 4;
-    const int n_out = ROWS || mn - r >= 4 ? 4 : (int)(mn - r);
+    int b = 0, n, r = id;
+    if (g.batch > 1) b = Divisor(groups, g.by.groups).div(id, r);
+    r *= 4;
+    int m = Divisor(g.N, g.by.row).div(r, n);
+    const int n_out = ROWS || mn - r >= 4 ? 4 : mn - r;
+    T *const c0 = (T *)g.C + (long)b * g.sC;
+    const bool whole = ROWS && !g.perm_OC && g.ldc % 4 == 0 && (((size_t)c0 | (size_t)g.bias) & (4 * sizeof(T) - 1)) == 0;
+    T4 *const c = (T4 *)(c0 + (long)m * g.ldc + n);
+    T4 old = {}, bias = {};
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    if (live) {
-        // (a last group of fewer than 4 is loaded with the outputs before it and moved down; an output of fewer than 4 in all
-        // is loaded one by one)
-        const bool tiny = !ROWS && mn < 4;
-        const int back = ROWS || tiny ? 0 : 4 - n_out;
-        const float *p = g.ws + (long)b * g.splits * mn + r - back;
-        auto piece = [&](int s) -> f32x4 {
-            const float *q = p + (long)s * mn;
-            if (!tiny) return *(const f32x4_any *)q;
-            f32x4 t = {q[0], 0.f, 0.f, 0.f};
-            if (n_out > 1) t[1] = q[1];
-            if (n_out > 2) t[2] = q[2];
-            return t;
+    const bool tiny = !ROWS && mn < 4;
+    if (live && whole && row == 0) {
+        if (g.beta != 0.f) old = *c;
+        if (g.bias) bias = *(const T4 *)((const T *)g.bias + n);
+    }
+    if (!tiny) {
+        // (a last group of fewer than 4 is loaded with the outputs before it and moved down.  Pieces past the last and groups past
+        // the last are fetched at an offset outside the buffer, as zeros: no load lies behind a branch)
+        const int back = ROWS ? 0 : 4 - n_out;
+        const unsigned bytes = (unsigned)(g.splits * g.batch) * (unsigned)mn * 4u, step = (unsigned)(LANES * mn) * 4u;
+        const __amdgpu_buffer_rsrc_t ws = __builtin_amdgcn_make_buffer_rsrc(g.ws, 0, (int)bytes, 0x00020000);
+        const unsigned at = live ? (unsigned)((b * g.splits + row) * mn + r - back) * 4u : 0x80000000u;
+        auto add = [&](auto in_flight, int s) {  // pieces s + row, s + row + LANES ...
+            constexpr int N = decltype(in_flight)::value;
+            u32x4 t[N];
+#pragma unroll
+            for (int u = 0; u < N; ++u)
+                t[u] = __builtin_amdgcn_raw_buffer_load_b128(ws, row + s + u * LANES < g.splits ? at : 0x80000000u, (s / LANES + u) * step, 0);
+#pragma unroll
+            for (int u = 0; u < N; ++u) v += __builtin_bit_cast(f32x4, t[u]);
         };
-        int s = row;
-        for (; s + 3 * LANES < g.splits; s += 4 * LANES) {
-            f32x4 t[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) t[u] = piece(s + u * LANES);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) v += t[u];
-        }
-        for (; s < g.splits; s += LANES) v += piece(s);
+        int s = 0;
+        for (; g.splits - s > 4 * LANES; s += 8 * LANES) add(std::integral_constant<int, 8>(), s);
+        if (g.splits - s > 2 * LANES) add(std::integral_constant<int, 4>(), s);
+        else if (g.splits - s > 0) add(std::integral_constant<int, 2>(), s);
         for (int k = 0; k < back; ++k) v = (f32x4){v[1], v[2], v[3], 0.f};
+    } else if (live) {  // an output of fewer than 4 in all
+        const float *p = g.ws + (long)b * g.splits * mn;
+        for (int s = row; s < g.splits; s += LANES)
+            for (int k = 0; k < n_out; ++k) v[k] += p[(long)s * mn + k];
     }
     if constexpr (LANES > 1) {
         part[row][lane] = v;
@@ -412,18 +431,13 @@ __device__ __forceinline__ void gemm_split_reduce_body(const GemmArgs &g, const 
         if constexpr (LANES > 1)
 #pragma unroll
             for (int k = 1; k < LANES; ++k) v += part[k][lane];
-        int m = (int)(r / g.N), n = (int)(r - (long)m * g.N);
-        T *c0 = (T *)g.C + (long)b * g.sC;
         auto finish = [&](float o, float old, float bias) {
             if (g.beta != 0.f) o += old;
             if (g.bias) o = (g.round_first ? to_f32((T)o) : o) + bias;
             return (T)(g.relu && !(o > 0.f) ? 0.f : o);
         };
-        if (ROWS && !g.perm_OC && g.ldc % 4 == 0 && (((size_t)c0 | (size_t)g.bias) & (4 * sizeof(T) - 1)) == 0) {
-            T4 *c = (T4 *)(c0 + (long)m * g.ldc + n);
-            T4 old = {}, bias = {}, out;
-            if (g.beta != 0.f) old = *c;
-            if (g.bias) bias = *(const T4 *)((const T *)g.bias + n);
+        if (whole) {
+            T4 out;
 #pragma unroll
             for (int k = 0; k < 4; ++k) out[k] = finish(v[k], to_f32(old[k]), to_f32(bias[k]));
             *c = out;
@@ -443,15 +457,16 @@ __device__ __forceinline__ void gemm_split_reduce_body(const GemmArgs &g, const 
 template <typename T, bool ROWS, int LANES>
 __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(GemmArgs g) {
     __shared__ f32x4 part[8][32];
-    gemm_split_reduce_body<T, ROWS, LANES>(g, (long)blockIdx.x, part);
+    gemm_split_reduce_body<T, ROWS, LANES>(g, (int)blockIdx.x, part);
 }
 
 // The reductions of two products in one launch: the first blocks0 workgroups are g0's, the rest g1's.
 template <typename T>
 __global__ __launch_bounds__(256) void gemm_split_reduce_pair_kernel(GemmArgs g0, GemmArgs g1, unsigned blocks0) {
     __shared__ f32x4 part[8][32];
-    const GemmArgs &g = blockIdx.x < blocks0 ? g0 : g1;
-    const long block = blockIdx.x < blocks0 ? blockIdx.x : blockIdx.x - blocks0;
+    const bool first = blockIdx.x < blocks0;
+    const GemmArgs &g = first ? g0 : g1;
+    const int block = (int)(first ? blockIdx.x : blockIdx.x - blocks0);
     if (reduce_lanes(g) == 1) gemm_split_reduce_body<T, true, 1>(g, block, part);
     else gemm_split_reduce_body<T, true, 8>(g, block, part);
 }
@@ -699,8 +714,12 @@ static long reduce_blocks(const GemmArgs &g, int lanes) {
     return (((long)g.M * g.N + 3) / 4 * g.batch + groups - 1) / groups;
 }
 
+static void set_reduce_reciprocals(GemmArgs &g) { g.by.row = reciprocal_of(g.N), g.by.groups = reciprocal_of((g.M * g.N + 3) / 4); }
+
 template <typename T>
-static int launch_reduce(const GemmArgs &g, hipStream_t stream) {
+static int launch_reduce(const GemmArgs &g0, hipStream_t stream) {
+    GemmArgs g = g0;
+    set_reduce_reciprocals(g);
     const int lanes = reduce_lanes(g);
     const dim3 grid((unsigned)reduce_blocks(g, lanes));
     if (g.N % 4 == 0 && lanes == 1) hipLaunchKernelGGL((gemm_split_reduce_kernel<T, true, 1>), grid, dim3(256), 0, stream, g);
@@ -713,7 +732,9 @@ static int launch_reduce(const GemmArgs &g, hipStream_t stream) {
 
 // The reductions that follow a launch of two products (either may be unsplit): one launch for both (whose rows are
 // multiples of 4, or they would not have shared the first).
-static int launch_reduce_pair(int dtype, const GemmArgs &g0, const GemmArgs &g1, hipStream_t stream) {
+static int launch_reduce_pair(int dtype, const GemmArgs &p0, const GemmArgs &p1, hipStream_t stream) {
+    GemmArgs g0 = p0, g1 = p1;
+    set_reduce_reciprocals(g0), set_reduce_reciprocals(g1);
     const bool r0 = g0.splits > 1, r1 = g1.splits > 1;
     const long b0 = reduce_blocks(g0, reduce_lanes(g0)), b1 = reduce_blocks(g1, reduce_lanes(g1));
     if (r0 && r1 && g0.N % 4 == 0 && g1.N % 4 == 0 && b0 + b1 < 0x7fffffffL) {
