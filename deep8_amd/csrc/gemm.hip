@@ -332,13 +332,13 @@ __global__ __launch_bounds__(SMALL_WAVES * 64) void gemm_small_kernel(GemmArgs g
 template <typename T>
 __global__ __launch_bounds__(SMALL_WAVES * 64) void gemm_small_pair_kernel(GemmArgs g0, GemmArgs g1, int nx0, int ny0, int n0, int nx1, int ny1) {
     __shared__ SmallParts part;
-    int id = (int)blockIdx.x;
-    if (id < n0) {
-        gemm_small_body<T, false, true>(g0, id % nx0, (id / nx0) % ny0, id / (nx0 * ny0), part);
-    } else {
-        id -= n0;
-        gemm_small_body<T, true, false>(g1, id % nx1, (id / nx1) % ny1, id / (nx1 * ny1), part);
-    }
+    const bool first = (int)blockIdx.x < n0;
+    const GemmArgs &g = first ? g0 : g1;
+    const int nx = first ? nx0 : nx1, ny = first ? ny0 : ny1;
+    int tile, bx;
+    const int b = Divisor(nx * ny, g.by.tiles).div((int)blockIdx.x - (first ? 0 : n0), tile), by = Divisor(nx, g.by.nbx).div(tile, bx);
+    if (first) gemm_small_body<T, false, true>(g0, bx, by, b, part);
+    else gemm_small_body<T, true, false>(g1, bx, by, b, part);
 }
 
 // Whether a product is small in the sense above: at most four 128 x 128 tiles of output and a reduction of
@@ -585,8 +585,9 @@ struct PackArgs {
     f16 *dst;
     int rows, cols, ld, pitch;  // rows of all matrices that follow each other, `per` of them `stride` elements from the next
     int per;
+    unsigned by_per;  // reciprocal_of(per)
     long stride;
-    int across;
+    int across;  // as a power of two
     unsigned first;  // workgroup
 };
 struct PackList {
@@ -594,36 +595,45 @@ struct PackList {
     int n;
 };
 
-// Bound by memory.  `across` threads (a power of two, at most 256) lie along a row, a thread copies 16 bytes of four rows before it
-// goes on along them, read at the alignment of an element.  Copied rows start at multiples of 128 bytes, as the K steps of
+// Bound by the way to memory and back.  2^across threads (at most 256) lie along a row, a thread copies 16 bytes of ROWS rows before
+// it goes on along them, read at the alignment of an element.  A row's last piece is read where it ends with the row and shifted
+// into place: element by element it kept the whole workgroup waiting for up to seven loads in a row (4096 x 1001 and 1024 x 1001
+// 8.4 -> 6.0 us, 1024 x 1001 alone 6.9 -> 4.5, 888 x 1255 6.7 -> 2.8).  Copied rows start at multiples of 128 bytes, as the K steps of
 // the product want them (pitch 1008 instead of 1024: 4096 x 1001 x 1024 loop of the product 9.7 us instead of 8.3).
-constexpr int PACK_ROWS = 4;
+template <int ROWS>
 __global__ __launch_bounds__(256) void pack_rows_kernel(PackList L) {
     typedef f16x8 f16x8_any __attribute__((aligned(2)));
     const int i = L.n > 2 && blockIdx.x >= L.m[2].first ? 2 : L.n > 1 && blockIdx.x >= L.m[1].first ? 1 : 0;
-    const PackArgs &a = L.m[i];
-    const int down = 256 / a.across, row0 = (int)(blockIdx.x - a.first) * PACK_ROWS * down + (int)threadIdx.x / a.across;
-    const f16 *src[PACK_ROWS];
+    const PackArgs a = L.m[i];
+    const int down = 256 >> a.across, row0 = (int)(blockIdx.x - a.first) * ROWS * down + ((int)threadIdx.x >> a.across);
+    const f16 *src[ROWS];
     f16 *const dst = a.dst + (long)row0 * a.pitch;
 #pragma unroll
-    for (int u = 0; u < PACK_ROWS; ++u) {
-        const int row = row0 + u * down, m = a.per < a.rows ? row / a.per : 0;
-        src[u] = row < a.rows ? a.src + (long)m * a.stride + (long)(row - m * a.per) * a.ld : nullptr;
+    for (int u = 0; u < ROWS; ++u) {
+        const int row = min(row0 + u * down, a.rows - 1);  // (rows past the last are read there and not written)
+        int m = 0, r = row;
+        if (a.per < a.rows) m = Divisor(a.per, a.by_per).div(row, r);
+        src[u] = a.src + (long)m * a.stride + (long)r * a.ld;
     }
-    for (int c = ((int)threadIdx.x & (a.across - 1)) * 8; c < a.pitch; c += a.across * 8) {
-        f16x8 v[PACK_ROWS];
+    const int step = 8 << a.across;
+    for (int c = ((int)threadIdx.x & ((1 << a.across) - 1)) * 8; c < a.pitch; c += step) {
+        u32x4 v[ROWS];
+        const int from = max(min(c, a.cols - 8), 0), left = a.cols - c, shift = c - from;  // elements of the piece that are the row's
 #pragma unroll
-        for (int u = 0; u < PACK_ROWS; ++u) {
-            v[u] = (f16x8)(f16)0.f;
-            if (!src[u]) continue;
-            if (c + 8 <= a.cols) v[u] = *(const f16x8_any *)(src[u] + c);
-            else
-                for (int e = 0; e < 8; ++e)
-                    if (c + e < a.cols) v[u][e] = src[u][c + e];
+        for (int u = 0; u < ROWS; ++u) v[u] = __builtin_bit_cast(u32x4, (f16x8)*(const f16x8_any *)(src[u] + from));
+        if (left < 8) {
+#pragma unroll
+            for (int u = 0; u < ROWS; ++u) {
+                u32x4 w = v[u];
+                if (shift & 4) w = (u32x4){w[2], w[3], 0u, 0u};
+                if (shift & 2) w = (u32x4){w[1], w[2], w[3], 0u};
+                if (shift & 1) w = (u32x4){w[0] >> 16 | w[1] << 16, w[1] >> 16 | w[2] << 16, w[2] >> 16 | w[3] << 16, w[3] >> 16};
+                v[u] = left > 0 ? w : (u32x4){0u, 0u, 0u, 0u};
+            }
         }
 #pragma unroll
-        for (int u = 0; u < PACK_ROWS; ++u)
-            if (src[u]) *(f16x8 *)(dst + (long)u * down * a.pitch + c) = v[u];
+        for (int u = 0; u < ROWS; ++u)
+            if (row0 + u * down < a.rows) *(u32x4 *)(dst + (long)u * down * a.pitch + c) = v[u];
     }
 }
 
@@ -658,37 +668,40 @@ struct PackPlan {
     size_t bytes;
 };
 
-// Whether copies pay: a product then saves some 0.13 us per K step of a 128 x 128 tile and round of the chip where one of its
-// operands is odd and 0.33 where both are; the copies take 3 us and 0.4 a MB, of which products that share a launch, which they would not
-// without copies, get the launch back.  1250 drawn calls with odd sizes, us on the kernels for rows that start anywhere / on copies
-// always / with this rule / with the better of the two, and how many lose more than 3 %:
-//   shared, both have operands to copy   15910 / 13579 / 13730 / 13475, 9 of 562 (with 0.25 a MB 14010, 5)
-//   shared, x alone                       7359 /  6896 /  6933 /  6754, 18 of 325 (by the line of the others 6946, 29; with 0.3 and 0.15 a MB throughout
-//                                         7048, 2: of more than 1700 columns x leaves both products many tiles, and less to gain from one launch)
-//   one after the other                  54096 / 47163 / 46767 / 46322, at most 1 of 365 (0.2 a MB and no launch: 35 of 199, 913 x 6859 x 177 26.4 -> 36.9)
-// 4096 rows, 1024 -> 1001: 44.6 -> 38.2 us.
-static bool pack_pays(const PackedProduct (&p)[2], const PackPlan &plan, bool shared) {
+// Whether copies pay: a product saves 0.2 us for each K step that a compute unit walks, 0.25 where both of its operands are odd, and a
+// MB of copies takes 0.3; a launch for them is what products save that share one, which they would not without copies, or that
+// are tiled finer.  Drawn calls with odd sizes, a third of them batched, us on the kernels for rows that start anywhere / on copies
+// always / by this rule / with the better of the two, and how many lose more than 3 % by it:
+//   330 calls of both gradients   10413 / 8937 / 8789 / 8672, 2
+//   330 forward products           5453 / 5457 / 5111 / 4981, 6
+// x alone to copy, in gradients: its products share a launch less often.  Forward: an output narrower than a tile is bound by its
+// operands' way from memory; a product that fills the chip with tiles of few steps has them hide each other's ways.
+// 4096 x 1024 x 1001 with bias and ReLu 21.1 -> 20.2, 883 x 624 x 334 17.1 -> 10.7, 107 x 1440 x 3121 36.2 -> 15.8.
+static bool pack_pays(const PackedProduct *p, int products, const PackPlan &plan) {
     const char *force = getenv("D8_GEMM_PACK");  // tuning and test aid (read at every call): 0 never, 1 always
     if (force) return atoi(force) != 0;
-    double saved = 0.0;
-    bool both = true;
-    for (int i = 0; i < 2; ++i) {
+    const double cus = cu_count();
+    double saved = 0.0, least = 0.5;
+    for (int i = 0; i < products; ++i) {
         const GemmArgs &g = *p[i].g;
-        const int odd = (plan.slot[i][0] >= 0) + (plan.slot[i][1] >= 0), shortest = g.M < g.N ? (g.M < g.K ? g.M : g.K) : (g.N < g.K ? g.N : g.K);
-        if (shortest < 64 || (double)g.M * g.N * g.K < (1 << 25)) return false;
-        const double steps = (double)ceil_div(g.M, 128) * ceil_div(g.N, 128) * g.batch * g.red * ceil_div(g.K, 64) / cu_count();
-        both = both && odd;
-        saved += (odd == 2 ? 0.33 : odd == 1 ? 0.13 : 0.0) * (steps < 1.0 ? 1.0 : steps);
+        const int odd = (plan.slot[i][0] >= 0) + (plan.slot[i][1] >= 0);
+        const long tiles = (long)ceil_div(g.M, 128) * ceil_div(g.N, 128) * g.batch, total = (long)g.red * ceil_div(g.K, 64);
+        const double share = tiles * total / cus, alone = total < 8 ? total : 8.0;
+        saved += (odd == 2 ? 0.25 : odd == 1 ? 0.2 : 0.0) * (share > alone ? share : alone);
+        if (products == 2 && i == 0 && odd) least = 0.0;
+        if (products == 1) {
+            if (g.M < 128 || g.N < 128) return false;
+            least = 4 * tiles >= cus && total <= 32 ? 1.7 : 0.2;
+        }
     }
-    if (!shared) return saved > 3.0 + 0.5e-6 * plan.bytes;
-    return both || p[0].g->N <= 1700 ? saved > 0.2e-6 * plan.bytes : saved > 0.3 + 0.15e-6 * plan.bytes;
+    return saved > least + 0.3e-6 * plan.bytes;
 }
 
 // (products on the tiled kernels; false: nothing to copy, or not with these)
-static bool pack_plan(int dtype, const PackedProduct (&p)[2], PackPlan &plan) {
+static bool pack_plan(int dtype, const PackedProduct *p, int products, PackPlan &plan) {
     plan.n = 0, plan.bytes = 0;
     if (dtype != D8_FLOAT16) return false;
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < products; ++i) {
         const GemmArgs &g = *p[i].g;
         if (g.virt != VIRT_NONE || g.K < 1 || g.batch > 448 || g.M > 65535 * 128 || gemm_is_small(g.M, g.N, g.K, g.batch, g.red) ||
             !gemm_tiled_eligible(dtype, g, p[i].ta, p[i].tb)) return false;
@@ -697,7 +710,7 @@ static bool pack_plan(int dtype, const PackedProduct (&p)[2], PackPlan &plan) {
             plan.slot[i][op] = -1;
             if (!(ops >> op & 1)) continue;
             const PackShape s = pack_shape(g, p[i].ta, p[i].tb, op);
-            if (pack_bytes(s) >= (1u << 31)) return false;  // (byte offsets inside an operand are 32-bit)
+            if (pack_bytes(s) >= (1u << 31) || s.cols < 8) return false;  // (byte offsets inside an operand are 32-bit; a row has a piece)
             int k = 0;
             while (k < plan.n && !(plan.shapes[k].p == s.p && plan.shapes[k].rows == s.rows && plan.shapes[k].cols == s.cols &&
                                    plan.shapes[k].ld == s.ld && plan.shapes[k].per == s.per && plan.shapes[k].stride == s.stride)) ++k;
@@ -980,6 +993,7 @@ bool gemm_small_pair_run(int dtype, const GemmArgs &g0, int ta0, int tb0, const 
     if (n0 + n1 > 0x7fffffffL) return false;
     GemmArgs a = g0, b = g1;
     a.splits = b.splits = 1;
+    a.by.nbx = reciprocal_of(nx0), a.by.tiles = reciprocal_of(nx0 * ny0), b.by.nbx = reciprocal_of(nx1), b.by.tiles = reciprocal_of(nx1 * ny1);
     if (dtype == D8_FLOAT16)
         hipLaunchKernelGGL((gemm_small_pair_kernel<f16>), dim3((unsigned)(n0 + n1)), dim3(SMALL_WAVES * 64), 0, stream, a, b, nx0, ny0, (int)n0, nx1, ny1);
     else
@@ -1121,44 +1135,67 @@ bool gemm_tiled_run_plain_pair(int dtype, GemmArgs &g0, int ta0, int tb0, GemmAr
     return true;
 }
 
-// The two products on copies, and how: whether they share a launch is known before anything is copied, because copies for products
-// that run one after the other have to save more (pack_pays), and then only those products read them that have something to copy.
-struct PackRun {
-    PackPlan plan;
+// Where the copies go, one behind the other.  A thread copies a piece of four rows, or of one where that leaves compute units without
+// two workgroups.
+struct PackLaunch {
     PackList list;
     unsigned blocks;
+    bool single;
+};
+static void pack_list(const PackPlan &plan, void *workspace, PackLaunch &p) {
+    auto lay_out = [&](int rows) {
+        p.blocks = 0;
+        char *to = (char *)workspace;
+        p.list.n = plan.n;
+        for (int k = 0; k < plan.n; ++k) {
+            const PackShape &s = plan.shapes[k];
+            int across = 3;
+            while (across < 8 && (8 << across) < pack_pitch(s)) ++across;
+            p.list.m[k] = {(const f16 *)s.p, (f16 *)to, (int)s.rows, s.cols, s.ld, pack_pitch(s), s.per, reciprocal_of(s.per), s.stride, across, p.blocks};
+            p.blocks += (unsigned)ceil_div(s.rows, rows * (256 >> across));
+            to += pack_bytes(s);
+        }
+    };
+    lay_out(4);
+    p.single = p.blocks < 2u * cu_count();
+    if (p.single) lay_out(1);
+}
+// The two products on copies, and how: whether they share a launch is known before anything is copied, because of products that run
+// one after the other only those read copies that have something to copy.
+struct PackRun {
+    PackPlan plan;
+    PackLaunch copies;
     GemmArgs g[2];
     bool shared;
 };
-static bool pack_run_plan(int dtype, const PackedProduct (&p)[2], void *workspace, size_t workspace_bytes, PackRun &r) {
-    if (!workspace || ((size_t)workspace & 15) || !pack_plan(dtype, p, r.plan) || r.plan.bytes > workspace_bytes) return false;
-    r.list.n = r.plan.n, r.blocks = 0;
-    char *to = (char *)workspace;
-    for (int k = 0; k < r.plan.n; ++k) {
-        const PackShape &s = r.plan.shapes[k];
-        int across = 8;
-        while (across < 256 && across * 8 < pack_pitch(s)) across *= 2;
-        r.list.m[k] = {(const f16 *)s.p, (f16 *)to, (int)s.rows, s.cols, s.ld, pack_pitch(s), s.per, s.stride, across, r.blocks};
-        r.blocks += (unsigned)ceil_div(s.rows, PACK_ROWS * (256 / across));
-        to += pack_bytes(s);
+// The product on its copies.
+static GemmArgs packed_args(GemmArgs g, const int (&slot)[2], const PackList &list) {
+    if (slot[0] >= 0) {
+        const PackArgs &a = list.m[slot[0]];
+        g.A = a.dst, g.lda = a.pitch, g.sA = g.sA ? (long)a.per * a.pitch : 0;
     }
-    auto packed = [&](int i) {
-        GemmArgs g = *p[i].g;
-        if (r.plan.slot[i][0] >= 0) {
-            const PackArgs &a = r.list.m[r.plan.slot[i][0]];
-            g.A = a.dst, g.lda = a.pitch, g.sA = g.sA ? (long)a.per * a.pitch : 0;
-        }
-        if (r.plan.slot[i][1] >= 0) {
-            const PackArgs &b = r.list.m[r.plan.slot[i][1]];
-            g.B = b.dst, g.ldb = b.pitch, g.sB = g.sB ? (long)b.per * b.pitch : 0;
-        }
-        g.packed = 1, g.padM = (g.M + 7) & ~7, g.padN = (g.N + 7) & ~7;
-        return g;
-    };
+    if (slot[1] >= 0) {
+        const PackArgs &b = list.m[slot[1]];
+        g.B = b.dst, g.ldb = b.pitch, g.sB = g.sB ? (long)b.per * b.pitch : 0;
+    }
+    g.packed = 1, g.padM = (g.M + 7) & ~7, g.padN = (g.N + 7) & ~7;
+    return g;
+}
+static int launch_pack(const PackLaunch &p, hipStream_t stream) {
+    if (p.single) hipLaunchKernelGGL(pack_rows_kernel<1>, dim3(p.blocks), dim3(256), 0, stream, p.list);
+    else hipLaunchKernelGGL(pack_rows_kernel<4>, dim3(p.blocks), dim3(256), 0, stream, p.list);
+    D8_LAUNCH_CHECK();
+    return 0;
+}
+static bool pack_run_plan(int dtype, const PackedProduct (&p)[2], void *workspace, size_t workspace_bytes, PackRun &r) {
+    if (!workspace || ((size_t)workspace & 15) || !pack_plan(dtype, p, 2, r.plan) || r.plan.bytes > workspace_bytes) return false;
+    char *const to = (char *)workspace + r.plan.bytes;
+    pack_list(r.plan, workspace, r.copies);
+    auto packed = [&](int i) { return packed_args(*p[i].g, r.plan.slot[i], r.copies.list); };
     r.g[0] = packed(0), r.g[1] = packed(1);
     const size_t rest = workspace_bytes - r.plan.bytes;
     r.shared = plain_pair_plan(dtype, r.g[0], p[0].ta, p[0].tb, r.g[1], p[1].ta, p[1].tb, to, rest);
-    if (!pack_pays(p, r.plan, r.shared)) return false;
+    if (!pack_pays(p, 2, r.plan)) return false;
     for (int i = 0; i < 2; ++i) {
         const GemmArgs &g = *p[i].g;  // (not at the cost of the pieces that it would run in without copies)
         if (d8_gemm_workspace_bytes(dtype, p[i].ta, p[i].tb, g.M, g.N, g.K, g.red > 1 ? g.red : g.batch, g.red > 1 ? 0 : 1) > rest) return false;
@@ -1176,15 +1213,35 @@ bool gemm_pack_run(int dtype, const PackedProduct (&p)[2], void *workspace, size
     PackRun r;
     if (!pack_run_plan(dtype, p, workspace, workspace_bytes, r)) return false;
     *shared = r.shared;
-    hipLaunchKernelGGL(pack_rows_kernel, dim3(r.blocks), dim3(256), 0, stream, r.list);
-    const hipError_t e = hipGetLastError();
-    *rc = e == hipSuccess ? 0 : fail((int)e, "kernel launch: %s", hipGetErrorString(e));
+    *rc = launch_pack(r.copies, stream);
     if (*rc == 0 && r.shared) *rc = plain_pair_run(dtype, r.g[0], r.g[1], stream);
     for (int i = 0; i < 2 && !r.shared && *rc == 0; ++i)
         *rc = gemm_tiled_run(dtype, r.g[i], p[i].ta, p[i].tb, (char *)workspace + r.plan.bytes, workspace_bytes - r.plan.bytes, stream);
     return true;
 }
 
+// A forward product by itself.
+static bool pack_one_plan(int dtype, const PackedProduct &p, size_t workspace_bytes, PackPlan &plan) {
+    if (!pack_plan(dtype, &p, 1, plan) || plan.bytes > workspace_bytes || !pack_pays(&p, 1, plan)) return false;
+    const GemmArgs &g = *p.g;  // (not at the cost of the pieces that it would run in without copies)
+    return d8_gemm_workspace_bytes(dtype, p.ta, p.tb, g.M, g.N, g.K, g.red > 1 ? g.red : g.batch, g.red > 1 ? 0 : 1) <= workspace_bytes - plan.bytes;
+}
+
+size_t gemm_pack_one_bytes(int dtype, const PackedProduct &p) {
+    PackPlan plan;
+    return pack_one_plan(dtype, p, (size_t)1 << 62, plan) ? plan.bytes : 0;
+}
+
+bool gemm_pack_run_one(int dtype, const PackedProduct &p, void *workspace, size_t workspace_bytes, hipStream_t stream, int *rc) {
+    PackPlan plan;
+    if (!workspace || ((size_t)workspace & 15) || !pack_one_plan(dtype, p, workspace_bytes, plan)) return false;
+    PackLaunch copies;
+    pack_list(plan, workspace, copies);
+    GemmArgs g = packed_args(*p.g, plan.slot[0], copies.list);
+    if ((*rc = launch_pack(copies, stream)) == 0)
+        *rc = gemm_tiled_run(dtype, g, p.ta, p.tb, (char *)workspace + plan.bytes, workspace_bytes - plan.bytes, stream);
+    return true;
+}
 
 bool gemm_fuses_store(int dtype, const GemmArgs &g, int transA, int transB, TiledRule rule) {
     // (a product beyond one launch's limits -- more than 448 outputs, more than 65535 * 128 rows -- is cut into several

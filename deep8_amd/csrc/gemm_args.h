@@ -219,6 +219,9 @@ struct PackedProduct {
 };
 bool gemm_pack_run(int dtype, const PackedProduct (&p)[2], void *workspace, size_t workspace_bytes, hipStream_t stream, bool *shared, int *rc);
 size_t gemm_pack_bytes(int dtype, const PackedProduct (&p)[2]);  // what it takes of the workspace (0: it does not pay)
+// The same for a forward product by itself (bias and ReLu included: the caller has checked gemm_fuses_store).
+bool gemm_pack_run_one(int dtype, const PackedProduct &p, void *workspace, size_t workspace_bytes, hipStream_t stream, int *rc);
+size_t gemm_pack_one_bytes(int dtype, const PackedProduct &p);
 
 // Plan the split of the reduction, launch the tiled kernel (which must be eligible) and reduce.
 int gemm_tiled_run(int dtype, GemmArgs &g, int transA, int transB, void *workspace, size_t workspace_bytes,

@@ -335,14 +335,32 @@ size_t d8_matmul_scratch_bytes(int dtype, int which, int xb, int xr, int xc, int
         return align256(d8_matmul_scratch_bytes(dtype, 1, xb, xr, xc, yb, yr, yc)) + d8_matmul_scratch_bytes(dtype, 2, xb, xr, xc, yb, yr, yc) +
                gemm_pack_bytes(dtype, both);
     }
-    return gemm_ws(dtype, mm_plan(which, nullptr, xb, xr, xc, nullptr, yb, yr, yc, nullptr));
+    const Gemm p = mm_plan(which, nullptr, xb, xr, xc, nullptr, yb, yr, yc, nullptr);
+    if (which != 0) return gemm_ws(dtype, p);
+    GemmArgs g = to_args(p);
+    return gemm_ws(dtype, p) + gemm_pack_one_bytes(dtype, {&g, p.ta, p.tb});
+}
+
+// A forward product (bias and relu: as its store may apply them) on copies of operands whose rows start anywhere; false, with
+// nothing launched, where that does not pay.
+static bool run_on_copies(int dtype, const Gemm &p, const void *bias, int relu, void *scratch, size_t scratch_bytes, void *stream, int *rc) {
+    GemmArgs g = to_args(p);
+    g.bias = bias, g.relu = relu;
+    if (bias || relu) {
+        g.round_first = !gemm_fuses_store(dtype, g, p.ta, p.tb, TILED_PIECES);
+        if (!gemm_fuses_store(dtype, g, p.ta, p.tb)) return false;
+    }
+    return gemm_pack_run_one(dtype, {&g, p.ta, p.tb}, scratch, scratch_bytes, as_stream(stream), rc);
 }
 
 int d8_matmul(int dtype, const void *x, int xb, int xr, int xc, const void *y, int yb, int yr, int yc,
               void *z, void *scratch, size_t scratch_bytes, void *stream) {
     if (int rc = check_mm("d8_matmul", dtype, xb, xr, xc, yb, yr, yc)) return rc;
     D8_REQUIRE(x && y && z, "d8_matmul: null tensor");
-    return run(dtype, mm_plan(0, x, xb, xr, xc, y, yb, yr, yc, z), scratch, scratch_bytes, stream);
+    const Gemm p = mm_plan(0, x, xb, xr, xc, y, yb, yr, yc, z);
+    int rc = 0;
+    if (run_on_copies(dtype, p, nullptr, 0, scratch, scratch_bytes, stream, &rc)) return rc;
+    return run(dtype, p, scratch, scratch_bytes, stream);
 }
 
 int d8_matmul_bias_relu(int dtype, const void *x, int xb, int xr, int xc, const void *y, int yb, int yr, int yc,
@@ -357,6 +375,8 @@ int d8_matmul_bias_relu(int dtype, const void *x, int xb, int xr, int xc, const 
         if (int rc = run(dtype, p, scratch, scratch_bytes, stream)) return rc;
         return launch_bias_relu(dtype, z, bias, (long)(xb > yb ? xb : yb), xr, relu, as_stream(stream));
     }
+    int rc = 0;
+    if (run_on_copies(dtype, p, bias, relu, scratch, scratch_bytes, stream, &rc)) return rc;
     return run_bias_relu(dtype, p, bias, relu, scratch, scratch_bytes, stream);
 }
 
