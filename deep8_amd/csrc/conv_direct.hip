@@ -35,6 +35,8 @@ struct DirectArgs {
     int rows, pitch;            // image rows of a tile, and elements an image row takes in LDS
     int vec_x, vec_z;           // elements a staging access of the image / of z moves
     unsigned mg_chunks, mg_tc;  // ceil(2^32 / (pitch / vec_x)), ceil(2^32 / TC or TCp)
+    unsigned mg_pieces;         // ceil(2^32 / P)
+    int zeros;                  // forward: element of LDS from which 32 bytes may be zeros
     int kb, pixels_p;           // gradient: blocks of 32 n; pixels of a tile with its rows filled up, a multiple of a k group
 };
 
@@ -127,24 +129,75 @@ __device__ __forceinline__ unsigned first_mask(int n, int d) {
 // start in the middle of a dword.  A workgroup walks every gridDim.x-th tile, its four waves every fourth block of 32 pixels.
 // Bound by the store of z and the latency of a tile's image rows, which two workgroups and more per compute unit hide from each
 // other; figures at conv_direct_forward.
-template <typename E, int G, int NB, bool ODD>
-__global__ __launch_bounds__(256, 2) void conv_direct_forward_kernel(DirectArgs a) {
+template <typename E, int G, int NB, bool ODD, int RESIDENT = 2>
+__global__ __launch_bounds__(256, RESIDENT) void conv_direct_forward_kernel(DirectArgs a) {
     typedef Elem<E> EL;
     typedef typename EL::Frag Frag;
-    constexpr int EPV = 16 / sizeof(E);
+    constexpr int EPV = 16 / sizeof(E), PITCH = 32 * EPV + EPV;  // a piece of 32 channels in LDS, and one to keep pieces in different banks
+    constexpr bool LONG = sizeof(E) == 2 && G * NB > 11;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_bytes[];
     __shared__ __attribute__((aligned(16))) float bias_s[NB * 32];
+    __shared__ __attribute__((aligned(16))) E bias_e[NB * 32];
     E *lds = (E *)lds_bytes;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, half = lane >> 5;
     const int oc0 = blockIdx.y * (NB * 32), ocs = min(NB * 32, a.s.OC - oc0);
 
-    // ---- the filter: through LDS (rows of K elements, as they lie in memory) into fragments; rows past OC and pieces past
-    // the last run are zeros
-    {
+    const int pieces = a.s.FH * a.P, tail = a.run - (a.P - 1) * EPV;  // elements of a run's last piece
+    unsigned tail_mask[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) tail_mask[d] = first_mask<E>(tail, d);
+    // ---- the filter.  Half: piece by piece from memory, with zeros behind the last run and behind each run's end, into LDS in the
+    // order of the fragments, and from there into registers (picked out of rows in LDS, five dwords and a shift each, they took
+    // 4.7 us of a 7x7x3 stem's 15.5, so 3.8).  fp32: through LDS as rows of K elements, as they lie in memory.
+    if constexpr (sizeof(E) == 2) {
+        typedef E EVec __attribute__((ext_vector_type(EPV)));
+        typedef EVec EVec_any __attribute__((aligned(sizeof(E))));
+        constexpr int N = NB * 32 * 2 * G, IT = (N + 255) / 256;
+        const E *const w = (const E *)a.w;
+        const int total = a.s.OC * a.K;
+        u32x4 v[IT];
+        int moved[IT];  // elements that a piece was read before its place (the last ones of the filter, which nothing follows)
+#pragma unroll
+        for (int u = 0; u < IT; ++u) {
+            moved[u] = 0;
+            const int i = u * 256 + threadIdx.x, ch = i / (2 * G), p = i - ch * (2 * G), fy = quotient(p, a.mg_pieces, a.P), j = p - fy * a.P;
+            // (channels past OC repeat the last: their results are not stored)
+            const int at = (oc0 + min(ch, ocs - 1)) * a.K + fy * a.run + j * EPV;
+            v[u] = (u32x4){0u, 0u, 0u, 0u};
+            if (p < pieces && ch < NB * 32) {
+                if (total >= EPV) {
+                    const int from = min(at, total - EPV), shift = at - from;
+                    u32x4 t = __builtin_bit_cast(u32x4, (EVec)*(const EVec_any *)(w + from));
+                    v[u] = t, moved[u] = shift;
+                } else {
+                    E t[EPV] = {};
+                    for (int e = 0; e < EPV; ++e)
+                        if (at + e < total) t[e] = w[at + e];
+                    v[u] = *(u32x4 *)t;
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < IT; ++u) {
+            const int i = u * 256 + threadIdx.x, ch = i / (2 * G), p = i - ch * (2 * G);
+            if (moved[u]) {
+                u32x4 t = v[u];
+                const int dwords = moved[u] * (int)sizeof(E) / 4;
+                if (dwords & 2) t = (u32x4){t[2], t[3], 0u, 0u};
+                if (dwords & 1) t = (u32x4){t[1], t[2], t[3], 0u};
+                if (sizeof(E) == 2 && (moved[u] & 1)) t = (u32x4){t[0] >> 16 | t[1] << 16, t[1] >> 16 | t[2] << 16, t[2] >> 16 | t[3] << 16, t[3] >> 16};
+                v[u] = t;
+            }
+            const unsigned all = (p + 1) - quotient(p + 1, a.mg_pieces, a.P) * a.P ? 0xffffffffu : 0u;  // (not a run's last piece)
+#pragma unroll
+            for (int d = 0; d < 4; ++d) v[u][d] &= tail_mask[d] | all;
+            if (ch < NB * 32) *(u32x4 *)(lds + ((ch >> 5) * (2 * G) + p) * PITCH + (ch & 31) * EPV) = v[u];
+        }
+    } else {
         const E *w = (const E *)a.w + (long)oc0 * a.K;
         const int n = ocs * a.K;
         if (((size_t)w & 15) == 0) {
-            constexpr int LOADS = 5;  // in flight at a time: all that a thread loads of 64 x 7x7x3 in half
+            constexpr int LOADS = 5;  // in flight at a time
             for (int i = threadIdx.x * EPV; i + EPV <= n; i += LOADS * 256 * EPV) {
                 u32x4 v[LOADS];
 #pragma unroll
@@ -158,16 +211,15 @@ __global__ __launch_bounds__(256, 2) void conv_direct_forward_kernel(DirectArgs 
         } else {
             for (int i = threadIdx.x; i < n; i += 256) lds[i] = w[i];
         }
-        if (threadIdx.x < NB * 32) bias_s[threadIdx.x] = a.bias && (int)threadIdx.x < ocs ? (float)((const E *)a.bias)[oc0 + threadIdx.x] : 0.f;
+    }
+    if (threadIdx.x < NB * 32) {
+        const E b = a.bias && (int)threadIdx.x < ocs ? ((const E *)a.bias)[oc0 + threadIdx.x] : (E)0.f;
+        bias_e[threadIdx.x] = b, bias_s[threadIdx.x] = (float)b;
     }
     __syncthreads();
     Frag wf[NB][G];
     int koff[G];              // element offset of this lane's piece of each group from its pixel's first element
     unsigned some = 0, all = 0;  // bit g: the piece has elements of the patch (may be a run's last one) / only such
-    const int tail = a.run - (a.P - 1) * EPV;  // elements of a run's last piece
-    unsigned tail_mask[4];
-#pragma unroll
-    for (int d = 0; d < 4; ++d) tail_mask[d] = first_mask<E>(tail, d);
     auto piece_mask = [&](int d, int g) -> unsigned {
         return (tail_mask[d] & (unsigned)((int)(some << (31 - g)) >> 31)) | (unsigned)((int)(all << (31 - g)) >> 31);
     };
@@ -181,24 +233,30 @@ __global__ __launch_bounds__(256, 2) void conv_direct_forward_kernel(DirectArgs 
         all |= in && !last ? 1u << g : 0u;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
-            // (channels past OC repeat the last: their results are not stored)
-            u32x4 v = piece_at<E, true>(lds, min(nb * 32 + l32, ocs - 1) * a.K + woff);
+            if constexpr (sizeof(E) == 2) {
+                wf[nb][g] = *(const Frag *)(lds + (nb * (2 * G) + 2 * g + half) * PITCH + l32 * EPV);
+            } else {
+                // (channels past OC repeat the last: their results are not stored)
+                u32x4 v = piece_at<E, true>(lds, min(nb * 32 + l32, ocs - 1) * a.K + woff);
 #pragma unroll
-            for (int d = 0; d < 4; ++d) v[d] &= piece_mask(d, g);
-            wf[nb][g] = __builtin_bit_cast(Frag, v);
+                for (int d = 0; d < 4; ++d) v[d] &= piece_mask(d, g);
+                wf[nb][g] = __builtin_bit_cast(Frag, v);
+            }
         }
-        if (g % 3 == 2) __builtin_amdgcn_sched_barrier(0);  // (all reads at once would not fit the registers)
+        if (sizeof(E) == 4 && g % 3 == 2) __builtin_amdgcn_sched_barrier(0);  // (all reads at once would not fit the registers)
         j += 2;
 #pragma unroll
         for (int u = 0; u < 2; ++u)
             if (j >= a.P) j -= a.P, ++fy;
     }
+    const int mine = pieces - half, zeros = a.zeros;
     const int blocks = (a.TR * a.TC + 31) / 32;
     const bool vec = a.s.OC % EPV == 0 && ((size_t)a.z & 15) == 0;
     for (int t = blockIdx.x; t < a.ntiles; t += gridDim.x) {
         const TileAt at = tile_at(a, t);
         __syncthreads();  // the filter's fragments have been read; every wave is done with the tile before
         stage_image<E>(a, at, lds);
+        if (LONG && threadIdx.x < 8) ((unsigned *)(lds + zeros))[threadIdx.x] = 0u;
         __syncthreads();
         E *const z0 = (E *)a.z + (((long)at.b * a.s.OH + at.oy0) * a.s.OW + at.ox0) * a.s.OC + oc0;
         const int rows_here = min(a.TR, a.s.OH - at.oy0), cols_here = min(a.TC, a.s.OW - at.ox0);
@@ -214,9 +272,17 @@ __global__ __launch_bounds__(256, 2) void conv_direct_forward_kernel(DirectArgs 
             if constexpr (G * NB > 11) asm volatile("" : "+v"(some), "+v"(all));
 #pragma unroll
             for (int g = 0; g < G; ++g) {
-                u32x4 v = piece_at<E, ODD>(lds, base + koff[g]);
+                u32x4 v;
+                if constexpr (LONG) {  // (pieces past the last are read where zeros lie: one instruction a dword is left of the masks)
+                    v = piece_at<E, ODD>(lds, 2 * g >= mine ? zeros : base + koff[g]);
+                    const unsigned whole = (unsigned)((int)(all << (31 - g)) >> 31);
 #pragma unroll
-                for (int d = 0; d < 4; ++d) v[d] &= piece_mask(d, g);
+                    for (int d = 0; d < 4; ++d) v[d] &= tail_mask[d] | whole;
+                } else {
+                    v = piece_at<E, ODD>(lds, base + koff[g]);
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) v[d] &= piece_mask(d, g);
+                }
                 const Frag f = __builtin_bit_cast(Frag, v);
 #pragma unroll
                 for (int e = 0; e < EL::MFMA_PER_FRAG; ++e)
@@ -229,23 +295,36 @@ __global__ __launch_bounds__(256, 2) void conv_direct_forward_kernel(DirectArgs 
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
                 // register i of the block is channel 8 * (i / 4) + 4 * half + i % 4 of this lane's pixel
-                E o[16];
-                f32x4 bias[4];
-                if (a.bias)
+                typedef E E2 __attribute__((ext_vector_type(2)));
+                E2 o[8];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) bias[i] = *(const f32x4 *)(bias_s + nb * 32 + 8 * i + 4 * half);
+                for (int q4 = 0; q4 < 4; ++q4) {
+                    const int at_bias = nb * 32 + 8 * q4 + 4 * half;
+                    f32x4 v = {acc[nb][4 * q4], acc[nb][4 * q4 + 1], acc[nb][4 * q4 + 2], acc[nb][4 * q4 + 3]};
+                    if (sizeof(E) == 2 && a.round_first) {  // (the half sum of two halfs is their fp32 sum rounded to half)
+                        o[2 * q4] = __builtin_convertvector(v.xy, E2), o[2 * q4 + 1] = __builtin_convertvector(v.zw, E2);
+                        if (a.bias) {
+                            typedef E E4 __attribute__((ext_vector_type(4)));
+                            const E4 add = *(const E4 *)(bias_e + at_bias);
+                            o[2 * q4] += add.xy, o[2 * q4 + 1] += add.zw;
+                        }
+                    } else {
+                        if (a.bias) v += *(const f32x4 *)(bias_s + at_bias);
+                        if (sizeof(E) == 4 && a.relu)
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    float v = acc[nb][i];
-                    if (a.bias) v = (sizeof(E) == 2 && a.round_first ? (float)(E)v : v) + bias[i >> 2][i & 3];
-                    o[i] = (E)(a.relu && !(v > 0.f) ? 0.f : v);
+                            for (int e = 0; e < 4; ++e) v[e] = !(v[e] > 0.f) ? 0.f : v[e];
+                        o[2 * q4] = __builtin_convertvector(v.xy, E2), o[2 * q4 + 1] = __builtin_convertvector(v.zw, E2);
+                    }
+                    if (sizeof(E) == 2 && a.relu)
+#pragma unroll
+                        for (int e = 0; e < 2; ++e) o[2 * q4 + e] = __builtin_elementwise_max(o[2 * q4 + e], (E2){(E)0.f, (E)0.f});
                 }
                 if (vec) {
                     if constexpr (sizeof(E) == 4) {
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
                             const int n = nb * 32 + 8 * i + 4 * half;
-                            if (px >= 0 && n < ocs) *(f32x4 *)(z + n) = (f32x4){(float)o[4 * i], (float)o[4 * i + 1], (float)o[4 * i + 2], (float)o[4 * i + 3]};
+                            if (px >= 0 && n < ocs) *(f32x4 *)(z + n) = (f32x4){(float)o[2 * i][0], (float)o[2 * i][1], (float)o[2 * i + 1][0], (float)o[2 * i + 1][1]};
                         }
                     } else {
                         // the lower half of the wave takes channels 16 i .. + 7 of its pixel, the upper 16 i + 8 .. + 15
@@ -254,8 +333,7 @@ __global__ __launch_bounds__(256, 2) void conv_direct_forward_kernel(DirectArgs 
                             u32x4 out;
 #pragma unroll
                             for (int d = 0; d < 2; ++d) {
-                                const f16x2 lo = {(f16)o[8 * i + 2 * d], (f16)o[8 * i + 2 * d + 1]}, hi = {(f16)o[8 * i + 4 + 2 * d], (f16)o[8 * i + 5 + 2 * d]};
-                                const auto s = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, lo), __builtin_bit_cast(unsigned, hi), false, false);
+                                const auto s = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, o[4 * i + d]), __builtin_bit_cast(unsigned, o[4 * i + 2 + d]), false, false);
                                 out[d] = s[0], out[d + 2] = s[1];
                             }
                             const int n = nb * 32 + 16 * i + 8 * half;
@@ -266,7 +344,7 @@ __global__ __launch_bounds__(256, 2) void conv_direct_forward_kernel(DirectArgs 
 #pragma unroll
                     for (int i = 0; i < 16; ++i) {
                         const int n = nb * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
-                        if (n < ocs) z[n] = o[i];
+                        if (n < ocs) z[n] = o[i >> 1][i & 1];
                     }
                 }
             }
@@ -480,9 +558,9 @@ bool plan_tiles(int dtype, const DirectShape &s, const void *x, int grain, int p
         long pitch = (long)(TCp - 1) * s.sx * s.C + (long)a.P * epv + (a.vec_x - 1) + 2;
         const int unit = a.vec_x > 2 / es ? a.vec_x : 2;
         pitch = (pitch + unit - 1) / unit * unit;
-        const long bytes = ((rows * pitch * es + 15) & ~15L) + 16 + px * px_bytes;
+        const long image = ((rows * pitch * es + 15) & ~15L) + 16, bytes = image + (grain > 1 ? px * px_bytes : 32);
         if (px > pixels + k_group || rows * pitch >= (1 << 15) || bytes > LDS_LIMIT) return false;
-        a.TR = TR, a.TC = TC, a.TCp = TCp, a.pixels_p = (int)px, a.rows = (int)rows, a.pitch = (int)pitch, lds = (size_t)bytes;
+        a.TR = TR, a.TC = TC, a.TCp = TCp, a.pixels_p = (int)px, a.rows = (int)rows, a.pitch = (int)pitch, a.zeros = (int)(image / es), lds = (size_t)bytes;
         return true;
     };
     int TC = a.TC;
@@ -500,6 +578,7 @@ bool plan_tiles(int dtype, const DirectShape &s, const void *x, int grain, int p
     if (tiles >= (1L << 30)) return false;
     a.ntiles = (int)tiles;
     a.mg_chunks = magic_up(a.pitch / a.vec_x);
+    a.mg_pieces = magic_up(a.P);
     a.mg_tc = magic_up(grain > 1 ? a.TCp : a.TC);
     if (lds < (size_t)min_bytes) lds = min_bytes;
     return lds <= (size_t)LDS_LIMIT;
@@ -508,7 +587,11 @@ bool plan_tiles(int dtype, const DirectShape &s, const void *x, int grain, int p
 template <typename E, int G, int NB>
 int launch_forward(const DirectArgs &a, size_t lds, bool odd, hipStream_t stream) {
     const dim3 grid((unsigned)(a.ntiles < 2 * cu_count() ? a.ntiles : 2 * cu_count()), (unsigned)ceil_div(a.s.OC, NB * 32));
+    // (fp32, ten groups: 135 registers let three workgroups share a compute unit; where there are more than that, the variant of 128
+    // takes all of a fourth round off, 43 x 133x133x1 -> 64 7x7 166 -> 119 us; where not, the other one is up to 3 % faster)
+    const bool many = sizeof(E) == 4 && G == 10 && (long)grid.x * grid.y > 3L * cu_count();
     if (sizeof(E) == 2 && odd) hipLaunchKernelGGL((conv_direct_forward_kernel<E, G, NB, sizeof(E) == 2>), grid, dim3(256), lds, stream, a);
+    else if (many) hipLaunchKernelGGL((conv_direct_forward_kernel<E, G, NB, false, sizeof(E) == 4 && G == 10 ? 4 : 2>), grid, dim3(256), lds, stream, a);
     else hipLaunchKernelGGL((conv_direct_forward_kernel<E, G, NB, false>), grid, dim3(256), lds, stream, a);
     D8_LAUNCH_CHECK();
     return 0;
@@ -517,8 +600,14 @@ int launch_forward(const DirectArgs &a, size_t lds, bool odd, hipStream_t stream
 // channels per workgroup: the filter's fragments are what fills the registers (8 dwords a group for 64 channels)
 int forward_channels(int dtype, const DirectShape &s) { return dtype == D8_FLOAT16 && s.OC > 32 ? 64 : 32; }
 
+// k groups that the kernel keeps of them
+int forward_groups(int dtype, const DirectShape &s) {
+    const int groups = ceil_div(pieces_of(dtype, s), 2);
+    return dtype == D8_FLOAT16 ? (groups <= 3 ? 3 : groups <= 5 ? 5 : 11) : (groups <= 5 ? 5 : groups <= 10 ? 10 : 21);
+}
+
 bool plan_forward(int dtype, const DirectShape &s, const void *x, DirectArgs &a, size_t &lds) {
-    const int es = (int)dtype_bytes(dtype), filter = (forward_channels(dtype, s) * s.FH * s.FW * s.C + 8) * es + 16;
+    const int ch = forward_channels(dtype, s), filter = dtype == D8_FLOAT16 ? ch / 32 * 2 * forward_groups(dtype, s) * 33 * 16 : (ch * s.FH * s.FW * s.C + 8) * 4 + 16;
     return plan_tiles(dtype, s, x, 1, 256, 0, filter, a, lds);
 }
 
@@ -556,8 +645,7 @@ double conv_direct_forward_us(int dtype, const DirectShape &s, const void *x) {
     size_t lds;
     if (!plan_forward(dtype, s, x, a, lds)) return INFINITY;
     const bool half = dtype == D8_FLOAT16;
-    const int es = half ? 2 : 4, ch = forward_channels(dtype, s), groups = ceil_div(pieces_of(dtype, s), 2), cus = cu_count();
-    const int kept = half ? (groups <= 3 ? 3 : groups <= 5 ? 5 : 11) : (groups <= 5 ? 5 : groups <= 10 ? 10 : 21);
+    const int es = half ? 2 : 4, ch = forward_channels(dtype, s), kept = forward_groups(dtype, s), cus = cu_count();
     const long wide = a.ntiles < 2 * cus ? a.ntiles : 2 * cus, wgs = wide * ceil_div(s.OC, ch), per_cu = (wgs + cus - 1) / cus;
     const double rounds = (double)((wgs + 2 * cus - 1) / (2 * cus)), tiles = (double)((a.ntiles + wide - 1) / wide);
     const double blocks = per_cu * tiles * ceil_div(ceil_div(a.TR * a.TC, 32), 4), accesses = rounds * tiles * ceil_div(a.rows * (a.pitch / a.vec_x), 256);
@@ -601,34 +689,38 @@ double conv_direct_grad_us(int dtype, const DirectShape &s, const void *x, const
 // 224x224x3 -> 64, 7x7 stride 2 (K = 147): patch matrix + padded filter + product 81 -> 23 us (26 MB are stored: 5 us at a
 // copy's rate; what the rest goes on is the filter's fragments and a block's chain of LDS reads, products and stores); fp32 64 x 28x28x1 -> 32,
 // 5x5: patch matrix + product 18 -> 11 us.
-// Now 19.7 and 7.3 us: the bias is read four values at a time, the filter's loads are in flight together, and masks are not kept for
+// Then 19.7 and 7.3 us: the bias is read four values at a time, the filter's loads are in flight together, and masks are not kept for
 // every group where the filter is long (two workgroups per compute unit need at most 256 registers; 295 gave 29.8 us).  A
 // block of z is stored from registers, 16 bytes a lane: turned around through LDS for whole lines it took 21.2 and 7.5 us, and the
 // LDS (8 - 16 KB) and registers kept workgroups off the compute unit (fp32 32 x 311x311x4 -> 64, 5x5 stride 4, 113 us, now 88).  Image
 // rows of the next tile fetched into registers gave nothing beside several workgroups.  248 drawn layers, all three against
 // none: with bias and ReLu 3142 us, now 2901; without 3098 us (125 layers more than 3 % slower than when z was not
-// turned around), now 2853 (one).
+// turned around), then 2853 (one).
+// Now 17.0 and 7.25 us: in half, filter fragments that are read from LDS whole, one mask instruction a dword where the filter is
+// long, and bias and ReLu on packed halfs, the bias read four values at a time (two at a time it is 18.2): 50 drawn half layers 10 %
+// faster at the mean, 40 in fp32 2 %, none more than 2 % slower.  Two blocks at a time for a wave gave nothing (the
+// instructions count, not their latencies) and took registers that workgroups need (32 x 163x145x3 -> 80 3x3 64 -> 98).
 int conv_direct_forward(int dtype, const DirectShape &s, const void *x, const void *w, void *z, const void *bias, int relu,
                         int round_first, hipStream_t stream) {
     DirectArgs a;
     size_t lds;
     D8_REQUIRE(conv_direct_eligible(dtype, s) && plan_forward(dtype, s, x, a, lds), "conv_direct_forward: the layer does not fit");
     a.w = w, a.z = z, a.bias = bias, a.relu = relu, a.round_first = round_first;
-    const int groups = ceil_div(pieces_of(dtype, s), 2);
+    const int groups = forward_groups(dtype, s);
     if (dtype == D8_FLOAT32) {
-        if (groups <= 5) return launch_forward<float, 5, 1>(a, lds, false, stream);
-        if (groups <= 10) return launch_forward<float, 10, 1>(a, lds, false, stream);
+        if (groups == 5) return launch_forward<float, 5, 1>(a, lds, false, stream);
+        if (groups == 10) return launch_forward<float, 10, 1>(a, lds, false, stream);
         return launch_forward<float, 21, 1>(a, lds, false, stream);
     }
     // every patch starts at an even element of an even pitch
     const bool odd = (s.sx * s.C) % 2 != 0 || (s.pl * s.C) % 2 != 0;
     if (s.OC > 32) {
-        if (groups <= 3) return launch_forward<f16, 3, 2>(a, lds, odd, stream);
-        if (groups <= 5) return launch_forward<f16, 5, 2>(a, lds, odd, stream);
+        if (groups == 3) return launch_forward<f16, 3, 2>(a, lds, odd, stream);
+        if (groups == 5) return launch_forward<f16, 5, 2>(a, lds, odd, stream);
         return launch_forward<f16, 11, 2>(a, lds, odd, stream);
     }
-    if (groups <= 3) return launch_forward<f16, 3, 1>(a, lds, odd, stream);
-    if (groups <= 5) return launch_forward<f16, 5, 1>(a, lds, odd, stream);
+    if (groups == 3) return launch_forward<f16, 3, 1>(a, lds, odd, stream);
+    if (groups == 5) return launch_forward<f16, 5, 1>(a, lds, odd, stream);
     return launch_forward<f16, 11, 1>(a, lds, odd, stream);
 }
 
