@@ -416,6 +416,20 @@ __device__ __forceinline__ void store_tile(f32x16 (&acc)[T::TM][T::TN], float *l
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, lhi = lane >> 5;
     if (!crow.perm_OC && (LOOSE || (aligned && N % 8 == 0 && ((size_t)bias & 15) == 0))) {
         float *patch = (wave < HALF_WAVES ? lds0 + wave * (32 * 36) : lds1 + (wave - HALF_WAVES) * (32 * 36));
+        // fp32: the bias of a lane's columns before the first store, because a load that is waited for behind a store waits for
+        // the store's acknowledgement too (51 drawn layers with bias and ReLu 1.7 % faster at the mean, Conv2d 13 x 10x9x64 -> 128
+        // 1x1 stride 2 11.4 -> 9.7 us; half, with half as many stores, 0.4 % slower)
+        constexpr bool BIAS_FIRST = sizeof(O) == 4;
+        OV bias_v[BIAS_FIRST ? TN : 1][8 / OPV];
+        if constexpr (BIAS_FIRST)
+            if (bias)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    const int n = o.n0 + o.wn0 + j * 32 + (lane & 3) * 8;
+                    if (n + 8 <= N)
+#pragma unroll
+                        for (int h = 0; h < 8 / OPV; ++h) bias_v[j][h] = *(const MV *)(bias + n + h * OPV);
+                }
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -441,7 +455,9 @@ __device__ __forceinline__ void store_tile(f32x16 (&acc)[T::TM][T::TN], float *l
                                 for (int e = 0; e < OPV; ++e) v[h * OPV + e] += as_f32(old[e]);
                             }
                             if (bias) {
-                                const OV bv = *(const MV *)(bias + n + h * OPV);
+                                OV bv;
+                                if constexpr (BIAS_FIRST) bv = bias_v[j][h];
+                                else bv = *(const MV *)(bias + n + h * OPV);
 #pragma unroll
                                 for (int e = 0; e < OPV; ++e) v[h * OPV + e] = (round_first ? as_f32((O)v[h * OPV + e]) : v[h * OPV + e]) + as_f32(bv[e]);
                             }
