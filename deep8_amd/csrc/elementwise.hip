@@ -107,41 +107,51 @@ __global__ __launch_bounds__(256) void accumulate_kernel(T *__restrict__ g, cons
     }
 }
 
-// The column sums of a block's 256 / TX row lanes meet in LDS, lane 0's first and the others' in their order, and every column's sum
-// is handed to done(column, sum).  `met` lanes had a row.  A thread adds one column at a time, eight lanes' sums in flight, where one
-// had VEC columns and waited for each lane's sums before it asked for the next's.  With the finishing kernel's loads all in flight,
-// ReLu gate and bias gradient of half 6272 x 256 7.3 -> 5.8 us, 13456 x 160 7.4 -> 5.9 (a launch takes 2.8 of the program's thread).
+// The column sums of a block's 256 / TX row lanes meet in LDS: 256 / (TX * VEC) threads a column take the lanes in as many runs, eight in
+// flight at a time, and the runs' sums are added in order; every column's sum is handed to done(column, sum).  `met` lanes had a
+// row.  (One thread had VEC columns and waited for each lane's sums before it asked for the next's.  With the finishing
+// kernel's loads all in flight, ReLu gate and bias gradient of half 6272 x 256 7.3 -> 5.8 us, 13456 x 160 7.4 -> 5.9.)
 // last_start: rows that start at any element, whose last columns' vector was moved back to start there; else 0.
 template <int VEC, class Done>
 __device__ __forceinline__ void meet_in_lds(float *part, const float (&acc)[VEC], int TX, int tx, int ty, int met, int C, int last_start, Done &&done) {
-    const int width = TX * VEC;
+    const int width = TX * VEC, bits = __builtin_ctz(width), i = threadIdx.x & (width - 1), seg = threadIdx.x >> bits, segs = 256 >> bits;
 #pragma unroll
     for (int e = 0; e < VEC; ++e) part[ty * width + tx * VEC + e] = acc[e];
     __syncthreads();
-    for (int i = threadIdx.x; i < width; i += 256) {
-        const long c = (long)blockIdx.x * width + i;
-        if (c >= C) break;
-        // (a vector that was moved back holds column c that much further on)
-        const int at = i + (last_start ? max(0, (int)(blockIdx.x * width + i / VEC * VEC) - last_start) : 0);
+    const long c = (long)blockIdx.x * width + i;
+    // (a vector that was moved back holds column c that much further on)
+    const int at = min(i + (last_start ? max(0, (int)(blockIdx.x * width + i / VEC * VEC) - last_start) : 0), width - 1);
+    const int run = width <= 8 && met <= 64 ? 64 : max(32, (met + segs - 1) >> (8 - bits));
+    // sum of n values `width` apart from p[0] on, eight in flight
+    auto sum = [&](const float *p, int n) -> float {
         float v = 0.f;
         int k = 0;
-        for (; k + 7 < met; k += 8) {
+        for (; k + 7 < n; k += 8) {
             float t[8];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) t[u] = part[(k + u) * width + at];
+            for (int u = 0; u < 8; ++u) t[u] = p[(k + u) * width];
 #pragma unroll
             for (int u = 0; u < 8; ++u) v += t[u];
         }
-        if (k < met) {
+        if (k < n) {
             float t[7];
 #pragma unroll
-            for (int u = 0; u < 7; ++u) t[u] = part[min(k + u, met - 1) * width + at];
+            for (int u = 0; u < 7; ++u) t[u] = p[min(k + u, n - 1) * width];
 #pragma unroll
             for (int u = 0; u < 7; ++u)
-                if (k + u < met) v += t[u];
+                if (k + u < n) v += t[u];
         }
-        done((int)c, v);
+        return v;
+    };
+    float v = sum(part + seg * run * width + at, min(met - seg * run, run));
+    if (run < met) {
+        __syncthreads();
+        part[threadIdx.x] = v;
+        __syncthreads();
+        v = sum(part + i, (met + run - 1) / run);
     }
+    if (seg > 0) return;
+    if (c < C) done((int)c, v);
 }
 
 // dz viewed [K0][R][C]; sums over R.  Block (x: column group, y: chunk of R, z: k0); TX threads
@@ -500,6 +510,16 @@ static ReducePlan plan_reduce(const int *d, const int *zd) {
     return p;
 }
 
+// Column sums of few rows in one launch: how many threads lie across a row's 16-byte pieces, so that the others take up to 64 rows
+// in flight each (0: more rows, which take chunks and a second launch).  The launch that it saves takes 2.5 us, a row of a block
+// of few pieces some 2 ns.  ReLu gate and bias gradient, us in chunks / so, with 4 and 8 across: half 128 x 1024 5.2 / 3.1, 2.9;
+// 256 x 1024 5.3 / 3.1, 3.4; 512 x 1024 5.5 / 3.8, 4.7; 1024 x 1024 5.55 / 5.1, 7.3.  Behind the layer's product, which leaves z in other XCDs'
+// caches, fewer rows: dense layers with their gradients of 128 rows 8 - 20 % faster, of 256 5 - 15 %, of 512 1 - 5 %, of 640 to 1024
+// level to 6 % slower.
+static int one_chunk_tx(long rows) {
+    return rows <= 64 || rows > 512 ? 0 : rows <= 128 ? 8 : 4;  // (up to 64 rows are one chunk anyway)
+}
+
 // g = keep * g + scale * (op(dz) summed over the axes where g has extent 1 and dz does not)
 template <typename T, int WIDE, int OP = LOAD_ID>
 static int reduce_t(T *g, const int *d, const T *dz, const int *zd, void *scratch, size_t scratch_bytes, hipStream_t s,
@@ -518,8 +538,9 @@ static int reduce_t(T *g, const int *d, const T *dz, const int *zd, void *scratc
         const bool wide = p.C % WIDE == 0 && al16(g) && al16(dz);
         const int vec = wide ? WIDE : 1;
         const long cvs = p.C / vec;
-        int TX = 1;
-        while (TX < 32 && TX < cvs) TX *= 2;
+        int TX = 1, most = 32;
+        if (const int narrow = wide && p.K0 == 1 ? one_chunk_tx(p.R) : 0) most = narrow, chunks = 1, rpc = (int)p.R;
+        while (TX < most && TX < cvs) TX *= 2;
         dim3 grid((unsigned)((cvs + TX - 1) / TX), (unsigned)chunks, (unsigned)p.K0);
         if (wide)
             hipLaunchKernelGGL((column_sum_kernel<T, WIDE, OP>), grid, dim3(256), 0, s, dz, g, (float *)scratch, (int)p.R, (int)p.C,
@@ -630,8 +651,11 @@ static int relu_gate_sum_t(const T *z, const T *dz, T *dpre, T *g, long rows, in
     const bool any = !wide && cols > 16 * WIDE;
     const int vec = wide || any ? WIDE : 1;
     const long cvs = ((long)cols + vec - 1) / vec;
-    int TX = 1;
-    while (TX < 32 && TX < cvs) TX *= 2;
+    int TX = 1, most = 32;
+    // (as d8_add_grad on dpre would)
+    const bool few = p.kind == 1 && cols % WIDE == 0 && al16(g) && al16(dpre);
+    if (const int narrow = few ? one_chunk_tx(rows) : 0) most = narrow, chunks = 1, rpc = (int)rows;
+    while (TX < most && TX < cvs) TX *= 2;
     dim3 grid((unsigned)((cvs + TX - 1) / TX), (unsigned)chunks, 1);
     if (any)
         hipLaunchKernelGGL((relu_gate_column_sum_kernel<T, WIDE, true>), grid, dim3(256), 0, s, z, dz, dpre, g, (float *)scratch, (int)rows, cols, TX, rpc, chunks, keep);
