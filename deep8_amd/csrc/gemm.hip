@@ -844,10 +844,10 @@ size_t gemm_tiled_workspace(int dtype, int M, int N, int K, int red, int virt) {
 // theirs is a quarter of the work; in half, whose step waits longer than it multiplies, half of it (through registers 0.25 us against
 // 0.38 for a 64 x 128 tile and 0.46 for 128 x 128).  The same pieces -- or none, and no second pass -- spread over four times as many
 // workgroups.  The estimate counts steps of a 128 x 128 tile (about 2 us of a CU in fp32, 0.5 us in half), for the plan that g
-// holds (splits set) and for 64 x 64 tiles in 1 .. as many pieces as that plan; 7 % or more decide.  It was fitted to half tiles
-// that pass through registers: straight into LDS the steps take 454, 620 and 1270 cycles (870 with four stages), i.e. 0.36 : 0.49 : 1
-// where 0.5 : 0.76 : 1 is counted, and the plans are still those of then.  A 64 x 128 half step is 0.76 here and 0.65 in plan_few_tiles, a half product's second pass 6.5 steps + 1
-// per 0.25e6 outputs and piece here, 14 + 1 per 0.5e6 there, which only chooses among 128-wide tiles.
+// holds (splits set) and for 64 x 64 tiles in 1 .. as many pieces as that plan; 7 % or more decide.  In half it was fitted to tiles
+// that pass through registers, and says only what a call takes (gemm_estimate_us); half_tile_us decides.  A 64 x 128 half step is 0.76
+// here and 0.65 in plan_few_tiles, a half product's second pass 6.5 steps + 1 per 0.25e6 outputs and piece here, 14 + 1 per 0.5e6
+// there, which only chooses among 128-wide tiles.
 // A narrow output (128 x 32 tiles, below) counts its pieces the same way.
 // NN, us before and after (M x K x N; NT and TN alike): fp32 512 x 512 x 512 16.4 -> 10.2, 784 x 1152 x 128 16.0 -> 10.3,
 // 1024 x 1024 x 1024 33.6 -> 23.5, 12544 x 800 x 64 24.0 -> 17.0, 3136 x 576 x 256 24.5 -> 12.7, 1536 x 1536 x 1536
@@ -867,6 +867,21 @@ static double tile_cost(bool half_elems, int bm, int bn, const GemmArgs &g, long
     return n * len * area * (n == 1 ? 1.1 : area < 0.3 ? 1.08 : 1.0) + 0.5 + 2.0 * sqrt(area) + 0.3 * (n - 1) + (s > 1 ? 2.0 + s * (mn / 2e6) : 0.0);
 }
 
+// ... in half, in microseconds, of tiles whose operands go straight into LDS: a workgroup's ends, its steps, a further round, what
+// patch rows take longer, and a second pass.  Fitted to 80 drawn forward products and convolutions of at most 255 128 x 128 tiles, each on three
+// tiles in 1 to 12 pieces; 5 % or more decide.  (The estimate above, which 7 % had to decide, counts the same ends for all
+// tiles, and for products of few steps those are most of the time.)  110 drawn half products and convolutions forward 1384 ->
+// 1358 us, 3.4 % at the mean, both gradients of 104 of them 2434 -> 2410, 1.9 %; three of the 214 calls more than 3 % slower (by 0.2
+// us): 218 x 64 x 1328 5.6 -> 4.0, 1504 x 3648 x 128 14.6 -> 10.8, Conv2d 37 x 8x8x64 -> 368 1x1 6.2 -> 4.7.
+static double half_tile_us(int bm, int bn, const GemmArgs &g, long total, long s) {
+    const long cus = cu_count(), n = (ceil_div(g.M, bm) * (long)ceil_div(g.N, bn) * g.batch * s + cus - 1) / cus, len = (total + s - 1) / s;
+    const int k = bm * bn == 128 * 128 ? 2 : bm * bn == 64 * 64 ? 0 : 1;
+    const double ends[3] = {3.6, 4.1, 4.1}, step[3] = {0.23, 0.31, 0.47}, rows[3] = {0.95, 1.25, 1.65};
+    const double far = k == 0 ? (2.0 * g.red * g.K * g.batch * ((double)g.M + g.N) - 4e6) / 8e6 : 0.0;  // (see above)
+    return ends[k] + n * len * (step[k] + 0.11 * (far < 0.0 ? 0.0 : far > 1.0 ? 1.0 : far)) + 0.2 * (n - 1) + (g.virt == VIRT_A_ROWS ? rows[k] : 0.0) +
+           (s > 1 ? 2.6 + 1.85e-6 * s * g.M * (double)g.N * g.batch : 0.0);
+}
+
 static void few_tiles_small(int dtype, GemmArgs &g, int transA, int transB, size_t usable) {
     // (a filter gradient's pieces stay those of the launch it may share with the input's: one sum, one result)
     if (g.virt == VIRT_A_CLASSES || g.virt == VIRT_B_KROWS || gemm_is_small(g.M, g.N, g.K, g.batch, g.red)) return;
@@ -879,16 +894,19 @@ static void few_tiles_small(int dtype, GemmArgs &g, int transA, int transB, size
     const long total = (long)g.red * ceil_div(g.K, BK);
     const bool half = g.splits == 1 && gemm_tiled_half_tiles(g.M, g.N, g.batch, total, BK);
     const bool narrow = g.tile_hint == HINT_128x32;
-    const double now = narrow ? 1e30 : g.N < 128 ? tile_cost(half_elems, 128, 64, g, total, g.splits) : tile_cost(half_elems, g.M < 128 || half ? 64 : 128, 128, g, total, g.splits);
+    auto cost = [&](int bm, int bn, long pieces) {
+        return half_elems ? half_tile_us(bm, bn, g, total, pieces) : tile_cost(false, bm, bn, g, total, pieces);
+    };
+    const double now = narrow ? 1e30 : g.N < 128 ? cost(128, 64, g.splits) : cost(g.M < 128 || half ? 64 : 128, 128, g.splits);
     long most = (long)(usable / ((size_t)g.batch * g.M * g.N * sizeof(float)));
     int tps;  // (no more pieces than the 128-wide plan would have: what the scratch queries provide for, whatever is passed)
     const long planned = plan_splits(BK, g.M, g.N, g.K, g.batch, g.red, (size_t)-1, &tps, g.virt);
     if (most > planned) most = planned;
     if (most > total / 2) most = total / 2;
-    double best = 0.93 * now;
+    double best = (half_elems ? 0.95 : 0.93) * now;
     long pieces = 0;
     for (long s = 1; s == 1 || s <= most; ++s)
-        if (const double c = narrow ? tile_cost(half_elems, 128, 32, g, total, s) : tile_cost(half_elems, 64, 64, g, total, s); c < best) best = c, pieces = s;
+        if (const double c = narrow ? cost(128, 32, s) : cost(64, 64, s); c < best) best = c, pieces = s;
     if (!pieces) return;
     if (!narrow) g.tile_hint = HINT_64x64;
     g.tiles_per_split = (int)((total + pieces - 1) / pieces);
