@@ -400,7 +400,7 @@ __device__ __forceinline__ void gemm_split_reduce_body(const GemmArgs &g, const 
     if (!tiny) {
         // (a last group of fewer than 4 is loaded with the outputs before it and moved down.  Pieces past the last and groups past
         // the last are fetched at an offset outside the buffer, as zeros: no load lies behind a branch)
-        const int back = ROWS ? 0 : 4 - n_out;
+        const int back = ROWS || !live ? 0 : 4 - n_out;
         const unsigned bytes = (unsigned)(g.splits * g.batch) * (unsigned)mn * 4u, step = (unsigned)(LANES * mn) * 4u;
         const __amdgpu_buffer_rsrc_t ws = __builtin_amdgcn_make_buffer_rsrc(g.ws, 0, (int)bytes, 0x00020000);
         const unsigned at = live ? (unsigned)((b * g.splits + row) * mn + r - back) * 4u : 0x80000000u;
@@ -417,7 +417,10 @@ __device__ __forceinline__ void gemm_split_reduce_body(const GemmArgs &g, const 
         for (; g.splits - s > 4 * LANES; s += 8 * LANES) add(std::integral_constant<int, 8>(), s);
         if (g.splits - s > 2 * LANES) add(std::integral_constant<int, 4>(), s);
         else if (g.splits - s > 0) add(std::integral_constant<int, 2>(), s);
-        for (int k = 0; k < back; ++k) v = (f32x4){v[1], v[2], v[3], 0.f};
+        if constexpr (!ROWS)
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                if (k < back) v = (f32x4){v[1], v[2], v[3], 0.f};
     } else if (live) {  // an output of fewer than 4 in all
         const float *p = g.ws + (long)b * g.splits * mn;
         for (int s = row; s < g.splits; s += LANES)
