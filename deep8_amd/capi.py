@@ -79,6 +79,7 @@ SIGNATURES = {
     "d8_conv_grad_kept_pair_launches": (ctypes.c_ulong, []),
     "d8_conv_route_calls": (ctypes.c_ulong, [_I]),
     "d8_matmul_grad_pair_launches": (ctypes.c_ulong, []),
+    "d8_matmul_grad_kept_pair_launches": (ctypes.c_ulong, []),
     "d8_matmul_grad_copied_calls": (ctypes.c_ulong, []),
     "d8_conv2d_grad_xy": (_I, [_I, _P, _P, _I, _I, _I, _I, _P, _P, _I, _I, _I, _P] + [_I] * 6 + [_P, _Z, _P]),
     "d8_deconv2d_grad_xy": (_I, [_I, _P, _P, _I, _I, _I, _I, _P, _P, _I, _I, _I, _P] + [_I] * 4 + [_P, _Z, _P]),

@@ -348,6 +348,7 @@ static bool gemm_is_small(int M, int N, int K, int batch, int red) {
            batch * 1L < 65536;
 }
 
+static long small_workgroups(const GemmArgs &g) { return (long)ceil_div(g.M, 32) * ceil_div(g.N, 32) * g.batch; }
 // C[b][m][n] = beta * C + sum_s ws[b][s][m][n].  A workgroup covers groups of 4 consecutive outputs.
 // Few pieces of many groups (LANES = 1): 256 groups, a thread adds all pieces of its group in order.  Else (LANES = 8): 32 groups, 8 thread rows each add every 8th piece, and the 8 sums meet in
 // LDS in a fixed order.  Either way the result does not depend on scheduling, and up to 8 pieces
@@ -769,18 +770,21 @@ static int launch_reduce_pair(int dtype, const GemmArgs &p0, const GemmArgs &p1,
 }
 
 template <typename T>
+static int launch_small(const GemmArgs &g, int transA, int transB, hipStream_t stream) {
+    dim3 grid(ceil_div(g.N, 32), ceil_div(g.M, 32), g.batch);
+    if (!transA && !transB)
+        hipLaunchKernelGGL((gemm_small_kernel<T, false, false>), grid, dim3(SMALL_WAVES * 64), 0, stream, g);
+    else if (!transA && transB)
+        hipLaunchKernelGGL((gemm_small_kernel<T, false, true>), grid, dim3(SMALL_WAVES * 64), 0, stream, g);
+    else
+        hipLaunchKernelGGL((gemm_small_kernel<T, true, false>), grid, dim3(SMALL_WAVES * 64), 0, stream, g);
+    D8_LAUNCH_CHECK();
+    return 0;
+}
+
+template <typename T>
 static int launch(GemmArgs &g, int transA, int transB, bool tiled, hipStream_t stream) {
-    if (g.virt == VIRT_NONE && g.splits == 1 && gemm_is_small(g.M, g.N, g.K, g.batch, g.red)) {
-        dim3 grid(ceil_div(g.N, 32), ceil_div(g.M, 32), g.batch);
-        if (!transA && !transB)
-            hipLaunchKernelGGL((gemm_small_kernel<T, false, false>), grid, dim3(SMALL_WAVES * 64), 0, stream, g);
-        else if (!transA && transB)
-            hipLaunchKernelGGL((gemm_small_kernel<T, false, true>), grid, dim3(SMALL_WAVES * 64), 0, stream, g);
-        else
-            hipLaunchKernelGGL((gemm_small_kernel<T, true, false>), grid, dim3(SMALL_WAVES * 64), 0, stream, g);
-        D8_LAUNCH_CHECK();
-        return 0;
-    }
+    if (g.virt == VIRT_NONE && g.splits == 1 && gemm_is_small(g.M, g.N, g.K, g.batch, g.red)) return launch_small<T>(g, transA, transB, stream);
     if (tiled) {
         if (int rc = gemm_tiled_launch(sizeof(T) == 2 ? D8_FLOAT16 : D8_FLOAT32, g, transA, transB, stream)) return rc;
     } else {
@@ -968,6 +972,10 @@ static int gemm_tiled_run_whole(int dtype, GemmArgs &g, int transA, int transB, 
     return dtype == D8_FLOAT16 ? launch<f16>(g, transA, transB, true, stream) : launch<float>(g, transA, transB, true, stream);
 }
 
+int gemm_small_run(int dtype, const GemmArgs &g, int transA, int transB, hipStream_t stream) {
+    return dtype == D8_FLOAT16 ? launch_small<f16>(g, transA, transB, stream) : launch_small<float>(g, transA, transB, stream);
+}
+
 int gemm_tiled_run(int dtype, GemmArgs &g, int transA, int transB, void *workspace, size_t workspace_bytes,
                    hipStream_t stream) {
     if (narrow_output(dtype, g)) g.tile_hint = HINT_128x32;
@@ -1003,15 +1011,25 @@ int gemm_tiled_run(int dtype, GemmArgs &g, int transA, int transB, void *workspa
     return gemm_tiled_run_whole(dtype, second, transA, transB, workspace, workspace_bytes, stream);
 }
 
-// The two gradients of a small MatrixMultiply (g0 = dZ . Y^T, NT; g1 = X^T . dZ, TN; both small in the sense of
-// gemm_is_small, neither Float64) as one launch.  False, with nothing launched, when they do not qualify.
-bool gemm_small_pair_run(int dtype, const GemmArgs &g0, int ta0, int tb0, const GemmArgs &g1, int ta1, int tb1, hipStream_t stream, int *rc) {
+// Whether the two gradients of a MatrixMultiply (g0 = dZ . Y^T, NT; g1 = X^T . dZ, TN) run on the kernel for small products, in
+// one launch where one call asks for both: both small in the sense of gemm_is_small.
+bool gemm_gradients_are_small(int dtype, const GemmArgs &g0, int ta0, int tb0, const GemmArgs &g1, int ta1, int tb1) {
     if (dtype == D8_FLOAT64 || ta0 || !tb0 || !ta1 || tb1) return false;
     if (g0.virt != VIRT_NONE || g1.virt != VIRT_NONE || g0.K < 1 || g1.K < 1) return false;
-    if (!gemm_is_small(g0.M, g0.N, g0.K, g0.batch, g0.red) || !gemm_is_small(g1.M, g1.N, g1.K, g1.batch, g1.red)) return false;
+    const long n = small_workgroups(g0) + small_workgroups(g1);
+    if (gemm_is_small(g0.M, g0.N, g0.K, g0.batch, g0.red) && gemm_is_small(g1.M, g1.N, g1.K, g1.batch, g1.red)) return n <= 0x7fffffffL;
+    return false;
+}
+
+static bool whole_steps(int dtype, const GemmArgs &g0, const GemmArgs &g1) {
+    const int BK = gemm_tiled_k_step(dtype);
+    return g0.K % BK == 0 && g1.K % BK == 0;
+}
+
+SharedLaunch gemm_small_pair_run(int dtype, const GemmArgs &g0, int ta0, int tb0, const GemmArgs &g1, int ta1, int tb1, hipStream_t stream, int *rc) {
+    if (!gemm_gradients_are_small(dtype, g0, ta0, tb0, g1, ta1, tb1)) return APART;
     const int nx0 = ceil_div(g0.N, 32), ny0 = ceil_div(g0.M, 32), nx1 = ceil_div(g1.N, 32), ny1 = ceil_div(g1.M, 32);
-    const long n0 = (long)nx0 * ny0 * g0.batch, n1 = (long)nx1 * ny1 * g1.batch;
-    if (n0 + n1 > 0x7fffffffL) return false;
+    const long n0 = small_workgroups(g0), n1 = small_workgroups(g1);
     GemmArgs a = g0, b = g1;
     a.splits = b.splits = 1;
     a.by.nbx = reciprocal_of(nx0), a.by.tiles = reciprocal_of(nx0 * ny0), b.by.nbx = reciprocal_of(nx1), b.by.tiles = reciprocal_of(nx1 * ny1);
@@ -1021,7 +1039,8 @@ bool gemm_small_pair_run(int dtype, const GemmArgs &g0, int ta0, int tb0, const 
         hipLaunchKernelGGL((gemm_small_pair_kernel<float>), dim3((unsigned)(n0 + n1)), dim3(SMALL_WAVES * 64), 0, stream, a, b, nx0, ny0, (int)n0, nx1, ny1);
     const hipError_t e = hipGetLastError();
     *rc = e == hipSuccess ? 0 : fail((int)e, "kernel launch: %s", hipGetErrorString(e));
-    return true;
+    const bool small = gemm_is_small(g0.M, g0.N, g0.K, g0.batch, g0.red) && gemm_is_small(g1.M, g1.N, g1.K, g1.batch, g1.red);
+    return small || whole_steps(dtype, g0, g1) ? SHARED : SHARED_KEPT;
 }
 
 // d8_conv_grad_pair_launches, d8_conv_grad_kept_pair_launches
@@ -1117,13 +1136,21 @@ int gemm_tiled_kept_pair_run(int dtype, const GemmArgs &gx, const GemmArgs &gy, 
     return launch_reduce_pair(dtype, gx, gy, stream);
 }
 
-static bool plain_pair_plan(int dtype, GemmArgs &g0, int ta0, int tb0, GemmArgs &g1, int ta1, int tb1, void *workspace, size_t workspace_bytes) {
+// Both gradients of a MatrixMultiply in one launch, each cut as it would be alone, whatever K leaves of a last step and however
+// many workgroups there are: a launch or two fewer, and one last round instead of two.  us apart / so: a K step cut short, of 90
+// drawn calls the 25 that are, 1.29 times as fast at the mean: fp32 448 x 304 x 152 15.8 / 10.2, 648 x 1128 x 64 15.4 / 11.5; half 368 x 824 x
+// 64 8.8 / 6.8, 5864 x 568 x 576 27.6 / 22.1.  More workgroups than the chip holds, longer ones first, 58 drawn calls in fp32 3750 / 3331:
+// 608 x 2816 x 768 61.5 / 46.4, 4096 x 2112 x 480 179 / 143, 4352 x 448 x 832 63.8 / 73.0, the others at least 0.96 times as fast; in half 4 x 3072 x
+// 680 x 1152 70.9 / 54.1, 3072 x 3584 x 744 59.0 / 48.4.
+static SharedLaunch plain_pair_plan(int dtype, GemmArgs &g0, int ta0, int tb0, GemmArgs &g1, int ta1, int tb1, void *workspace, size_t workspace_bytes) {
     const bool off = getenv("D8_MATMUL_GRADS_APART") != nullptr;  // tuning and test aid (read at every call)
-    if (off || dtype == D8_FLOAT64 || ta0 || !tb0 || !ta1 || tb1) return false;
-    if (g0.virt != VIRT_NONE || g1.virt != VIRT_NONE || g0.K < 1 || g1.K < 1) return false;
-    if (!g0.packed && !g1.packed && (!gemm_tiled_eligible(dtype, g0, ta0, tb0, TILED_PIECES) || !gemm_tiled_eligible(dtype, g1, ta1, tb1, TILED_PIECES))) return false;
-    if (gemm_is_small(g0.M, g0.N, g0.K, g0.batch, g0.red) || gemm_is_small(g1.M, g1.N, g1.K, g1.batch, g1.red)) return false;
-    if (balanced_rows(g0) || balanced_rows(g1)) return false;
+    if (off || dtype == D8_FLOAT64 || ta0 || !tb0 || !ta1 || tb1) return APART;
+    if (g0.virt != VIRT_NONE || g1.virt != VIRT_NONE || g0.K < 1 || g1.K < 1) return APART;
+    for (const GemmArgs *g : {&g0, &g1})
+        if (g->batch > 448 || g->M > 65535 * 128) return APART;  // (beyond one launch's limits: d8_gemm cuts it into several)
+    if (!g0.packed && !g1.packed && (!gemm_tiled_eligible(dtype, g0, ta0, tb0, TILED_PIECES) || !gemm_tiled_eligible(dtype, g1, ta1, tb1, TILED_PIECES))) return APART;
+    if (gemm_is_small(g0.M, g0.N, g0.K, g0.batch, g0.red) || gemm_is_small(g1.M, g1.N, g1.K, g1.batch, g1.red)) return APART;
+    if (balanced_rows(g0) || balanced_rows(g1)) return APART;
     const size_t usable = (workspace && ((size_t)workspace & 15) == 0) ? workspace_bytes : 0;
     const int BK = gemm_tiled_k_step(dtype);
     // each split as it would be alone, the partial sums of the two side by side in the workspace
@@ -1137,11 +1164,12 @@ static bool plain_pair_plan(int dtype, GemmArgs &g0, int ta0, int tb0, GemmArgs 
     }
     const size_t need0 = g0.splits > 1 ? ((size_t)g0.splits * g0.batch * g0.M * g0.N * sizeof(float) + 255) & ~(size_t)255 : 0;
     const size_t need1 = g1.splits > 1 ? (size_t)g1.splits * g1.batch * g1.M * g1.N * sizeof(float) : 0;
-    if (need0 + need1 > usable) return false;
+    if (need0 + need1 > usable) return APART;
     g0.ws = (float *)workspace, g1.ws = (float *)((char *)workspace + need0);
     g0.tail_splits = g1.tail_splits = 0;
     const long wgs = gemm_tiled_plain_pair_workgroups(dtype, g0, g1);
-    return wgs > 0 && wgs <= 2L * cu_count();
+    if (wgs <= 0 || wgs > 0x7fffffffL) return APART;
+    return wgs <= 2L * cu_count() && (g0.packed || whole_steps(dtype, g0, g1)) ? SHARED : SHARED_KEPT;
 }
 
 static int plain_pair_run(int dtype, const GemmArgs &g0, const GemmArgs &g1, hipStream_t stream) {
@@ -1149,11 +1177,11 @@ static int plain_pair_run(int dtype, const GemmArgs &g0, const GemmArgs &g1, hip
     return launch_reduce_pair(dtype, g0, g1, stream);
 }
 
-bool gemm_tiled_run_plain_pair(int dtype, GemmArgs &g0, int ta0, int tb0, GemmArgs &g1, int ta1, int tb1, void *workspace,
-                               size_t workspace_bytes, hipStream_t stream, int *rc) {
-    if (!plain_pair_plan(dtype, g0, ta0, tb0, g1, ta1, tb1, workspace, workspace_bytes)) return false;
-    *rc = plain_pair_run(dtype, g0, g1, stream);
-    return true;
+SharedLaunch gemm_tiled_run_plain_pair(int dtype, GemmArgs &g0, int ta0, int tb0, GemmArgs &g1, int ta1, int tb1, void *workspace,
+                                       size_t workspace_bytes, hipStream_t stream, int *rc) {
+    const SharedLaunch shared = plain_pair_plan(dtype, g0, ta0, tb0, g1, ta1, tb1, workspace, workspace_bytes);
+    if (shared) *rc = plain_pair_run(dtype, g0, g1, stream);
+    return shared;
 }
 
 // Where the copies go, one behind the other.  A thread copies a piece of four rows, or of one where that leaves compute units without
@@ -1187,7 +1215,7 @@ struct PackRun {
     PackPlan plan;
     PackLaunch copies;
     GemmArgs g[2];
-    bool shared;
+    SharedLaunch shared;
 };
 // The product on its copies.
 static GemmArgs packed_args(GemmArgs g, const int (&slot)[2], const PackList &list) {
@@ -1230,7 +1258,7 @@ size_t gemm_pack_bytes(int dtype, const PackedProduct (&p)[2]) {
     return pack_run_plan(dtype, p, (void *)4096, (size_t)1 << 62, r) ? r.plan.bytes : 0;
 }
 
-bool gemm_pack_run(int dtype, const PackedProduct (&p)[2], void *workspace, size_t workspace_bytes, hipStream_t stream, bool *shared, int *rc) {
+bool gemm_pack_run(int dtype, const PackedProduct (&p)[2], void *workspace, size_t workspace_bytes, hipStream_t stream, SharedLaunch *shared, int *rc) {
     PackRun r;
     if (!pack_run_plan(dtype, p, workspace, workspace_bytes, r)) return false;
     *shared = r.shared;

@@ -134,6 +134,9 @@ struct GemmArgs {
 
 enum { HINT_NONE = 0, HINT_64x64 = 1, HINT_128x32 = 2 };  // GemmArgs::tile_hint
 
+// Whether two gradients have run as one launch: SHARED if their reductions are whole K steps (or both are small, or copies) and all their
+// workgroups fit the chip at once, else SHARED_KEPT.  The two are counted apart (d8_matmul_grad_pair_launches, ..._kept_pair_launches).
+enum SharedLaunch { APART = 0, SHARED, SHARED_KEPT };
 enum TiledRule { TILED_ANY, TILED_PIECES, TILED_WHOLE };  // see gemm_tiled_eligible
 
 // Whether a product with these arguments would run on a kernel that applies GemmArgs::bias / relu in its store
@@ -180,6 +183,8 @@ int gemm_tiled_pair_classes_f32(const GemmArgs &gx, const GemmArgs &gy, hipStrea
 // (g.splits / tiles_per_split / ws set; the caller reduces).
 long gemm_tiled_plain_pair_workgroups(int dtype, const GemmArgs &g0, const GemmArgs &g1);
 int gemm_tiled_plain_pair_launch(int dtype, const GemmArgs &g0, const GemmArgs &g1, hipStream_t stream);
+int gemm_tiled_plain_pair_pieces_f16(const GemmArgs &g0, const GemmArgs &g1, hipStream_t stream);
+int gemm_tiled_plain_pair_pieces_f32(const GemmArgs &g0, const GemmArgs &g1, hipStream_t stream);
 // Where the next launches write their per-workgroup phase records (GemmArgs::phase_rec); null switches them off.
 void gemm_tiled_phase_record(void *records, size_t bytes);
 
@@ -194,9 +199,11 @@ int gemm_wide_launch(const GemmArgs &g, int transA, int transB, hipStream_t stre
 int gemm_wide_pair_launch(const GemmArgs &g0, int transA0, int transB0, const GemmArgs &g1, int transA1, int transB1,
                           hipStream_t stream);
 
-// The two gradients of a small MatrixMultiply (NT then TN, both on the small-product kernel) as ONE launch; false, with
-// nothing launched, when they do not qualify.
-bool gemm_small_pair_run(int dtype, const GemmArgs &g0, int ta0, int tb0, const GemmArgs &g1, int ta1, int tb1, hipStream_t stream, int *rc);
+// Whether the two gradients of a MatrixMultiply (NT, TN) run on the small-product kernel, and one of them on it.
+bool gemm_gradients_are_small(int dtype, const GemmArgs &g0, int ta0, int tb0, const GemmArgs &g1, int ta1, int tb1);
+int gemm_small_run(int dtype, const GemmArgs &g, int transA, int transB, hipStream_t stream);
+// Both as ONE launch; APART, with nothing launched, when they do not qualify.
+SharedLaunch gemm_small_pair_run(int dtype, const GemmArgs &g0, int ta0, int tb0, const GemmArgs &g1, int ta1, int tb1, hipStream_t stream, int *rc);
 
 // fp64 kernel (64 x 64 or 128 x 128 tiles, v_mfma_f64_16x16x4_f64): any shape; plans its own split of the
 // reduction from g.ws / g.ws_bytes (double partial sums) and reduces.
@@ -217,7 +224,7 @@ struct PackedProduct {
     GemmArgs *g;
     int ta, tb;
 };
-bool gemm_pack_run(int dtype, const PackedProduct (&p)[2], void *workspace, size_t workspace_bytes, hipStream_t stream, bool *shared, int *rc);
+bool gemm_pack_run(int dtype, const PackedProduct (&p)[2], void *workspace, size_t workspace_bytes, hipStream_t stream, SharedLaunch *shared, int *rc);
 size_t gemm_pack_bytes(int dtype, const PackedProduct (&p)[2]);  // what it takes of the workspace (0: it does not pay)
 // The same for a forward product by itself (bias and ReLu included: the caller has checked gemm_fuses_store).
 bool gemm_pack_run_one(int dtype, const PackedProduct &p, void *workspace, size_t workspace_bytes, hipStream_t stream, int *rc);
@@ -233,7 +240,7 @@ bool gemm_tiled_run_pair(int dtype, GemmArgs &gx, GemmArgs &gy, void *workspace,
 // The two gradients of a mid-size MatrixMultiply (g0 = dZ . Y^T, NT; g1 = X^T . dZ, TN; both on the tiled kernels, all their
 // workgroups resident at once) as one launch plus their split reductions; false, with nothing launched, otherwise.
 // The workspace holds both products' partial sums side by side.
-bool gemm_tiled_run_plain_pair(int dtype, GemmArgs &g0, int ta0, int tb0, GemmArgs &g1, int ta1, int tb1, void *workspace,
+SharedLaunch gemm_tiled_run_plain_pair(int dtype, GemmArgs &g0, int ta0, int tb0, GemmArgs &g1, int ta1, int tb1, void *workspace,
                                size_t workspace_bytes, hipStream_t stream, int *rc);
 // Microseconds that a product is expected to take with all the workspace it asks for (which of two ways a convolution goes).
 double gemm_estimate_us(int dtype, const GemmArgs &g, int transA, int transB);

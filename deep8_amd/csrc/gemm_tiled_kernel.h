@@ -1031,13 +1031,13 @@ __global__ __launch_bounds__(T::NT, T::VIRT == VIRT_A_CLASSES && T::BN == 128 ||
 // that nothing hides when a compute unit holds one workgroup), and side by side on a compute unit one's waits are
 // the other's issue slots.  The operand areas are as large as the larger tile needs.
 template <typename T0, typename T1, int EDGE = EDGE_NONE>
-__global__ __launch_bounds__(T0::NT, T0::TWO_FIT && T1::TWO_FIT ? 2 : 1) void gemm_tiled_pair_kernel(GemmArgs g0, GemmArgs g1, int tilesM0, int tilesN0, int nx0, int nz0,
-                                                                 int tilesM1, int tilesN1, int nx1) {
+__global__ __launch_bounds__(T0::NT, T0::TWO_FIT && T1::TWO_FIT ? 2 : 1) void gemm_tiled_pair_kernel(int ahead, int nx0, int nz0, int nx1, int tilesM0, int tilesN0,
+                                                                 int tilesM1, int tilesN1, GemmArgs g0, GemmArgs g1) {
     typedef typename T0::E E;
     static_assert(T0::NT == T1::NT && sizeof(typename T0::E) == sizeof(typename T1::E) && T0::DMA == T1::DMA, "one workgroup shape, one element type");
     if constexpr (T0::DMA) {
         __shared__ __attribute__((aligned(1024))) E stages[(T0::LDS_BYTES > T1::LDS_BYTES ? T0::LDS_BYTES : T1::LDS_BYTES) / T0::ES];
-        const int id = (int)blockIdx.x, first = nx0 * nz0, j = id - first;
+        const int at = (int)blockIdx.x, first = nx0 * nz0, id = at < ahead ? at + first : at - ahead, j = id - first;
         int bx;
         if (id < first) {
             const int bz = Divisor(nx0, g0.by.nbx).div(id, bx);
@@ -1052,7 +1052,7 @@ __global__ __launch_bounds__(T0::NT, T0::TWO_FIT && T1::TWO_FIT ? 2 : 1) void ge
         __shared__ __attribute__((aligned(16))) E As1[A_SZ];
         __shared__ __attribute__((aligned(16))) E Bs0[B_SZ];
         __shared__ __attribute__((aligned(16))) E Bs1[B_SZ];
-        const int id = (int)blockIdx.x, first = nx0 * nz0;
+        const int at = (int)blockIdx.x, first = nx0 * nz0, id = at < ahead ? at + first : at - ahead;
         int bx;
         if (id < first) {
             const int bz = Divisor(nx0, g0.by.nbx).div(id, bx);
@@ -1174,7 +1174,6 @@ static int launch_pair_tiles(const GemmArgs &gx0, const GemmArgs &gy0, hipStream
     const bool tail = gx.tail_splits > 0;
     const int tMx = ceil_div(tail ? gx.tail_m0 : gx.M, TX::BM), tNx = ceil_div(gx.N, TX::BN), tMy = ceil_div(gy.M, TY::BM), tNy = ceil_div(gy.N, TY::BN);
     const int extra = tail ? ceil_div(gx.M - gx.tail_m0, TX::BM) * tNx * gx.tail_splits : 0;
-    // the longer-running product first: gy's pieces, then gx's tiles
     const int ny = tMy * tNy, nzy = gy.batch * gy.splits, nx = tMx * tNx + extra;
     const int nzx = TX::VIRT == VIRT_A_CLASSES ? gx.ncls : tail ? 1 : gx.batch * gx.splits;
     // phase records (a measurement aid): gy's workgroups first, then gx's, tagged 0 and 1
@@ -1188,9 +1187,20 @@ static int launch_pair_tiles(const GemmArgs &gx0, const GemmArgs &gy0, hipStream
     else lds = 2L * ((TX::A_SZ > TY::A_SZ ? TX::A_SZ : TY::A_SZ) + (TX::B_SZ > TY::B_SZ ? TX::B_SZ : TY::B_SZ)) * TX::ES;
     const long wgs = (long)ny * nzy + (long)nx * nzx, cus = cu_count();
     const unsigned pad = lds <= third && wgs > cus && wgs <= 2 * cus ? (unsigned)(third + 512 - lds) : 0u;
+    // Of more workgroups than compute units the longer ones first, gx's (`ahead` of them) or gy's: what starts last runs alone at the end.
+    auto time = [](const GemmArgs &g, int bm, int bn, int bk, double red) {
+        const double steps = g.splits > 1 ? g.tiles_per_split : red * ceil_div(g.K, bk);
+        return steps * (TX::DMA ? bm + bn : bm * bn);  // (half waits for its loads, fp32 for its matrix instructions)
+    };
+    double red = gx.red;
+    if constexpr (TX::VIRT == VIRT_A_CLASSES) {  // (at the mean)
+        red = 0;
+        for (int i = 0; i < gx.ncls; ++i) red += (double)gx.cls[i].red / gx.ncls;
+    }
+    const int ahead = wgs > cus && time(gx, TX::BM, TX::BN, TX::BK, red) > time(gy, TY::BM, TY::BN, TY::BK, gy.red) ? nx * nzx : 0;
     set_reciprocals(gy, tMy, tNy, TY::BM, TY::BK, ny);
     set_reciprocals(gx, tMx, tNx, TX::BM, TX::BK, nx);
-    hipLaunchKernelGGL((gemm_tiled_pair_kernel<TY, TX, EDGE>), dim3(ny * nzy + nx * nzx), dim3(TX::NT), pad, stream, gy, gx, tMy, tNy, ny, nzy, tMx, tNx, nx);
+    hipLaunchKernelGGL((gemm_tiled_pair_kernel<TY, TX, EDGE>), dim3(ny * nzy + nx * nzx), dim3(TX::NT), pad, stream, ahead, ny, nzy, nx, tMy, tNy, tMx, tNx, gy, gx);
     D8_LAUNCH_CHECK();
     return 0;
 }

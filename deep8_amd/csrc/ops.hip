@@ -380,39 +380,53 @@ int d8_matmul_bias_relu(int dtype, const void *x, int xb, int xr, int xc, const 
     return run_bias_relu(dtype, p, bias, relu, scratch, scratch_bytes, stream);
 }
 
+// The gradient of input `which` alone: on the kernel that a call for both gradients takes, for the same bits.
+static int run_gradient(int dtype, int which, const Gemm &p, int xb, int xr, int xc, int yb, int yr, int yc, void *scratch, size_t scratch_bytes, void *stream) {
+    const Gemm other = mm_plan(3 - which, nullptr, xb, xr, xc, nullptr, yb, yr, yc, nullptr);
+    const GemmArgs g = to_args(p), h = to_args(other);
+    const bool small = which == 1 ? gemm_gradients_are_small(dtype, g, p.ta, p.tb, h, other.ta, other.tb)
+                                  : gemm_gradients_are_small(dtype, h, other.ta, other.tb, g, p.ta, p.tb);
+    return small ? gemm_small_run(dtype, g, p.ta, p.tb, as_stream(stream)) : run(dtype, p, scratch, scratch_bytes, stream);
+}
+
 int d8_matmul_grad_x(int dtype, void *dx, int xb, int xr, int xc, const void *y, int yb, int yr, int yc,
                      const void *dz, void *scratch, size_t scratch_bytes, void *stream) {
     if (int rc = check_mm("d8_matmul_grad_x", dtype, xb, xr, xc, yb, yr, yc)) return rc;
     D8_REQUIRE(dx && y && dz, "d8_matmul_grad_x: null tensor");
-    return run(dtype, mm_plan(1, dx, xb, xr, xc, y, yb, yr, yc, dz), scratch, scratch_bytes, stream);
+    return run_gradient(dtype, 1, mm_plan(1, dx, xb, xr, xc, y, yb, yr, yc, dz), xb, xr, xc, yb, yr, yc, scratch, scratch_bytes, stream);
 }
 
 int d8_matmul_grad_y(int dtype, const void *x, int xb, int xr, int xc, void *dy, int yb, int yr, int yc,
                      const void *dz, void *scratch, size_t scratch_bytes, void *stream) {
     if (int rc = check_mm("d8_matmul_grad_y", dtype, xb, xr, xc, yb, yr, yc)) return rc;
     D8_REQUIRE(x && dy && dz, "d8_matmul_grad_y: null tensor");
-    return run(dtype, mm_plan(2, x, xb, xr, xc, dy, yb, yr, yc, dz), scratch, scratch_bytes, stream);
+    return run_gradient(dtype, 2, mm_plan(2, x, xb, xr, xc, dy, yb, yr, yc, dz), xb, xr, xc, yb, yr, yc, scratch, scratch_bytes, stream);
 }
 
 int d8_matmul_grad_x_overwrite(int dtype, void *dx, int xb, int xr, int xc, const void *y, int yb, int yr, int yc,
                                const void *dz, void *scratch, size_t scratch_bytes, void *stream) {
     if (int rc = check_mm("d8_matmul_grad_x_overwrite", dtype, xb, xr, xc, yb, yr, yc)) return rc;
     D8_REQUIRE(dx && y && dz, "d8_matmul_grad_x_overwrite: null tensor");
-    return run(dtype, mm_plan(1, dx, xb, xr, xc, y, yb, yr, yc, dz, 0.f), scratch, scratch_bytes, stream);
+    return run_gradient(dtype, 1, mm_plan(1, dx, xb, xr, xc, y, yb, yr, yc, dz, 0.f), xb, xr, xc, yb, yr, yc, scratch, scratch_bytes, stream);
 }
 
 int d8_matmul_grad_y_overwrite(int dtype, const void *x, int xb, int xr, int xc, void *dy, int yb, int yr, int yc,
                                const void *dz, void *scratch, size_t scratch_bytes, void *stream) {
     if (int rc = check_mm("d8_matmul_grad_y_overwrite", dtype, xb, xr, xc, yb, yr, yc)) return rc;
     D8_REQUIRE(x && dy && dz, "d8_matmul_grad_y_overwrite: null tensor");
-    return run(dtype, mm_plan(2, x, xb, xr, xc, dy, yb, yr, yc, dz, 0.f), scratch, scratch_bytes, stream);
+    return run_gradient(dtype, 2, mm_plan(2, x, xb, xr, xc, dy, yb, yr, yc, dz, 0.f), xb, xr, xc, yb, yr, yc, scratch, scratch_bytes, stream);
 }
 
 unsigned long d8_conv_route_calls(int route) { return route >= 0 && route < 3 ? route_calls[route].load() : 0; }
 
-static std::atomic<unsigned long> matmul_pair_launches{0}, matmul_copied_calls{0};
+static std::atomic<unsigned long> matmul_pair_launches{0}, matmul_kept_pair_launches{0}, matmul_copied_calls{0};
 unsigned long d8_matmul_grad_copied_calls(void) { return matmul_copied_calls.load(); }
 unsigned long d8_matmul_grad_pair_launches(void) { return matmul_pair_launches.load(); }
+unsigned long d8_matmul_grad_kept_pair_launches(void) { return matmul_kept_pair_launches.load(); }
+static void count_shared(SharedLaunch shared) {
+    if (shared == SHARED) ++matmul_pair_launches;
+    if (shared == SHARED_KEPT) ++matmul_kept_pair_launches;
+}
 
 int d8_matmul_grad_xy(int dtype, const void *x, void *dx, int xb, int xr, int xc, const void *y, void *dy, int yb, int yr,
                       int yc, const void *dz, int overwrite, void *scratch, size_t scratch_bytes, void *stream) {
@@ -437,27 +451,24 @@ int d8_matmul_grad_xy(int dtype, const void *x, void *dx, int xb, int xr, int xc
             return gemm_wide_pair_launch(gx, px.ta, px.tb, gy, py.ta, py.tb, as_stream(stream));
         }
     }
-    {  // both products small: one launch of the small-product kernel's workgroups for both
-        int rc = 0;
-        if (gemm_small_pair_run(dtype, to_args(px), px.ta, px.tb, to_args(py), py.ta, py.tb, as_stream(stream), &rc)) {
-            ++matmul_pair_launches;
-            return rc;
-        }
+    int rc = 0;
+    GemmArgs gx = to_args(px), gy = to_args(py);
+    // both products small: one launch of the small-product kernel's workgroups for both
+    if (const SharedLaunch shared = gemm_small_pair_run(dtype, gx, px.ta, px.tb, gy, py.ta, py.tb, as_stream(stream), &rc)) {
+        count_shared(shared);
+        return rc;
     }
-    {  // both on the tiled kernels with all their workgroups resident at once: one launch, then their split reductions
-        int rc = 0;
-        GemmArgs gx = to_args(px), gy = to_args(py);
-        const PackedProduct both[2] = {{&gx, px.ta, px.tb}, {&gy, py.ta, py.tb}};
-        bool shared = false;
-        if (gemm_pack_run(dtype, both, scratch, scratch_bytes, as_stream(stream), &shared, &rc)) {
-            ++matmul_copied_calls;
-            if (shared) ++matmul_pair_launches;
-            return rc;
-        }
-        if (gemm_tiled_run_plain_pair(dtype, gx, px.ta, px.tb, gy, py.ta, py.tb, scratch, scratch_bytes, as_stream(stream), &rc)) {
-            ++matmul_pair_launches;
-            return rc;
-        }
+    // both on the tiled kernels: one launch, then their split reductions
+    const PackedProduct both[2] = {{&gx, px.ta, px.tb}, {&gy, py.ta, py.tb}};
+    SharedLaunch shared = APART;
+    if (gemm_pack_run(dtype, both, scratch, scratch_bytes, as_stream(stream), &shared, &rc)) {
+        ++matmul_copied_calls;
+        count_shared(shared);
+        return rc;
+    }
+    if ((shared = gemm_tiled_run_plain_pair(dtype, gx, px.ta, px.tb, gy, py.ta, py.tb, scratch, scratch_bytes, as_stream(stream), &rc))) {
+        count_shared(shared);
+        return rc;
     }
     if (int rc = run(dtype, px, scratch, scratch_bytes, stream)) return rc;
     return run(dtype, py, scratch, scratch_bytes, stream);

@@ -176,8 +176,9 @@ int d8_matmul_grad_y_overwrite(int dtype, const void *x, int xb, int xr, int xc,
  * _overwrite forms above).  scratch: d8_matmul_scratch_bytes(which = 3), room for both gradients' scratch side by
  * side and, in Float16, for copies of the operands whose rows do not start at multiples of 16 bytes, where copies
  * pay; with less, but at least the larger of which = 1 and which = 2, the call still works (mid-size products
- * then run as two launches, and such operands are read as they lie, which takes longer).  Two small products (each at most four 128 x 128 tiles over a reduction of at most
- * 512) share a launch as well, and so do two mid-size ones whose workgroups all fit the chip at once.          */
+ * then run as two launches, and such operands are read as they lie, which takes longer).  Two small products share a launch as
+ * well (each at most four 128 x 128 tiles over a reduction of at most 512, or reductions of at most 512 -- in Float16 1024 --
+ * and no more 32 x 32 tiles than run at once), and so do two mid-size ones.                                             */
 int d8_matmul_grad_xy(int dtype, const void *x, void *dx, int xb, int xr, int xc,
                       const void *y, void *dy, int yb, int yr, int yc, const void *dz, int overwrite,
                       void *scratch, size_t scratch_bytes, void *stream);
@@ -302,7 +303,8 @@ int d8_deconv2d_grad_xy_ex(int dtype, const void *x, void *gx, int B, int IH, in
  * those whose two products are tiled and cut as they would be alone.  A call counts in one of them at most.        */
 unsigned long d8_conv_grad_pair_launches(void);
 unsigned long d8_conv_grad_kept_pair_launches(void);
-unsigned long d8_matmul_grad_pair_launches(void);  /* ... and of the d8_matmul_grad_xy calls */
+unsigned long d8_matmul_grad_pair_launches(void);  /* ... and of the d8_matmul_grad_xy calls: whole K steps, and no more workgroups than run at once; */
+unsigned long d8_matmul_grad_kept_pair_launches(void);  /* the others: a K step (64 in Float16, 32 in Float32) that is cut short, or more workgroups */
 unsigned long d8_matmul_grad_copied_calls(void);   /* d8_matmul_grad_xy calls that ran on copies of their odd operands */
 /* How many Conv2d / DeConv2d calls have run (each gradient is one; both gradients from one call are two), by route: 0 on an
  * interim matrix in scratch, 1 with the patches read by the GEMM's loader, 2 on the kernels for images of few channels. */
