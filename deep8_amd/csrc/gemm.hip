@@ -348,7 +348,23 @@ static bool gemm_is_small(int M, int N, int K, int batch, int red) {
            batch * 1L < 65536;
 }
 
+// Larger outputs of as short a reduction: what the kernel can hold, on as many workgroups as run at once.  Beyond that the loads of a
+// 32 x 32 tile, which a larger one would share, take longer than the way from memory that all of them wait for once.
+// us, tiled / so, by workgroups; 70 drawn forward products: fp32 64 x 200 x 640 (40) 7.8 / 4.5, 2824 x 272 x 64 (178) 9.0 / 5.2, 3 x 192 x 192 x 704
+// (396) 7.2 / 6.3, 2944 x 64 x 64, 3 of them (552) 5.1 / 5.7, 28 x 225 x 192 x 128 (896) 7.8 / 10.7; half 64 x 352 x 896 (56) 5.1 / 4.2, 317 x 128
+// x 592 (190) 4.3 / 3.6, 3520 x 576 x 46 (220) 11.8 / 5.3, 3 x 968 x 200 x 72 (279) 4.5 / 5.6, 2560 x 448 x 192 (480) 5.5 / 8.3; at the
+// mean 1.45 times as fast in fp32, 1.2 times in half.
+static bool gemm_fits_small(int dtype, const GemmArgs &g) {
+    const int KG = dtype == D8_FLOAT16 ? SmallOp<f16>::KG : SmallOp<float>::KG;
+    return dtype != D8_FLOAT64 && g.virt == VIRT_NONE && !g.packed && !g.perm_OC && g.K >= 1 && (long)g.red * ceil_div(g.K, KG) <= SMALL_WAVES * SMALL_MAXC;
+}
 static long small_workgroups(const GemmArgs &g) { return (long)ceil_div(g.M, 32) * ceil_div(g.N, 32) * g.batch; }
+// (products of rows by rows only: a gradient, which may share a launch, has a rule for the two of them, gemm_gradients_are_small)
+static bool gemm_is_short(int dtype, const GemmArgs &g) {
+    const long cus = cu_count();
+    return gemm_fits_small(dtype, g) && small_workgroups(g) <= (dtype == D8_FLOAT16 ? cus : cus * 3 / 2);
+}
+
 // C[b][m][n] = beta * C + sum_s ws[b][s][m][n].  A workgroup covers groups of 4 consecutive outputs.
 // Few pieces of many groups (LANES = 1): 256 groups, a thread adds all pieces of its group in order.  Else (LANES = 8): 32 groups, 8 thread rows each add every 8th piece, and the 8 sums meet in
 // LDS in a fixed order.  Either way the result does not depend on scheduling, and up to 8 pieces
@@ -694,7 +710,7 @@ static bool pack_pays(const PackedProduct *p, int products, const PackPlan &plan
         saved += (odd == 2 ? 0.25 : odd == 1 ? 0.2 : 0.0) * (share > alone ? share : alone);
         if (products == 2 && i == 0 && odd) least = 0.0;
         if (products == 1) {
-            if (g.M < 128 || g.N < 128) return false;
+            if (g.M < 128 || g.N < 128 || (gemm_is_short(D8_FLOAT16, g) && (long)g.red * g.K <= 512)) return false;
             least = 4 * tiles >= cus && total <= 32 ? 1.7 : 0.2;
         }
     }
@@ -978,6 +994,7 @@ int gemm_small_run(int dtype, const GemmArgs &g, int transA, int transB, hipStre
 
 int gemm_tiled_run(int dtype, GemmArgs &g, int transA, int transB, void *workspace, size_t workspace_bytes,
                    hipStream_t stream) {
+    if (!transA && !transB && gemm_is_short(dtype, g)) return gemm_small_run(dtype, g, transA, transB, stream);
     if (narrow_output(dtype, g)) g.tile_hint = HINT_128x32;
     static const bool no_cut = getenv("D8_GEMM_NO_ROW_CUT") != nullptr;  // tuning and test aid
     const int head = (no_cut || transA) ? 0 : balanced_rows(g);
@@ -1012,13 +1029,19 @@ int gemm_tiled_run(int dtype, GemmArgs &g, int transA, int transB, void *workspa
 }
 
 // Whether the two gradients of a MatrixMultiply (g0 = dZ . Y^T, NT; g1 = X^T . dZ, TN) run on the kernel for small products, in
-// one launch where one call asks for both: both small in the sense of gemm_is_small.
+// one launch where one call asks for both, and so that a call for one leaves the same bits: both small in the sense of
+// gemm_is_small, or both short and with no more workgroups than run at once.  us, as they ran before (two launches, or one of tiles
+// and a pass over partial sums) / so, by workgroups; 70 drawn calls: fp32 280 x 192 x 64 (66) 9.8 / 5.3, 64 x 704 x 336 (286)
+// 10.4 / 6.5, 64 x 2525 x 120 (474) 13.3 / 5.1, 128 x 3200 x 64 (600) 6.6 / 7.1; half 336 x 320 x 14 (120) 11.7 / 4.5, 640 x 320 x 128 (240)
+// 9.4 / 5.8, 384 x 832 x 64 (364) 6.2 / 6.6, 3 x 64 x 832 x 640 (676) 9.3 / 10.2.
 bool gemm_gradients_are_small(int dtype, const GemmArgs &g0, int ta0, int tb0, const GemmArgs &g1, int ta1, int tb1) {
     if (dtype == D8_FLOAT64 || ta0 || !tb0 || !ta1 || tb1) return false;
     if (g0.virt != VIRT_NONE || g1.virt != VIRT_NONE || g0.K < 1 || g1.K < 1) return false;
     const long n = small_workgroups(g0) + small_workgroups(g1);
     if (gemm_is_small(g0.M, g0.N, g0.K, g0.batch, g0.red) && gemm_is_small(g1.M, g1.N, g1.K, g1.batch, g1.red)) return n <= 0x7fffffffL;
-    return false;
+    const char *copies = getenv("D8_GEMM_PACK");  // (see pack_pays; both are tuning and test aids, read at every call)
+    if (getenv("D8_MATMUL_GRADS_APART") != nullptr || (copies && atoi(copies) != 0)) return false;
+    return gemm_fits_small(dtype, g0) && gemm_fits_small(dtype, g1) && n <= (dtype == D8_FLOAT16 ? 1L : 2L) * cu_count();
 }
 
 static bool whole_steps(int dtype, const GemmArgs &g0, const GemmArgs &g1) {
