@@ -704,18 +704,15 @@ static int d8_conv2d_grad_x_impl(int dtype, void *gx, int B, int IH, int IW, int
             if (int rc = launch_pad_rows(dtype, w, wp, OC, K, pitch, as_stream(stream))) return rc;
             Gemm plan = conv_plan(1, M, pitch, OC, colp, wp, gz);  // dxcol [M][pitch] = dz W, the padding columns come out 0
             if (int rc = run(dtype, plan, ws, scratch_bytes - ps.col - ps.filt, stream)) return rc;
-            if (beta == 0.f)  // col2im adds into its destination
-                if (int rc = d8_fill(dtype, gx, (size_t)B * IH * IW * IC, 0.f, stream)) return rc;
             const MapGeom mg = {B, IH, IW, IC, g[0], g[1], FH, FW, sy, sx, dy, dx, g[2], g[3], pitch};
-            return launch_col2im(dtype, colp, gx, mg, true, as_stream(stream));
+            return launch_col2im(dtype, colp, gx, mg, beta != 0.f, as_stream(stream));
         }
     }
     const size_t ws = scratch_bytes > col ? scratch_bytes - col : 0;
     if (int rc = run(dtype, conv_plan(1, M, K, OC, scratch, w, gz), ws ? (char *)scratch + col : nullptr, ws, stream))
         return rc;
-    if (beta == 0.f)  // col2im adds into its destination
-        if (int rc = d8_fill(dtype, gx, (size_t)B * IH * IW * IC, 0.f, stream)) return rc;
-    return d8_col2im(dtype, scratch, gx, B, IH, IW, IC, g[0], g[1], FH, FW, sy, sx, dy, dx, g[2], g[3], stream);
+    const MapGeom mg = {B, IH, IW, IC, g[0], g[1], FH, FW, sy, sx, dy, dx, g[2], g[3]};
+    return launch_col2im(dtype, scratch, gx, mg, beta != 0.f, as_stream(stream));
 }
 
 static int d8_conv2d_grad_y_impl(int dtype, const void *x, int B, int IH, int IW, int IC,
