@@ -77,6 +77,7 @@ SIGNATURES = {
     "d8_conv2d": (_I, [_I, _P, _I, _I, _I, _I, _P, _I, _I, _I, _P, _I, _I, _I, _I, _I, _P, _Z, _P]),
     "d8_conv_grad_pair_launches": (ctypes.c_ulong, []),
     "d8_conv_grad_kept_pair_launches": (ctypes.c_ulong, []),
+    "d8_conv_grad_crowded_pair_launches": (ctypes.c_ulong, []),
     "d8_conv_route_calls": (ctypes.c_ulong, [_I]),
     "d8_matmul_grad_pair_launches": (ctypes.c_ulong, []),
     "d8_matmul_grad_kept_pair_launches": (ctypes.c_ulong, []),

@@ -1066,8 +1066,8 @@ SharedLaunch gemm_small_pair_run(int dtype, const GemmArgs &g0, int ta0, int tb0
     return small || whole_steps(dtype, g0, g1) ? SHARED : SHARED_KEPT;
 }
 
-// d8_conv_grad_pair_launches, d8_conv_grad_kept_pair_launches
-static std::atomic<unsigned long> pair_launches{0}, kept_pair_launches{0};
+// d8_conv_grad_pair_launches, d8_conv_grad_kept_pair_launches, d8_conv_grad_crowded_pair_launches
+static std::atomic<unsigned long> pair_launches{0}, kept_pair_launches{0}, crowded_pair_launches{0};
 
 // Both gradients of a convolution as one launch (gemm_tiled_pair_launch) when that fills compute units the two
 // products would each leave idle: gx is not cut into a band and not split, the workgroups of both fit the chip
@@ -1138,7 +1138,7 @@ bool gemm_tiled_kept_pair_plan(int dtype, GemmArgs &gx, GemmArgs &gy, void *work
     gy.ws = (float *)workspace;
     gy.splits = plan_splits(BK, gy.M, gy.N, gy.K, 1, gy.red, usable, &gy.tiles_per_split, gy.virt);
     const auto tiles = dtype == D8_FLOAT16 ? gemm_tiled_kept_pair_tiles_f16 : gemm_tiled_kept_pair_tiles_f32;
-    if (gx.virt == VIRT_A_CLASSES) return tiles(gx, gy);
+    if (gx.virt == VIRT_A_CLASSES) return tiles(gx, gy) != APART;
     if (narrow_output(dtype, gx)) gx.tile_hint = HINT_128x32;
     if (gx.virt != VIRT_A_ROWS || balanced_rows(gx) || !gemm_tiled_eligible(dtype, gx, 0, 0) || gemm_is_small(gx.M, gx.N, gx.K, gx.batch, gx.red)) return false;
     gx.splits = plan_splits(BK, gx.M, gx.N, gx.K, 1, gx.red, usable, &gx.tiles_per_split, gx.virt);
@@ -1148,13 +1148,14 @@ bool gemm_tiled_kept_pair_plan(int dtype, GemmArgs &gx, GemmArgs &gy, void *work
     const size_t gx_bytes = gx.splits > 1 ? (size_t)gx.splits * gx.M * gx.N * sizeof(float) : 0;
     if (gy_bytes + gx_bytes > usable) return false;
     gx.ws = (float *)((char *)workspace + gy_bytes);
-    return tiles(gx, gy);
+    return tiles(gx, gy) != APART;
 }
 
 int gemm_tiled_kept_pair_run(int dtype, const GemmArgs &gx, const GemmArgs &gy, hipStream_t stream) {
     const bool classes = gx.virt == VIRT_A_CLASSES;
     const auto pair = dtype == D8_FLOAT16 ? (classes ? gemm_tiled_pair_classes_f16 : gemm_tiled_pair_rows_f16) : (classes ? gemm_tiled_pair_classes_f32 : gemm_tiled_pair_rows_f32);
-    ++kept_pair_launches;
+    const SharedLaunch shared = dtype == D8_FLOAT16 ? gemm_tiled_kept_pair_tiles_f16(gx, gy) : gemm_tiled_kept_pair_tiles_f32(gx, gy);
+    ++(shared == SHARED ? kept_pair_launches : crowded_pair_launches);
     if (int rc = pair(gx, gy, stream)) return rc;
     return launch_reduce_pair(dtype, gx, gy, stream);
 }
@@ -1399,6 +1400,7 @@ static int gemm_one(int dtype, int transA, int transB, int M, int N, int K,
 
 unsigned long d8_conv_grad_pair_launches(void) { return pair_launches.load(); }
 unsigned long d8_conv_grad_kept_pair_launches(void) { return kept_pair_launches.load(); }
+unsigned long d8_conv_grad_crowded_pair_launches(void) { return crowded_pair_launches.load(); }
 
 int d8_gemm_phase_record(void *records, size_t bytes) {
     D8_REQUIRE(((size_t)records & 7) == 0, "d8_gemm_phase_record: the record buffer is not 8-byte aligned");

@@ -173,8 +173,8 @@ int gemm_tiled_pair_launch(int dtype, const GemmArgs &gx, const GemmArgs &gy, hi
 // cut; _run launches and reduces.
 bool gemm_tiled_kept_pair_plan(int dtype, GemmArgs &gx, GemmArgs &gy, void *workspace, size_t workspace_bytes);
 int gemm_tiled_kept_pair_run(int dtype, const GemmArgs &gx, const GemmArgs &gy, hipStream_t stream);
-bool gemm_tiled_kept_pair_tiles_f16(const GemmArgs &gx, const GemmArgs &gy);
-bool gemm_tiled_kept_pair_tiles_f32(const GemmArgs &gx, const GemmArgs &gy);
+SharedLaunch gemm_tiled_kept_pair_tiles_f16(const GemmArgs &gx, const GemmArgs &gy);
+SharedLaunch gemm_tiled_kept_pair_tiles_f32(const GemmArgs &gx, const GemmArgs &gy);
 int gemm_tiled_pair_rows_f16(const GemmArgs &gx, const GemmArgs &gy, hipStream_t stream);
 int gemm_tiled_pair_rows_f32(const GemmArgs &gx, const GemmArgs &gy, hipStream_t stream);
 int gemm_tiled_pair_classes_f16(const GemmArgs &gx, const GemmArgs &gy, hipStream_t stream);

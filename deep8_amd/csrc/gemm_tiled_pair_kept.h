@@ -9,37 +9,45 @@
 namespace d8 {
 
 template <typename E>
-static bool kept_tiles(const GemmArgs &gx, const GemmArgs &gy, TileId &tx, TileId &ty) {
-    if (gy.virt != VIRT_B_KROWS || gx.batch != 1 || gy.batch != 1 || gx.tail_splits || gy.tail_splits) return false;
+static SharedLaunch kept_tiles(const GemmArgs &gx, const GemmArgs &gy, TileId &tx, TileId &ty) {
+    if (gy.virt != VIRT_B_KROWS || gx.batch != 1 || gy.batch != 1 || gx.tail_splits || gy.tail_splits) return APART;
     if (gx.virt == VIRT_A_CLASSES) {  // (the tiles of gemm_tiled_launch.h)
-        if (gx.splits != 1) return false;
+        if (gx.splits != 1) return APART;
         tx = sizeof(E) == 4 && gx.N <= 32 ? TILE_128x32 : gx.N < 128 ? TILE_128x64 : TILE_128x128;
     } else if (gx.virt == VIRT_A_ROWS) {
         tx = choose_tile<E, true, false, VIRT_A_ROWS>(gx);
     } else {
-        return false;
+        return APART;
     }
     ty = choose_tile<E, false, false, VIRT_B_KROWS>(gy);
     const bool x_ok = tx == TILE_64x64 || tx == TILE_64x128 || tx == TILE_128x128 || tx == TILE_128x64 || (sizeof(E) == 4 && tx == TILE_128x32);
-    if (!x_ok || (ty != TILE_128x128 && ty != TILE_64x128 && ty != TILE_64x64)) return false;
-    // (fp32 on 128 x 128 tiles in both: bound by the matrix pipe either way, and side by side they miss the caches more often.
-    // DeConv2d 59 x 7x7x256 -> 240 4x4 stride 2 124.4 us apart, 135.9 in one launch)
-    if (sizeof(E) == 4 && gx.virt == VIRT_A_ROWS && tx == TILE_128x128 && ty == TILE_128x128) return false;
+    if (!x_ok || (ty != TILE_128x128 && ty != TILE_64x128 && ty != TILE_64x64)) return APART;
     int mx, nx, my, ny;
     grid_of(ty, gy, my, ny);
+    if (tx == TILE_128x32) mx = ceil_div(gx.M, 128), nx = ceil_div(gx.N, 32);
+    else grid_of(tx, gx, mx, nx);
+    const long wx = (long)mx * nx * (gx.virt == VIRT_A_CLASSES ? gx.ncls : gx.splits), wy = (long)my * ny * gy.splits;
+    if (wx + wy >= 0x7fffffffL) return APART;
     if (sizeof(E) == 4 && gx.virt == VIRT_A_ROWS) {
-        // (fp32: all workgroups at once, two to a compute unit.  With more a smaller tile's product, of which three would fit,
-        // loses by the larger one's LDS, Conv2d 4 x 62x62x64 -> 384 3x3 132.6 us apart, 142.7 in one launch, and 128 x 64 tiles by
-        // an uneven end, 6 x 67x67x64 -> 64 50.9 and 54.0.  Smaller tiles of x's product beside small areas: any number,
-        // 64 x 14x14x32 -> 64 5x5 48.0 and 37.1)
-        if (tx == TILE_128x32) mx = ceil_div(gx.M, 128), nx = ceil_div(gx.N, 32);
-        else grid_of(tx, gx, mx, nx);
         auto long_m = [](TileId t) { return t == TILE_128x128 || t == TILE_128x64 || t == TILE_128x32; };
         auto long_n = [](TileId t) { return t == TILE_128x128 || t == TILE_64x128; };
-        const bool rows = long_m(tx) || long_m(ty), cols = long_n(tx) || long_n(ty);
-        if ((rows && cols) || (tx != TILE_64x64 && tx != TILE_128x32)) return (long)mx * nx * gx.splits + (long)my * ny * gy.splits <= 2L * cu_count();
+        const bool rows = long_m(tx) || long_m(ty), cols = long_n(tx) || long_n(ty), both = tx == TILE_128x128 && ty == TILE_128x128;
+        // fp32, more workgroups than two to a compute unit, of which smaller tiles would have three, or 128 x 128 tiles in both: as long
+        // as no workgroup runs longer than 24 steps of a 128 x 128 tile would (the longer workgroups start first: launch_pair_tiles).
+        // 90 drawn layers apart 9351 us, in one launch 9205 without that line; 7 x 35x35x64 -> 64 5x5 50.4 / 40.4, 17 x 17x17x200 -> 148
+        // 100 / 85.5, and of longer workgroups DeConv2d 27 x 21x21x320 -> 64 4x4 stride 2 217 / 187, but Conv2d 1 x 93x54x320 -> 64 5x5 107 /
+        // 117, 4 x 82x82x64 -> 168 148 / 157.  Slower by more than 3 % with it: 56 x 17x17x256 -> 64, 98 / 103.
+        // (Smaller tiles of x's product beside small areas: any number, 64 x 14x14x32 -> 64 5x5 48.0 and 37.1.)
+        if (both || (((rows && cols) || (tx != TILE_64x64 && tx != TILE_128x32)) && wx + wy > 2L * cu_count())) {
+            auto work = [](const GemmArgs &g, long m, long n) {
+                return (g.splits > 1 ? g.tiles_per_split : (long)g.red * ceil_div(g.K, 32)) * m * n;
+            };
+            const long most = 24 * 128 * 128;
+            const bool brief = work(gx, long_m(tx) ? 128 : 64, tx == TILE_128x32 ? 32 : long_n(tx) ? 128 : 64) <= most && work(gy, long_m(ty) ? 128 : 64, long_n(ty) ? 128 : 64) <= most;
+            return brief ? SHARED_KEPT : APART;
+        }
     }
-    return (long)ceil_div(gx.M, 64) * ceil_div(gx.N, 32) * (gx.virt == VIRT_A_CLASSES ? gx.ncls : gx.splits) + (long)my * ny * gy.splits < 0x7fffffffL;
+    return SHARED;
 }
 
 template <typename E, typename X, int EDGE>
@@ -73,7 +81,7 @@ static int kept_launch_x(TileId tx, TileId ty, const GemmArgs &gx, const GemmArg
 template <typename E, int VIRT>
 static int kept_launch(const GemmArgs &gx, const GemmArgs &gy, hipStream_t stream) {
     TileId tx, ty;
-    if (!kept_tiles<E>(gx, gy, tx, ty)) return fail(D8_ERR_ARGUMENT, "gemm_tiled_kept_pair_launch: no kernel for this pair of tiles");
+    if (kept_tiles<E>(gx, gy, tx, ty) == APART) return fail(D8_ERR_ARGUMENT, "gemm_tiled_kept_pair_launch: no kernel for this pair of tiles");
     return gx.K % (128 / (int)sizeof(E)) ? kept_launch_x<E, VIRT, EDGE_PIECES>(tx, ty, gx, gy, stream) : kept_launch_x<E, VIRT, EDGE_NONE>(tx, ty, gx, gy, stream);
 }
 

@@ -3,7 +3,7 @@
 
 namespace d8 {
 
-bool gemm_tiled_kept_pair_tiles_f32(const GemmArgs &gx, const GemmArgs &gy) {
+SharedLaunch gemm_tiled_kept_pair_tiles_f32(const GemmArgs &gx, const GemmArgs &gy) {
     TileId tx, ty;
     return kept_tiles<float>(gx, gy, tx, ty);
 }

@@ -300,9 +300,10 @@ int d8_deconv2d_grad_xy_ex(int dtype, const void *x, void *gx, int B, int IH, in
 
 /* Test and measurement aid: how many of the _grad_xy calls above have run as one launch since the library was
  * loaded (no counterpart in the reference): those whose gradient of x runs whole, or with its remainder band, and
- * those whose two products are tiled and cut as they would be alone.  A call counts in one of them at most.        */
+ * those whose two products are tiled and cut as they would be alone.  A call counts in one of the three at most.   */
 unsigned long d8_conv_grad_pair_launches(void);
 unsigned long d8_conv_grad_kept_pair_launches(void);
+unsigned long d8_conv_grad_crowded_pair_launches(void);  /* likewise, Float32, more workgroups than run at once */
 unsigned long d8_matmul_grad_pair_launches(void);  /* ... and of the d8_matmul_grad_xy calls: whole K steps, and no more workgroups than run at once; */
 unsigned long d8_matmul_grad_kept_pair_launches(void);  /* the others: a K step (64 in Float16, 32 in Float32) that is cut short, or more workgroups */
 unsigned long d8_matmul_grad_copied_calls(void);   /* d8_matmul_grad_xy calls that ran on copies of their odd operands */
