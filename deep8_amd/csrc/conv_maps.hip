@@ -162,6 +162,54 @@ __global__ __launch_bounds__(256) void im2col_padded_kernel(const V *__restrict_
     }
 }
 
+// Rows of odd length side by side (dense: no padding), on a 16-byte aligned matrix: a thread gathers the NV elements of a 16-byte piece of
+// the whole matrix, which may begin in one row and end in the next, and stores them at once.  (BIG: 2^31 elements or more.)
+// From three quarters of a workgroup per compute unit on; a thread per element, which fewer pieces leave to it, has a shorter chain.  Layers, us a thread per
+// element / so: half DeConv2d 22 x 15x15x64 -> 324 3x3 (1.8e6 pieces) 154 / 97, Conv2d 36 x 64x64x258 -> 39 3x3 stride 2 1005 / 669, fp32 DeConv2d 24
+// x 7x7x64 -> 155 5x5 stride 2 127 / 107; 28 x 26x26x128 -> 3 (63882) 59.9 / 59.0, 2 x 51x51x384 -> 3 (31212) 74.9 / 75.3, 8 x 31x31x46 -> 1 (15376)
+// 51.9 / 54.1, 1 x 10x10x152 -> 1 (112) 23.3 / 25.3.
+struct Im2colFlat {
+    FastDiv by_K, by_OW, by_OH, by_C, by_FW;
+};
+
+template <typename V, int NV, bool BIG>
+__global__ __launch_bounds__(256) void im2col_flat_kernel(const V *__restrict__ im, V *__restrict__ col, MapGeom g, Im2colFlat by, long total) {
+    typedef V VV __attribute__((ext_vector_type(NV)));
+    typedef std::conditional_t<BIG, long, unsigned> Index;
+    auto over = [](Index n, int d, FastDiv f) -> Index {
+        if constexpr (BIG) return n / d;
+        else return div_by(n, f);
+    };
+    const int K = g.FH * g.FW * g.C;
+    const long pieces = (total + NV - 1) / NV;
+    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < pieces; i += (long)gridDim.x * blockDim.x) {
+        const Index first = (Index)(i * NV), r = over(first, K, by.by_K), q = over(r, g.OW, by.by_OW), image = over(q, g.OH, by.by_OH);
+        int ox = (int)(r - q * g.OW), oy = (int)(q - image * g.OH), b = (int)image;
+        const int j = (int)(first - r * K), tap = (int)div_by((unsigned)j, by.by_C);
+        int c = j - tap * g.C, fy = (int)div_by((unsigned)tap, by.by_FW), fx = tap - fy * g.FW;
+        V s[NV];
+        bool inside[NV];
+#pragma unroll
+        for (int e = 0; e < NV; ++e) {
+            const int iy = oy * g.sy + fy * g.dy - g.pt, ix = ox * g.sx + fx * g.dx - g.pl;
+            inside[e] = i * NV + e < total && (unsigned)iy < (unsigned)g.IH && (unsigned)ix < (unsigned)g.IW;
+            s[e] = im[inside[e] ? (((long)b * g.IH + iy) * g.IW + ix) * g.C + c : 0L];
+            const bool next = ++c == g.C, row = next && fx + 1 == g.FW, end = row && fy + 1 == g.FH, line = end && ox + 1 == g.OW, whole = line && oy + 1 == g.OH;
+            c = next ? 0 : c, fx = row ? 0 : fx + next, fy = end ? 0 : fy + row, ox = line ? 0 : ox + end, oy = whole ? 0 : oy + line, b += whole;
+        }
+        VV v;
+#pragma unroll
+        for (int e = 0; e < NV; ++e) v[e] = inside[e] ? s[e] : (V)0;
+        if (i * NV + NV <= total) {
+            *(VV *)(col + i * NV) = v;
+        } else {
+#pragma unroll
+            for (int e = 0; e < NV; ++e)
+                if (i * NV + e < total) col[i * NV + e] = v[e];
+        }
+    }
+}
+
 template <typename V>
 __global__ __launch_bounds__(256) void pad_rows_kernel(const V *__restrict__ src, V *__restrict__ dst, int K, int pitch, long total) {
     for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += (long)gridDim.x * blockDim.x) {
@@ -745,6 +793,14 @@ static void launch_im2col_padded(const void *im, void *col, const MapGeom &g, lo
     else hipLaunchKernelGGL((im2col_padded_kernel<V, NV, true>), grid, dim3(256), 0, s, (const V *)im, (V *)col, g, by, total);
 }
 
+template <typename V, int NV>
+static void launch_im2col_flat(const void *im, void *col, const MapGeom &g, long total, hipStream_t s) {
+    const Im2colFlat by = {fast_div(g.FH * g.FW * g.C), fast_div(g.OW), fast_div(g.OH), fast_div(g.C), fast_div(g.FW)};
+    const dim3 grid(grid_for((total + NV - 1) / NV, 256));
+    if (total < (1L << 31) - NV) hipLaunchKernelGGL((im2col_flat_kernel<V, NV, false>), grid, dim3(256), 0, s, (const V *)im, (V *)col, g, by, total);
+    else hipLaunchKernelGGL((im2col_flat_kernel<V, NV, true>), grid, dim3(256), 0, s, (const V *)im, (V *)col, g, by, total);
+}
+
 int launch_im2col(int dtype, const void *im, void *col, const MapGeom &g, hipStream_t s) {
     if (g.B == 0) return 0;
     const size_t es = dtype_bytes(dtype);
@@ -778,6 +834,9 @@ int launch_im2col(int dtype, const void *im, void *col, const MapGeom &g, hipStr
         const long total = elems / (16 / es);
         hipLaunchKernelGGL((im2col_kernel<uint4>), dim3(grid_for(total, 256)), dim3(256), 0, s,
                            (const uint4 *)im, (uint4 *)col, g, CV, total);
+    } else if (es < 8 && aligned16(col) && elems / (16 / (long)es) >= 192L * cu_count()) {  // (see im2col_flat_kernel)
+        if (es == 4) launch_im2col_flat<unsigned, 4>(im, col, g, elems, s);
+        else launch_im2col_flat<unsigned short, 8>(im, col, g, elems, s);
     } else if (es == 8) {
         hipLaunchKernelGGL((im2col_kernel<unsigned long long>), dim3(grid_for(elems, 256)), dim3(256), 0, s,
                            (const unsigned long long *)im, (unsigned long long *)col, g, g.C, elems);
