@@ -344,6 +344,7 @@ size_t d8_matmul_scratch_bytes(int dtype, int which, int xb, int xr, int xc, int
 // A forward product (bias and relu: as its store may apply them) on copies of operands whose rows start anywhere; false, with
 // nothing launched, where that does not pay.
 static bool run_on_copies(int dtype, const Gemm &p, const void *bias, int relu, void *scratch, size_t scratch_bytes, void *stream, int *rc) {
+    if (dtype != D8_FLOAT16) return false;  // (no copies of others: nothing to plan)
     GemmArgs g = to_args(p);
     g.bias = bias, g.relu = relu;
     if (bias || relu) {
