@@ -327,15 +327,15 @@ extern "C" {
 // ---------------------------------------------------------------------------------------------
 size_t d8_matmul_scratch_bytes(int dtype, int which, int xb, int xr, int xc, int yb, int yr, int yc) {
     if (check_mm("d8_matmul_scratch_bytes", dtype, xb, xr, xc, yb, yr, yc)) return 0;
+    const char *const base = (const char *)4096;  // (three matrices, none of them the same: one that is read twice is copied once)
     if (which == 3) {  // for d8_matmul_grad_xy: both gradients' scratch side by side (they may share a launch), and their copies
-        const char *const base = (const char *)4096;  // (three matrices, none of them the same)
         const Gemm px = mm_plan(1, nullptr, xb, xr, xc, base, yb, yr, yc, base + 4096), py = mm_plan(2, base + 8192, xb, xr, xc, nullptr, yb, yr, yc, base + 4096);
         GemmArgs gx = to_args(px), gy = to_args(py);
         const PackedProduct both[2] = {{&gx, px.ta, px.tb}, {&gy, py.ta, py.tb}};
         return align256(d8_matmul_scratch_bytes(dtype, 1, xb, xr, xc, yb, yr, yc)) + d8_matmul_scratch_bytes(dtype, 2, xb, xr, xc, yb, yr, yc) +
                gemm_pack_bytes(dtype, both);
     }
-    const Gemm p = mm_plan(which, nullptr, xb, xr, xc, nullptr, yb, yr, yc, nullptr);
+    const Gemm p = mm_plan(which, base, xb, xr, xc, base + 4096, yb, yr, yc, base + 8192);
     if (which != 0) return gemm_ws(dtype, p);
     GemmArgs g = to_args(p);
     return gemm_ws(dtype, p) + gemm_pack_one_bytes(dtype, {&g, p.ta, p.tb});
