@@ -646,15 +646,14 @@ static int relu_gate_sum_t(const T *z, const T *dz, T *dpre, T *g, long rows, in
     const size_t need = (size_t)chunks * cols * sizeof(float);
     if (chunks > 1 && (!scratch || scratch_bytes < need || !al16(scratch))) chunks = 1, rpc = (int)rows;
     const bool wide = cols % WIDE == 0 && al16(g) && al16(dz) && al16(z) && al16(dpre);
-    // rows that start at any element: 16-byte accesses too where a row is more than sixteen of them, so that 32 threads lie
-    // across the columns as they do in d8_add_grad's single-element pass over such a tensor and the sums stay its own
-    const bool any = !wide && cols > 16 * WIDE;
+    // The sums have the order of d8_add_grad on dpre.  It moves 16 bytes at a time where dpre and g are aligned, whatever z and dz
+    // are; and where a row is more than sixteen pieces, 32 threads lie across the columns in its single-element pass as well.
+    const bool sums_wide = p.kind == 1 && cols % WIDE == 0 && al16(g) && al16(dpre);
+    const bool any = !wide && (sums_wide || cols > 16 * WIDE);
     const int vec = wide || any ? WIDE : 1;
     const long cvs = ((long)cols + vec - 1) / vec;
     int TX = 1, most = 32;
-    // (as d8_add_grad on dpre would)
-    const bool few = p.kind == 1 && cols % WIDE == 0 && al16(g) && al16(dpre);
-    if (const int narrow = few ? one_chunk_tx(rows) : 0) most = narrow, chunks = 1, rpc = (int)rows;
+    if (const int narrow = sums_wide ? one_chunk_tx(rows) : 0) most = narrow, chunks = 1, rpc = (int)rows;
     while (TX < most && TX < cvs) TX *= 2;
     dim3 grid((unsigned)((cvs + TX - 1) / TX), (unsigned)chunks, 1);
     if (any)
