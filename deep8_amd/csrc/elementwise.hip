@@ -510,14 +510,19 @@ static ReducePlan plan_reduce(const int *d, const int *zd) {
     return p;
 }
 
-// Column sums of few rows in one launch: how many threads lie across a row's 16-byte pieces, so that the others take up to 64 rows
-// in flight each (0: more rows, which take chunks and a second launch).  The launch that it saves takes 2.5 us, a row of a block
-// of few pieces some 2 ns.  ReLu gate and bias gradient, us in chunks / so, with 4 and 8 across: half 128 x 1024 5.2 / 3.1, 2.9;
-// 256 x 1024 5.3 / 3.1, 3.4; 512 x 1024 5.5 / 3.8, 4.7; 1024 x 1024 5.55 / 5.1, 7.3.  Behind the layer's product, which leaves z in other XCDs'
-// caches, fewer rows: dense layers with their gradients of 128 rows 8 - 20 % faster, of 256 5 - 15 %, of 512 1 - 5 %, of 640 to 1024
-// level to 6 % slower.
-static int one_chunk_tx(long rows) {
-    return rows <= 64 || rows > 512 ? 0 : rows <= 128 ? 8 : 4;  // (up to 64 rows are one chunk anyway)
+// Column sums of few rows in one launch: how many threads lie across a row's 16-byte pieces (of which it has `pieces`), so that the
+// others take up to 64 rows in flight each (0: more rows, which take chunks and a second launch).  The launch that it saves takes 2.5
+// us, a row of a block of few pieces some 2 ns.  8 across read whole 128-byte lines; 4 give narrow outputs twice the blocks, and
+// cost half of every line read where those are more than the loads' latency wants; from 4097 pieces on 32 across are blocks enough.
+// ReLu gate and bias gradient, us, chunks and a second launch / 4 / 8 / 32 across: half 128 x 1024 4.6 / 3.0 / 2.7 / 3.8, 512 x 1024 4.8 / 3.5 /
+// 4.2 / 9.7, 512 x 4096 5.3 / 4.0 / 4.6 / 10.0, 512 x 8192 6.6 / 8.2 / 5.0 / 10.5, 512 x 16384 11.7 / 14.4 / 9.5 / 13.5, 512 x 65536 34.2 / 50.2 / 32.6 /
+// 30.7, 256 x 262144 86.9 / 127 / 89.3 / 86.7; fp32 512 x 4096 6.3 / 8.0 / 4.7 / 8.9, 512 x 65536 84.8 / 123 / 91.6 / 79.9.  (4 across whatever the width,
+// as it was first from 129 rows on, took 1.1 to 1.5 times as long as the chunks from 8192 columns in half, 4096 in fp32.)
+// Behind the layer's product, which leaves z in other XCDs' caches, fewer rows: dense layers with their gradients of 128 rows 8 - 20 %
+// faster, of 256 5 - 15 %, of 512 1 - 5 %, of 640 to 1024 level to 6 % slower.
+static int one_chunk_tx(long rows, long pieces) {
+    if (rows <= 64 || rows > 512) return 0;  // (up to 64 rows are one chunk anyway)
+    return pieces > 4096 ? 32 : rows > 128 && pieces <= 512 ? 4 : 8;
 }
 
 // g = keep * g + scale * (op(dz) summed over the axes where g has extent 1 and dz does not)
@@ -539,7 +544,7 @@ static int reduce_t(T *g, const int *d, const T *dz, const int *zd, void *scratc
         const int vec = wide ? WIDE : 1;
         const long cvs = p.C / vec;
         int TX = 1, most = 32;
-        if (const int narrow = wide && p.K0 == 1 ? one_chunk_tx(p.R) : 0) most = narrow, chunks = 1, rpc = (int)p.R;
+        if (const int narrow = wide && p.K0 == 1 ? one_chunk_tx(p.R, cvs) : 0) most = narrow, chunks = 1, rpc = (int)p.R;
         while (TX < most && TX < cvs) TX *= 2;
         dim3 grid((unsigned)((cvs + TX - 1) / TX), (unsigned)chunks, (unsigned)p.K0);
         if (wide)
@@ -653,7 +658,7 @@ static int relu_gate_sum_t(const T *z, const T *dz, T *dpre, T *g, long rows, in
     const int vec = wide || any ? WIDE : 1;
     const long cvs = ((long)cols + vec - 1) / vec;
     int TX = 1, most = 32;
-    if (const int narrow = sums_wide ? one_chunk_tx(rows) : 0) most = narrow, chunks = 1, rpc = (int)rows;
+    if (const int narrow = sums_wide ? one_chunk_tx(rows, cvs) : 0) most = narrow, chunks = 1, rpc = (int)rows;
     while (TX < most && TX < cvs) TX *= 2;
     dim3 grid((unsigned)((cvs + TX - 1) / TX), (unsigned)chunks, 1);
     if (any)
