@@ -869,7 +869,7 @@ size_t gemm_tiled_workspace(int dtype, int M, int N, int K, int red, int virt) {
 // 0.38 for a 64 x 128 tile and 0.46 for 128 x 128).  The same pieces -- or none, and no second pass -- spread over four times as many
 // workgroups.  The estimate counts steps of a 128 x 128 tile (about 2 us of a CU in fp32, 0.5 us in half), for the plan that g
 // holds (splits set) and for 64 x 64 tiles in 1 .. as many pieces as that plan; 7 % or more decide.  In half it was fitted to tiles
-// that pass through registers, and says only what a call takes (gemm_estimate_us); half_tile_us decides.  A 64 x 128 half step is 0.76
+// that pass through registers; forward products are decided by half_tile_us.  A 64 x 128 half step is 0.76
 // here and 0.65 in plan_few_tiles, a half product's second pass 6.5 steps + 1 per 0.25e6 outputs and piece here, 14 + 1 per 0.5e6
 // there, which only chooses among 128-wide tiles.
 // A narrow output (128 x 32 tiles, below) counts its pieces the same way.
@@ -895,8 +895,7 @@ static double tile_cost(bool half_elems, int bm, int bn, const GemmArgs &g, long
 // patch rows take longer, and a second pass.  Fitted to 80 drawn forward products and convolutions of at most 255 128 x 128 tiles, each on three
 // tiles in 1 to 12 pieces; 5 % or more decide.  (The estimate above, which 7 % had to decide, counts the same ends for all
 // tiles, and for products of few steps those are most of the time.)  110 drawn half products and convolutions forward 1384 ->
-// 1358 us, 3.4 % at the mean, both gradients of 104 of them 2434 -> 2410, 1.9 %; three of the 214 calls more than 3 % slower (by 0.2
-// us): 218 x 64 x 1328 5.6 -> 4.0, 1504 x 3648 x 128 14.6 -> 10.8, Conv2d 37 x 8x8x64 -> 368 1x1 6.2 -> 4.7.
+// 1358 us, 3.4 % at the mean: 218 x 64 x 1328 5.6 -> 4.0, 1504 x 3648 x 128 14.6 -> 10.8, Conv2d 37 x 8x8x64 -> 368 1x1 6.2 -> 4.7.
 static double half_tile_us(int bm, int bn, const GemmArgs &g, long total, long s) {
     const long cus = cu_count(), n = (ceil_div(g.M, bm) * (long)ceil_div(g.N, bn) * g.batch * s + cus - 1) / cus, len = (total + s - 1) / s;
     const int k = bm * bn == 128 * 128 ? 2 : bm * bn == 64 * 64 ? 0 : 1;
@@ -905,6 +904,12 @@ static double half_tile_us(int bm, int bn, const GemmArgs &g, long total, long s
     return ends[k] + n * len * (step[k] + 0.11 * (far < 0.0 ? 0.0 : far > 1.0 ? 1.0 : far)) + 0.2 * (n - 1) + (g.virt == VIRT_A_ROWS ? rows[k] : 0.0) +
            (s > 1 ? 2.6 + 1.85e-6 * s * g.M * (double)g.N * g.batch : 0.0);
 }
+
+// It plans forward products only (a convolution on the interim matrix has a gradient's operands and counts as one).  A gradient is cut as
+// its launch alone would be, also where it shares one with the other gradient, whose workgroups run longer than its own: there a second
+// pass, for pieces that alone are worth it, comes on top (4 x 320 x 128 x 1408 8.2 -> 11.7 us, 1792 x 256 x 1088 15.2 -> 18.2, 576 x 128 x 1216 8.7 ->
+// 11.1, Conv2d 2 x 19x19x64 -> 128 3x3 11.6 -> 13.6), which the estimate above finds worth it less often.
+static bool is_gradient(const GemmArgs &g, int transA, int transB) { return g.virt == VIRT_A_ROWS ? !transB : transA || transB; }
 
 static void few_tiles_small(int dtype, GemmArgs &g, int transA, int transB, size_t usable) {
     // (a filter gradient's pieces stay those of the launch it may share with the input's: one sum, one result)
@@ -918,16 +923,15 @@ static void few_tiles_small(int dtype, GemmArgs &g, int transA, int transB, size
     const long total = (long)g.red * ceil_div(g.K, BK);
     const bool half = g.splits == 1 && gemm_tiled_half_tiles(g.M, g.N, g.batch, total, BK);
     const bool narrow = g.tile_hint == HINT_128x32;
-    auto cost = [&](int bm, int bn, long pieces) {
-        return half_elems ? half_tile_us(bm, bn, g, total, pieces) : tile_cost(false, bm, bn, g, total, pieces);
-    };
+    const bool by_time = half_elems && !is_gradient(g, transA, transB);
+    auto cost = [&](int bm, int bn, long pieces) { return by_time ? half_tile_us(bm, bn, g, total, pieces) : tile_cost(half_elems, bm, bn, g, total, pieces); };
     const double now = narrow ? 1e30 : g.N < 128 ? cost(128, 64, g.splits) : cost(g.M < 128 || half ? 64 : 128, 128, g.splits);
     long most = (long)(usable / ((size_t)g.batch * g.M * g.N * sizeof(float)));
     int tps;  // (no more pieces than the 128-wide plan would have: what the scratch queries provide for, whatever is passed)
     const long planned = plan_splits(BK, g.M, g.N, g.K, g.batch, g.red, (size_t)-1, &tps, g.virt);
     if (most > planned) most = planned;
     if (most > total / 2) most = total / 2;
-    double best = (half_elems ? 0.95 : 0.93) * now;
+    double best = (by_time ? 0.95 : 0.93) * now;
     long pieces = 0;
     for (long s = 1; s == 1 || s <= most; ++s)
         if (const double c = narrow ? cost(128, 32, s) : cost(64, 64, s); c < best) best = c, pieces = s;
