@@ -869,7 +869,7 @@ size_t gemm_tiled_workspace(int dtype, int M, int N, int K, int red, int virt) {
 // 0.38 for a 64 x 128 tile and 0.46 for 128 x 128).  The same pieces -- or none, and no second pass -- spread over four times as many
 // workgroups.  The estimate counts steps of a 128 x 128 tile (about 2 us of a CU in fp32, 0.5 us in half), for the plan that g
 // holds (splits set) and for 64 x 64 tiles in 1 .. as many pieces as that plan; 7 % or more decide.  In half it was fitted to tiles
-// that pass through registers; forward products are decided by half_tile_us.  A 64 x 128 half step is 0.76
+// that pass through registers; most products are decided by half_tile_us.  A 64 x 128 half step is 0.76
 // here and 0.65 in plan_few_tiles, a half product's second pass 6.5 steps + 1 per 0.25e6 outputs and piece here, 14 + 1 per 0.5e6
 // there, which only chooses among 128-wide tiles.
 // A narrow output (128 x 32 tiles, below) counts its pieces the same way.
@@ -896,20 +896,18 @@ static double tile_cost(bool half_elems, int bm, int bn, const GemmArgs &g, long
 // tiles in 1 to 12 pieces; 5 % or more decide.  (The estimate above, which 7 % had to decide, counts the same ends for all
 // tiles, and for products of few steps those are most of the time.)  110 drawn half products and convolutions forward 1384 ->
 // 1358 us, 3.4 % at the mean: 218 x 64 x 1328 5.6 -> 4.0, 1504 x 3648 x 128 14.6 -> 10.8, Conv2d 37 x 8x8x64 -> 368 1x1 6.2 -> 4.7.
+// What a workgroup takes besides its steps, and a step (128 x 128 and 64 x 64 tiles, and the two between).
+static double half_ends_us(int bm, int bn) { return bm * bn == 64 * 64 ? 3.6 : 4.1; }
+static double half_step_us(int bm, int bn, const GemmArgs &g) {
+    const double far = bm * bn == 64 * 64 ? (2.0 * g.red * g.K * g.batch * ((double)g.M + g.N) - 4e6) / 8e6 : 0.0;  // (see above)
+    return (bm * bn == 128 * 128 ? 0.47 : bm * bn == 64 * 64 ? 0.23 : 0.31) + 0.11 * (far < 0.0 ? 0.0 : far > 1.0 ? 1.0 : far);
+}
+static double half_rows_us(int bm, int bn) { return bm * bn == 128 * 128 ? 1.65 : bm * bn == 64 * 64 ? 0.95 : 1.25; }
 static double half_tile_us(int bm, int bn, const GemmArgs &g, long total, long s) {
     const long cus = cu_count(), n = (ceil_div(g.M, bm) * (long)ceil_div(g.N, bn) * g.batch * s + cus - 1) / cus, len = (total + s - 1) / s;
-    const int k = bm * bn == 128 * 128 ? 2 : bm * bn == 64 * 64 ? 0 : 1;
-    const double ends[3] = {3.6, 4.1, 4.1}, step[3] = {0.23, 0.31, 0.47}, rows[3] = {0.95, 1.25, 1.65};
-    const double far = k == 0 ? (2.0 * g.red * g.K * g.batch * ((double)g.M + g.N) - 4e6) / 8e6 : 0.0;  // (see above)
-    return ends[k] + n * len * (step[k] + 0.11 * (far < 0.0 ? 0.0 : far > 1.0 ? 1.0 : far)) + 0.2 * (n - 1) + (g.virt == VIRT_A_ROWS ? rows[k] : 0.0) +
+    return half_ends_us(bm, bn) + n * len * half_step_us(bm, bn, g) + 0.2 * (n - 1) + (g.virt == VIRT_A_ROWS ? half_rows_us(bm, bn) : 0.0) +
            (s > 1 ? 2.6 + 1.85e-6 * s * g.M * (double)g.N * g.batch : 0.0);
 }
-
-// It plans forward products only (a convolution on the interim matrix has a gradient's operands and counts as one).  A gradient is cut as
-// its launch alone would be, also where it shares one with the other gradient, whose workgroups run longer than its own: there a second
-// pass, for pieces that alone are worth it, comes on top (4 x 320 x 128 x 1408 8.2 -> 11.7 us, 1792 x 256 x 1088 15.2 -> 18.2, 576 x 128 x 1216 8.7 ->
-// 11.1, Conv2d 2 x 19x19x64 -> 128 3x3 11.6 -> 13.6), which the estimate above finds worth it less often.
-static bool is_gradient(const GemmArgs &g, int transA, int transB) { return g.virt == VIRT_A_ROWS ? !transB : transA || transB; }
 
 static void few_tiles_small(int dtype, GemmArgs &g, int transA, int transB, size_t usable) {
     // (a filter gradient's pieces stay those of the launch it may share with the input's: one sum, one result)
@@ -923,7 +921,7 @@ static void few_tiles_small(int dtype, GemmArgs &g, int transA, int transB, size
     const long total = (long)g.red * ceil_div(g.K, BK);
     const bool half = g.splits == 1 && gemm_tiled_half_tiles(g.M, g.N, g.batch, total, BK);
     const bool narrow = g.tile_hint == HINT_128x32;
-    const bool by_time = half_elems && !is_gradient(g, transA, transB);
+    const bool by_time = half_elems && g.pieces_by == BY_TILE_TIMES;
     auto cost = [&](int bm, int bn, long pieces) { return by_time ? half_tile_us(bm, bn, g, total, pieces) : tile_cost(half_elems, bm, bn, g, total, pieces); };
     const double now = narrow ? 1e30 : g.N < 128 ? cost(128, 64, g.splits) : cost(g.M < 128 || half ? 64 : 128, 128, g.splits);
     long most = (long)(usable / ((size_t)g.batch * g.M * g.N * sizeof(float)));
@@ -945,6 +943,90 @@ static void few_tiles_small(int dtype, GemmArgs &g, int transA, int transB, size
 // matrix instructions would multiply columns that are not there.  50000 x 288 x 32: 22.0 -> 14.3 us.
 static bool narrow_output(int dtype, const GemmArgs &g) {
     return dtype == D8_FLOAT32 && g.N <= 32 && g.M >= 128 && (g.virt == VIRT_NONE || g.virt == VIRT_A_ROWS);
+}
+
+static void plan_pieces(int dtype, GemmArgs &g, int ta, int tb, size_t usable) {
+    g.splits = plan_splits(gemm_tiled_k_step(dtype), g.M, g.N, g.K, g.batch, g.red, usable, &g.tiles_per_split, g.virt);
+    few_tiles_small(dtype, g, ta, tb, usable);
+}
+
+// A planned half product as one of two that share a launch.  One that runs whole may take larger tiles than alone, which sum in the same
+// order: fewer steps for the chip, where the smaller ones make shorter workgroups.
+struct HalfShare {
+    double longest[2], share[2];  // us of a workgroup, and a compute unit's share of all steps; on its tiles and on larger ones
+    double pass;                  // over its partial sums, the launch left out
+    bool larger;                  // whether there is the choice
+};
+static HalfShare half_share(const GemmArgs &g) {
+    const long total = (long)g.red * ceil_div(g.K, 64), len = g.splits > 1 ? g.tiles_per_split : total;
+    const bool small = g.tile_hint == HINT_64x64 || (g.virt == VIRT_B_KROWS && ((g.M < 128 && g.N < 128) || gemm_tiled_krows_64(g.virt, g.M, g.N)));
+    HalfShare h;
+    h.larger = g.virt == VIRT_NONE && g.splits == 1 && g.tile_hint == HINT_64x64;
+    h.pass = g.splits > 1 ? 1.85e-6 * g.splits * g.M * (double)g.N * g.batch : 0.0;
+    for (int i = 0; i < (h.larger ? 2 : 1); ++i) {
+        const bool t64 = small && i == 0;
+        const int bn = t64 || g.N < 128 ? 64 : 128;
+        const int bm = t64 || (bn == 128 && (g.M < 128 || (g.splits == 1 && gemm_tiled_half_tiles(g.M, g.N, g.batch, total, 64)))) ? 64 : 128;
+        const double steps = len * half_step_us(bm, bn, g);
+        h.longest[i] = half_ends_us(bm, bn) + steps + (g.virt != VIRT_NONE ? half_rows_us(bm, bn) : 0.0);
+        h.share[i] = (double)ceil_div(g.M, bm) * ceil_div(g.N, bn) * g.batch * g.splits * steps / cu_count();
+    }
+    return h;
+}
+// What the launch takes with the pass after it: its longest workgroup or a compute unit's share, whichever is more; bit i of tiles: product i on
+// larger ones.
+static double half_pair_us(const HalfShare &a, const HalfShare &b, int &tiles) {
+    double best = INFINITY;
+    for (int t = 0; t < 4; ++t) {
+        const int i = t & 1, j = t >> 1;
+        if (i > a.larger || j > b.larger) continue;
+        const double longest = a.longest[i] > b.longest[j] ? a.longest[i] : b.longest[j], share = 4.0 + a.share[i] + b.share[j];
+        if (const double us = longest > share ? longest : share; us < best) best = us, tiles = t;
+    }
+    return best + (a.pass + b.pass > 0.0 ? 3.5 + a.pass + b.pass : 0.0);
+}
+
+// Plans the two half gradients of a MatrixMultiply for a launch that they share.  Which estimate plans the pieces of each (and of each alone, for
+// the same bits: by the shapes only): by its tiles' times a product is cut where that pays in a launch of its own; beside another one that runs
+// as long anyway, a second pass comes on top.  Both by the tiles' times and on larger tiles where they run whole, as it was, / so, us: 4 x 320 x
+// 128 x 1408 12.6 / 9.0, 960 x 128 x 1872 18.4 / 11.4 (apart 15.2), 3 x 384 x 768 x 264 16.2 / 9.7 (12.8), 4 x 832 x 448 x 160 14.2 / 8.8 (12.1), 1216 x
+// 128 x 256 10.3 / 7.7, 1856 x 128 x 3200 14.9 / 14.5 (by its steps 18.4); 500 drawn calls of both gradients 6083 / 5739.
+static void half_pair_plan(GemmArgs &g0, GemmArgs &g1, size_t usable) {
+    GemmArgs *const g[2] = {&g0, &g1};
+    HalfShare plan[2][2];
+    int tiles = 0, choice = 0;
+    for (int i = 0; i < 2; ++i)
+        for (int by : {BY_TILE_TIMES, BY_STEPS}) {
+            GemmArgs p = *g[i];
+            p.pieces_by = by;
+            plan_pieces(D8_FLOAT16, p, i, !i, (size_t)-1);
+            plan[i][by] = half_share(p);
+        }
+    double best = INFINITY;
+    for (int c = 0; c < 4; ++c)
+        if (const double us = half_pair_us(plan[0][c & 1], plan[1][c >> 1], tiles); us < best) best = us, choice = c;
+    g0.pieces_by = choice & 1, g1.pieces_by = choice >> 1;
+    plan_pieces(D8_FLOAT16, g0, 0, 1, usable), plan_pieces(D8_FLOAT16, g1, 1, 0, usable);
+    half_pair_us(half_share(g0), half_share(g1), tiles);
+    for (int i = 0; i < 2; ++i)
+        if (tiles >> i & 1) g[i]->tile_hint = HINT_NONE;
+}
+
+// (Conv2d 2 x 19x19x64 -> 128 3x3, both gradients, by its tiles' times 14.8 us, so 12.7; 217 drawn layers level)
+void gemm_conv_pieces(int dtype, GemmArgs &gx, const GemmArgs &gy) {
+    if (dtype != D8_FLOAT16 || gx.virt != VIRT_A_ROWS || gy.virt != VIRT_B_KROWS) return;
+    GemmArgs y = gy;
+    y.splits = plan_splits(gemm_tiled_k_step(dtype), y.M, y.N, y.K, 1, y.red, (size_t)-1, &y.tiles_per_split, y.virt);
+    const HalfShare other = half_share(y);
+    double us[2];
+    for (int by : {BY_TILE_TIMES, BY_STEPS}) {
+        GemmArgs x = gx;
+        int tiles;
+        x.pieces_by = by;
+        plan_pieces(dtype, x, 0, 0, (size_t)-1);
+        us[by] = half_pair_us(half_share(x), other, tiles);
+    }
+    gx.pieces_by = us[BY_STEPS] < us[BY_TILE_TIMES] ? BY_STEPS : BY_TILE_TIMES;
 }
 
 // What the planners above count for the plan that they make, in microseconds.  (Over 3100 calls on drawn layers the time
@@ -972,8 +1054,7 @@ double gemm_estimate_us(int dtype, const GemmArgs &g0, int transA, int transB) {
     if (g0.virt == VIRT_NONE && gemm_is_small(g0.M, g0.N, g0.K, g0.batch, g0.red)) return 4.0;
     GemmArgs g = g0;
     g.tile_hint = narrow_output(dtype, g) ? HINT_128x32 : HINT_NONE;
-    g.splits = plan_splits(BK, g.M, g.N, g.K, g.batch, g.red, (size_t)-1, &g.tiles_per_split, g.virt);
-    few_tiles_small(dtype, g, transA, transB, (size_t)-1);
+    plan_pieces(dtype, g, transA, transB, (size_t)-1);
     const long total = (long)g.red * ceil_div(g.K, BK);
     int bm = 128, bn = 128;
     if (g.tile_hint) bm = g.tile_hint == HINT_64x64 ? 64 : 128, bn = g.tile_hint == HINT_64x64 ? 64 : 32;
@@ -988,8 +1069,7 @@ static int gemm_tiled_run_whole(int dtype, GemmArgs &g, int transA, int transB, 
                                 hipStream_t stream) {
     g.ws = (float *)workspace;
     const size_t usable = (workspace && ((size_t)workspace & 15) == 0) ? workspace_bytes : 0;
-    g.splits = plan_splits(gemm_tiled_k_step(dtype), g.M, g.N, g.K, g.batch, g.red, usable, &g.tiles_per_split, g.virt);
-    few_tiles_small(dtype, g, transA, transB, usable);
+    plan_pieces(dtype, g, transA, transB, usable);
     return dtype == D8_FLOAT16 ? launch<f16>(g, transA, transB, true, stream) : launch<float>(g, transA, transB, true, stream);
 }
 
@@ -1033,6 +1113,8 @@ int gemm_tiled_run(int dtype, GemmArgs &g, int transA, int transB, void *workspa
     return gemm_tiled_run_whole(dtype, second, transA, transB, workspace, workspace_bytes, stream);
 }
 
+static bool grads_apart() { return getenv("D8_MATMUL_GRADS_APART") != nullptr; }  // tuning and test aid (read at every call)
+
 // Whether the two gradients of a MatrixMultiply (g0 = dZ . Y^T, NT; g1 = X^T . dZ, TN) run on the kernel for small products, in
 // one launch where one call asks for both, and so that a call for one leaves the same bits: both small in the sense of
 // gemm_is_small, or both short and with no more workgroups than run at once.  us, as they ran before (two launches, or one of tiles
@@ -1045,7 +1127,7 @@ bool gemm_gradients_are_small(int dtype, const GemmArgs &g0, int ta0, int tb0, c
     const long n = small_workgroups(g0) + small_workgroups(g1);
     if (gemm_is_small(g0.M, g0.N, g0.K, g0.batch, g0.red) && gemm_is_small(g1.M, g1.N, g1.K, g1.batch, g1.red)) return n <= 0x7fffffffL;
     const char *copies = getenv("D8_GEMM_PACK");  // (see pack_pays; both are tuning and test aids, read at every call)
-    if (getenv("D8_MATMUL_GRADS_APART") != nullptr || (copies && atoi(copies) != 0)) return false;
+    if (grads_apart() || (copies && atoi(copies) != 0)) return false;
     return gemm_fits_small(dtype, g0) && gemm_fits_small(dtype, g1) && n <= (dtype == D8_FLOAT16 ? 1L : 2L) * cu_count();
 }
 
@@ -1146,8 +1228,8 @@ bool gemm_tiled_kept_pair_plan(int dtype, GemmArgs &gx, GemmArgs &gy, void *work
     if (gx.virt == VIRT_A_CLASSES) return tiles(gx, gy) != APART;
     if (narrow_output(dtype, gx)) gx.tile_hint = HINT_128x32;
     if (gx.virt != VIRT_A_ROWS || balanced_rows(gx) || !gemm_tiled_eligible(dtype, gx, 0, 0) || gemm_is_small(gx.M, gx.N, gx.K, gx.batch, gx.red)) return false;
-    gx.splits = plan_splits(BK, gx.M, gx.N, gx.K, 1, gx.red, usable, &gx.tiles_per_split, gx.virt);
-    few_tiles_small(dtype, gx, 0, 0, usable);
+    gemm_conv_pieces(dtype, gx, gy);
+    plan_pieces(dtype, gx, 0, 0, usable);
     // the partial sums side by side
     const size_t gy_bytes = gy.splits > 1 ? ((size_t)gy.splits * gy.M * gy.N * sizeof(float) + 255) & ~(size_t)255 : 0;
     const size_t gx_bytes = gx.splits > 1 ? (size_t)gx.splits * gx.M * gx.N * sizeof(float) : 0;
@@ -1172,8 +1254,7 @@ int gemm_tiled_kept_pair_run(int dtype, const GemmArgs &gx, const GemmArgs &gy, 
 // 608 x 2816 x 768 61.5 / 46.4, 4096 x 2112 x 480 179 / 143, 4352 x 448 x 832 63.8 / 73.0, the others at least 0.96 times as fast; in half 4 x 3072 x
 // 680 x 1152 70.9 / 54.1, 3072 x 3584 x 744 59.0 / 48.4.
 static SharedLaunch plain_pair_plan(int dtype, GemmArgs &g0, int ta0, int tb0, GemmArgs &g1, int ta1, int tb1, void *workspace, size_t workspace_bytes) {
-    const bool off = getenv("D8_MATMUL_GRADS_APART") != nullptr;  // tuning and test aid (read at every call)
-    if (off || dtype == D8_FLOAT64 || ta0 || !tb0 || !ta1 || tb1) return APART;
+    if (dtype == D8_FLOAT64 || ta0 || !tb0 || !ta1 || tb1) return APART;
     if (g0.virt != VIRT_NONE || g1.virt != VIRT_NONE || g0.K < 1 || g1.K < 1) return APART;
     for (const GemmArgs *g : {&g0, &g1})
         if (g->batch > 448 || g->M > 65535 * 128) return APART;  // (beyond one launch's limits: d8_gemm cuts it into several)
@@ -1181,16 +1262,9 @@ static SharedLaunch plain_pair_plan(int dtype, GemmArgs &g0, int ta0, int tb0, G
     if (gemm_is_small(g0.M, g0.N, g0.K, g0.batch, g0.red) || gemm_is_small(g1.M, g1.N, g1.K, g1.batch, g1.red)) return APART;
     if (balanced_rows(g0) || balanced_rows(g1)) return APART;
     const size_t usable = (workspace && ((size_t)workspace & 15) == 0) ? workspace_bytes : 0;
-    const int BK = gemm_tiled_k_step(dtype);
     // each split as it would be alone, the partial sums of the two side by side in the workspace
-    g0.splits = plan_splits(BK, g0.M, g0.N, g0.K, g0.batch, g0.red, usable, &g0.tiles_per_split);
-    g1.splits = plan_splits(BK, g1.M, g1.N, g1.K, g1.batch, g1.red, usable, &g1.tiles_per_split);
-    // (in half the two products fill the chip together on larger tiles, which sum an unsplit reduction in the same order)
-    for (GemmArgs *g : {&g0, &g1}) {
-        const int whole = g->splits == 1 && dtype == D8_FLOAT16;
-        few_tiles_small(dtype, *g, g == &g1, g == &g0, usable);
-        if (whole) g->tile_hint = HINT_NONE;
-    }
+    if (dtype == D8_FLOAT16) half_pair_plan(g0, g1, usable);
+    else plan_pieces(dtype, g0, 0, 1, usable), plan_pieces(dtype, g1, 1, 0, usable);
     const size_t need0 = g0.splits > 1 ? ((size_t)g0.splits * g0.batch * g0.M * g0.N * sizeof(float) + 255) & ~(size_t)255 : 0;
     const size_t need1 = g1.splits > 1 ? (size_t)g1.splits * g1.batch * g1.M * g1.N * sizeof(float) : 0;
     if (need0 + need1 > usable) return APART;
@@ -1201,6 +1275,14 @@ static SharedLaunch plain_pair_plan(int dtype, GemmArgs &g0, int ta0, int tb0, G
     return wgs <= 2L * cu_count() && (g0.packed || whole_steps(dtype, g0, g1)) ? SHARED : SHARED_KEPT;
 }
 
+bool gemm_gradients_share(int dtype, GemmArgs &g0, int ta0, int tb0, GemmArgs &g1, int ta1, int tb1) {
+    GemmArgs a = g0, b = g1;
+    for (GemmArgs *g : {&a, &b}) g->A = g->B = nullptr, g->C = nullptr;
+    if (plain_pair_plan(dtype, a, ta0, tb0, b, ta1, tb1, (void *)4096, (size_t)1 << 62) == APART) return false;
+    g0.pieces_by = a.pieces_by, g1.pieces_by = b.pieces_by;
+    return true;
+}
+
 static int plain_pair_run(int dtype, const GemmArgs &g0, const GemmArgs &g1, hipStream_t stream) {
     if (int rc = gemm_tiled_plain_pair_launch(dtype, g0, g1, stream)) return rc;
     return launch_reduce_pair(dtype, g0, g1, stream);
@@ -1208,6 +1290,7 @@ static int plain_pair_run(int dtype, const GemmArgs &g0, const GemmArgs &g1, hip
 
 SharedLaunch gemm_tiled_run_plain_pair(int dtype, GemmArgs &g0, int ta0, int tb0, GemmArgs &g1, int ta1, int tb1, void *workspace,
                                        size_t workspace_bytes, hipStream_t stream, int *rc) {
+    if (grads_apart()) return APART;
     const SharedLaunch shared = plain_pair_plan(dtype, g0, ta0, tb0, g1, ta1, tb1, workspace, workspace_bytes);
     if (shared) *rc = plain_pair_run(dtype, g0, g1, stream);
     return shared;
@@ -1272,7 +1355,7 @@ static bool pack_run_plan(int dtype, const PackedProduct (&p)[2], void *workspac
     auto packed = [&](int i) { return packed_args(*p[i].g, r.plan.slot[i], r.copies.list); };
     r.g[0] = packed(0), r.g[1] = packed(1);
     const size_t rest = workspace_bytes - r.plan.bytes;
-    r.shared = plain_pair_plan(dtype, r.g[0], p[0].ta, p[0].tb, r.g[1], p[1].ta, p[1].tb, to, rest);
+    r.shared = grads_apart() ? APART : plain_pair_plan(dtype, r.g[0], p[0].ta, p[0].tb, r.g[1], p[1].ta, p[1].tb, to, rest);
     if (!pack_pays(p, 2, r.plan)) return false;
     for (int i = 0; i < 2; ++i) {
         const GemmArgs &g = *p[i].g;  // (not at the cost of the pieces that it would run in without copies)

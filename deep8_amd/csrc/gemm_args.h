@@ -117,6 +117,9 @@ struct GemmArgs {
     // a smaller tile than the shape's own (128 x 32: fp32 only), chosen by gemm_tiled_run and gemm_tiled_run_plain_pair
     // (few_tiles_small, narrow_output)
     int tile_hint;
+    // half: which estimate plans the pieces (few_tiles_small).  Of two gradients that share a launch, or would, the one that suits
+    // the two of them (half_pair_plan)
+    int pieces_by;
     // Remainder band in the same launch (tail_splits > 0; unsplit, unbatched products only): rows tail_m0 .. M - 1
     // are not tiled by the launch's first tiles(tail_m0) x tiles(N) workgroups but by further ones, tail_splits per
     // tile, each walking tail_tps K steps and writing fp32 partial sums to ws[piece][row - tail_m0][n].  They start
@@ -133,6 +136,7 @@ struct GemmArgs {
 };
 
 enum { HINT_NONE = 0, HINT_64x64 = 1, HINT_128x32 = 2 };  // GemmArgs::tile_hint
+enum { BY_TILE_TIMES = 0, BY_STEPS = 1 };                  // GemmArgs::pieces_by
 
 // Whether two gradients have run as one launch: SHARED if their reductions are whole K steps (or both are small, or copies) and all their
 // workgroups fit the chip at once, else SHARED_KEPT.  The two are counted apart (d8_matmul_grad_pair_launches, ..._kept_pair_launches).
@@ -202,6 +206,10 @@ int gemm_wide_pair_launch(const GemmArgs &g0, int transA0, int transB0, const Ge
 // Whether the two gradients of a MatrixMultiply (NT, TN) run on the small-product kernel, and one of them on it.
 bool gemm_gradients_are_small(int dtype, const GemmArgs &g0, int ta0, int tb0, const GemmArgs &g1, int ta1, int tb1);
 int gemm_small_run(int dtype, const GemmArgs &g, int transA, int transB, hipStream_t stream);
+// Whether the two by their shapes share a launch of the tiled kernels, given aligned tensors and scratch enough; their pieces_by is set if so.
+bool gemm_gradients_share(int dtype, GemmArgs &g0, int ta0, int tb0, GemmArgs &g1, int ta1, int tb1);
+// The pieces_by of a convolution's gradient of x on patch rows, beside the filter's gradient gy (half; else nothing is set).
+void gemm_conv_pieces(int dtype, GemmArgs &gx, const GemmArgs &gy);
 // Both as ONE launch; APART, with nothing launched, when they do not qualify.
 SharedLaunch gemm_small_pair_run(int dtype, const GemmArgs &g0, int ta0, int tb0, const GemmArgs &g1, int ta1, int tb1, hipStream_t stream, int *rc);
 

@@ -381,13 +381,20 @@ int d8_matmul_bias_relu(int dtype, const void *x, int xb, int xr, int xc, const 
     return run_bias_relu(dtype, p, bias, relu, scratch, scratch_bytes, stream);
 }
 
+// A gradient in a launch of its own, planned as where it shares one (planned: its shapes would; half), for the same bits.
+static int run_apart(int dtype, const Gemm &p, GemmArgs &g, bool planned, void *scratch, size_t scratch_bytes, void *stream) {
+    if (planned && gemm_tiled_eligible(dtype, g, p.ta, p.tb, TILED_PIECES)) return gemm_tiled_run(dtype, g, p.ta, p.tb, scratch, scratch_bytes, as_stream(stream));
+    return run(dtype, p, scratch, scratch_bytes, stream);
+}
+
 // The gradient of input `which` alone: on the kernel that a call for both gradients takes, for the same bits.
 static int run_gradient(int dtype, int which, const Gemm &p, int xb, int xr, int xc, int yb, int yr, int yc, void *scratch, size_t scratch_bytes, void *stream) {
     const Gemm other = mm_plan(3 - which, nullptr, xb, xr, xc, nullptr, yb, yr, yc, nullptr);
-    const GemmArgs g = to_args(p), h = to_args(other);
-    const bool small = which == 1 ? gemm_gradients_are_small(dtype, g, p.ta, p.tb, h, other.ta, other.tb)
-                                  : gemm_gradients_are_small(dtype, h, other.ta, other.tb, g, p.ta, p.tb);
-    return small ? gemm_small_run(dtype, g, p.ta, p.tb, as_stream(stream)) : run(dtype, p, scratch, scratch_bytes, stream);
+    const Gemm &px = which == 1 ? p : other, &py = which == 1 ? other : p;
+    GemmArgs gx = to_args(px), gy = to_args(py);
+    if (gemm_gradients_are_small(dtype, gx, px.ta, px.tb, gy, py.ta, py.tb)) return gemm_small_run(dtype, to_args(p), p.ta, p.tb, as_stream(stream));
+    const bool planned = dtype == D8_FLOAT16 && gemm_gradients_share(dtype, gx, px.ta, px.tb, gy, py.ta, py.tb);
+    return run_apart(dtype, p, which == 1 ? gx : gy, planned, scratch, scratch_bytes, stream);
 }
 
 int d8_matmul_grad_x(int dtype, void *dx, int xb, int xr, int xc, const void *y, int yb, int yr, int yc,
@@ -471,8 +478,10 @@ int d8_matmul_grad_xy(int dtype, const void *x, void *dx, int xb, int xr, int xc
         count_shared(shared);
         return rc;
     }
-    if (int rc = run(dtype, px, scratch, scratch_bytes, stream)) return rc;
-    return run(dtype, py, scratch, scratch_bytes, stream);
+    gx = to_args(px), gy = to_args(py);
+    const bool planned = dtype == D8_FLOAT16 && gemm_gradients_share(dtype, gx, px.ta, px.tb, gy, py.ta, py.tb);
+    if ((rc = run_apart(dtype, px, gx, planned, scratch, scratch_bytes, stream))) return rc;
+    return run_apart(dtype, py, gy, planned, scratch, scratch_bytes, stream);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -682,7 +691,9 @@ static int d8_conv2d_grad_x_impl(int dtype, void *gx, int B, int IH, int IW, int
             !prefer_interim(dtype, ga, ta, tb, product, (double)M * K, IC, 1, scratch, scratch_bytes)) {
             ++route_calls[ROUTE_PATCH];
             ga.beta = beta;
-            return implicit_run(dtype, ga, ta, tb, scratch, scratch_bytes, as_stream(stream));
+            GemmArgs other;  // the filter's gradient, beside which this one is planned
+            if (dtype == D8_FLOAT16 && conv_implicit_plan(dtype, 2, cs, nullptr, nullptr, gz, other, ta, tb)) gemm_conv_pieces(dtype, ga, other);
+            return implicit_run(dtype, ga, 0, 0, scratch, scratch_bytes, as_stream(stream));
         }
         bool untouched = false;
         if (conv_classes_grad_x(dtype, cs, gx, w, gz, ga, &untouched) &&
@@ -977,6 +988,8 @@ static int deconv2d_grad_x_geo(int dtype, void *gx, int B, int IH, int IW, int I
             !prefer_interim(dtype, ga, 0, 0, deconv_plan(1, M, T, OC, IC, scratch, w, gx), (double)M * T * OC, OC, 0, scratch, scratch_bytes)) {
             ++route_calls[ROUTE_PATCH];
             ga.beta = beta;
+            GemmArgs other;  // the filter's gradient, beside which this one is planned
+            if (dtype == D8_FLOAT16 && deconv_implicit_grad_y(dtype, B, IH, IW, IC, OC, FH, FW, sy, sx, g, (const void *)4096, nullptr, gz, other)) gemm_conv_pieces(dtype, ga, other);
             return implicit_run(dtype, ga, 0, 0, scratch, scratch_bytes, as_stream(stream));
         }
     }
