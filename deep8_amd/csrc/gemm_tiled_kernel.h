@@ -1188,6 +1188,9 @@ static int launch_pair_tiles(const GemmArgs &gx0, const GemmArgs &gy0, hipStream
     const long wgs = (long)ny * nzy + (long)nx * nzx, cus = cu_count();
     const unsigned pad = lds <= third && wgs > cus && wgs <= 2 * cus ? (unsigned)(third + 512 - lds) : 0u;
     // Of more workgroups than compute units the longer ones first, gx's (`ahead` of them) or gy's: what starts last runs alone at the end.
+    // fp32 classes, whose longest run up to twice their mean, only where the chip cannot hold all workgroups at once: two of them on a compute
+    // unit end later than one beside a shorter one of gy's (Conv2d, both gradients, gx's first / gy's: 31 x 15x15x64 -> 320 5x5 stride 2 120 /
+    // 101 us, 27 x 24x18x120 -> 128 3x3 stride 2 34.5 / 29.0; of more, 26 x 28x28x256 -> 96 61 / 77; in half either may be first).
     auto time = [](const GemmArgs &g, int bm, int bn, int bk, double red) {
         const double steps = g.splits > 1 ? g.tiles_per_split : red * ceil_div(g.K, bk);
         return steps * (TX::DMA ? bm + bn : bm * bn);  // (half waits for its loads, fp32 for its matrix instructions)
@@ -1197,7 +1200,8 @@ static int launch_pair_tiles(const GemmArgs &gx0, const GemmArgs &gy0, hipStream
         red = 0;
         for (int i = 0; i < gx.ncls; ++i) red += (double)gx.cls[i].red / gx.ncls;
     }
-    const int ahead = wgs > cus && time(gx, TX::BM, TX::BN, TX::BK, red) > time(gy, TY::BM, TY::BN, TY::BK, gy.red) ? nx * nzx : 0;
+    const bool crowded = wgs > (TX::VIRT == VIRT_A_CLASSES && !TX::DMA ? 2 * cus : cus);
+    const int ahead = crowded && time(gx, TX::BM, TX::BN, TX::BK, red) > time(gy, TY::BM, TY::BN, TY::BK, gy.red) ? nx * nzx : 0;
     set_reciprocals(gy, tMy, tNy, TY::BM, TY::BK, ny);
     set_reciprocals(gx, tMx, tNx, TX::BM, TX::BK, nx);
     hipLaunchKernelGGL((gemm_tiled_pair_kernel<TY, TX, EDGE>), dim3(ny * nzy + nx * nzx), dim3(TX::NT), pad, stream, ahead, ny, nzy, nx, tMy, tNy, tMx, tNx, gy, gx);
