@@ -3,7 +3,7 @@
 #ifndef DEEP8_AMD_GEMM_TILED_PAIR_PLAIN_H
 #define DEEP8_AMD_GEMM_TILED_PAIR_PLAIN_H
 
-#include "gemm_tiled_kernel.h"
+#include "gemm_tiled_pair_tail.h"
 
 namespace d8 {
 
