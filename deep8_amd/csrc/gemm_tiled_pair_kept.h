@@ -4,7 +4,7 @@
 #ifndef DEEP8_AMD_GEMM_TILED_PAIR_KEPT_H
 #define DEEP8_AMD_GEMM_TILED_PAIR_KEPT_H
 
-#include "gemm_tiled_kernel.h"
+#include "gemm_tiled_pair_tail.h"
 
 namespace d8 {
 
@@ -36,7 +36,7 @@ static SharedLaunch kept_tiles(const GemmArgs &gx, const GemmArgs &gy, TileId &t
         // as no workgroup runs longer than 24 steps of a 128 x 128 tile would (the longer workgroups start first: launch_pair_tiles).
         // 90 drawn layers apart 9351 us, in one launch 9205 without that line; 7 x 35x35x64 -> 64 5x5 50.4 / 40.4, 17 x 17x17x200 -> 148
         // 100 / 85.5, and of longer workgroups DeConv2d 27 x 21x21x320 -> 64 4x4 stride 2 217 / 187, but Conv2d 1 x 93x54x320 -> 64 5x5 107 /
-        // 117, 4 x 82x82x64 -> 168 148 / 157.  Slower by more than 3 % with it: 56 x 17x17x256 -> 64, 98 / 103.
+        // 117, 4 x 82x82x64 -> 168 148 / 157.  And none that leaves a tail behind (leaves_a_tail).
         // (Smaller tiles of x's product beside small areas: any number, 64 x 14x14x32 -> 64 5x5 48.0 and 37.1.)
         if (both || (((rows && cols) || (tx != TILE_64x64 && tx != TILE_128x32)) && wx + wy > 2L * cu_count())) {
             auto work = [](const GemmArgs &g, long m, long n) {
@@ -44,7 +44,7 @@ static SharedLaunch kept_tiles(const GemmArgs &gx, const GemmArgs &gy, TileId &t
             };
             const long most = 24 * 128 * 128;
             const bool brief = work(gx, long_m(tx) ? 128 : 64, tx == TILE_128x32 ? 32 : long_n(tx) ? 128 : 64) <= most && work(gy, long_m(ty) ? 128 : 64, long_n(ty) ? 128 : 64) <= most;
-            return brief ? SHARED_KEPT : APART;
+            return brief && !leaves_a_tail(gx, tx, wx, gy, ty, wy) ? SHARED_KEPT : APART;
         }
     }
     return SHARED;

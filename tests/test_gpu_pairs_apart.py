@@ -22,3 +22,24 @@ def test_matmul(R, I, O, shared):
     check(lib.d8_matmul_grad_xy(capi.FLOAT32, dx.ptr, gx.ptr, 1, R, I, dy.ptr, gy.ptr, 1, I, O, dd.ptr, 3, ws.ptr, nb, None))
     assert lib.d8_matmul_grad_kept_pair_launches() - before == shared
     assert np.array_equal(gx.numpy(), dz @ y.T) and np.array_equal(gy.numpy(), x.T @ dz)
+
+
+@pytest.mark.parametrize("B,size,IC,OC,F,shared", [(2, 97, 384, 192, 1, 0), (7, 35, 64, 64, 5, 1)])
+def test_conv2d(oracle_port, B, size, IC, OC, F, shared):
+    from deep8_amd import capi
+    from deep8_amd.capi import DeviceArray, check
+    lib = capi.init()
+    image, filt, geo = (B, size, size, IC), (OC, F, F), (1, 1, 1, 1, 1)
+    r = rng(size)
+    x, w, dz = (ints(r, s, 3).astype(np.float32) for s in (image, filt + (IC,), (B, size, size, OC)))
+    nb = lib.d8_conv2d_scratch_bytes(capi.FLOAT32, 3, *image, *filt, *geo)
+    dx, dw, dd, ws = DeviceArray.from_numpy(x), DeviceArray.from_numpy(w), DeviceArray.from_numpy(dz), DeviceArray((max(nb, 16),), np.uint8)
+    gx, gw = DeviceArray.from_numpy(np.full(x.shape, np.nan, np.float32)), DeviceArray.from_numpy(np.full(w.shape, np.nan, np.float32))
+    before = lib.d8_conv_grad_crowded_pair_launches()
+    check(lib.d8_conv2d_grad_xy(capi.FLOAT32, dx.ptr, gx.ptr, *image, dw.ptr, gw.ptr, *filt, dd.ptr, *geo, 3, ws.ptr, nb, None))
+    assert lib.d8_conv_grad_crowded_pair_launches() - before == shared
+    if F == 1:
+        wx, ww = dz.reshape(-1, OC) @ w.reshape(OC, IC), dz.reshape(-1, OC).T @ x.reshape(-1, IC)
+    else:
+        wx, ww = oracle_port.conv2d_grad_x(x, w, dz, *geo), oracle_port.conv2d_grad_y(x, w, dz, *geo)
+    assert np.array_equal(gx.numpy().ravel(), wx.ravel()) and np.array_equal(gw.numpy().ravel(), ww.ravel())
