@@ -341,6 +341,9 @@ size_t d8_matmul_scratch_bytes(int dtype, int which, int xb, int xr, int xc, int
     return gemm_ws(dtype, p) + gemm_pack_one_bytes(dtype, {&g, p.ta, p.tb});
 }
 
+static std::atomic<unsigned long> matmul_pair_launches{0}, matmul_kept_pair_launches{0}, matmul_copied_calls{0}, forward_copied_calls{0};
+unsigned long d8_matmul_copied_calls(void) { return forward_copied_calls.load(); }
+
 // A forward product (bias and relu: as its store may apply them) on copies of operands whose rows start anywhere; false, with
 // nothing launched, where that does not pay.
 static bool run_on_copies(int dtype, const Gemm &p, const void *bias, int relu, void *scratch, size_t scratch_bytes, void *stream, int *rc) {
@@ -351,7 +354,9 @@ static bool run_on_copies(int dtype, const Gemm &p, const void *bias, int relu, 
         g.round_first = !gemm_fuses_store(dtype, g, p.ta, p.tb, TILED_PIECES);
         if (!gemm_fuses_store(dtype, g, p.ta, p.tb)) return false;
     }
-    return gemm_pack_run_one(dtype, {&g, p.ta, p.tb}, scratch, scratch_bytes, as_stream(stream), rc);
+    if (!gemm_pack_run_one(dtype, {&g, p.ta, p.tb}, scratch, scratch_bytes, as_stream(stream), rc)) return false;
+    ++forward_copied_calls;
+    return true;
 }
 
 int d8_matmul(int dtype, const void *x, int xb, int xr, int xc, const void *y, int yb, int yr, int yc,
@@ -427,7 +432,6 @@ int d8_matmul_grad_y_overwrite(int dtype, const void *x, int xb, int xr, int xc,
 
 unsigned long d8_conv_route_calls(int route) { return route >= 0 && route < 3 ? route_calls[route].load() : 0; }
 
-static std::atomic<unsigned long> matmul_pair_launches{0}, matmul_kept_pair_launches{0}, matmul_copied_calls{0};
 unsigned long d8_matmul_grad_copied_calls(void) { return matmul_copied_calls.load(); }
 unsigned long d8_matmul_grad_pair_launches(void) { return matmul_pair_launches.load(); }
 unsigned long d8_matmul_grad_kept_pair_launches(void) { return matmul_kept_pair_launches.load(); }

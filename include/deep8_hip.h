@@ -303,10 +303,11 @@ int d8_deconv2d_grad_xy_ex(int dtype, const void *x, void *gx, int B, int IH, in
  * those whose two products are tiled and cut as they would be alone.  A call counts in one of the three at most.   */
 unsigned long d8_conv_grad_pair_launches(void);
 unsigned long d8_conv_grad_kept_pair_launches(void);
-unsigned long d8_conv_grad_crowded_pair_launches(void);  /* likewise, Float32, more workgroups than run at once */
+unsigned long d8_conv_grad_crowded_pair_launches(void);  /* likewise, Float32: 128 x 128 tiles in both, or more workgroups than run at once */
 unsigned long d8_matmul_grad_pair_launches(void);  /* ... and of the d8_matmul_grad_xy calls: whole K steps, and no more workgroups than run at once; */
 unsigned long d8_matmul_grad_kept_pair_launches(void);  /* the others: a K step (64 in Float16, 32 in Float32) that is cut short, or more workgroups */
 unsigned long d8_matmul_grad_copied_calls(void);   /* d8_matmul_grad_xy calls that ran on copies of their odd operands */
+unsigned long d8_matmul_copied_calls(void);        /* ... and d8_matmul and d8_matmul_bias_relu calls */
 /* How many Conv2d / DeConv2d calls have run (each gradient is one; both gradients from one call are two), by route: 0 on an
  * interim matrix in scratch, 1 with the patches read by the GEMM's loader, 2 on the kernels for images of few channels. */
 unsigned long d8_conv_route_calls(int route);

@@ -1,6 +1,6 @@
 """A half MatrixMultiply whose rows start anywhere, forward, on copies of the operands with rows of whole pieces: every remainder of
-a row's last piece, batches, tensors that start at any element, with bias and ReLu, with room for the copies and without.
-Integers, bit for bit; what lies around the tensors is NaN."""
+a row's last piece, batches, square products, tensors that start at any element, with bias and ReLu, with room for the copies and
+without.  Integers, bit for bit; what lies around the tensors is NaN; the calls that ran on copies are counted."""
 import numpy as np
 import pytest
 
@@ -17,7 +17,8 @@ def _lay(a, before):
 
 
 SHAPES = [(1, 300, 640, 1, 128 + n) for n in range(1, 8)] + [(1, 300, 512 + n, 1, 136) for n in (1, 3, 7)] + \
-         [(1, 1000, 521, 1, 1001), (3, 150, 330, 3, 203), (2, 515, 131, 1, 645), (1, 260, 1100, 3, 257), (1, 2600, 200, 1, 2049), (1, 129, 4001, 1, 130)]
+         [(1, 1000, 521, 1, 1001), (3, 150, 330, 3, 203), (2, 515, 131, 1, 645), (1, 260, 1100, 3, 257), (1, 2600, 200, 1, 2049), (1, 129, 4001, 1, 130), (1, 515, 515, 1, 515),
+          (3, 203, 203, 3, 203)]
 
 
 @pytest.mark.parametrize("xb,R,I,yb,O", SHAPES)
@@ -47,6 +48,7 @@ def test_forward(monkeypatch, xb, R, I, yb, O, before, copies):
         ws = DeviceArray.from_numpy(np.full(max(nb, 16), 0xff, np.uint8))
         for relu in (None, 0, 1):
             dz = _lay(np.full((zb, R, O), 7), 0)
+            count = lib.d8_matmul_copied_calls()
             if relu is None:
                 check(lib.d8_matmul(capi.FLOAT16, dx[1], xb, R, I, dy[1], yb, I, O, dz[1], ws.ptr if nb else None, nb, None))
                 want = z
@@ -54,6 +56,11 @@ def test_forward(monkeypatch, xb, R, I, yb, O, before, copies):
                 check(lib.d8_matmul_bias_relu(capi.FLOAT16, dx[1], xb, R, I, dy[1], yb, I, O, db.ptr, relu, dz[1], ws.ptr if nb else None, nb, None))
                 want = z + bias
                 want = np.maximum(want, 0) if relu else want
+            count = lib.d8_matmul_copied_calls() - count
+            if nb <= plain or copies == "0":
+                assert count == 0, (nb, relu)
+            elif copies == "1" and (nb > asked or not any(before)):  # (at odd addresses more may be copied than was asked for)
+                assert count == 1, (nb, relu)
             got = f(dz[0].numpy())
             assert np.array_equal(got[:want.size].reshape(want.shape), want), (nb, relu)
             assert np.isnan(got[want.size:]).all(), (nb, relu)
