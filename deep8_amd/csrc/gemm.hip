@@ -684,7 +684,7 @@ static PackShape pack_shape(const GemmArgs &g, int ta, int tb, int op) {
 static int pack_pitch(const PackShape &s) { return (s.cols + 63) & ~63; }
 static size_t pack_bytes(const PackShape &s) { return (size_t)s.rows * pack_pitch(s) * 2; }  // (a multiple of 128)
 
-// What is to be copied for two products: a matrix that both read is copied once.
+// What is to be copied for one product or two: a matrix that is read twice is copied once.
 struct PackPlan {
     PackShape shapes[4];
     int n, slot[2][2];
@@ -1032,9 +1032,10 @@ void gemm_conv_pieces(int dtype, GemmArgs &gx, const GemmArgs &gy) {
     gx.pieces_by = us[BY_STEPS] < us[BY_TILE_TIMES] ? BY_STEPS : BY_TILE_TIMES;
 }
 
-// What the planners above count for the plan that they make, in microseconds.  (Over 3100 calls on drawn layers the time
-// measured was 1.0 - 1.2 of this at the median in fp32, 1.1 - 1.5 in half, for products and patch products alike, before half
-// tiles went straight into LDS.)
+// Microseconds of a product in steps of its tiles, for the choice between two ways of a convolution (products and patch products alike,
+// so what counts is their ratio).  Over 3100 calls on drawn layers the time measured was 1.0 - 1.2 of this at the median in fp32, 1.1 - 1.5
+// in half, before half tiles went straight into LDS.  Later kernels are not in it: a half plan may have been made by half_tile_us, and a
+// product that gemm_is_short takes is counted as a tiled one; of 300 drawn layers none runs slower than before them for that.
 double gemm_estimate_us(int dtype, const GemmArgs &g0, int transA, int transB) {
     const bool half_elems = dtype == D8_FLOAT16;
     const int BK = gemm_tiled_k_step(dtype);

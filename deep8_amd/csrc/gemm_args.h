@@ -138,8 +138,10 @@ struct GemmArgs {
 enum { HINT_NONE = 0, HINT_64x64 = 1, HINT_128x32 = 2 };  // GemmArgs::tile_hint
 enum { BY_TILE_TIMES = 0, BY_STEPS = 1 };                  // GemmArgs::pieces_by
 
-// Whether two gradients have run as one launch: SHARED if their reductions are whole K steps (or both are small, or copies) and all their
-// workgroups fit the chip at once, else SHARED_KEPT.  The two are counted apart (d8_matmul_grad_pair_launches, ..._kept_pair_launches).
+// Whether two gradients have run as one launch.  Of a MatrixMultiply: SHARED if their reductions are whole K steps (or both are small, or
+// copies) and all their workgroups fit the chip at once, else SHARED_KEPT.  Of a convolution, tiled and cut as alone: SHARED_KEPT if in fp32
+// both have 128 x 128 tiles or there are more workgroups than run at once, else SHARED.  The two are counted apart
+// (d8_matmul_grad_pair_launches, ..._kept_pair_launches; d8_conv_grad_kept_pair_launches, ..._crowded_pair_launches).
 enum SharedLaunch { APART = 0, SHARED, SHARED_KEPT };
 enum TiledRule { TILED_ANY, TILED_PIECES, TILED_WHOLE };  // see gemm_tiled_eligible
 
@@ -245,9 +247,10 @@ int gemm_tiled_run(int dtype, GemmArgs &g, int transA, int transB, void *workspa
 // into the filter's) as one launch where that pays; false, with nothing launched, where it does not (the caller then
 // runs them one after the other).  The workspace is gy's.
 bool gemm_tiled_run_pair(int dtype, GemmArgs &gx, GemmArgs &gy, void *workspace, size_t workspace_bytes, hipStream_t stream, int *rc);
-// The two gradients of a mid-size MatrixMultiply (g0 = dZ . Y^T, NT; g1 = X^T . dZ, TN; both on the tiled kernels, all their
-// workgroups resident at once) as one launch plus their split reductions; false, with nothing launched, otherwise.
-// The workspace holds both products' partial sums side by side.
+// The two gradients of a MatrixMultiply (g0 = dZ . Y^T, NT; g1 = X^T . dZ, TN; both on the tiled kernels, their operands in whole pieces or
+// copies) as one launch plus their split reductions, whatever K leaves of a last step and, but for fp32 pairs that leave a tail
+// behind, however many workgroups there are; APART, with nothing launched, otherwise.  The workspace holds both products' partial
+// sums side by side.
 SharedLaunch gemm_tiled_run_plain_pair(int dtype, GemmArgs &g0, int ta0, int tb0, GemmArgs &g1, int ta1, int tb1, void *workspace,
                                size_t workspace_bytes, hipStream_t stream, int *rc);
 // Microseconds that a product is expected to take with all the workspace it asks for (which of two ways a convolution goes).
