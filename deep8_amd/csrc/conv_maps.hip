@@ -222,8 +222,8 @@ __global__ __launch_bounds__(256) void pad_rows_kernel(const V *__restrict__ src
 // ---- col2im: one thread owns VEC channels of one image pixel; taps are added in (fy, fx)
 // ascending order into registers, then the pixel is written once.
 // Bound by latencies: five taps are asked for at once, one that does not reach the pixel at the matrix's first row and left out of the
-// sum, so that no load lies behind a branch; and pixels and taps are found by multiplications (BIG: by divisions, from 2^31
-// outputs on).  Both gradients of half Conv2d 18 x 12x12x134 -> 40, 3x3 stride 2, whose dx is written and not cleared first:
+// sum, so that no load lies behind a branch; and pixels and taps are found by multiplications (BIG: by divisions and with 64-bit
+// offsets, from 2^31 outputs or elements of a patch row on).  Both gradients of half Conv2d 18 x 12x12x134 -> 40, 3x3 stride 2, whose dx is written and not cleared first:
 // 30.0 -> 27.0 us, of half 50 x 59x59x62 -> 64 3x3 455 -> 381, fp32 2 x 56x56x91 -> 64 5x5 128 -> 116, before loads one by one behind 64-bit
 // divisions.
 struct Col2im {
@@ -264,7 +264,7 @@ __global__ __launch_bounds__(256) void col2im_kernel(const T *__restrict__ col, 
                 const int ty = iy + g.pt - fy * g.dy, tx = ix + g.pl - fx * g.dx;
                 const int oy = (int)div_by((unsigned)max(ty, 0), by.by_sy), ox = (int)div_by((unsigned)max(tx, 0), by.by_sx);
                 reaches[u] = t0 + u < taps && oy * g.sy == ty && oy < g.OH && ox * g.sx == tx && ox < g.OW;
-                v[u] = *(const VT *)(image + (reaches[u] ? ((long)oy * g.OW + ox) * K + (fy * g.FW + fx) * g.C : 0L));
+                v[u] = *(const VT *)(image + (reaches[u] ? ((long)oy * g.OW + ox) * K + (Index)(fy * g.FW + fx) * g.C : 0L));
                 if (++fx == g.FW) fx = 0, ++fy;
             }
 #pragma unroll
@@ -834,7 +834,7 @@ int launch_im2col(int dtype, const void *im, void *col, const MapGeom &g, hipStr
         const long total = elems / (16 / es);
         hipLaunchKernelGGL((im2col_kernel<uint4>), dim3(grid_for(total, 256)), dim3(256), 0, s,
                            (const uint4 *)im, (uint4 *)col, g, CV, total);
-    } else if (es < 8 && aligned16(col) && elems / (16 / (long)es) >= 192L * cu_count()) {  // (see im2col_flat_kernel)
+    } else if (es < 8 && aligned16(col) && elems / (16 / (long)es) >= 192L * cu_count() && (long)g.FH * g.FW * g.C < (1L << 31)) {  // (see im2col_flat_kernel)
         if (es == 4) launch_im2col_flat<unsigned, 4>(im, col, g, elems, s);
         else launch_im2col_flat<unsigned short, 8>(im, col, g, elems, s);
     } else if (es == 8) {
@@ -855,7 +855,7 @@ template <typename T, int VEC, bool ACC>
 static void launch_col2im_t(const void *col, void *im, const MapGeom &g, long elems, hipStream_t s) {
     const Col2im by = {fast_div(g.C / VEC), fast_div(g.IW), fast_div(g.IH), fast_div(g.sy), fast_div(g.sx)};
     const dim3 grid(grid_for(elems / VEC, 256));
-    if (elems / VEC < (1L << 31)) hipLaunchKernelGGL((col2im_kernel<T, VEC, ACC, false>), grid, dim3(256), 0, s, (const T *)col, (T *)im, g, by, elems / VEC);
+    if (elems / VEC < (1L << 31) && (long)g.FH * g.FW * g.C < (1L << 31)) hipLaunchKernelGGL((col2im_kernel<T, VEC, ACC, false>), grid, dim3(256), 0, s, (const T *)col, (T *)im, g, by, elems / VEC);
     else hipLaunchKernelGGL((col2im_kernel<T, VEC, ACC, true>), grid, dim3(256), 0, s, (const T *)col, (T *)im, g, by, elems / VEC);
 }
 

@@ -1,5 +1,5 @@
-"""im2col and col2im of 2^31 elements and more, whose indices do not fit 32 bits: a filter of one row and three columns over a wide
-image, so that what every element has to be follows from its neighbours.  Bit for bit (small integers)."""
+"""im2col and col2im of 2^31 elements and more, whose indices do not fit 32 bits, also within one patch row: a filter of one row and
+three columns over a wide image, so that what every element has to be follows from its neighbours.  Bit for bit (small integers)."""
 import numpy as np
 import pytest
 
@@ -43,3 +43,19 @@ def test_taps_added_into_the_image():
         im[b, :, :-1] += col[b, :, 1:, 0]
         im[b, :, 1:] += col[b, :, :-1, 2]
         assert np.array_equal(got[b], im[b])
+
+
+@pytest.mark.parametrize("C", [(1 << 30) + 1, 1 << 30])
+def test_patch_rows_beyond_31_bits(C):
+    from deep8_amd import capi
+    lib = capi.init()
+    assert 3 * C >= 1 << 31
+    x, before = _image(1, 1, C), _image(1, 1, C)[..., ::-1]
+    dx, dcol, dim = capi.DeviceArray.from_numpy(x), capi.DeviceArray((3, C), np.float16), capi.DeviceArray.from_numpy(np.ascontiguousarray(before))
+    geo = (1, 1, 1, C, 1, 1, 1, 3, 1, 1, 1, 1, 0, 2)  # one pixel, which only the last tap of a row of three reaches
+    capi.check(lib.d8_im2col(capi.FLOAT16, dx.ptr, dcol.ptr, *geo, None))
+    col = dcol.numpy()
+    assert not col[:2].any() and np.array_equal(col[2], x[0, 0])
+    del col
+    capi.check(lib.d8_col2im(capi.FLOAT16, dcol.ptr, dim.ptr, *geo, None))
+    assert np.array_equal(dim.numpy(), x + before)
