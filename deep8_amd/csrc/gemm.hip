@@ -350,12 +350,15 @@ static bool gemm_is_small(int M, int N, int K, int batch, int red) {
 
 // Larger outputs of as short a reduction: what the kernel can hold, on as many workgroups as run at once, and no longer reductions on many of
 // them than 400 elements a compute unit.  Beyond that the loads of a 32 x 32 tile, which a larger one would share, take longer than the
-// way from memory that all of them wait for once.  us, tiled / so, by workgroups; 570 drawn forward products, three sets of tensors in turn:
+// way from memory that all of them wait for once.  In half up to 128 rows of a wider output have 240: the second operand is most of what is read,
+// in half cache lines that no other row of tiles asks for meanwhile.  And rows that start anywhere have no line, because the larger tiles
+// have no whole pieces to load there.  us, tiled / so, by workgroups; 570 drawn forward products, three sets of tensors in turn:
 // fp32 64 x 200 x 640 (40) 7.8 / 4.5, 2824 x 272 x 64 (178) 9.0 / 5.2, 3 x 192 x 192 x 704 (396) 7.2 / 6.3, 13 x 112 x 496 x 152 (260) 11.4 / 12.9, 11 x
 // 128 x 352 x 208 (308) 9.0 / 10.1, 28 x 225 x 192 x 128 (896) 7.8 / 10.7; half 64 x 352 x 896 (56) 5.1 / 4.2, 3520 x 576 x 46 (220) 11.8 / 5.3, 10 x 104 x
 // 736 x 176 (240) 6.1 / 7.9, 720 x 896 x 304 (230) 6.1 / 7.0, 3 x 968 x 200 x 72 (279) 4.5 / 5.6.  Workgroups times elements: up to 60000 all faster,
 // 1.3 to 1.6 times at the mean; up to 100000 half 1.3, fp32 1.4; up to 120000 half 1.10; beyond half 0.92 to 1.01, fp32 on more workgroups than
-// compute units 1.02 (on at most as many 1.3).
+// compute units 1.02 (on at most as many 1.3).  Half, up to 128 rows, 61000 to 102000: 41 of them 0.98 (64 x 832 x 1920 6.4 / 7.5, 64 x 488 x 3176 5.7 /
+// 6.7), other shapes 1.05.  Half rows that start anywhere, from 102000 on: 19 of them 1.14 (43 x 64 x 704 x 34 9.0 / 5.2).
 static bool gemm_fits_small(int dtype, const GemmArgs &g) {
     const int KG = dtype == D8_FLOAT16 ? SmallOp<f16>::KG : SmallOp<float>::KG;
     return dtype != D8_FLOAT64 && g.virt == VIRT_NONE && !g.packed && !g.perm_OC && g.K >= 1 && (long)g.red * ceil_div(g.K, KG) <= SMALL_WAVES * SMALL_MAXC;
@@ -365,7 +368,8 @@ static long small_workgroups(const GemmArgs &g) { return (long)ceil_div(g.M, 32)
 static bool gemm_is_short(int dtype, const GemmArgs &g) {
     if (!gemm_fits_small(dtype, g)) return false;
     const long cus = cu_count(), n = small_workgroups(g), most = 400 * cus / ((long)g.red * g.K);
-    return dtype == D8_FLOAT16 ? n <= cus && n <= most : n <= cus || (n <= cus * 3 / 2 && n <= most);
+    if (dtype == D8_FLOAT32) return n <= cus || (n <= cus * 3 / 2 && n <= most);
+    return n <= cus && (n <= (g.M <= 128 && g.N > 64 ? most * 3 / 5 : most) || !gemm_tiled_eligible(dtype, g, 0, 0, TILED_PIECES));
 }
 
 // C[b][m][n] = beta * C + sum_s ws[b][s][m][n].  A workgroup covers groups of 4 consecutive outputs.

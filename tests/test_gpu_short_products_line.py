@@ -1,5 +1,6 @@
 """Forward products on both sides of the line that workgroups times the reduction draw for the kernel for small products (400 elements a
-compute unit: 256 and 384 workgroups of 32 x 32 outputs).  Integers against numpy, bit for bit."""
+compute unit: 256 and 384 workgroups of 32 x 32 outputs; 240 for up to 128 rows in half, none for rows that start anywhere).  Integers
+against numpy, bit for bit."""
 import numpy as np
 import pytest
 
@@ -9,6 +10,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype,xb,R,K,O", [(np.float16, 1, 512, K, 512) for K in (399, 400, 401, 408)] + [(np.float16, 10, 104, 736, 176), (np.float16, 1, 250, 1000, 344)] +
+                         [(np.float16, 1, 128, K, 2048) for K in (232, 240, 248)] + [(np.float16, 1, 129, 248, 1632), (np.float16, 1, 64, 832, 1920), (np.float16, 2, 64, 1000, 64)] +
+                         [(np.float16, 1, 512, K, 511) for K in (399, 400, 405)] + [(np.float16, 43, 64, 704, 34), (np.float16, 1, 77, 1021, 2047)] +
                          [(np.float32, 1, 512, K, 760) for K in (265, 266, 267, 268)] + [(np.float32, 1, 512, 512, 512), (np.float32, 13, 112, 496, 152)])
 def test_forward(dtype, xb, R, K, O):
     from deep8_amd import capi
