@@ -695,13 +695,14 @@ struct PackPlan {
     size_t bytes;
 };
 
-// Whether copies pay.  Both gradients: a product saves 0.5 us for each K step that a compute unit walks, or 0.25 where both of its
-// operands are odd, and a MB of copies takes 0.2; on copies the two mostly share a launch, which they would not without.  A forward
+// Whether copies pay.  Both gradients: a product saves 0.5 us for each K step that a compute unit walks (0.3 on tiles of 64 columns or rows), or
+// 0.25 where both of its operands are odd, and a MB of copies takes 0.2; on copies the two mostly share a launch, which they would not without.  A forward
 // product by itself: 0.2 and 0.25 us a step, 0.3 a MB, and a launch for the copies; an output narrower than a tile is bound by its operands' way
 // from memory, and a product that fills the chip with tiles of few steps has them hide each other's ways.
 // Drawn calls with odd sizes, a third of them batched, three sets of tensors in turn, us on the kernels for rows that start anywhere /
 // on copies always / by this rule / with the better of the two, and how many lose more than 3 % to the better one by the rule:
-//   330 calls of both gradients   12488 / 9805 / 9846 / 9766, 18 (10257, 76 with the forward products' rates for both)
+//   594 calls of both gradients   17168 / 13523 / 13697 / 13474, 59 (4 of them to the way without copies, at most 12 %; 0.5 us a step for narrow
+//                                 tiles too: 12)
 //   330 forward products           5774 / 5491 / 5351 / 5183, 85 (6 lose more than 3 % to the way without copies, at most 10 %)
 // Gradients of 3039 x 376 x 2289 52.7 -> 34.8, 6 x 1005 x 368 x 1211 45.1 -> 33.0; forward 4096 x 1024 x 1001 with bias and ReLu 21.1 -> 20.2, 883 x 624 x 334
 // 17.1 -> 10.7, 107 x 1440 x 3121 36.2 -> 15.8.
@@ -716,7 +717,8 @@ static bool pack_pays(const PackedProduct *p, int products, const PackPlan &plan
         const int odd = (plan.slot[i][0] >= 0) + (plan.slot[i][1] >= 0);
         const long tiles = (long)ceil_div(g.M, 128) * ceil_div(g.N, 128) * g.batch, total = (long)g.red * ceil_div(g.K, 64);
         const double share = tiles * total / cus, alone = total < 8 ? total : 8.0;
-        saved += (odd == 2 ? 0.25 : odd == 1 ? (both ? 0.5 : 0.2) : 0.0) * (share > alone ? share : alone);
+        const double one = !both ? 0.2 : g.M <= 64 || g.N <= 64 ? 0.3 : 0.5;
+        saved += (odd == 2 ? 0.25 : odd == 1 ? one : 0.0) * (share > alone ? share : alone);
         if (!both) {
             if (g.M < 128 || g.N < 128 || (gemm_is_short(D8_FLOAT16, g) && (long)g.red * g.K <= 512)) return false;
             least = 4 * tiles >= cus && total <= 32 ? 1.7 : 0.2;
