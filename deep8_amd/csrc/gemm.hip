@@ -1261,7 +1261,7 @@ int gemm_tiled_kept_pair_run(int dtype, const GemmArgs &gx, const GemmArgs &gy, 
 // many workgroups there are: a launch or two fewer, and one last round instead of two.  us apart / so: a K step cut short, of 90
 // drawn calls the 25 that are, 1.29 times as fast at the mean: fp32 448 x 304 x 152 15.8 / 10.2, 648 x 1128 x 64 15.4 / 11.5; half 368 x 824 x
 // 64 8.8 / 6.8, 5864 x 568 x 576 27.6 / 22.1.  More workgroups than the chip holds, longer ones first, 58 drawn calls in fp32 3750 / 3331:
-// 608 x 2816 x 768 61.5 / 46.4, 4096 x 2112 x 480 179 / 143, and apart where one launch leaves a tail behind (leaves_a_tail); in half 4 x 3072 x
+// 608 x 2816 x 768 61.5 / 46.4, 4096 x 2112 x 480 179 / 143, and apart where one launch leaves a tail behind (leaves_a_tail, leaves_a_half_tail); in half 4 x 3072 x
 // 680 x 1152 70.9 / 54.1, 3072 x 3584 x 744 59.0 / 48.4.
 static SharedLaunch plain_pair_plan(int dtype, GemmArgs &g0, int ta0, int tb0, GemmArgs &g1, int ta1, int tb1, void *workspace, size_t workspace_bytes) {
     if (dtype == D8_FLOAT64 || ta0 || !tb0 || !ta1 || tb1) return APART;

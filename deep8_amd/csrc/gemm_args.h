@@ -248,7 +248,7 @@ int gemm_tiled_run(int dtype, GemmArgs &g, int transA, int transB, void *workspa
 // runs them one after the other).  The workspace is gy's.
 bool gemm_tiled_run_pair(int dtype, GemmArgs &gx, GemmArgs &gy, void *workspace, size_t workspace_bytes, hipStream_t stream, int *rc);
 // The two gradients of a MatrixMultiply (g0 = dZ . Y^T, NT; g1 = X^T . dZ, TN; both on the tiled kernels, their operands in whole pieces or
-// copies) as one launch plus their split reductions, whatever K leaves of a last step and, but for fp32 pairs that leave a tail
+// copies) as one launch plus their split reductions, whatever K leaves of a last step and, but for pairs that leave a tail
 // behind, however many workgroups there are; APART, with nothing launched, otherwise.  The workspace holds both products' partial
 // sums side by side.
 SharedLaunch gemm_tiled_run_plain_pair(int dtype, GemmArgs &g0, int ta0, int tb0, GemmArgs &g1, int ta1, int tb1, void *workspace,

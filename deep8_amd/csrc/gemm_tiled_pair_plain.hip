@@ -11,7 +11,9 @@ long gemm_tiled_plain_pair_workgroups(int dtype, const GemmArgs &g0, const GemmA
     grid_of(t0, g0, m0, n0);
     grid_of(t1, g1, m1, n1);
     const long wg0 = (long)m0 * n0 * g0.batch * g0.splits, wg1 = (long)m1 * n1 * g1.batch * g1.splits;
-    return dtype == D8_FLOAT32 && wg0 + wg1 > 2L * cu_count() && leaves_a_tail(g0, t0, wg0, g1, t1, wg1) ? 0 : wg0 + wg1;
+    if (wg0 + wg1 <= 2L * cu_count() || g0.packed) return wg0 + wg1;
+    const bool tail = dtype == D8_FLOAT32 ? leaves_a_tail(g0, t0, wg0, g1, t1, wg1) : leaves_a_half_tail(g0, t0, wg0, g1, t1, wg1);
+    return tail ? 0 : wg0 + wg1;
 }
 
 int gemm_tiled_plain_pair_launch(int dtype, const GemmArgs &g0, const GemmArgs &g1, hipStream_t stream) {
