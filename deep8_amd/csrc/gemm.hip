@@ -962,7 +962,8 @@ static void plan_pieces(int dtype, GemmArgs &g, int ta, int tb, size_t usable) {
 // A planned half product as one of two that share a launch.  One that runs whole may take larger tiles than alone, which sum in the same
 // order: fewer steps for the chip, where the smaller ones make shorter workgroups.
 struct HalfShare {
-    double longest[2], share[2];  // us of a workgroup, and a compute unit's share of all steps; on its tiles and on larger ones
+    // us of a workgroup and of its steps, workgroups, and a compute unit's share of all steps; on its tiles and on larger ones
+    double longest[2], steps[2], workgroups[2], share[2];
     double pass;                  // over its partial sums, the launch left out
     bool larger;                  // whether there is the choice
 };
@@ -977,19 +978,23 @@ static HalfShare half_share(const GemmArgs &g) {
         const int bn = t64 || g.N < 128 ? 64 : 128;
         const int bm = t64 || (bn == 128 && (g.M < 128 || (g.splits == 1 && gemm_tiled_half_tiles(g.M, g.N, g.batch, total, 64)))) ? 64 : 128;
         const double steps = len * half_step_us(bm, bn, g);
-        h.longest[i] = half_ends_us(bm, bn) + steps + (g.virt != VIRT_NONE ? half_rows_us(bm, bn) : 0.0);
-        h.share[i] = (double)ceil_div(g.M, bm) * ceil_div(g.N, bn) * g.batch * g.splits * steps / cu_count();
+        const double slow = bm * bn == 128 * 128 ? 1.4 : bm * bn == 64 * 64 ? 1.0 : 1.3;  // (four waves and fewer stages than in a launch alone)
+        h.longest[i] = half_ends_us(bm, bn) + slow * steps + (g.virt != VIRT_NONE ? half_rows_us(bm, bn) : 0.0);
+        h.steps[i] = steps, h.workgroups[i] = (double)ceil_div(g.M, bm) * ceil_div(g.N, bn) * g.batch * g.splits;
+        h.share[i] = h.workgroups[i] * steps / cu_count();
     }
     return h;
 }
 // What the launch takes with the pass after it: its longest workgroup or a compute unit's share, whichever is more; bit i of tiles: product i on
-// larger ones.
+// larger ones.  Some more workgroups than compute units lie beside a longest one (3 x 2600 x 128 x 2176 29.1 us on 63 + 204 workgroups, 21.7 on 246 + 204).
 static double half_pair_us(const HalfShare &a, const HalfShare &b, int &tiles) {
     double best = INFINITY;
     for (int t = 0; t < 4; ++t) {
         const int i = t & 1, j = t >> 1;
         if (i > a.larger || j > b.larger) continue;
-        const double longest = a.longest[i] > b.longest[j] ? a.longest[i] : b.longest[j], share = 4.0 + a.share[i] + b.share[j];
+        const double rounds = (a.workgroups[i] + b.workgroups[j]) / cu_count(), shorter = a.steps[i] < b.steps[j] ? a.steps[i] : b.steps[j];
+        const double longest = (a.longest[i] > b.longest[j] ? a.longest[i] : b.longest[j]) + (rounds > 1.0 && rounds <= 1.5 ? 0.75 * shorter : 0.0);
+        const double share = 4.0 + a.share[i] + b.share[j];
         if (const double us = longest > share ? longest : share; us < best) best = us, tiles = t;
     }
     return best + (a.pass + b.pass > 0.0 ? 3.5 + a.pass + b.pass : 0.0);
@@ -1000,6 +1005,8 @@ static double half_pair_us(const HalfShare &a, const HalfShare &b, int &tiles) {
 // as long anyway, a second pass comes on top.  Both by the tiles' times and on larger tiles where they run whole, as it was, / so, us: 4 x 320 x
 // 128 x 1408 12.6 / 9.0, 960 x 128 x 1872 18.4 / 11.4 (apart 15.2), 3 x 384 x 768 x 264 16.2 / 9.7 (12.8), 4 x 832 x 448 x 160 14.2 / 8.8 (12.1), 1216 x
 // 128 x 256 10.3 / 7.7, 1856 x 128 x 3200 14.9 / 14.5 (by its steps 18.4); 500 drawn calls of both gradients 6083 / 5739.
+// Within 5 % of each other the tiles' times decide: without that line 34 of 378 drawn calls whose plans differ were more than 3 % slower than by the
+// tiles' times alone (more pieces of larger tiles, whose pass takes longer: 4560 x 1216 x 64 15.3 / 16.6, 4056 x 1416 x 64 15.9 / 17.2), with it 16.
 static void half_pair_plan(GemmArgs &g0, GemmArgs &g1, size_t usable) {
     GemmArgs *const g[2] = {&g0, &g1};
     HalfShare plan[2][2];
@@ -1013,7 +1020,7 @@ static void half_pair_plan(GemmArgs &g0, GemmArgs &g1, size_t usable) {
         }
     double best = INFINITY;
     for (int c = 0; c < 4; ++c)
-        if (const double us = half_pair_us(plan[0][c & 1], plan[1][c >> 1], tiles); us < best) best = us, choice = c;
+        if (const double us = half_pair_us(plan[0][c & 1], plan[1][c >> 1], tiles) * (c ? 1.05 : 1.0); us < best) best = us, choice = c;
     g0.pieces_by = choice & 1, g1.pieces_by = choice >> 1;
     plan_pieces(D8_FLOAT16, g0, 0, 1, usable), plan_pieces(D8_FLOAT16, g1, 1, 0, usable);
     half_pair_us(half_share(g0), half_share(g1), tiles);

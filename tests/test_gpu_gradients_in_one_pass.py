@@ -1,5 +1,5 @@
 """Both gradients of half layers of few tiles: what shares a launch with a longer product is not cut into pieces for it, so nothing is
-written to the scratch and there is no second pass.  Integers, bit for bit."""
+written to the scratch and there is no second pass; and into no more than its tiles' times ask for.  Integers, bit for bit."""
 import numpy as np
 import pytest
 
@@ -29,6 +29,26 @@ def test_matmul(xb, R, I, O):
     check(lib.d8_matmul_grad_xy(capi.FLOAT16, dx.ptr, gx.ptr, xb, R, I, dy.ptr, gy.ptr, xb, I, O, dd.ptr, 3, ws.ptr, nb, None))
     assert np.array_equal(gx.numpy(), wx.astype(np.float16)) and np.array_equal(gy.numpy(), wy.astype(np.float16))
     assert _untouched(ws)
+
+
+@pytest.mark.parametrize("R,I,O,pieces", [(4560, 1216, 64, 12), (4056, 1416, 64, 11)])
+def test_pieces_of_the_second_gradient(R, I, O, pieces):
+    from deep8_amd import capi
+    from deep8_amd.capi import DeviceArray, check
+    lib = capi.init()
+    r = rng(R)
+    sparse = lambda *s: ints(r, s, 2) * (r.random(s) < 0.25)
+    x, y, dz = sparse(R, I), sparse(I, O), sparse(R, O)
+    wx, wy = dz @ y.T, x.T @ dz
+    assert max(np.abs(wx).max(), np.abs(wy).max()) < 2048
+    nb = lib.d8_matmul_scratch_bytes(capi.FLOAT16, 3, 1, R, I, 1, I, O)
+    dx, dy, dd = (DeviceArray.from_numpy(t.astype(np.float16)) for t in (x, y, dz))
+    gx, gy = DeviceArray.from_numpy(np.full(x.shape, np.nan, np.float16)), DeviceArray.from_numpy(np.full(y.shape, np.nan, np.float16))
+    ws = DeviceArray.from_numpy(np.full(nb // 4, np.nan, np.float32))
+    check(lib.d8_matmul_grad_xy(capi.FLOAT16, dx.ptr, gx.ptr, 1, R, I, dy.ptr, gy.ptr, 1, I, O, dd.ptr, 3, ws.ptr, nb, None))
+    assert np.array_equal(gx.numpy(), wx.astype(np.float16)) and np.array_equal(gy.numpy(), wy.astype(np.float16))
+    written = ~np.isnan(ws.numpy())
+    assert written[:pieces * I * O].all() and not written[pieces * I * O:].any()
 
 
 def test_conv2d(oracle_port):
