@@ -701,7 +701,7 @@ struct PackPlan {
 // from memory, and a product that fills the chip with tiles of few steps has them hide each other's ways.
 // Drawn calls with odd sizes, a third of them batched, three sets of tensors in turn, us on the kernels for rows that start anywhere /
 // on copies always / by this rule / with the better of the two, and how many lose more than 3 % to the better one by the rule:
-//   594 calls of both gradients   17168 / 13523 / 13697 / 13474, 59 (4 of them to the way without copies, at most 12 %; 0.5 us a step for narrow
+//   691 calls of both gradients   19571 / 15311 / 15516 / 15220, 69 (4 of them to the way without copies, at most 12 %; 0.5 us a step for narrow
 //                                 tiles too: 12)
 //   330 forward products           5774 / 5491 / 5351 / 5183, 85 (6 lose more than 3 % to the way without copies, at most 10 %)
 // Gradients of 3039 x 376 x 2289 52.7 -> 34.8, 6 x 1005 x 368 x 1211 45.1 -> 33.0; forward 4096 x 1024 x 1001 with bias and ReLu 21.1 -> 20.2, 883 x 624 x 334
@@ -711,7 +711,7 @@ static bool pack_pays(const PackedProduct *p, int products, const PackPlan &plan
     if (force) return atoi(force) != 0;
     const double cus = cu_count();
     const bool both = products == 2;
-    double saved = 0.0, least = both && (plan.slot[0][0] >= 0 || plan.slot[0][1] >= 0) ? 0.5 : 1.0;
+    double saved = 0.0, least = both && (plan.slot[0][0] >= 0 || plan.slot[0][1] >= 0) ? 0.2 : 1.0;
     for (int i = 0; i < products; ++i) {
         const GemmArgs &g = *p[i].g;
         const int odd = (plan.slot[i][0] >= 0) + (plan.slot[i][1] >= 0);

@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("xb,R,I,O,copied", [(1, 3039, 376, 2289, 1), (6, 1005, 368, 1211, 1), (4, 174, 1524, 872, 1), (1, 2375, 369, 1146, 1),
-                                             (1, 4288, 878, 64, 0), (58, 1888, 46, 64, 0)])
+                                             (1, 4288, 878, 64, 0), (58, 1888, 46, 64, 0), (1, 64, 3712, 15, 1)])
 def test_calls_that_run_on_copies(monkeypatch, xb, R, I, O, copied):
     from deep8_amd import capi
     from deep8_amd.capi import DeviceArray, check
