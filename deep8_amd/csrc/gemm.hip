@@ -907,14 +907,16 @@ static double tile_cost(bool half_elems, int bm, int bn, const GemmArgs &g, long
 // 1358 us, 3.4 % at the mean: 218 x 64 x 1328 5.6 -> 4.0, 1504 x 3648 x 128 14.6 -> 10.8, Conv2d 37 x 8x8x64 -> 368 1x1 6.2 -> 4.7.
 // What a workgroup takes besides its steps, and a step (128 x 128 and 64 x 64 tiles, and the two between).
 static double half_ends_us(int bm, int bn) { return bm * bn == 64 * 64 ? 3.6 : 4.1; }
-static double half_step_us(int bm, int bn, const GemmArgs &g) {
+// (operands of more than 4 MB are farther away, for two products at once more so: 4352 x 1152 x 192 8.1 us on 64 x 64 tiles, 10.0 on those that 0.11 chooses,
+// 2304 x 2560 x 320 12.1 and 17.0; 1828 drawn forward products and convolutions 18821 -> 18716 us.  43 x 64 x 248 x 512, both gradients, by 0.06 10.1 -> 12.4)
+static double half_step_us(int bm, int bn, const GemmArgs &g, bool shared) {
     const double far = bm * bn == 64 * 64 ? (2.0 * g.red * g.K * g.batch * ((double)g.M + g.N) - 4e6) / 8e6 : 0.0;  // (see above)
-    return (bm * bn == 128 * 128 ? 0.47 : bm * bn == 64 * 64 ? 0.23 : 0.31) + 0.11 * (far < 0.0 ? 0.0 : far > 1.0 ? 1.0 : far);
+    return (bm * bn == 128 * 128 ? 0.47 : bm * bn == 64 * 64 ? 0.23 : 0.31) + (shared ? 0.11 : 0.06) * (far < 0.0 ? 0.0 : far > 1.0 ? 1.0 : far);
 }
 static double half_rows_us(int bm, int bn) { return bm * bn == 128 * 128 ? 1.65 : bm * bn == 64 * 64 ? 0.95 : 1.25; }
 static double half_tile_us(int bm, int bn, const GemmArgs &g, long total, long s) {
     const long cus = cu_count(), n = (ceil_div(g.M, bm) * (long)ceil_div(g.N, bn) * g.batch * s + cus - 1) / cus, len = (total + s - 1) / s;
-    return half_ends_us(bm, bn) + n * len * half_step_us(bm, bn, g) + 0.2 * (n - 1) + (g.virt == VIRT_A_ROWS ? half_rows_us(bm, bn) : 0.0) +
+    return half_ends_us(bm, bn) + n * len * half_step_us(bm, bn, g, g.pieces_by == BY_SHARED_TIMES) + 0.2 * (n - 1) + (g.virt == VIRT_A_ROWS ? half_rows_us(bm, bn) : 0.0) +
            (s > 1 ? 2.6 + 1.85e-6 * s * g.M * (double)g.N * g.batch : 0.0);
 }
 
@@ -930,7 +932,7 @@ static void few_tiles_small(int dtype, GemmArgs &g, int transA, int transB, size
     const long total = (long)g.red * ceil_div(g.K, BK);
     const bool half = g.splits == 1 && gemm_tiled_half_tiles(g.M, g.N, g.batch, total, BK);
     const bool narrow = g.tile_hint == HINT_128x32;
-    const bool by_time = half_elems && g.pieces_by == BY_TILE_TIMES;
+    const bool by_time = half_elems && g.pieces_by != BY_STEPS;
     auto cost = [&](int bm, int bn, long pieces) { return by_time ? half_tile_us(bm, bn, g, total, pieces) : tile_cost(half_elems, bm, bn, g, total, pieces); };
     const double now = narrow ? 1e30 : g.N < 128 ? cost(128, 64, g.splits) : cost(g.M < 128 || half ? 64 : 128, 128, g.splits);
     long most = (long)(usable / ((size_t)g.batch * g.M * g.N * sizeof(float)));
@@ -977,7 +979,7 @@ static HalfShare half_share(const GemmArgs &g) {
         const bool t64 = small && i == 0;
         const int bn = t64 || g.N < 128 ? 64 : 128;
         const int bm = t64 || (bn == 128 && (g.M < 128 || (g.splits == 1 && gemm_tiled_half_tiles(g.M, g.N, g.batch, total, 64)))) ? 64 : 128;
-        const double steps = len * half_step_us(bm, bn, g);
+        const double steps = len * half_step_us(bm, bn, g, true);
         const double slow = bm * bn == 128 * 128 ? 1.4 : bm * bn == 64 * 64 ? 1.0 : 1.3;  // (four waves and fewer stages than in a launch alone)
         h.longest[i] = half_ends_us(bm, bn) + slow * steps + (g.virt != VIRT_NONE ? half_rows_us(bm, bn) : 0.0);
         h.steps[i] = steps, h.workgroups[i] = (double)ceil_div(g.M, bm) * ceil_div(g.N, bn) * g.batch * g.splits;
@@ -1010,18 +1012,19 @@ static double half_pair_us(const HalfShare &a, const HalfShare &b, int &tiles) {
 static void half_pair_plan(GemmArgs &g0, GemmArgs &g1, size_t usable) {
     GemmArgs *const g[2] = {&g0, &g1};
     HalfShare plan[2][2];
+    const int ways[2] = {BY_SHARED_TIMES, BY_STEPS};
     int tiles = 0, choice = 0;
     for (int i = 0; i < 2; ++i)
-        for (int by : {BY_TILE_TIMES, BY_STEPS}) {
+        for (int k = 0; k < 2; ++k) {
             GemmArgs p = *g[i];
-            p.pieces_by = by;
+            p.pieces_by = ways[k];
             plan_pieces(D8_FLOAT16, p, i, !i, (size_t)-1);
-            plan[i][by] = half_share(p);
+            plan[i][k] = half_share(p);
         }
     double best = INFINITY;
     for (int c = 0; c < 4; ++c)
         if (const double us = half_pair_us(plan[0][c & 1], plan[1][c >> 1], tiles) * (c ? 1.05 : 1.0); us < best) best = us, choice = c;
-    g0.pieces_by = choice & 1, g1.pieces_by = choice >> 1;
+    g0.pieces_by = ways[choice & 1], g1.pieces_by = ways[choice >> 1];
     plan_pieces(D8_FLOAT16, g0, 0, 1, usable), plan_pieces(D8_FLOAT16, g1, 1, 0, usable);
     half_pair_us(half_share(g0), half_share(g1), tiles);
     for (int i = 0; i < 2; ++i)
@@ -1034,15 +1037,16 @@ void gemm_conv_pieces(int dtype, GemmArgs &gx, const GemmArgs &gy) {
     GemmArgs y = gy;
     y.splits = plan_splits(gemm_tiled_k_step(dtype), y.M, y.N, y.K, 1, y.red, (size_t)-1, &y.tiles_per_split, y.virt);
     const HalfShare other = half_share(y);
+    const int ways[2] = {BY_SHARED_TIMES, BY_STEPS};
     double us[2];
-    for (int by : {BY_TILE_TIMES, BY_STEPS}) {
+    for (int k = 0; k < 2; ++k) {
         GemmArgs x = gx;
         int tiles;
-        x.pieces_by = by;
+        x.pieces_by = ways[k];
         plan_pieces(dtype, x, 0, 0, (size_t)-1);
-        us[by] = half_pair_us(half_share(x), other, tiles);
+        us[k] = half_pair_us(half_share(x), other, tiles);
     }
-    gx.pieces_by = us[BY_STEPS] < us[BY_TILE_TIMES] ? BY_STEPS : BY_TILE_TIMES;
+    gx.pieces_by = ways[us[1] < us[0]];
 }
 
 // Microseconds of a product in steps of its tiles, for the choice between two ways of a convolution (products and patch products alike,

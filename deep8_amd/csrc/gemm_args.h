@@ -136,7 +136,7 @@ struct GemmArgs {
 };
 
 enum { HINT_NONE = 0, HINT_64x64 = 1, HINT_128x32 = 2 };  // GemmArgs::tile_hint
-enum { BY_TILE_TIMES = 0, BY_STEPS = 1 };                  // GemmArgs::pieces_by
+enum { BY_TILE_TIMES = 0, BY_STEPS = 1, BY_SHARED_TIMES = 2 };  // GemmArgs::pieces_by
 
 // Whether two gradients have run as one launch.  Of a MatrixMultiply: SHARED if their reductions are whole K steps (or both are small, or
 // copies) and all their workgroups fit the chip at once, else SHARED_KEPT.  Of a convolution, tiled and cut as alone: SHARED_KEPT if in fp32

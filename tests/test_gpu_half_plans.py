@@ -29,3 +29,21 @@ def test_pieces_that_fit(M, K, N, trans):
         dC = DeviceArray.from_numpy(np.full((M, N), np.nan, np.float16))
         check(lib.d8_gemm(capi.FLOAT16, tA, tB, M, N, K, dA.ptr, M if tA else K, 0, dB.ptr, K if tB else N, 0, 0.0, dC.ptr, N, 0, 1, ws.ptr if nb else None, nb, None))
         assert np.array_equal(dC.numpy().astype(np.float64), want), pieces
+
+
+@pytest.mark.parametrize("R,I,O", [(128, 1664, 2752), (3968, 1712, 96)])
+def test_forward_products_that_run_whole(R, I, O):
+    """more than 4 MB of operands: by 64 x 64 tiles in one pass, so nothing is written to the scratch"""
+    from deep8_amd import capi
+    from deep8_amd.capi import DeviceArray, check
+    lib = capi.init()
+    r = rng(R + I + O)
+    x, y = (ints(r, s, 2) * (r.random(s) < 0.25) for s in ((R, I), (I, O)))
+    z = x.astype(np.float32) @ y.astype(np.float32)
+    assert np.abs(z).max() < 2048
+    nb = lib.d8_matmul_scratch_bytes(capi.FLOAT16, 0, 1, R, I, 1, I, O)
+    dx, dy, ws = DeviceArray.from_numpy(x.astype(np.float16)), DeviceArray.from_numpy(y.astype(np.float16)), DeviceArray.from_numpy(np.full(nb // 4, np.nan, np.float32))
+    dz = DeviceArray.from_numpy(np.full(z.shape, np.nan, np.float16))
+    check(lib.d8_matmul(capi.FLOAT16, dx.ptr, 1, R, I, dy.ptr, 1, I, O, dz.ptr, ws.ptr, nb, None))
+    assert nb > 0 and np.isnan(ws.numpy()).all()
+    assert np.array_equal(dz.numpy(), z.astype(np.float16))
