@@ -357,7 +357,8 @@ static bool gemm_is_small(int M, int N, int K, int batch, int red) {
 // 128 x 352 x 208 (308) 9.0 / 10.1, 28 x 225 x 192 x 128 (896) 7.8 / 10.7; half 64 x 352 x 896 (56) 5.1 / 4.2, 3520 x 576 x 46 (220) 11.8 / 5.3, 10 x 104 x
 // 736 x 176 (240) 6.1 / 7.9, 720 x 896 x 304 (230) 6.1 / 7.0, 3 x 968 x 200 x 72 (279) 4.5 / 5.6.  Workgroups times elements: up to 60000 all faster,
 // 1.3 to 1.6 times at the mean; up to 100000 half 1.3, fp32 1.4; up to 120000 half 1.10; beyond half 0.92 to 1.01, fp32 on more workgroups than
-// compute units 1.02 (on at most as many 1.3).  Half, up to 128 rows, 61000 to 102000: 41 of them 0.98 (64 x 832 x 1920 6.4 / 7.5, 64 x 488 x 3176 5.7 /
+// compute units 1.02 (on at most as many 1.3).  Replayed from a graph, where launches do not count, up to 60000 and 102000: fp32 1.25 and 1.13, half 1.07 and
+// 1.03, half rows that start anywhere 1.5 and 1.4.  Half, up to 128 rows, 61000 to 102000: 41 of them 0.98 (64 x 832 x 1920 6.4 / 7.5, 64 x 488 x 3176 5.7 /
 // 6.7), other shapes 1.05.  Half rows that start anywhere, from 102000 on: 19 of them 1.14 (43 x 64 x 704 x 34 9.0 / 5.2).
 static bool gemm_fits_small(int dtype, const GemmArgs &g) {
     const int KG = dtype == D8_FLOAT16 ? SmallOp<f16>::KG : SmallOp<float>::KG;
