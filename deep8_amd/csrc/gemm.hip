@@ -1052,8 +1052,10 @@ void gemm_conv_pieces(int dtype, GemmArgs &gx, const GemmArgs &gy) {
 
 // Microseconds of a product in steps of its tiles, for the choice between two ways of a convolution (products and patch products alike,
 // so what counts is their ratio).  Over 3100 calls on drawn layers the time measured was 1.0 - 1.2 of this at the median in fp32, 1.1 - 1.5
-// in half, before half tiles went straight into LDS.  Later kernels are not in it: a half plan may have been made by half_tile_us, and a
-// product that gemm_is_short takes is counted as a tiled one; of 300 drawn layers none runs slower than before them for that.
+// in half, before half tiles went straight into LDS.  Later kernels are not in it: a half plan may have been made by half_tile_us and is priced in
+// steps all the same, and a product that gemm_is_short takes is counted as a tiled one.  Of 5440 drawn half layers one goes the wrong way for that
+// (both gradients of DeConv2d 2 x 7x7x64 -> 448 5x5 stride 2, 9.9 us through the loader, 18.7 on an interim matrix) and several go the right way (Conv2d
+// 1 x 50x50x80 -> 136 5x5 34 and 21.9).  Plans in steps here, for either kind of product or both, or the lower of the two prices, were no better.
 double gemm_estimate_us(int dtype, const GemmArgs &g0, int transA, int transB) {
     const bool half_elems = dtype == D8_FLOAT16;
     const int BK = gemm_tiled_k_step(dtype);
