@@ -208,17 +208,19 @@ __global__ __launch_bounds__(256) void column_sum_kernel(const T *__restrict__ d
 }
 
 // g[k0][c] += sum over chunks of partial[k0][chunk][c].  A block covers 16 outputs of k0 = blockIdx.y, or of several k0 (`outputs` in all, else 0)
-// where C is so small that a block each would fetch the same lines; 16 lanes per output each add every 16th chunk, sixteen, four or one at a time
-// in flight, and meet in LDS in a fixed order.  (Sixteen whatever their number, the ones past the last asked for again, and a block for every k0:
-// 13 chunks of an L2 norm of 24 x 771 3.3 us instead of 1.7; with that mended but for the blocks 5.9 us for both launches instead of 5.4.)
-template <typename T, int OP = LOAD_ID>
+// where C is so small that a block each would fetch the same lines; 16 lanes per output each add every 16th chunk, sixteen at a time in
+// flight, FEW (at most 64 chunks): four or one, and meet in LDS in a fixed order.  (Sixteen whatever their number, the ones past the last asked
+// for again, and a block for every k0: 13 chunks of an L2 norm of 24 x 771 3.3 us instead of 1.7; with that mended but for the blocks 5.9 us for
+// both launches instead of 5.4.  One kernel for few and many chunks took the many longer: a training call of half Conv2d 16 x 224x224x3 -> 64,
+// 7x7 stride 2, 61.9 instead of 61.35 us in four of four comparisons; half Conv2d 32 x 14x14x256 3x3 49.3 with either.)
+template <typename T, int OP = LOAD_ID, bool FEW = false>
 __global__ __launch_bounds__(256) void column_sum_finish_kernel(const float *__restrict__ partial, T *__restrict__ g,
                                                                 int C, int outputs, int chunks, float scale, float keep) {
     __shared__ float part[16][16];
     const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4, at = blockIdx.x * 16 + tx;
     int k0 = blockIdx.y, c = at;
-    if (outputs) k0 = at / C, c = at - k0 * C;
-    const bool live = at < (outputs ? outputs : C);
+    if (FEW && outputs) k0 = at / C, c = at - k0 * C;
+    const bool live = at < (FEW && outputs ? outputs : C);
     float v = 0.f;
     if (live) {
         const float *p = partial + (long)k0 * chunks * C + c;
@@ -231,10 +233,12 @@ __global__ __launch_bounds__(256) void column_sum_finish_kernel(const float *__r
             for (int u = 0; u < N; ++u)
                 if (k + u * 16 < chunks) v += t[u];
         };
-        int k = 0;
-        for (; chunks - k > 4 * 16; k += 16 * 16) add(std::integral_constant<int, 16>(), k + ty);
-        if (chunks - k > 16) add(std::integral_constant<int, 4>(), k + ty);
-        else if (chunks > k) add(std::integral_constant<int, 1>(), k + ty);
+        if constexpr (FEW) {
+            if (chunks > 16) add(std::integral_constant<int, 4>(), ty);
+            else add(std::integral_constant<int, 1>(), ty);
+        } else {
+            for (int k = ty; k < chunks; k += 16 * 16) add(std::integral_constant<int, 16>(), k);
+        }
     }
     part[ty][tx] = v;
     __syncthreads();
@@ -244,6 +248,16 @@ __global__ __launch_bounds__(256) void column_sum_finish_kernel(const float *__r
         T *o = g + (long)k0 * C + c;
         *o = ew_result<T, OP>((keep != 0.f ? ew_f32(*o) : 0.f) + scale * v);
     }
+}
+
+template <typename T, int OP = LOAD_ID>
+static void launch_column_sum_finish(const float *partial, T *g, long K0, int C, int chunks, float scale, float keep, hipStream_t s) {
+    const bool several = K0 > 1 && C <= 4 && chunks <= 64;  // rows of the output in a block
+    const dim3 blocks = several ? dim3((unsigned)((K0 * C + 15) / 16)) : dim3((unsigned)((C + 15) / 16), (unsigned)K0);
+    if (chunks <= 64)
+        hipLaunchKernelGGL((column_sum_finish_kernel<T, OP, true>), blocks, dim3(256), 0, s, partial, g, C, several ? (int)(K0 * C) : 0, chunks, scale, keep);
+    else
+        hipLaunchKernelGGL((column_sum_finish_kernel<T, OP>), blocks, dim3(256), 0, s, partial, g, C, 0, chunks, scale, keep);
 }
 
 // ReLuGrad and the bias gradient in one pass over a [R][C] gradient: dpre = z > 0 ? dz : 0 is written out and its
@@ -566,9 +580,7 @@ static int reduce_t(T *g, const int *d, const T *dz, const int *zd, void *scratc
                                TX, rpc, chunks, scale, keep);
         if (chunks > 1) {
             D8_LAUNCH_CHECK();
-            const bool several = p.K0 > 1 && p.C <= 4;  // rows of the output in a block
-            const dim3 blocks = several ? dim3((unsigned)((ng + 15) / 16)) : dim3((unsigned)((p.C + 15) / 16), (unsigned)p.K0);
-            hipLaunchKernelGGL((column_sum_finish_kernel<T, OP>), blocks, dim3(256), 0, s, (const float *)scratch, g, (int)p.C, several ? (int)ng : 0, chunks, scale, keep);
+            launch_column_sum_finish<T, OP>((const float *)scratch, g, p.K0, (int)p.C, chunks, scale, keep, s);
         }
     } else {
         ReduceGeom q;
@@ -681,8 +693,7 @@ static int relu_gate_sum_t(const T *z, const T *dz, T *dpre, T *g, long rows, in
         hipLaunchKernelGGL((relu_gate_column_sum_kernel<T, 1, false>), grid, dim3(256), 0, s, z, dz, dpre, g, (float *)scratch, (int)rows, cols, TX, rpc, chunks, keep);
     D8_LAUNCH_CHECK();
     if (chunks > 1) {
-        hipLaunchKernelGGL((column_sum_finish_kernel<T>), dim3((unsigned)((cols + 15) / 16)), dim3(256), 0, s,
-                           (const float *)scratch, g, cols, 0, chunks, 1.f, keep);
+        launch_column_sum_finish<T>((const float *)scratch, g, 1, cols, chunks, 1.f, keep, s);
         D8_LAUNCH_CHECK();
     }
     return 0;
